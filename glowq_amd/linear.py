@@ -253,11 +253,15 @@ class CudaW4A16Linear(nn.Module):
         x2d = self._as_rows(x)
         self._require_gpu(x2d)
         KNOBS.sync()
-        if KNOBS.force_gemm or (not self._prefer_gemv(x2d.size(0))):
+        m = x2d.size(0)
+        if KNOBS.force_gemm or (m <= DEFAULT_GEMV_M_MAX and not self._prefer_gemv(m)):
+            # the GEMM entry point asked for where the row count alone would not take it
             out = self._get_ext().w4a16_gemm_forward_cuda(x2d, self.qweight_i32, self.scales_f16, self.qzeros_i32,
                                                           self.group_size, KNOBS.split_k_iters)
             return self._finish(out, lead)
-        # the decode kernels through descriptors validated once (the bias rides in the kernel's epilogue)
+        # Through descriptors validated once (the bias rides in the kernel's epilogue).  From 65 rows this is the same MFMA
+        # GEMM as the entry point above, but on the tiled copy of the weights and with the stream's workspace for its splits
+        # of K: two 14B layers with half of their groups bare at 1500 rows 2362 -> 2048 us.
         return self._finish(self._bare_group().run(x2d)[0], lead, bias_applied=KNOBS.out_dtype == torch.float16)
 
     def dequantize(self) -> torch.Tensor:

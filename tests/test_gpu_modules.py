@@ -201,3 +201,20 @@ def test_dequant_chunk_rows_match_the_reference_vectors(golden):
     for start, end in ((0, n), (3, 17), (n - 1, n), (5, 5), (30, n + 10)):
         got = mod._dequant_chunk(start, end).cpu().numpy()
         np.testing.assert_array_equal(got.view(np.uint16), want[start:min(end, n)].view(np.uint16))
+
+
+@pytest.mark.parametrize("rows", [64, 65, 129, 300])
+@pytest.mark.parametrize("K,N", [(512, 96), (384, 40)])  # with and without a tiled copy of the weights (K % 256)
+def test_bare_linear_around_the_gemm_threshold(fp16_out, monkeypatch, rows, K, N):
+    """From 65 rows a bare module runs the MFMA GEMM on its tiled copy; a lower W4A16_GEMV_M_MAX keeps the GEMM entry point."""
+    torch.manual_seed(rows)
+    lin = nn.Linear(K, N, bias=True).half()
+    monkeypatch.setenv("W4A16_GEMV_M_MAX", "8" if rows == 64 else "")
+    mod = linear.CudaW4A16Linear.from_float(lin, 128).cuda()
+    x = torch.randn(rows, K).half()
+    want = _ref(x.numpy(), mod)
+    assert_close(mod(x.cuda()).cpu().numpy(), want, f"{rows} rows, fp16")
+    monkeypatch.setenv("W4A16_KERNEL_OUT_DTYPE", "fp32")
+    y32 = mod(x.cuda())
+    assert y32.dtype == torch.float32
+    assert_close(y32.cpu().numpy(), want, f"{rows} rows, fp32")
