@@ -255,6 +255,31 @@ def test_appended_key_is_bit_identical_to_the_tensor_expression(ext, fp16_out):
         run(d, 8, 8, 200, int(rng.integers(0, 200)), 1000 + i, int(rng.choice([2, 4])))
 
 
+@pytest.mark.parametrize("heads,kvh,splits", [(6, 3, 1), (28, 4, 4), (10, 1, 3), (5, 5, 7), (40, 8, 8)])
+def test_every_head_and_split_is_taken_once(ext, fp16_out, heads, kvh, splits):
+    """Workgroups are numbered by (member of the KV group, split, KV head): each partial is written by its own head and split."""
+    d, max_len, pos = 64, 96, 61
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    q, k, v = (torch.randn(n, d, device="cuda", generator=g).half() for n in (heads, kvh, kvh))
+    ck, cv = (torch.randn(kvh, max_len, d, device="cuda", generator=g).half() for _ in range(2))
+    cos, sin = torch.ones(max_len, d, device="cuda"), torch.zeros(max_len, d, device="cuda")  # no rotation
+    part = torch.full((heads, splits, d + 4), float("nan"), device="cuda")
+    ck2, cv2 = ck.clone(), cv.clone()
+    ext.rope_attend_split(q.reshape(-1), k.reshape(-1), v.reshape(-1), cos, sin, torch.tensor([pos], device="cuda"), ck2, cv2, part, d ** -0.5)
+    ck[:, pos], cv[:, pos] = k, v
+    assert torch.equal(ck2, ck) and torch.equal(cv2, cv)
+    for h in range(heads):
+        for s in range(splits):
+            rows = list(range(s, pos, splits)) + ([pos] if s == splits - 1 else [])
+            score = (ck[h // (heads // kvh), rows].double() @ q[h].double()) * d ** -0.5
+            w = torch.exp(score - score.max())
+            got = part[h, s].double()
+            # fp32 sums of 64 and of up to 62 terms, exp in fp32: well under 1e-4 of the largest entry
+            want = w @ cv[h // (heads // kvh), rows].double()
+            assert abs(got[0] - score.max()) <= 1e-4 and abs(got[1] - w.sum()) <= 1e-4 * w.sum()
+            assert (got[4:] - want).abs().max() <= 1e-4 * w.sum() * 4
+
+
 def test_position_outside_the_cache_touches_no_cache_row_and_poisons_the_output(ext, fp16_out):
     heads, kvh, d, max_len = 8, 2, 64, 96
     g = torch.Generator(device="cuda").manual_seed(1)
