@@ -948,6 +948,50 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// What a launch of gemm_tiled_kernel takes, in us: a fit over 250 (group, rows) pairs -- 21 groups of 1.5B to 14B shapes,
+// 65 to 1024 rows, with and without slices of K, 8400 timings, 7 % rms -- used to compare ways to cut one product.  A half-step
+// (128 columns of K) of a tile costs `step` on the first workgroup of a compute unit and `step_more` on every further one
+// (they share its matrix cores, but fill each other's waits); a split of K pays the launch that adds the slices and the
+// traffic of their fp32 tiles.
+struct GemmCost {
+  int mt, nt, wk;
+  float fixed, rank_block, step, step_more, reduce, partial_mb, output_mb;
+};
+constexpr GemmCost kGemmCost[] = {
+    {1, 1, 1, 1.6f, 1.9f, 0.45f, 0.27f, 1.7f, 0.50f, 0.80f}, {1, 2, 1, 2.1f, 3.3f, 0.69f, 0.53f, 2.3f, 0.28f, 0.65f},
+    {2, 1, 1, 2.2f, 2.1f, 0.60f, 0.39f, 1.6f, 0.37f, 0.64f}, {2, 1, 2, 2.0f, 3.0f, 0.96f, 0.88f, 2.3f, 0.34f, 0.96f},
+    {2, 2, 1, 2.9f, 3.3f, 0.90f, 0.77f, 1.6f, 0.29f, 0.52f}, {4, 1, 1, 3.1f, 2.8f, 1.00f, 0.73f, 1.9f, 0.24f, 0.59f},
+    {4, 2, 1, 5.0f, 4.0f, 1.43f, 1.27f, 1.1f, 0.23f, 0.58f}, {4, 2, 2, 6.0f, 5.5f, 2.46f, 3.10f, 1.3f, 0.25f, 0.92f}};
+
+static long gemm_tiles(const GemmGroup& gg, int mt, int nt) {
+  long tiles = 0;
+  for (int i = 0; i < gg.n; ++i) tiles += (long)((gg.m[0].M + 32 * mt - 1) / (32 * mt)) * ((gg.m[i].N + 128 * nt - 1) / (128 * nt));
+  return tiles;
+}
+
+// `tail_slices` > 1: the tiles past the last multiple of the compute-unit count are cut into that many (slices is then 1)
+static float gemm_cost(const GemmGroup& gg, const GemmCost& c, int slices, int tail_slices, int num_cus) {
+  const int sb = gg.m[0].K >> 8;
+  const long tiles = gemm_tiles(gg, c.mt, c.nt);
+  const auto half_steps = [&](int s) { return (float)(2 * ((((sb + s - 1) / s) + c.wk - 1) / c.wk)); };
+  const float tile_mb = (float)(32 * c.mt) * (128 * c.nt) * 4e-6f;
+  int rank = 0;
+  float out_mb = 0.f;
+  for (int i = 0; i < gg.n; ++i) {
+    if (gg.m[i].r != nullptr) rank = gg.m[i].rank;
+    out_mb += (float)gg.m[i].N * (float)gg.m[i].M * 2e-6f;
+  }
+  float us = c.fixed + c.rank_block * (float)((rank + 127) / 128) + c.output_mb * out_mb;
+  if (tail_slices > 1) {
+    const long tail = tiles % num_cus;
+    return us + half_steps(1) * (c.step + (float)(tiles / num_cus - 1) * c.step_more) + half_steps(tail_slices) * c.step_more + c.reduce +
+           c.partial_mb * tile_mb * (float)(tail * tail_slices);
+  }
+  us += half_steps(slices) * (c.step + (float)((tiles * slices + num_cus - 1) / num_cus - 1) * c.step_more);
+  if (slices > 1) us += c.reduce + c.partial_mb * tile_mb * (float)(tiles * slices);
+  return us;
+}
+
 static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes, hipStream_t stream) {
   // Tile choice: the largest tile (most reuse of both operands) whose workgroup count still fills the chip; when
   // none does, the one with the most workgroups.  Row tiles are capped by M (and at 4: 8 spills), column tiles at
@@ -1067,7 +1111,38 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
       }
     }
   }
-  if (wk == 2) return launch_gemm_t<4, 2, true, true, true, 2>(gg, stream);
+  // From 65 rows on the tiled copy the cut above stands unless another one is predicted 7 % faster: the choice above fills the
+  // chip with tiles first and cuts K only where that leaves most of it idle, but up to about a thousand rows one round of
+  // workgroups made of smaller tiles and slices of K is often the shorter way (8B o_proj at 100 rows 18.4 -> 15.1 us, down_proj
+  // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  Over the timings behind kGemmCost this takes
+  // 9 % off the mean and costs more than 1 % on one pair of 250; without the margin it costs more than 1 % on 30.
+  if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
+    float best_us = 0.f;
+    for (const GemmCost& c : kGemmCost)
+      if (c.mt == mt && c.nt == nt && c.wk == wk) best_us = 0.93f * gemm_cost(gg, c, gg.slices, gg.tail_slices, num_cus);
+    static const int tried[4][3] = {{1, 1, 1}, {2, 1, 1}, {2, 1, 2}, {4, 2, 1}};
+    const int sb_total = gg.m[0].K >> 8;
+    for (const auto& t : tried) {
+      for (const GemmCost& c : kGemmCost) {
+        if (c.mt != t[0] || c.nt != t[1] || c.wk != t[2]) continue;
+        const long tiles = gemm_tiles(gg, c.mt, c.nt);
+        for (int s = 1; s <= 16 && s * 2 <= std::max(sb_total, 2); ++s) {  // two super-blocks and more to a slice, three rounds at most
+          const int per = (sb_total + s - 1) / s;
+          if ((sb_total + per - 1) / per != s) continue;  // a slice without super-blocks
+          if (s > 1 && (env_split == 0 || tiles * s > 3L * num_cus || (size_t)(tiles * s) * (32 * c.mt) * (128 * c.nt) * sizeof(float) > ws_bytes)) break;
+          const float us = gemm_cost(gg, c, s, 0, num_cus);
+          if (us >= best_us) continue;
+          best_us = us;
+          mt = c.mt;
+          nt = c.nt;
+          wk = c.wk;
+          gg.slices = s;
+          gg.full = gg.tail_slices = 0;
+        }
+      }
+    }
+  }
+  if (wk == 2) return mt == 2 ? launch_gemm_t<2, 1, true, true, true, 2>(gg, stream) : launch_gemm_t<4, 2, true, true, true, 2>(gg, stream);
 #define GLOWQ_GEMM_CASE(MT, NT)                                                            \
   if (mt == MT && nt == NT)                                                                \
     return tiled_ok ? launch_gemm_t<MT, NT, true, true, true>(gg, stream)                  \

@@ -4,6 +4,8 @@ import pytest
 import torch
 
 import glowq_oracle as oracle
+from glowq_amd.kernels import PreparedGroup
+from glowq_amd.linear import CudaW4A16Linear
 from helpers import assert_close, dev, make_group, tuning
 
 pytestmark = pytest.mark.gpu
@@ -299,3 +301,39 @@ def test_gemm_tail_tiles_split_along_k(ext, M, K, Ns, rank):
         ext.WORKSPACE_BYTES = saved[0]
         ext._workspaces.clear()
         ext._workspaces.update(saved[1])
+
+
+@pytest.mark.parametrize("M,K,Ns,rank,kernel", [
+    (65, 3840, [1000, 130], 64, None), (100, 4096, [4096], 128, "gemm_tiled_kernel<2,1,1>"), (129, 5376, [2000], 40, None),
+    (256, 4096, [4096, 1024, 1024], 128, "gemm_tiled_kernel<2,1,2>"), (250, 5376, [5000, 1100], 0, "gemm_tiled_kernel<2,1,2>"),
+    (333, 17408, [2600], 256, None), (512, 512, [16000], 64, None), (700, 256, [300], 8, None)])
+def test_cut_of_products_of_a_few_hundred_rows(ext, M, K, Ns, rank, kernel):
+    """The cut (tile, K groups of a workgroup, slices of K) that the cost rule picks from 65 rows on: with the workspace, with one
+    that holds few slices and with none, odd numbers of super-blocks and ragged last tiles among them."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half() if rank else None
+    members, want = [], []
+    for N in Ns:
+        lin = torch.nn.Linear(K, N, bias=True, device="cuda", dtype=torch.float16)
+        mod = CudaW4A16Linear.from_float(lin, 128)
+        L = (torch.randn(N, rank, device="cuda", generator=g) * 0.01).half() if rank else None
+        members.append({"qweight": mod.qweight_i32, "scales": mod.scales_f16, "qzeros": mod.qzeros_i32, "L": L, "bias": mod.bias.data})
+        y = x.double() @ mod.dequantize().double().t() + mod.bias.data.double()
+        want.append(y if not rank else y + (x.double() @ R.double().t()) @ L.double().t())
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if rank else 0.0, R=R)
+    saved = ext.WORKSPACE_BYTES
+    try:
+        for nbytes in (saved, 4 << 20, 16):
+            ext.WORKSPACE_BYTES = nbytes
+            ext._workspaces.clear()
+            outs = [[y.clone() for y in pg.run(x)] for _ in range(2)]
+            torch.cuda.synchronize()
+            if nbytes == saved and kernel is not None:
+                assert ext.last_launch()["kernel"] == kernel
+            for a, b, w in zip(*outs, want):
+                assert torch.equal(a, b)
+                assert_close(a.cpu().numpy(), w.cpu().numpy(), f"M={M} K={K} workspace {nbytes}")
+    finally:
+        ext.WORKSPACE_BYTES = saved
+        ext._workspaces.clear()
