@@ -58,6 +58,16 @@ class _Glue:
         self.ext, self.cos_t, self.sin_t, self.pos = ext, cos_t, sin_t, pos
 
 
+def _row_kernels(*tensors) -> bool:
+    """Whether several token rows may go through the library's kernels instead of tensor expressions: plain fp16 tensors on the
+    GPU, and nobody who needs to see the expressions -- no gradients in either direction, no tracing, no function transforms."""
+    for t in tensors:
+        if not (t.is_cuda and t.device == tensors[0].device and t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            return False
+    return not (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+                or torch._C._len_torch_dispatch_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float):
         super().__init__()
@@ -73,7 +83,25 @@ class RMSNorm(nn.Module):
             return h
         if delta is not None:
             x.add_(delta)
+        if self._takes_rows(x):
+            h = torch.empty_like(x)
+            load_w4a16_extension().add_rmsnorm(x, None, self.weight, h, self.eps)
+            return h
         return F.rms_norm(x, (x.size(-1),), self.weight, self.eps)
+
+    def _takes_rows(self, *xs) -> bool:
+        x = xs[0]
+        return (x.dim() == 2 and x.size(0) > 1 and x.size(1) % 8 == 0 and all(t.shape == x.shape and t.device == x.device for t in xs)
+                and self.weight.device == x.device and self.weight.numel() == x.size(1) and _row_kernels(*xs, self.weight))
+
+    def forward_add(self, x, delta):
+        """(x + delta, rmsnorm(x + delta) * weight), one launch for several token rows."""
+        if self._takes_rows(x, delta):
+            out, h = torch.empty_like(x), torch.empty_like(x)
+            load_w4a16_extension().add_rmsnorm_out(x, delta, self.weight, out, h, self.eps)
+            return out, h
+        out = x + delta
+        return out, self.forward(out)
 
 
 class Attention(nn.Module):
@@ -101,12 +129,21 @@ class Attention(nn.Module):
                 self.glue.ext.rope_attend(q[0], k[0], v[0], self.glue.cos_t, self.glue.sin_t, pos_idx, cache_k, cache_v, out[0],
                                           cfg.head_dim ** -0.5)
                 return self.o_proj(out)
-        q = self.q_proj(x).view(T, cfg.heads, cfg.head_dim).transpose(0, 1)      # [H, T, d]
-        k = self.k_proj(x).view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)   # [KV, T, d]
-        v = self.v_proj(x).view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)
-        q, k = _rope(q, cos, sin), _rope(k, cos, sin)
-        cache_k.index_copy_(1, pos_idx, k.to(cache_k.dtype))
-        cache_v.index_copy_(1, pos_idx, v.to(cache_v.dtype))
+        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        if (T > 1 and x.dim() == 2 and cfg.head_dim % 16 == 0 and pos_idx.dtype == torch.int64 and pos_idx.device == q.device and tuple(pos_idx.shape) == (T,) and pos_idx.is_contiguous()
+                and cos.shape == sin.shape == (T, cfg.head_dim) and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
+            # rotary embedding and cache append in one launch; the heads stay side by side in a row
+            q_rot, k_rot = torch.empty_like(q), torch.empty_like(k)
+            load_w4a16_extension().rope_append(q, k, v, cos, sin, pos_idx, q_rot, k_rot, cache_k, cache_v)
+            q, k = q_rot.view(T, cfg.heads, cfg.head_dim).transpose(0, 1), k_rot.view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)
+            v = v.view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)
+        else:
+            q = q.view(T, cfg.heads, cfg.head_dim).transpose(0, 1)      # [H, T, d]
+            k = k.view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)   # [KV, T, d]
+            v = v.view(T, cfg.kv_heads, cfg.head_dim).transpose(0, 1)
+            q, k = _rope(q, cos, sin), _rope(k, cos, sin)
+            cache_k.index_copy_(1, pos_idx, k.to(cache_k.dtype))
+            cache_v.index_copy_(1, pos_idx, v.to(cache_v.dtype))
         if mask is None:
             out = F.scaled_dot_product_attention(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), is_causal=True, enable_gqa=True)
         else:
@@ -136,7 +173,19 @@ class MLP(nn.Module):
             act = torch.empty_like(gate)
             self.glue.ext.silu_mul(gate, up, act)
             return self.down_proj(act)
+        if x.dim() == 2 and x.size(0) > 1 and gate.shape == up.shape and gate.numel() % 8 == 0 and _row_kernels(gate, up):
+            act = torch.empty_like(gate)
+            load_w4a16_extension().silu_mul(gate, up, act)
+            return self.down_proj(act)
         return self.down_proj(F.silu(gate) * up)
+
+
+def _hooked(mod: nn.Module) -> bool:
+    """Whether calling `mod` does more than its forward, or it is another module than the decoder's own norm."""
+    glob = torch.nn.modules.module
+    return not (type(mod) is RMSNorm and "forward" not in mod.__dict__) or bool(
+        mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+        or glob._global_forward_hooks or glob._global_forward_pre_hooks or glob._global_backward_hooks or glob._global_backward_pre_hooks)
 
 
 class DecoderLayer(nn.Module):
@@ -153,8 +202,13 @@ class DecoderLayer(nn.Module):
             attn = self.self_attn(self.input_layernorm(x), cos, sin, cache_k, cache_v, pos_idx, mask)
             h = self.post_attention_layernorm(x, delta=attn.to(x.dtype))
             return x.add_(self.mlp(h).to(x.dtype))
-        x = x + self.self_attn(self.input_layernorm(x), cos, sin, cache_k, cache_v, pos_idx, mask)
-        return x + self.mlp(self.post_attention_layernorm(x))
+        attn = self.self_attn(self.input_layernorm(x), cos, sin, cache_k, cache_v, pos_idx, mask)
+        if x.size(0) > 1 and not _hooked(self.post_attention_layernorm):
+            x, h = self.post_attention_layernorm.forward_add(x, attn)  # the residual add rides on the norm's launch
+        else:
+            x = x + attn
+            h = self.post_attention_layernorm(x)
+        return x + self.mlp(h)
 
 
 class _Body(nn.Module):

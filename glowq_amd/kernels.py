@@ -87,6 +87,8 @@ _SIGNATURES = {
     "glowq_pack_tiled_left": (_I, [_P, _P, _I, _I, _P]),
     "glowq_set_tuning": (_I, [ctypes.c_char_p, _I]),
     "glowq_add_rmsnorm": (_I, [_P, _P, _P, _P, _I, _I, ctypes.c_float, _P]),
+    "glowq_add_rmsnorm_out": (_I, [_P, _P, _P, _P, _P, _I, _I, ctypes.c_float, _P]),
+    "glowq_rope_append": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "glowq_silu_mul": (_I, [_P, _P, _P, ctypes.c_long, _P]),
     "glowq_add_rmsnorm_proj": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, ctypes.c_float, _P]),
     "glowq_silu_mul_proj": (_I, [_P, _P, _P, _P, _P, _I, _I, _P]),
@@ -445,6 +447,37 @@ class W4A16Extension:
                                             h.data_ptr(), x.size(0), x.size(1), float(eps), self._stream(x.device))
         if rc:
             self._raise(rc, "add_rmsnorm")
+
+    def add_rmsnorm_out(self, x, delta, weight, x_out, h, eps: float) -> None:
+        """x_out = x + delta, h = rmsnorm(x_out) * weight over [M, H] rows, x untouched."""
+        for t, n in ((x, "x"), (delta, "delta"), (weight, "weight"), (x_out, "x_out"), (h, "h")):
+            self._f16(t, n)
+        _check(x.dim() == 2 and delta.shape == x.shape and x_out.shape == x.shape and h.shape == x.shape and weight.numel() == x.size(1),
+               "add_rmsnorm_out: shape mismatch")
+        with torch.cuda.device(x.device):
+            rc = self.lib.glowq_add_rmsnorm_out(x.data_ptr(), delta.data_ptr(), weight.data_ptr(), x_out.data_ptr(), h.data_ptr(), x.size(0),
+                                                x.size(1), float(eps), self._stream(x.device))
+        if rc:
+            self._raise(rc, "add_rmsnorm_out")
+
+    def rope_append(self, q, k, v, cos_rows, sin_rows, pos, q_out, k_out, cache_k, cache_v) -> None:
+        """T token rows: q_out = rope(q), k_out = rope(k), and rows pos[t] of the caches [kv_heads, max_len, d] = (k_out, v).
+        q [T, heads d], k / v [T, kv_heads d], cos_rows / sin_rows [T, d] fp16, pos int64 [T] on the device."""
+        for t, n in ((q, "q"), (k, "k"), (v, "v"), (cos_rows, "cos_rows"), (sin_rows, "sin_rows"), (q_out, "q_out"), (k_out, "k_out"),
+                     (cache_k, "cache_k"), (cache_v, "cache_v")):
+            self._f16(t, n)
+        kv_heads, max_len, d = cache_k.shape
+        T = pos.numel()
+        _check(pos.is_cuda and pos.dtype == torch.int64 and pos.is_contiguous(), "rope_append: pos must be int64 [T] on the device")
+        _check(q.dim() == 2 and q.size(0) == T and q.size(1) % d == 0 and q_out.shape == q.shape and tuple(k.shape) == (T, kv_heads * d)
+               and v.shape == k.shape and k_out.shape == k.shape and tuple(cos_rows.shape) == (T, d) and sin_rows.shape == cos_rows.shape
+               and cache_v.shape == cache_k.shape, "rope_append: shape mismatch")
+        with torch.cuda.device(q.device):
+            rc = self.lib.glowq_rope_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_rows.data_ptr(), sin_rows.data_ptr(), pos.data_ptr(),
+                                            q_out.data_ptr(), k_out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), T, q.size(1) // d,
+                                            kv_heads, d, max_len, self._stream(q.device))
+        if rc:
+            self._raise(rc, "rope_append")
 
     def silu_mul(self, gate, up, out) -> None:
         for t, n in ((gate, "gate"), (up, "up"), (out, "out")):

@@ -310,6 +310,13 @@ int glowq_set_tuning(const char* key, int value);
 
 /* x[m] += delta[m] (skipped when delta is NULL), h[m] = rmsnorm(x[m]) * weight; x [M, H] is updated in place. */
 int glowq_add_rmsnorm(void* x, const void* delta, const void* weight, void* h, int M, int H, float eps, void* stream);
+/* the same with the sum in x_out (x_out may be x; without delta x_out is not written and may be NULL) */
+int glowq_add_rmsnorm_out(const void* x, const void* delta, const void* weight, void* x_out, void* h, int M, int H, float eps, void* stream);
+/* T token rows: q_out = rope(q) [T, heads d], k_out = rope(k) [T, kv_heads d], rows pos[t] of the caches [kv_heads, max_len, d] =
+   (k_out, v); cos_rows / sin_rows [T, d] fp16 are the tables at the tokens' positions; a position outside the cache writes no row.
+   head_dim % 16 == 0, tensors contiguous fp16, 16-byte aligned. */
+int glowq_rope_append(const void* q, const void* k, const void* v, const void* cos_rows, const void* sin_rows, const int64_t* pos, void* q_out,
+                      void* k_out, void* cache_k, void* cache_v, int T, int heads, int kv_heads, int head_dim, int max_len, void* stream);
 
 /* out = silu(gate) * up over n elements (n % 8 == 0). */
 int glowq_silu_mul(const void* gate, const void* up, void* out, long n, void* stream);

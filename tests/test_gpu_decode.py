@@ -560,3 +560,64 @@ def test_glue_with_projection_matches_separate_launches(ext, fp16_out):
     ext.silu_mul_proj(gate, up, act, R2, r2)
     assert torch.equal(act, act_ref)
     assert (r2.float() - r2_ref.float()).abs().max() <= 2e-3 * r2_ref.float().abs().max() + 1e-3
+
+
+@pytest.mark.parametrize("T,heads,kvh,d", [(2, 4, 2, 64), (65, 6, 3, 128), (300, 5, 1, 48), (1, 2, 2, 16)])
+def test_rope_append_matches_the_expression(ext, T, heads, kvh, d):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    max_len = T + 9
+    q, k, v = (torch.randn(T, n * d, device="cuda", generator=g).half() for n in (heads, kvh, kvh))
+    ang = torch.rand(T, d, device="cuda", generator=g) * 6.0  # the halves differ: each dimension has its own angle
+    cos, sin = ang.cos().half(), ang.sin().half()
+    pos = torch.randperm(max_len, device="cuda", generator=g)[:T].contiguous()
+    pos[0] = max_len  # outside: no row is written
+    ck, cv = (torch.randn(kvh, max_len, d, device="cuda", generator=g).half() for _ in range(2))
+    ck2, cv2, q_out, k_out = ck.clone(), cv.clone(), torch.empty_like(q), torch.empty_like(k)
+    ext.rope_append(q, k, v, cos, sin, pos, q_out, k_out, ck2, cv2)
+
+    def rope(t, n):
+        t = t.view(T, n, d).double()
+        rot = torch.cat((-t[..., d // 2:], t[..., :d // 2]), dim=-1)
+        return (t * cos.double()[:, None] + rot * sin.double()[:, None]).reshape(T, n * d)
+    # two products and a sum in fp32, one rounding to fp16: an fp16 ulp of the largest term where the products cancel
+    for got, want in ((q_out, rope(q, heads)), (k_out, rope(k, kvh))):
+        assert ((got.double() - want).abs() <= 2.0 ** -10 * want.abs() + 2e-6).all()
+    ok = pos < max_len
+    ck[:, pos[ok]] = k_out.view(T, kvh, d)[ok].transpose(0, 1)
+    cv[:, pos[ok]] = v.view(T, kvh, d)[ok].transpose(0, 1)
+    assert torch.equal(ck2, ck) and torch.equal(cv2, cv)
+
+
+@pytest.mark.parametrize("T", [2, 33, 130])
+@pytest.mark.parametrize("from_empty", [True, False])
+def test_rows_through_the_kernels_match_the_tensor_expressions(fp16_out, T, from_empty):
+    """Several token rows run norm, rotary embedding, cache append and gate as kernels; with gradients on, as expressions."""
+    cfg = decode.DecoderConfig(hidden=512, layers=2, heads=8, kv_heads=2, head_dim=64, intermediate=1280, vocab=320, max_len=160, rank=32)
+    with torch.device("cuda"):
+        model, _, _ = decode.build_decoder(cfg, seed=5)
+    cos, sin = model.rope_tables("cuda")
+    tokens, pos = torch.randint(0, cfg.vocab, (T,), device="cuda"), torch.arange(T, device="cuda")
+    res = []
+    for grad in (False, True):
+        caches = [tuple(torch.zeros(cfg.kv_heads, cfg.max_len, cfg.head_dim, dtype=torch.float16, device="cuda") for _ in range(2)) for _ in range(2)]
+        with torch.set_grad_enabled(grad):
+            for p in model.parameters():
+                p.requires_grad_(False)
+            logits = model.forward_tokens(tokens, pos, caches, cos, sin, from_empty_cache=from_empty)
+        res.append([logits] + [t for pair in caches for t in pair])
+    for a, b in zip(*res):
+        # both round every activation to fp16 several times a layer (2^-11 each): well under 1e-2 of the result
+        assert (a.double() - b.double()).norm() <= 1e-2 * b.double().norm()
+
+
+def test_norm_hooks_still_see_the_residual_norm(fp16_out):
+    cfg = decode.DecoderConfig(hidden=256, layers=1, heads=4, kv_heads=2, head_dim=64, intermediate=512, vocab=64, max_len=32, rank=32)
+    with torch.device("cuda"):
+        model, _, _ = decode.build_decoder(cfg, seed=6)
+    cos, sin = model.rope_tables("cuda")
+    caches = [tuple(torch.zeros(2, 32, 64, dtype=torch.float16, device="cuda") for _ in range(2))]
+    seen = []
+    model.model.layers[0].post_attention_layernorm.register_forward_hook(lambda m, i, o: seen.append((i[0].shape, o.shape)))
+    with torch.no_grad():
+        model.forward_tokens(torch.arange(5, device="cuda"), torch.arange(5, device="cuda"), caches, cos, sin, from_empty_cache=True)
+    assert seen == [(torch.Size([5, 256]), torch.Size([5, 256]))]
