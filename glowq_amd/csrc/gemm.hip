@@ -1111,15 +1111,17 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
       }
     }
   }
-  // From 65 rows on the tiled copy the cut above stands unless another one is predicted 7 % faster: the choice above fills the
+  // From 65 rows on the tiled copy the cut above stands unless another one is predicted 9 % faster: the choice above fills the
   // chip with tiles first and cuts K only where that leaves most of it idle, but up to about a thousand rows one round of
   // workgroups made of smaller tiles and slices of K is often the shorter way (8B o_proj at 100 rows 18.4 -> 15.1 us, down_proj
   // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  Over the timings behind kGemmCost this takes
-  // 9 % off the mean and costs more than 1 % on one pair of 250; without the margin it costs more than 1 % on 30.
+  // 9 % off the mean and costs nowhere more than 1 %; without the margin it costs more than that on 30 pairs of 250.  Cuts that
+  // send more than 32 MB of fp32 tiles through the workspace are not tried: there the fit is off by up to 15 % (1B fc2 at 1500
+  // rows in five slices 70.6 us against 65.1 in two).
   if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
     float best_us = 0.f;
     for (const GemmCost& c : kGemmCost)
-      if (c.mt == mt && c.nt == nt && c.wk == wk) best_us = 0.93f * gemm_cost(gg, c, gg.slices, gg.tail_slices, num_cus);
+      if (c.mt == mt && c.nt == nt && c.wk == wk) best_us = 0.91f * gemm_cost(gg, c, gg.slices, gg.tail_slices, num_cus);
     static const int tried[4][3] = {{1, 1, 1}, {2, 1, 1}, {2, 1, 2}, {4, 2, 1}};
     const int sb_total = gg.m[0].K >> 8;
     for (const auto& t : tried) {
@@ -1129,7 +1131,8 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
         for (int s = 1; s <= 16 && s * 2 <= std::max(sb_total, 2); ++s) {  // two super-blocks and more to a slice, three rounds at most
           const int per = (sb_total + s - 1) / s;
           if ((sb_total + per - 1) / per != s) continue;  // a slice without super-blocks
-          if (s > 1 && (env_split == 0 || tiles * s > 3L * num_cus || (size_t)(tiles * s) * (32 * c.mt) * (128 * c.nt) * sizeof(float) > ws_bytes)) break;
+          const size_t partial_bytes = (size_t)(tiles * s) * (32 * c.mt) * (128 * c.nt) * sizeof(float);
+          if (s > 1 && (env_split == 0 || tiles * s > 3L * num_cus || partial_bytes > std::min(ws_bytes, (size_t)32 << 20))) break;
           const float us = gemm_cost(gg, c, s, 0, num_cus);
           if (us >= best_us) continue;
           best_us = us;
@@ -1392,6 +1395,124 @@ __global__ __launch_bounds__(256) void proj_reduce_kernel(const float* __restric
   if (m < M && n < rank) r[(size_t)m * rank + n] = (half_t)v;
 }
 
+// ---- shared projection, 65 rows and more: tiles of 64 x 64 or 128 x 128, both operands through LDS --------------------
+// proj_mfma_kernel's 32-row tiles read R once per 32 rows and x once per 32 or 64 columns, 16 or 8 products for every element
+// that a compute unit pulls in, two blocks in flight.  Here a workgroup of four waves (two by two) takes 64 kA rows of x and 64 kB rows
+// of R in stages of 128 columns that go from memory straight into LDS (kSt stages in a ring, swizzled like the activations of
+// gemm_tiled_kernel: slot c' of row q holds the row's 16-byte piece c' ^ (q % 16)), and K is cut over gridDim.z workgroups
+// whose fp32 tiles [slice][M][rank] meet in proj_sum_kernel, in slice order.
+template <int kA>
+__global__ __launch_bounds__(256) void proj_tile_kernel(const half_t* __restrict__ x, const half_t* __restrict__ R, half_t* __restrict__ r,
+                                                        float* __restrict__ partials, int M, int K, int rank) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int kB = kA, kSt = 2;  // (three and four stages measured the same or slower; the second workgroup of a compute unit fills the waits)
+  constexpr int BM = 64 * kA, BN = 64 * kB;
+  constexpr int kStage = (BM + BN) * kTRow;
+  constexpr int kLoads = (BM + BN) / 16;  // 16-byte loads of a thread per stage
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, lh = lane >> 5;
+  const int m0 = (int)blockIdx.x * BM, n0 = (int)blockIdx.y * BN;
+  const int all = K >> 7, per = (all + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int first = min((int)blockIdx.z * per, all), n = min(per, all - first);  // this workgroup's stages
+  const auto rsrc = [](const void* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rs_x = rsrc(x, (size_t)M * K * 2), rs_r = rsrc(R, (size_t)rank * K * 2);
+  const int srow = tid >> 4, spiece = (tid & 15) ^ srow;
+  uint32_t off[kLoads];
+#pragma unroll
+  for (int q = 0; q < kLoads; ++q) {
+    const int row = q < BM / 16 ? min(m0 + 16 * q + srow, M - 1) : min(n0 + 16 * (q - BM / 16) + srow, rank - 1);  // past the end: dropped results
+    off[q] = ((uint32_t)row * (uint32_t)K + (uint32_t)spiece * 8u) * 2u;
+  }
+  auto request = [&](int st) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+    unsigned char* dst = smem + (size_t)(st % kSt) * kStage + 4 * wave * kTRow;
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(q < BM / 16 ? rs_x : rs_r, (lds_ptr_t)(dst + 16 * q * kTRow), 16, (int)off[q], (first + st) * 256, 0, 0);
+  };
+  f16v acc[kA][kB];
+#pragma unroll
+  for (int a = 0; a < kA; ++a)
+#pragma unroll
+    for (int b = 0; b < kB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+#pragma unroll
+  for (int st = 0; st < kSt - 1; ++st)
+    if (st < n) request(st);
+  const int wr = (wave >> 1) * (32 * kA), wc = (wave & 1) * (32 * kB);
+  for (int st = 0; st < n; ++st) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of stage st has landed, behind the barrier everybody's
+    __syncthreads();
+    if (st + kSt - 1 < n) request(st + kSt - 1);  // into the stage that everybody is done with
+    const unsigned char* base = smem + (size_t)(st % kSt) * kStage;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int slot = ((2 * t + lh) ^ (ln & 15)) << 4;
+      h8 af[kA], bf[kB];
+#pragma unroll
+      for (int a = 0; a < kA; ++a) af[a] = *reinterpret_cast<const h8*>(base + (wr + 32 * a + ln) * kTRow + slot);
+#pragma unroll
+      for (int b = 0; b < kB; ++b) bf[b] = *reinterpret_cast<const h8*>(base + (BM + wc + 32 * b + ln) * kTRow + slot);
+#pragma unroll
+      for (int a = 0; a < kA; ++a)
+#pragma unroll
+        for (int b = 0; b < kB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a], bf[b], acc[a][b], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < kA; ++a)
+#pragma unroll
+    for (int b = 0; b < kB; ++b) {
+      const int col = n0 + wc + 32 * b + ln;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int m = m0 + wr + 32 * a + 8 * (i >> 2) + 4 * lh + (i & 3);
+        if (m >= M || col >= rank) continue;
+        if (gridDim.z == 1) r[(size_t)m * rank + col] = (half_t)acc[a][b][i];
+        else partials[((size_t)blockIdx.z * M + m) * rank + col] = acc[a][b][i];
+      }
+    }
+}
+
+// r = fp16(sum of the slices in slice order); four elements to a thread, one wave to a workgroup (a few hundred waves at most)
+__global__ __launch_bounds__(64) void proj_sum_kernel(const float* __restrict__ partials, half_t* __restrict__ r, long n4, int slices) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n4) return;
+  const f4* src = reinterpret_cast<const f4*>(partials) + i;
+  f4 v = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kBatch = 8;  // slices in flight
+  for (int z = 0; z < slices; z += kBatch) {
+    f4 t[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) t[u] = src[(size_t)min(z + u, slices - 1) * n4];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += z + u < slices ? t[u][e] : 0.f;
+  }
+  h4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (half_t)v[e];
+  reinterpret_cast<h4*>(r)[i] = o;
+}
+
+template <int kA>
+static hipError_t launch_proj_tile(const half_t* x, const half_t* R, half_t* r, int M, int K, int rank, int slices, float* ws, hipStream_t stream) {
+  auto kern = proj_tile_kernel<kA>;
+  constexpr size_t lds = (size_t)2 * (128 * kA) * kTRow;
+  static LdsLimit lds_limit;
+  if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((M + 64 * kA - 1) / (64 * kA), (rank + 64 * kA - 1) / (64 * kA), slices), dim3(256), lds, stream, x, R, r, ws, M, K,
+                     rank);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || slices == 1) return e;
+  const long n4 = (long)M * rank / 4;
+  hipLaunchKernelGGL(proj_sum_kernel, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, stream, ws, r, n4, slices);
+  return hipGetLastError();
+}
+
 // How a projection is cut: columns per workgroup (32 * nt) and K slices.  The tile width follows the workgroup count
 // (narrow tiles where 64 columns each would leave CUs idle; R is small, re-reading it is cheap).  K is split only with a
 // workspace, where the tiles alone fill less than half the chip and K is long enough for the second launch to pay
@@ -1431,6 +1552,42 @@ static ProjPlan plan_proj(int M, int K, int rank, int num_cus, size_t ws_bytes) 
   return best;
 }
 
+// Which of the two kernels, and how the tiles are cut: by what they are predicted to take, in us -- fits over 204 (M, K, rank),
+// 65 to 2048 rows, 7 % rms, of the same form as kGemmCost: a block (256 columns) or stage (128) of K on the first workgroup of
+// a compute unit, on every further one, the second launch, its walk over the slices, the traffic of the fp32 tiles, x.  The
+// tile kernel has to be 7 % ahead; by that rule it takes 18 % off the mean and loses nowhere by more than 1 %.  us, this / 32-row tiles:
+// K = 18944, rank 128 at 100 / 333 / 2048 rows 11.1 / 14.7, 15.3 / 21.1, 30 / 37; K = 17408, rank 256 at 200 / 1500 rows 14.4 / 26.9,
+// 34 / 78; K = 4096, rank 128 at 100 / 1500 rows 7.3 / 8.6, 12.0 / 17.1; K = 1536, rank 256 at 512 rows 8.9 / 6.9 (not taken).
+struct ProjTilePlan {
+  int a, slices;  // a = 0: the 32-row tiles
+};
+static ProjTilePlan plan_proj_tile(const ProjPlan& p, int M, int K, int rank, int num_cus, size_t ws_bytes) {
+  const auto rounds_more = [&](long wgs) { return (float)((wgs + num_cus - 1) / num_cus - 1); };
+  const float slice_mb = (float)M * (float)rank * 4e-6f;
+  const int blocks = (K + kPK - 1) / kPK, stages = K >> 7;
+  const float per = (float)((blocks + p.slices - 1) / p.slices);
+  const long wgs = (long)((M + 31) / 32) * ((rank + 32 * p.nt - 1) / (32 * p.nt)) * p.slices;
+  float best = 3.9f + per * (p.nt == 1 ? 0.48f : 0.81f) + per * 0.52f * rounds_more(wgs);
+  if (p.slices > 1) best += 1.6f + 0.09f * (float)p.slices + 1.5f * slice_mb * (float)p.slices;
+  best *= 0.93f;
+  ProjTilePlan plan = {0, 1};
+  for (int a = 1; a <= 2; ++a) {
+    const long tiles = (long)((M + 64 * a - 1) / (64 * a)) * ((rank + 64 * a - 1) / (64 * a));
+    for (int s = 1; s <= 32 && s <= stages && tiles * s <= 4L * num_cus; ++s) {
+      const int depth = (stages + s - 1) / s;
+      if ((stages + depth - 1) / depth != s) continue;  // a slice without stages
+      if (s > 1 && (size_t)s * M * rank * sizeof(float) > ws_bytes) break;
+      float us = (a == 1 ? 2.1f : 5.4f) + (float)depth * ((a == 1 ? 0.62f : 1.05f) + (a == 1 ? 0.29f : 1.66f) * rounds_more(tiles * s)) +
+                 0.07f * (float)M * (float)K * 2e-6f;
+      if (s > 1) us += 2.5f + (a == 1 ? 0.074f : 0.043f) * (float)s + (a == 1 ? 0.56f : 0.43f) * slice_mb * (float)s;
+      if (us >= best) continue;
+      best = us;
+      plan = {a, s};
+    }
+  }
+  return plan;
+}
+
 size_t proj_workspace_bytes(int M, int K, int rank, int num_cus) {
   if (M <= 16 || (K % kBK) != 0) return 0;
   const ProjPlan p = plan_proj(M, K, rank, num_cus, ~(size_t)0 >> 8);
@@ -1462,6 +1619,14 @@ hipError_t launch_shared_proj_mfma(const half_t* x, const half_t* R, half_t* r, 
   if ((K % kBK) != 0 || K < kBK) return hipErrorInvalidValue;
   if (ws == nullptr || (reinterpret_cast<uintptr_t>(ws) & 15u) != 0) ws_bytes = 0;
   const ProjPlan p = plan_proj(M, K, rank, num_cus, ws_bytes);
+  const bool tiles_ok = (K & 127) == 0 && (rank & 3) == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)rank * K * 2 < (1ull << 32) &&
+                        (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(R) & 15u) == 0 &&
+                        (reinterpret_cast<uintptr_t>(r) & 7u) == 0;
+  if (tiles_ok) {
+    const ProjTilePlan t = plan_proj_tile(p, M, K, rank, num_cus, ws_bytes);
+    if (t.a == 1) return launch_proj_tile<1>(x, R, r, M, K, rank, t.slices, static_cast<float*>(ws), stream);
+    if (t.a == 2) return launch_proj_tile<2>(x, R, r, M, K, rank, t.slices, static_cast<float*>(ws), stream);
+  }
   if (p.nt == 2) return launch_proj_t<2>(x, R, r, M, K, rank, p.slices, ws, stream);
   return launch_proj_t<1>(x, R, r, M, K, rank, p.slices, ws, stream);
 }

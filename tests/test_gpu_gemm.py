@@ -337,3 +337,25 @@ def test_cut_of_products_of_a_few_hundred_rows(ext, M, K, Ns, rank, kernel):
     finally:
         ext.WORKSPACE_BYTES = saved
         ext._workspaces.clear()
+
+
+@pytest.mark.parametrize("M,K,rank", [(65, 1408, 100), (130, 4096, 68), (257, 17408, 260), (1000, 384, 32), (333, 18944, 128), (90, 4160, 64),
+                                      (2048, 5120, 256), (64, 17408, 256), (129, 128, 4), (700, 2048, 6)])
+def test_shared_proj_tiles(ext, M, K, rank):
+    """The tile kernel of the projection and its neighbours (K not a multiple of 128, ranks not of 4): ragged tiles, with the
+    workspace, with one that holds a few slices and with none; the same bits on every call."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half()
+    want = (x.double() @ R.double().t()).cpu().numpy()
+    saved = ext.WORKSPACE_BYTES
+    try:
+        for nbytes in (saved, 3 * M * rank * 4, 16):
+            ext.WORKSPACE_BYTES = nbytes
+            ext._workspaces.clear()
+            r = [ext.shared_proj(x, R) for _ in range(2)]
+            assert torch.equal(*r)
+            assert_close(r[0].cpu().numpy(), want, f"M={M} K={K} rank={rank} workspace {nbytes}")
+    finally:
+        ext.WORKSPACE_BYTES = saved
+        ext._workspaces.clear()
