@@ -199,8 +199,8 @@ class AddSVDCorrection(nn.Module):
                     return self._finish(y, lead_shape)
             pg = self._prepared(ext, [self], True)
             if ok and same_x and r is not None:
-                return self._finish(pg.run(x2d, r=r, project=False)[0], lead_shape)
-            return self._finish(pg.run(x2d)[0], lead_shape)  # the reference's recompute-on-miss: r from this module's own R
+                return self._finish(pg.run(x2d, r=r, project=False, out_dtype=KNOBS.out_dtype)[0], lead_shape)
+            return self._finish(pg.run(x2d, out_dtype=KNOBS.out_dtype)[0], lead_shape)  # the reference's recompute-on-miss: r from this module's own R
 
         if cache is not None and self.role in _LEADER_USES:
             # who joins the leader's launch is decided once per state of the group (members, their alpha switches,
@@ -213,7 +213,7 @@ class AddSVDCorrection(nn.Module):
                 self.__dict__["_group_memo"] = memo
             group = memo[1]
             pg = self._prepared(ext, group, True)
-            outs = pg.run(x2d)  # r = x R^T and every member of the group in one call
+            outs = pg.run(x2d, out_dtype=KNOBS.out_dtype)  # r = x R^T and every member of the group in one call
             cache.clear()
             cache.set(pg.last_r, _LEADER_USES[self.role])
             cache.x_key = _x_key(x2d)
@@ -221,7 +221,7 @@ class AddSVDCorrection(nn.Module):
             for w, y in zip(group[1:], outs[1:]):
                 cache.outputs[id(w)] = y
             return self._finish(outs[0], lead_shape)
-        return self._finish(self._prepared(ext, [self], True).run(x2d)[0], lead_shape)
+        return self._finish(self._prepared(ext, [self], True).run(x2d, out_dtype=KNOBS.out_dtype)[0], lead_shape)
 
 
 def ext_max_members() -> int:

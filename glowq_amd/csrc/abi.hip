@@ -41,6 +41,7 @@ bool skinny_raw_form(const GroupDev& g);
 hipError_t launch_skinny(GroupDev& g, int num_cus, hipStream_t stream, bool raw);
 bool gemm_supported(const GroupDev& g);
 hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream);
+bool gemm_widens(const GroupDev& g);
 // misc.hip
 hipError_t launch_probe_read(const void* src, size_t bytes, void* sink, int grid, int block, hipStream_t stream);
 hipError_t launch_probe_empty(int grid, int block, hipStream_t stream);
@@ -236,6 +237,7 @@ void to_dev(const glowq_member_t& s, MemberDev& d) {
   d.lds = s.lds;
   d.ldz = s.ldz_i32;
   d.ldy = s.ldy;
+  d.y32 = s.y_type == GLOWQ_Y_FP32;
 }
 
 //   stream_max_m    token rows up to which the stream GEMV (every request of a wave in flight up front) is used where it
@@ -400,6 +402,8 @@ int pick_route_rounded(const GroupDev& g, int force) {
 // Runs one group through the chosen route.  Routes with a row capacity smaller than M walk the
 // token rows in chunks (weights are re-read once per chunk).
 int run_group(GroupDev g, int route, hipStream_t stream) {
+  for (int i = 0; i < g.n_members; ++i)
+    if (g.mem[i].y32 && !(route == kRouteGemm && gemm_widens(g))) return fail(GLOWQ_EUNSUPPORTED, "fp32 outputs: only where the GEMM on the tiled weights takes the call, and for all members alike");
   const int cus = num_cus();
   hipError_t e = hipSuccess;
   g.pub = nullptr;
@@ -608,6 +612,7 @@ int glowq_w4a16_group_forward_chained(const void* x, const void* r, const glowq_
     rc = check_member(m, K, group_size, i);
     if (rc) return rc;
     if (m.L == nullptr) return fail(GLOWQ_EUNSUPPORTED, "chained: member %d has no L", i);
+    if (m.y_type == GLOWQ_Y_FP32) return fail(GLOWQ_EUNSUPPORTED, "chained: outputs are fp16");
     if (y_optional) m.y = nullptr;
     to_dev(m, g.mem[i]);
     g.mem[i].side = nullptr;

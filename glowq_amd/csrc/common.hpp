@@ -35,6 +35,7 @@ struct MemberDev {
   const void* tiled_L;        // its tiled left factor or nullptr
   int tiled_rank;             // the rank tiled_L was packed for
   int N, ldw, lds, ldz, ldy;
+  int y32;                    // y is fp32 and receives the fp16 result widened (GEMM route)
 };
 
 struct GroupDev {

@@ -37,13 +37,20 @@ struct GemmArgs {
   const int32_t* qzeros;
   const half_t* bmat;     // [N, ldb] fp16 B operand: L for the correction, or the whole B of a plain GEMM
   const half_t* bias;
-  half_t* y;              // [M, ldy]
+  half_t* y;              // [M, ldy] (fp32 in the kernels with YT = float)
   const unsigned char* wt;  // the member's tiled weights (tiled.hpp) or nullptr
   const unsigned char* lt;  // its tiled left factor or nullptr
   int M, N, K, group_size, rank;
   int ldw, lds, ldz, ldb, ldy;
   float alpha;
 };
+
+// The result is rounded to fp16 in either form; fp32 outputs hold that value widened, which a caller that wants them would
+// otherwise do in a launch and two passes of its own (Qwen2.5-7B layer at 333 rows: 34 us of 326).  The form is a template argument of
+// the kernels on the tiled copy: a branch on it around every store costs 5 to 8 % of a launch, one per column far more (the
+// accumulators leave the registers).
+__device__ __forceinline__ void store_y(half_t* y, float v) { *y = (half_t)v; }
+__device__ __forceinline__ void store_y(float* y, float v) { *y = (float)(half_t)v; }
 
 // One launch covers every member of a group: workgroup b serves member i for blk_end[i-1] <= b < blk_end[i].
 struct GemmGroup {
@@ -550,7 +557,7 @@ constexpr int kTRow = 256;  // bytes of a staged row: 128 halves, swizzled inste
 // of their own, and the two accumulator sets meet in LDS before the epilogue.  For launches with about one tile per
 // compute unit: a SIMD then holds two waves of the one workgroup it has, instead of one wave with nothing to overlap its
 // waits with, and the K loop of a tile takes half as many steps.
-template <int kMT, int kNT, int kWk>
+template <int kMT, int kNT, int kWk, typename YT>
 __global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : 2), (kMT * kNT >= 16 ? 1 : 8))))
 void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   int wg = (int)blockIdx.x, slice = (int)blockIdx.y, nslices = gg.slices, part_tile = (int)blockIdx.x, part_tiles = (int)gridDim.x;
@@ -864,7 +871,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int m = m0 + tm * 32 + 8 * (i >> 2) + 4 * lh + (i & 3);
-        if (m < a.M) a.y[(size_t)m * a.ldy + n] = (half_t)(acc[tm][tn][i] + b);
+        if (m < a.M) store_y(reinterpret_cast<YT*>(a.y) + (size_t)m * a.ldy + n, acc[tm][tn][i] + b);
       }
     }
   }
@@ -874,7 +881,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
 // in x, same workgroup -> (member, row block, column block) map and accumulator-register order as the producer.
 // gridDim.y = kMT * kNT: workgroup y of a tile sums one 32 x 32 accumulator tile of each wave (a tile per workgroup
 // left the sum of 64 tail tiles to 64 workgroups: 20 us for 34 MB).
-template <int kMT, int kNT>
+template <int kMT, int kNT, typename YT>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmGroup gg, const int m_blocks) {
   // uniform split: one workgroup per tile of the producer; tail split: one per tail tile (tiles full, full + 1, ...)
   const bool tail = gg.tail_slices > 1;
@@ -908,19 +915,19 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmGroup gg, co
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int m = m0 + tm * 32 + 8 * (i >> 2) + 4 * lh + (i & 3);
-        if (m < a.M && n < a.N) a.y[(size_t)m * a.ldy + n] = (half_t)(v[i] + b);
+        if (m < a.M && n < a.N) store_y(reinterpret_cast<YT*>(a.y) + (size_t)m * a.ldy + n, v[i] + b);
       }
     }
   }
 }
 
 // ---- host side ------------------------------------------------------------------------------------
-template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1>
+template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1, typename YT = half_t>
 static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   static_assert(!kTiled || (kQuant && kSuper), "the tiled copy serves the super-block form");
-  static_assert(kWk == 1 || kTiled, "K groups inside a workgroup: the tiled-copy kernel");
+  static_assert(kTiled || (kWk == 1 && std::is_same_v<YT, half_t>), "K groups inside a workgroup and fp32 outputs: the tiled-copy kernel");
   constexpr int BM = 32 * kMT, BN = 128 * kNT;
-  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
+  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk, YT> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
   size_t lds = kTiled ? (size_t)kWk * 2 * BM * kTRow
                       : (size_t)2 * BM * kARow * sizeof(half_t) + (kSuper ? (size_t)4 * (32 * kNT) * 144 : 0);
   if (kWk > 1 && lds < (size_t)BM * BN * sizeof(float)) lds = (size_t)BM * BN * sizeof(float);  // the hand-over of the accumulators
@@ -939,12 +946,12 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
     const int tail_tiles = total - gg.full;
     hipLaunchKernelGGL(kern, dim3(gg.full + tail_tiles * gg.tail_slices, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT>), dim3(tail_tiles, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
+    hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(tail_tiles, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(kern, dim3(total, gg.slices), dim3(256 * kWk), lds, stream, gg, m_blocks);
   if (hipError_t e = hipGetLastError(); e != hipSuccess || gg.slices == 1) return e;
-  hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT>), dim3(total, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
+  hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(total, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
   return hipGetLastError();
 }
 
@@ -992,7 +999,27 @@ static float gemm_cost(const GemmGroup& gg, const GemmCost& c, int slices, int t
   return us;
 }
 
-static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes, hipStream_t stream) {
+// the super-block form: addresses its operands with 32-bit byte offsets
+static bool gemm_super_form(const GemmGroup& gg) {
+  static const int env_super = getenv("GLOWQ_GEMM_SUPER") ? atoi(getenv("GLOWQ_GEMM_SUPER")) : 1;
+  bool fits32 = (size_t)gg.m[0].M * gg.m[0].K * 2 < (1ull << 32);
+  for (int i = 0; i < gg.n; ++i) {
+    const size_t rows = (size_t)gg.m[i].N;
+    fits32 = fits32 && rows * gg.m[i].ldw * 4 < (1ull << 32) && rows * gg.m[i].lds * 2 < (1ull << 32) && rows * gg.m[i].ldz * 4 < (1ull << 32);
+  }
+  return env_super != 0 && (gg.m[0].K & 255) == 0 && gg.m[0].group_size >= 128 && fits32;
+}
+
+// the tiled copy of the weights where every member brings one (and its tiled left factor where it is corrected)
+static bool gemm_tiled_form(const GemmGroup& gg) {
+  static const int env_tiled = getenv("GLOWQ_GEMM_TILED") ? atoi(getenv("GLOWQ_GEMM_TILED")) : 1;
+  bool ok = gemm_super_form(gg) && env_tiled != 0 && tiled::applies(gg.m[0].K, gg.m[0].group_size);
+  for (int i = 0; i < gg.n; ++i)
+    ok = ok && gg.m[i].wt != nullptr && (gg.m[i].r == nullptr || gg.m[i].lt != nullptr) && tiled::weight_bytes(gg.m[i].N, gg.m[i].K) < (1ull << 32);
+  return ok;
+}
+
+static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes, bool y32, hipStream_t stream) {
   // Tile choice: the largest tile (most reuse of both operands) whose workgroup count still fills the chip; when
   // none does, the one with the most workgroups.  Row tiles are capped by M (and at 4: 8 spills), column tiles at
   // 2 per wave unless every member is narrow.
@@ -1027,20 +1054,8 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   static const int force_nt = getenv("GLOWQ_GEMM_FORCE_NT") ? atoi(getenv("GLOWQ_GEMM_FORCE_NT")) : 0;
   if (force_mt > 0 && force_mt <= mt_cap) mt = force_mt;
   if (force_nt > 0 && force_nt <= nt_cap) nt = force_nt;
-  static const int env_super = getenv("GLOWQ_GEMM_SUPER") ? atoi(getenv("GLOWQ_GEMM_SUPER")) : 1;
-  // the super-block form addresses its operands with 32-bit byte offsets
-  bool fits32 = (size_t)M * gg.m[0].K * 2 < (1ull << 32);
-  for (int i = 0; i < gg.n; ++i) {
-    const size_t rows = (size_t)gg.m[i].N;
-    fits32 = fits32 && rows * gg.m[i].ldw * 4 < (1ull << 32) && rows * gg.m[i].lds * 2 < (1ull << 32) && rows * gg.m[i].ldz * 4 < (1ull << 32);
-  }
-  const bool super = env_super != 0 && (gg.m[0].K & 255) == 0 && gg.m[0].group_size >= 128 && fits32;
-  // the tiled copy of the weights where every member brings one (and its tiled left factor where it is corrected)
-  static const int env_tiled = getenv("GLOWQ_GEMM_TILED") ? atoi(getenv("GLOWQ_GEMM_TILED")) : 1;
-  bool tiled_ok = super && env_tiled != 0 && tiled::applies(gg.m[0].K, gg.m[0].group_size);
-  for (int i = 0; i < gg.n; ++i)
-    tiled_ok = tiled_ok && gg.m[i].wt != nullptr && (gg.m[i].r == nullptr || gg.m[i].lt != nullptr) &&
-               tiled::weight_bytes(gg.m[i].N, gg.m[i].K) < (1ull << 32);
+  const bool super = gemm_super_form(gg);
+  const bool tiled_ok = gemm_tiled_form(gg);
   // About one 128 x 256 tile per compute unit and a long K (where K would otherwise be cut into slices over workgroups,
   // with fp32 partial tiles through the workspace and a second launch for their sum): eight waves per tile, the K range
   // dealt to two groups of four inside the workgroup (gemm_tiled_kernel's kWk = 2), the sum in LDS.  Qwen2.5-7B down_proj at
@@ -1145,12 +1160,16 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
       }
     }
   }
-  if (wk == 2) return mt == 2 ? launch_gemm_t<2, 1, true, true, true, 2>(gg, stream) : launch_gemm_t<4, 2, true, true, true, 2>(gg, stream);
+#define GLOWQ_GEMM_TILED_CASE(MT, NT, WK)                                                  \
+  if (tiled_ok && mt == MT && nt == NT && wk == WK)                                        \
+    return y32 ? launch_gemm_t<MT, NT, true, true, true, WK, float>(gg, stream) : launch_gemm_t<MT, NT, true, true, true, WK>(gg, stream);
+  GLOWQ_GEMM_TILED_CASE(8, 2, 1) GLOWQ_GEMM_TILED_CASE(4, 2, 1) GLOWQ_GEMM_TILED_CASE(2, 2, 1) GLOWQ_GEMM_TILED_CASE(1, 2, 1)
+  GLOWQ_GEMM_TILED_CASE(8, 1, 1) GLOWQ_GEMM_TILED_CASE(4, 1, 1) GLOWQ_GEMM_TILED_CASE(2, 1, 1) GLOWQ_GEMM_TILED_CASE(1, 1, 1)
+  GLOWQ_GEMM_TILED_CASE(4, 2, 2) GLOWQ_GEMM_TILED_CASE(2, 1, 2)
+#undef GLOWQ_GEMM_TILED_CASE
+  if (y32) return hipErrorInvalidValue;  // (gemm_widens said no)
 #define GLOWQ_GEMM_CASE(MT, NT)                                                            \
-  if (mt == MT && nt == NT)                                                                \
-    return tiled_ok ? launch_gemm_t<MT, NT, true, true, true>(gg, stream)                  \
-           : super  ? launch_gemm_t<MT, NT, true, true>(gg, stream)                        \
-                    : launch_gemm_t<MT, NT, true>(gg, stream);
+  if (mt == MT && nt == NT) return super ? launch_gemm_t<MT, NT, true, true>(gg, stream) : launch_gemm_t<MT, NT, true>(gg, stream);
   GLOWQ_GEMM_CASE(8, 2) GLOWQ_GEMM_CASE(4, 2) GLOWQ_GEMM_CASE(2, 2) GLOWQ_GEMM_CASE(1, 2)
   GLOWQ_GEMM_CASE(8, 1) GLOWQ_GEMM_CASE(4, 1) GLOWQ_GEMM_CASE(2, 1) GLOWQ_GEMM_CASE(1, 1)
 #undef GLOWQ_GEMM_CASE
@@ -1174,14 +1193,13 @@ bool gemm_supported(const GroupDev& g) {
   return true;
 }
 
-hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
-  GemmGroup gg;
+static void fill_gemm_group(const GroupDev& g, GemmGroup& gg) {
   gg.n = g.n_members;
   for (int i = 0; i < g.n_members; ++i) {
     const MemberDev& m = g.mem[i];
     GemmArgs& a = gg.m[i];
     a.x = g.x;
-    a.r = (m.L != nullptr) ? g.r : nullptr;
+    a.r = (m.L != nullptr) ? (g.r != nullptr ? g.r : g.r_out) : nullptr;  // (given, or produced by the launch ahead)
     a.qweight = m.qweight;
     a.scales = m.scales;
     a.qzeros = m.qzeros;
@@ -1202,6 +1220,20 @@ hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
     a.ldy = m.ldy;
     a.alpha = g.alpha;
   }
+}
+
+// whether a call can have fp32 outputs: the kernels on the tiled copy have them
+bool gemm_widens(const GroupDev& g) {
+  GemmGroup gg;
+  fill_gemm_group(g, gg);
+  for (int i = 1; i < g.n_members; ++i)
+    if ((g.mem[i].y32 != 0) != (g.mem[0].y32 != 0)) return false;
+  return gemm_supported(g) && gemm_tiled_form(gg);
+}
+
+hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
+  GemmGroup gg;
+  fill_gemm_group(g, gg);
   // slices of the padded output (rows to a multiple of 128, columns of every member to a multiple of 256) that fit the
   // workspace; launch_gemm_group turns this into the slice count
   size_t padded = 0;
@@ -1209,7 +1241,7 @@ hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
   const bool ws_ok = g.ws != nullptr && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0;
   gg.slices = ws_ok ? (int)std::min<size_t>(g.ws_bytes / (padded * sizeof(float)), 64) : 0;
   gg.partials = static_cast<float*>(g.ws);
-  return launch_gemm_group(gg, num_cus, ws_ok ? g.ws_bytes : 0, stream);
+  return launch_gemm_group(gg, num_cus, ws_ok ? g.ws_bytes : 0, g.mem[0].y32 != 0, stream);
 }
 
 // ---- shared projection for many rows: r[M, rank] = fp16(x[M, K] . R[rank, K]^T) ---------------------------

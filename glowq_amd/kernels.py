@@ -36,8 +36,13 @@ class _Member(ctypes.Structure):
         ("qweight", _P), ("scales", _P), ("qzeros", _P), ("L", _P), ("bias", _P), ("y", _P),
         ("N", ctypes.c_int32), ("ldw_i32", ctypes.c_int32), ("lds", ctypes.c_int32),
         ("ldz_i32", ctypes.c_int32), ("ldy", ctypes.c_int32), ("side_rank", ctypes.c_int32),
-        ("side", _P), ("tiled", _P), ("tiled_L", _P), ("tiled_rank", ctypes.c_int32), ("reserved", ctypes.c_int32),
+        ("side", _P), ("tiled", _P), ("tiled_L", _P), ("tiled_rank", ctypes.c_int32), ("y_type", ctypes.c_int32),
     ]
+
+
+Y_FP32 = 0x32335946   # y_type of a member whose output is fp32 (GLOWQ_Y_FP32)
+EUNSUPPORTED = -4
+GEMM_MIN_ROWS = 65    # from here on the GEMM takes a call whose layout it supports
 
 
 class _Chain(ctypes.Structure):
@@ -688,10 +693,11 @@ class PreparedGroup:
         self._n_total = sum(self.Ns)
 
     def run(self, x: torch.Tensor, r: Optional[torch.Tensor] = None, outs: Optional[List[torch.Tensor]] = None,
-            project: bool = True) -> List[torch.Tensor]:
+            project: bool = True, out_dtype: torch.dtype = torch.float16) -> List[torch.Tensor]:
         """x [M, K] contiguous fp16 on the group's device.  With a right factor and `project`, r = x R^T is computed by
         the call (into `r`, allocated when not given, and kept as `self.last_r`); otherwise `r` is an input (needed when
-        the group is corrected).  Returns the members' [M, N_i] outputs (`outs` when given)."""
+        the group is corrected).  Returns the members' [M, N_i] outputs (`outs` when given).  `out_dtype` fp32: the GEMM
+        writes its fp16 results widened; a call that another kernel takes still returns fp16."""
         if not (x.is_cuda and x.dtype is torch.float16 and x.dim() == 2 and x.size(1) == self.K and x.is_contiguous()):
             raise RuntimeError("inputs must be contiguous CUDA fp16 [M, IC]")
         M = x.size(0)
@@ -701,8 +707,9 @@ class PreparedGroup:
             self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
                                 for e, k in zip(self.arr, self.keep)]
         Ns = self.Ns
+        widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:
-            outs = [torch.empty((M, N), dtype=torch.float16, device=dev) for N in Ns]
+            outs = [torch.empty((M, N), dtype=torch.float32 if widen else torch.float16, device=dev) for N in Ns]
             for e, y in zip(self.arr, outs):
                 e.y, e.ldy = y.data_ptr(), y.stride(0)
         else:
@@ -729,6 +736,9 @@ class PreparedGroup:
         try:
             ws, ws_bytes = ext._workspace(dev, M)
             stream = ext._stream(dev)
+            if widen:
+                for e in self.arr:
+                    e.y_type = Y_FP32
             if fused:
                 rc = self.lib.glowq_w4a16_group_forward_fused_ws(
                     x.data_ptr(), self.R.data_ptr(), r.data_ptr(), self.arr, len(Ns), M, self.K, self.group_size,
@@ -738,8 +748,13 @@ class PreparedGroup:
                     x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, self.arr, len(Ns), M,
                     self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
         finally:
+            if widen:
+                for e in self.arr:
+                    e.y_type = 0
             if ctx is not None:
                 ctx.__exit__(None, None, None)
+        if rc == EUNSUPPORTED and widen:  # not the GEMM's call: nothing has been launched
+            return self.run(x, r=r, project=project)
         if rc:
             ext._raise(rc, "w4a16_group_forward")
         return outs

@@ -262,7 +262,7 @@ class CudaW4A16Linear(nn.Module):
         # Through descriptors validated once (the bias rides in the kernel's epilogue).  From 65 rows this is the same MFMA
         # GEMM as the entry point above, but on the tiled copy of the weights and with the stream's workspace for its splits
         # of K: two 14B layers with half of their groups bare at 1500 rows 2362 -> 2048 us.
-        return self._finish(self._bare_group().run(x2d)[0], lead, bias_applied=KNOBS.out_dtype == torch.float16)
+        return self._finish(self._bare_group().run(x2d, out_dtype=KNOBS.out_dtype)[0], lead, bias_applied=KNOBS.out_dtype == torch.float16)
 
     def dequantize(self) -> torch.Tensor:
         """fp16 [out_features, in_features] weight, fp16((code - zero) * scale); the device twin of the

@@ -55,8 +55,11 @@ typedef struct glowq_member {
   const void* tiled;      /* the member's tiled weights written by glowq_pack_tiled for this K and group_size, or NULL */
   const void* tiled_L;    /* its tiled left factor written by glowq_pack_tiled_left for tiled_rank, or NULL */
   int32_t tiled_rank;
-  int32_t reserved;
+  int32_t y_type;         /* GLOWQ_Y_FP32: y is [M, N] fp32 and receives the fp16 result widened; only calls that
+                             the GEMM takes (65 token rows and more) with the tiled weights given, and all members alike; others
+                             are refused with GLOWQ_EUNSUPPORTED.  Any other value: fp16 */
 } glowq_member_t;
+#define GLOWQ_Y_FP32 0x32335946
 
 /* Library / device information. */
 int glowq_version(void);

@@ -218,3 +218,23 @@ def test_bare_linear_around_the_gemm_threshold(fp16_out, monkeypatch, rows, K, N
     y32 = mod(x.cuda())
     assert y32.dtype == torch.float32
     assert_close(y32.cpu().numpy(), want, f"{rows} rows, fp32")
+
+
+@pytest.mark.parametrize("rows", [5, 64, 65, 129, 300])
+@pytest.mark.parametrize("K,Ns,gs", [(512, (96, 40), 128), (4096, (256, 130), 128), (200, (37,), 40)])  # tiled, split over K, generic
+def test_fp32_outputs_are_the_fp16_results_widened(monkeypatch, rows, K, Ns, gs):
+    torch.manual_seed(rows)
+    mods = []
+    cache = corr.MiniGroupCache()
+    R = (torch.randn(32, K) * K ** -0.5).half().cuda()
+    for N, role in zip(Ns, ("gate", "up")):
+        inner = linear.CudaW4A16Linear.from_float(nn.Linear(K, N, bias=True).half(), gs).cuda()
+        mods.append(corr.AddSVDCorrection(inner, (torch.randn(N, 32) * 0.01).half().cuda(), R, role, True, cache, 1.0))
+    x = torch.randn(rows, K).half().cuda()
+    got = {}
+    for dtype in ("fp16", "fp32"):
+        monkeypatch.setenv("W4A16_KERNEL_OUT_DTYPE", dtype)
+        got[dtype] = [m(x) for m in mods]
+    for a, b in zip(got["fp16"], got["fp32"]):
+        assert a.dtype == torch.float16 and b.dtype == torch.float32
+        assert torch.equal(a.float(), b)
