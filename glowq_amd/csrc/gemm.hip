@@ -861,6 +861,25 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
         for (int i = 0; i < 16; ++i) part[((tm * kNT + tn) * 16 + i) * 256 + tid] = acc[tm][tn][i];
     return;
   }
+  if (m0 + BM <= a.M && (bn + 1) * BN <= a.N) {
+    // A tile inside the output: no test per element, and a row's address is a scalar base plus one lane offset for all of them.
+    // With a test and a 64-bit address per element the 32 kMT kNT stores of a wave are some twelve instructions each, 3 to 6 us of
+    // a tile that takes 50 (Qwen2.5-7B layer at 2048 rows 965 -> 928 us, 8B o_proj at 2048 rows 74.5 -> 69.5).
+    YT* corner = reinterpret_cast<YT*>(a.y) + (size_t)m0 * a.ldy + (bn * BN + wave * (32 * kNT));
+    const uint32_t lane_off = (uint32_t)(4 * lh) * (uint32_t)a.ldy + (uint32_t)ln;
+    float b[kNT];
+#pragma unroll
+    for (int tn = 0; tn < kNT; ++tn) b[tn] = a.bias ? (float)a.bias[bn * BN + wave * (32 * kNT) + tn * 32 + ln] : 0.f;
+#pragma unroll
+    for (int tm = 0; tm < kMT; ++tm)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        YT* row = corner + (size_t)(tm * 32 + 8 * (i >> 2) + (i & 3)) * a.ldy;
+#pragma unroll
+        for (int tn = 0; tn < kNT; ++tn) store_y(row + tn * 32 + lane_off, acc[tm][tn][i] + b[tn]);
+      }
+    return;
+  }
 #pragma unroll
   for (int tn = 0; tn < kNT; ++tn) {
     const int n = bn * BN + wave * (32 * kNT) + tn * 32 + ln;
