@@ -989,33 +989,33 @@ constexpr GemmCost kGemmCost[] = {
     {2, 2, 1, 2.9f, 3.3f, 0.90f, 0.77f, 1.6f, 0.29f, 0.52f}, {4, 1, 1, 3.1f, 2.8f, 1.00f, 0.73f, 1.9f, 0.24f, 0.59f},
     {4, 2, 1, 5.0f, 4.0f, 1.43f, 1.27f, 1.1f, 0.23f, 0.58f}, {4, 2, 2, 6.0f, 5.5f, 2.46f, 3.10f, 1.3f, 0.25f, 0.92f}};
 
-static long gemm_tiles(const GemmGroup& gg, int mt, int nt) {
-  long tiles = 0;
-  for (int i = 0; i < gg.n; ++i) tiles += (long)((gg.m[0].M + 32 * mt - 1) / (32 * mt)) * ((gg.m[i].N + 128 * nt - 1) / (128 * nt));
-  return tiles;
+static int gemm_tiles(const GemmGroup& gg, int mt, int nt) {
+  int cols = 0;
+  for (int i = 0; i < gg.n; ++i) cols += (gg.m[i].N + 128 * nt - 1) / (128 * nt);
+  return (gg.m[0].M + 32 * mt - 1) / (32 * mt) * cols;
+}
+
+// The part of a launch's cost that no cut changes needs the group; the rest needs its tiles.  (Calls from Python are often bound by
+// the host: the rule looks at some forty cuts in under a microsecond.)
+static float gemm_cost_fixed(const GemmGroup& gg, const GemmCost& c) {
+  int rank = 0;
+  float cols = 0.f;
+  for (int i = 0; i < gg.n; ++i) {
+    if (gg.m[i].r != nullptr) rank = gg.m[i].rank;
+    cols += (float)gg.m[i].N;
+  }
+  return c.fixed + c.rank_block * (float)((rank + 127) / 128) + c.output_mb * cols * (float)gg.m[0].M * 2e-6f;
 }
 
 // `tail_slices` > 1: the tiles past the last multiple of the compute-unit count are cut into that many (slices is then 1)
-static float gemm_cost(const GemmGroup& gg, const GemmCost& c, int slices, int tail_slices, int num_cus) {
-  const int sb = gg.m[0].K >> 8;
-  const long tiles = gemm_tiles(gg, c.mt, c.nt);
-  const auto half_steps = [&](int s) { return (float)(2 * ((((sb + s - 1) / s) + c.wk - 1) / c.wk)); };
+static float gemm_cost_cut(const GemmCost& c, int tiles, int sb, int slices, int tail_slices, int num_cus) {
+  const auto half_steps = [&](int s) { return (float)(2 * (((sb + s - 1) / s + c.wk - 1) / c.wk)); };
   const float tile_mb = (float)(32 * c.mt) * (128 * c.nt) * 4e-6f;
-  int rank = 0;
-  float out_mb = 0.f;
-  for (int i = 0; i < gg.n; ++i) {
-    if (gg.m[i].r != nullptr) rank = gg.m[i].rank;
-    out_mb += (float)gg.m[i].N * (float)gg.m[i].M * 2e-6f;
-  }
-  float us = c.fixed + c.rank_block * (float)((rank + 127) / 128) + c.output_mb * out_mb;
-  if (tail_slices > 1) {
-    const long tail = tiles % num_cus;
-    return us + half_steps(1) * (c.step + (float)(tiles / num_cus - 1) * c.step_more) + half_steps(tail_slices) * c.step_more + c.reduce +
-           c.partial_mb * tile_mb * (float)(tail * tail_slices);
-  }
-  us += half_steps(slices) * (c.step + (float)((tiles * slices + num_cus - 1) / num_cus - 1) * c.step_more);
-  if (slices > 1) us += c.reduce + c.partial_mb * tile_mb * (float)(tiles * slices);
-  return us;
+  if (tail_slices > 1)
+    return half_steps(1) * (c.step + (float)(tiles / num_cus - 1) * c.step_more) + half_steps(tail_slices) * c.step_more + c.reduce +
+           c.partial_mb * tile_mb * (float)(tiles % num_cus * tail_slices);
+  const float us = half_steps(slices) * (c.step + (float)((tiles * slices + num_cus - 1) / num_cus - 1) * c.step_more);
+  return slices > 1 ? us + c.reduce + c.partial_mb * tile_mb * (float)(tiles * slices) : us;
 }
 
 // the super-block form: addresses its operands with 32-bit byte offsets
@@ -1153,29 +1153,31 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   // send more than 32 MB of fp32 tiles through the workspace are not tried: there the fit is off by up to 15 % (1B fc2 at 1500
   // rows in five slices 70.6 us against 65.1 in two).
   if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
+    const int sb_total = gg.m[0].K >> 8;
     float best_us = 0.f;
     for (const GemmCost& c : kGemmCost)
-      if (c.mt == mt && c.nt == nt && c.wk == wk) best_us = 0.91f * gemm_cost(gg, c, gg.slices, gg.tail_slices, num_cus);
-    static const int tried[4][3] = {{1, 1, 1}, {2, 1, 1}, {2, 1, 2}, {4, 2, 1}};
-    const int sb_total = gg.m[0].K >> 8;
-    for (const auto& t : tried) {
-      for (const GemmCost& c : kGemmCost) {
-        if (c.mt != t[0] || c.nt != t[1] || c.wk != t[2]) continue;
-        const long tiles = gemm_tiles(gg, c.mt, c.nt);
-        for (int s = 1; s <= 16 && s * 2 <= std::max(sb_total, 2); ++s) {  // two super-blocks and more to a slice, three rounds at most
-          const int per = (sb_total + s - 1) / s;
-          if ((sb_total + per - 1) / per != s) continue;  // a slice without super-blocks
-          const size_t partial_bytes = (size_t)(tiles * s) * (32 * c.mt) * (128 * c.nt) * sizeof(float);
-          if (s > 1 && (env_split == 0 || tiles * s > 3L * num_cus || partial_bytes > std::min(ws_bytes, (size_t)32 << 20))) break;
-          const float us = gemm_cost(gg, c, s, 0, num_cus);
-          if (us >= best_us) continue;
-          best_us = us;
-          mt = c.mt;
-          nt = c.nt;
-          wk = c.wk;
-          gg.slices = s;
-          gg.full = gg.tail_slices = 0;
-        }
+      if (c.mt == mt && c.nt == nt && c.wk == wk)
+        best_us = 0.91f * (gemm_cost_fixed(gg, c) + gemm_cost_cut(c, gemm_tiles(gg, mt, nt), sb_total, gg.slices, gg.tail_slices, num_cus));
+    // a second launch where there was none also takes the host's time, which calls from Python at the small end wait for
+    const float second = gg.slices > 1 || gg.tail_slices > 1 ? 0.f : 1.5f;
+    for (const GemmCost& c : kGemmCost) {
+      if (!((c.nt == 1 && c.mt <= 2) || (c.mt == 4 && c.nt == 2 && c.wk == 1))) continue;  // <1,1,1>, <2,1,1>, <2,1,2>, <4,2,1>
+      const int tiles = gemm_tiles(gg, c.mt, c.nt);
+      const float fixed = gemm_cost_fixed(gg, c);
+      if (tiles > 64 * num_cus) continue;
+      for (int s = 1; s <= 16 && s * 2 <= std::max(sb_total, 2); ++s) {  // two super-blocks and more to a slice, three rounds at most
+        const size_t partial_bytes = (size_t)(tiles * s) * (32 * c.mt) * (128 * c.nt) * sizeof(float);
+        if (s > 1 && (env_split == 0 || tiles * s > 3 * num_cus || partial_bytes > std::min(ws_bytes, (size_t)32 << 20))) break;
+        const int per = (sb_total + s - 1) / s;
+        if ((sb_total + per - 1) / per != s) continue;  // a slice without super-blocks
+        const float us = fixed + gemm_cost_cut(c, tiles, sb_total, s, 0, num_cus) + (s > 1 ? second : 0.f);
+        if (us >= best_us) continue;
+        best_us = us;
+        mt = c.mt;
+        nt = c.nt;
+        wk = c.wk;
+        gg.slices = s;
+        gg.full = gg.tail_slices = 0;
       }
     }
   }
@@ -1623,17 +1625,19 @@ static ProjTilePlan plan_proj_tile(const ProjPlan& p, int M, int K, int rank, in
   best *= 0.93f;
   ProjTilePlan plan = {0, 1};
   for (int a = 1; a <= 2; ++a) {
-    const long tiles = (long)((M + 64 * a - 1) / (64 * a)) * ((rank + 64 * a - 1) / (64 * a));
-    for (int s = 1; s <= 32 && s <= stages && tiles * s <= 4L * num_cus; ++s) {
+    const long row_tiles = (M + 64 * a - 1) / (64 * a), col_tiles = (rank + 64 * a - 1) / (64 * a);
+    if (row_tiles * col_tiles > 4L * num_cus) continue;
+    const int tiles = (int)(row_tiles * col_tiles);
+    for (const int s : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32}) {
+      if (s > stages || tiles * s > 4 * num_cus || (s > 1 && (size_t)s * M * rank * sizeof(float) > ws_bytes)) break;
       const int depth = (stages + s - 1) / s;
-      if ((stages + depth - 1) / depth != s) continue;  // a slice without stages
-      if (s > 1 && (size_t)s * M * rank * sizeof(float) > ws_bytes) break;
       float us = (a == 1 ? 2.1f : 5.4f) + (float)depth * ((a == 1 ? 0.62f : 1.05f) + (a == 1 ? 0.29f : 1.66f) * rounds_more(tiles * s)) +
                  0.07f * (float)M * (float)K * 2e-6f;
       if (s > 1) us += 2.5f + (a == 1 ? 0.074f : 0.043f) * (float)s + (a == 1 ? 0.56f : 0.43f) * slice_mb * (float)s;
+      if (s > 1 && p.slices == 1) us += 1.5f;  // a second launch where there was none also takes the host's time
       if (us >= best) continue;
       best = us;
-      plan = {a, s};
+      plan = {a, (stages + depth - 1) / depth};  // no slice without stages
     }
   }
   return plan;
