@@ -41,8 +41,10 @@ __device__ __forceinline__ float block_max(float v, float* red, int nwaves) {
 }  // namespace
 
 // x_out[m] = fp16(x[m] + delta[m]) (when delta != nullptr; x_out may be x), h[m] = fp16(x_out[m] * rsqrt(mean(x_out[m]^2) +
-// eps) * w), one workgroup per token row, statistics in fp32.  Many rows: bound by its 2 to 4 passes over [M, H] fp16 (512 rows
+// eps) * w), one workgroup per token row, statistics in fp32.  kOnce: the product is rounded once, as torch's rms_norm does, not
+// also before the weight (the decode step's norm, which follows the Llama module).  Many rows: bound by its 2 to 4 passes over [M, H] fp16 (512 rows
 // of 4096: 4.8 us with the add, where the two launches of the tensor expressions take 4.7 + 6.2).
+template <bool kOnce>
 __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(const half_t* x, const half_t* __restrict__ delta,
                                                             const half_t* __restrict__ w, half_t* x_out,
                                                             half_t* __restrict__ h, int H, float eps) {
@@ -70,7 +72,10 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(const half_t* x, cons
     const h8 ww = *reinterpret_cast<const h8*>(w + i);
     h8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)(half_t)((float)v[j] * inv) * (float)ww[j]);
+    for (int j = 0; j < 8; ++j) {
+      const float n = (float)v[j] * inv;
+      o[j] = (half_t)((kOnce ? n : (float)(half_t)n) * (float)ww[j]);
+    }
     *reinterpret_cast<h8*>(hr + i) = o;
   }
 }
@@ -645,11 +650,12 @@ __global__ __launch_bounds__(1024) void argmax_advance_kernel(const half_t* __re
 
 // ---- launchers ------------------------------------------------------------------------------
 hipError_t launch_add_rmsnorm(const half_t* x, const half_t* delta, const half_t* w, half_t* x_out, half_t* h, int M, int H, float eps,
-                              hipStream_t stream) {
+                              bool once, hipStream_t stream) {
   int threads = ((H / 8 + 63) / 64) * 64;
   if (threads > 1024) threads = 1024;
   if (threads < 64) threads = 64;
-  hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(M), dim3(threads), 0, stream, x, delta, w, x_out, h, H, eps);
+  auto kern = once ? add_rmsnorm_kernel<true> : add_rmsnorm_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(M), dim3(threads), 0, stream, x, delta, w, x_out, h, H, eps);
   return hipGetLastError();
 }
 
@@ -757,16 +763,25 @@ using namespace glowq;
 
 extern "C" {
 
-int glowq_add_rmsnorm_out(const void* x, const void* delta, const void* weight, void* x_out, void* h, int M, int H, float eps, void* stream) {
+}  // extern "C"
+
+static int add_rmsnorm_impl(const void* x, const void* delta, const void* weight, void* x_out, void* h, int M, int H, float eps, bool once,
+                            void* stream) {
   if (!x || !weight || !h || (delta && !x_out)) return fail(GLOWQ_EINVAL, "add_rmsnorm: x, weight, h and, with delta, x_out must be device pointers");
   if (M <= 0 || H <= 0 || (H & 7)) return fail(GLOWQ_EINVAL, "add_rmsnorm: M > 0 and H a positive multiple of 8 (got M=%d, H=%d)", M, H);
   hipError_t e = launch_add_rmsnorm(static_cast<const half_t*>(x), static_cast<const half_t*>(delta), static_cast<const half_t*>(weight),
-                                    static_cast<half_t*>(x_out), static_cast<half_t*>(h), M, H, eps, static_cast<hipStream_t>(stream));
+                                    static_cast<half_t*>(x_out), static_cast<half_t*>(h), M, H, eps, once, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? GLOWQ_OK : fail(GLOWQ_ELAUNCH, "add_rmsnorm launch failed: %s", hipGetErrorString(e));
 }
 
+extern "C" {
+
+int glowq_add_rmsnorm_out(const void* x, const void* delta, const void* weight, void* x_out, void* h, int M, int H, float eps, void* stream) {
+  return add_rmsnorm_impl(x, delta, weight, x_out, h, M, H, eps, true, stream);
+}
+
 int glowq_add_rmsnorm(void* x, const void* delta, const void* weight, void* h, int M, int H, float eps, void* stream) {
-  return glowq_add_rmsnorm_out(x, delta, weight, x, h, M, H, eps, stream);
+  return add_rmsnorm_impl(x, delta, weight, x, h, M, H, eps, false, stream);
 }
 
 int glowq_rope_append(const void* q, const void* k, const void* v, const void* cos_rows, const void* sin_rows, const int64_t* pos, void* q_out,

@@ -10,8 +10,9 @@ src/step2_rsvd.py:487-527 for the low-rank factors.
 
     python -m glowq_amd.decode --layers 32 --prompt 512 --new 256        # Llama-3.1-8B shape, batch 1
 
-Two ways to run a token: the module path (`Decoder.forward_tokens`: the patched linears inside plain torch norms, RoPE
-and attention; used for prefill and as the yardstick) and `FusedStep` (single-token decode as a fixed chain of this
+Two ways to run a token: the module path (`Decoder.forward_tokens`: the patched linears with, for several token rows, the
+library's norm, rotary / cache append and gate kernels around torch's attention -- tensor expressions where gradients,
+tracing or other types ask for them, and for a single token, where they are the yardstick) and `FusedStep` (single-token decode as a fixed chain of this
 library's launches: add+RMSNorm, group linears, RoPE+cache append+attention, SwiGLU gating, greedy pick; only the
 lm_head matmul and the embedding lookup stay torch ops).
 """
@@ -85,7 +86,7 @@ class RMSNorm(nn.Module):
             x.add_(delta)
         if self._takes_rows(x):
             h = torch.empty_like(x)
-            load_w4a16_extension().add_rmsnorm(x, None, self.weight, h, self.eps)
+            load_w4a16_extension().add_rmsnorm_out(x, None, self.weight, None, h, self.eps)
             return h
         return F.rms_norm(x, (x.size(-1),), self.weight, self.eps)
 

@@ -454,14 +454,14 @@ class W4A16Extension:
             self._raise(rc, "add_rmsnorm")
 
     def add_rmsnorm_out(self, x, delta, weight, x_out, h, eps: float) -> None:
-        """x_out = x + delta, h = rmsnorm(x_out) * weight over [M, H] rows, x untouched."""
-        for t, n in ((x, "x"), (delta, "delta"), (weight, "weight"), (x_out, "x_out"), (h, "h")):
+        """x_out = x + delta (both None: no sum), h = rmsnorm(x_out) * weight over [M, H] rows rounded once, x untouched."""
+        for t, n in ((x, "x"), (weight, "weight"), (h, "h")) + (() if delta is None else ((delta, "delta"), (x_out, "x_out"))):
             self._f16(t, n)
-        _check(x.dim() == 2 and delta.shape == x.shape and x_out.shape == x.shape and h.shape == x.shape and weight.numel() == x.size(1),
-               "add_rmsnorm_out: shape mismatch")
+        _check(x.dim() == 2 and (delta is None or (delta.shape == x.shape and x_out.shape == x.shape)) and h.shape == x.shape
+               and weight.numel() == x.size(1), "add_rmsnorm_out: shape mismatch")
         with torch.cuda.device(x.device):
-            rc = self.lib.glowq_add_rmsnorm_out(x.data_ptr(), delta.data_ptr(), weight.data_ptr(), x_out.data_ptr(), h.data_ptr(), x.size(0),
-                                                x.size(1), float(eps), self._stream(x.device))
+            rc = self.lib.glowq_add_rmsnorm_out(x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(),
+                                                None if delta is None else x_out.data_ptr(), h.data_ptr(), x.size(0), x.size(1), float(eps), self._stream(x.device))
         if rc:
             self._raise(rc, "add_rmsnorm_out")
 

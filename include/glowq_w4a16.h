@@ -120,8 +120,9 @@ int glowq_shared_proj(const void* x, const void* R, void* r, int M, int K, int r
  * The same with a caller-provided workspace (same reference lines).  With more than 16 token rows (more than 64, or
  * M * K * rank above 90 million, from where the MFMA projection is used) the output [M, rank] is too small to fill the chip, so K is split over workgroups that leave fp32 partial tiles in `workspace`; a second
  * small launch adds them in slice order (results do not depend on scheduling) and writes r.
- * `workspace`: 16-byte aligned device memory, contents irrelevant; glowq_proj_workspace_bytes gives the size that lets
- * the split go as far as it is useful for a shape -- a smaller one splits less, NULL or 0 bytes is glowq_shared_proj.
+ * `workspace`: 16-byte aligned device memory, contents irrelevant; glowq_proj_workspace_bytes gives the size that the
+ * 32-row tiles split through -- a smaller one splits less, NULL or 0 bytes is glowq_shared_proj.  The tile kernel for many rows
+ * takes up to 32 slices of 4 M rank bytes where a larger one holds them.
  * Calls that share a workspace must not overlap (one workspace per stream).
  */
 int glowq_shared_proj_ws(const void* x, const void* R, void* r, int M, int K, int rank, void* workspace,
@@ -313,7 +314,8 @@ int glowq_set_tuning(const char* key, int value);
 
 /* x[m] += delta[m] (skipped when delta is NULL), h[m] = rmsnorm(x[m]) * weight; x [M, H] is updated in place. */
 int glowq_add_rmsnorm(void* x, const void* delta, const void* weight, void* h, int M, int H, float eps, void* stream);
-/* the same with the sum in x_out (x_out may be x; without delta x_out is not written and may be NULL) */
+/* the same with the sum in x_out (x_out may be x; without delta x_out is not written and may be NULL), and with h rounded once, as
+   torch's rms_norm does, where glowq_add_rmsnorm also rounds before the weight */
 int glowq_add_rmsnorm_out(const void* x, const void* delta, const void* weight, void* x_out, void* h, int M, int H, float eps, void* stream);
 /* T token rows: q_out = rope(q) [T, heads d], k_out = rope(k) [T, kv_heads d], rows pos[t] of the caches [kv_heads, max_len, d] =
    (k_out, v); cos_rows / sin_rows [T, d] fp16 are the tables at the tokens' positions; a position outside the cache writes no row.

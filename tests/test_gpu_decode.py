@@ -621,3 +621,20 @@ def test_norm_hooks_still_see_the_residual_norm(fp16_out):
     with torch.no_grad():
         model.forward_tokens(torch.arange(5, device="cuda"), torch.arange(5, device="cuda"), caches, cos, sin, from_empty_cache=True)
     assert seen == [(torch.Size([5, 256]), torch.Size([5, 256]))]
+
+
+@pytest.mark.parametrize("M,H", [(2, 8), (3, 1544), (130, 4096), (5, 16384)])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_row_norm_rounds_once(fp16_out, M, H, with_delta):
+    """Several rows through the norm: as close to 64 bits as torch's rms_norm, half an fp16 ulp and the fp32 sum of squares."""
+    g = torch.Generator(device="cuda").manual_seed(H)
+    x, d = (torch.randn(M, H, device="cuda", generator=g).half() for _ in range(2))
+    norm = decode.RMSNorm(H, 1e-5).cuda()
+    norm.weight.data.normal_(1.0, 0.2, generator=g)
+    with torch.no_grad():
+        out, h = norm.forward_add(x, d) if with_delta else (x, norm(x))
+    want_x = (x + d) if with_delta else x
+    assert torch.equal(out, want_x)
+    t = want_x.double()
+    want = t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
+    assert ((h.double() - want).abs() <= (2.0 ** -11 + 2.0 ** -20) * want.abs() + 2.0 ** -25).all()
