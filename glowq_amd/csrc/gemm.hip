@@ -1150,8 +1150,8 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   // workgroups made of smaller tiles and slices of K is often the shorter way (8B o_proj at 100 rows 18.4 -> 15.1 us, down_proj
   // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  Over the timings behind kGemmCost this takes
   // 9 % off the mean and costs nowhere more than 1 %; without the margin it costs more than that on 30 pairs of 250.  Cuts that
-  // send more than 32 MB of fp32 tiles through the workspace are not tried: there the fit is off by up to 15 % (1B fc2 at 1500
-  // rows in five slices 70.6 us against 65.1 in two).
+  // send more than 32 MB of fp32 tiles through the workspace are not tried: from there the fit scatters by 7 to 11 %
+  // (standard deviation) instead of 3 to 5.
   if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
     const int sb_total = gg.m[0].K >> 8;
     float best_us = 0.f;
