@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from operator import attrgetter
 from typing import List, Optional, Sequence
 
 import torch
@@ -116,6 +117,23 @@ def tiled_enabled() -> bool:
 # The raw handle of torch's current stream of a device: the accessor behind `torch.cuda.current_stream(dev).cuda_stream`,
 # without building the Stream object (a forward makes this call once).
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda idx: torch.cuda.current_stream(idx).cuda_stream)
+
+
+_version_of = attrgetter("_version")
+
+
+class _Packed:
+    """A packed copy `out` of a few tensors, kept on the first of them.  `key` says what it was made from: addresses and
+    versions (every in-place write through torch raises a tensor's version), so that a write to a source is seen.  Holding the
+    other sources keeps their addresses from being given to new tensors."""
+
+    __slots__ = ("key", "others", "out")
+
+    def __init__(self, key, others, out):
+        self.key, self.others, self.out = key, others, out
+
+    def __reduce__(self):
+        return set, ()  # a deep copy or a saved file of the tensor starts without one
 
 
 def _check(cond: bool, msg: str) -> None:
@@ -273,54 +291,72 @@ class W4A16Extension:
             self._raise(rc, "pack_side")
         return out
 
-    def pack_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[torch.Tensor]:
-        """The tiled copy of a member's weights for the matrix-core routes (a uint8 tensor; layout in csrc/tiled.hpp), or
-        None where the layout does not apply.  Built once per weight tensor and kept on it (`qweight._glowq_tiled`) until
-        the tensor is written to in place; a module moved with `.to()` gets new tensors and with them a new copy."""
+    def _packed_copy(self, sources, shape_key, nbytes: int, pack) -> Optional[_Packed]:
+        """The copy of `sources` kept on the first of them, made by `pack(out, stream)` where there is none or a source has been
+        written to since.  After a write the copy is made again in its old place, so that launches recorded into graphs read
+        the new one too.  None where it would have to be made under a graph capture (it would come from the graph's own memory
+        pool, or be made at every replay)."""
+        owner = sources[0]
+        ptrs, versions = [t.data_ptr() for t in sources], [t._version for t in sources]
+        shape_key += (nbytes,)
+        key = (ptrs, versions, shape_key)
+        hit = getattr(owner, "_glowq_tiled", None)
+        if not isinstance(hit, _Packed):
+            hit = None
+        if hit is not None and hit.key == key:
+            return hit
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        if hit is not None and hit.key[0] == ptrs and hit.key[2] == shape_key:
+            out = hit.out
+        else:
+            out = torch.empty(nbytes, dtype=torch.uint8, device=owner.device)
+        with torch.cuda.device(owner.device):
+            rc = pack(out.data_ptr(), self._stream(owner.device))
+        if rc:
+            self._raise(rc, "pack_tiled")
+        packed = _Packed(key, sources[1:], out)
+        owner._glowq_tiled = packed
+        return packed
+
+    def _packed_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[_Packed]:
         if not tiled_enabled():
             return None
         N = qweight.size(0)
         nbytes = self.lib.glowq_tiled_bytes(N, int(in_features), int(group_size))
         if nbytes == 0 or not qweight.is_cuda:
             return None
-        key = (qweight._version, scales.data_ptr(), scales._version, qzeros.data_ptr(), qzeros._version, int(in_features), int(group_size))
-        hit = getattr(qweight, "_glowq_tiled", None)
-        if hit is not None and hit[0] == key:
-            return hit[1]
-        if torch.cuda.is_current_stream_capturing():
-            return None  # not under a graph capture: the copy would come from the graph's own memory pool
         _check(qweight.dtype == torch.int32 and scales.dtype == torch.float16 and qzeros.dtype == torch.int32 and
                qweight.is_contiguous() and scales.is_contiguous() and qzeros.is_contiguous(), "pack_tiled: contiguous canonical buffers")
-        out = torch.empty(nbytes, dtype=torch.uint8, device=qweight.device)
-        with torch.cuda.device(qweight.device):
-            rc = self.lib.glowq_pack_tiled(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), out.data_ptr(), N, int(in_features),
-                                           int(group_size), qweight.size(1), scales.size(1), qzeros.size(1), self._stream(qweight.device))
-        if rc:
-            self._raise(rc, "pack_tiled")
-        qweight._glowq_tiled = (key, out)
-        return out
+        return self._packed_copy(
+            (qweight, scales, qzeros), (int(in_features), int(group_size)), nbytes,
+            lambda out, stream: self.lib.glowq_pack_tiled(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), out, N, int(in_features),
+                                                          int(group_size), qweight.size(1), scales.size(1), qzeros.size(1), stream))
 
-    def pack_tiled_left(self, L) -> Optional[torch.Tensor]:
-        """The tiled copy of a left factor [N, rank] (fp16 B operand of the correction blocks), kept on the tensor."""
+    def _packed_tiled_left(self, L) -> Optional[_Packed]:
         if not tiled_enabled() or L is None or not L.is_cuda:
             return None
         N, rank = L.shape
         nbytes = self.lib.glowq_tiled_left_bytes(int(N), int(rank))
         if nbytes == 0:
             return None
-        hit = getattr(L, "_glowq_tiled", None)
-        if hit is not None and hit[0] == L._version:
-            return hit[1]
-        if torch.cuda.is_current_stream_capturing():
-            return None
         _check(L.dtype == torch.float16 and L.is_contiguous(), "pack_tiled_left: contiguous fp16 [OC, rank]")
-        out = torch.empty(nbytes, dtype=torch.uint8, device=L.device)
-        with torch.cuda.device(L.device):
-            rc = self.lib.glowq_pack_tiled_left(L.data_ptr(), out.data_ptr(), int(N), int(rank), self._stream(L.device))
-        if rc:
-            self._raise(rc, "pack_tiled_left")
-        L._glowq_tiled = (L._version, out)
-        return out
+        return self._packed_copy((L,), (int(N), int(rank)), nbytes,
+                                 lambda out, stream: self.lib.glowq_pack_tiled_left(L.data_ptr(), out, int(N), int(rank), stream))
+
+    def pack_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[torch.Tensor]:
+        """The tiled copy of a member's weights for the matrix-core routes (a uint8 tensor; layout in csrc/tiled.hpp), or
+        None where the layout does not apply.  Built once per weight tensor and kept on it (`qweight._glowq_tiled`) until
+        one of the three tensors is written to in place, then made again by the next call; a module moved with `.to()` gets new
+        tensors and with them a new copy.  Writes that torch does not count (through `.data`, a raw pointer or a collective) are
+        not seen: after those, call `torch.autograd.graph.increment_version` on the tensor."""
+        packed = self._packed_tiled(qweight, scales, qzeros, in_features, group_size)
+        return packed.out if packed is not None else None
+
+    def pack_tiled_left(self, L) -> Optional[torch.Tensor]:
+        """The tiled copy of a left factor [N, rank] (fp16 B operand of the correction blocks), kept on the tensor."""
+        packed = self._packed_tiled_left(L)
+        return packed.out if packed is not None else None
 
     def wants_tiled(self, M: int, K: int, N_total: int, group_size: int, ldw_i32: int) -> bool:
         """Whether a group of this shape would take the route that reads the tiled copies: they are built (and kept in device
@@ -333,15 +369,15 @@ class W4A16Extension:
         return route == 8 or (route == 2 and self.lib.glowq_tiled_bytes(int(N_total), int(K), int(group_size)) > 0)
 
     def _set_tiled(self, e, qw, sc, qz, L, in_features: int, group_size: int):
-        """Fills the tiled fields of descriptor `e`; returns what has to stay alive with it."""
-        tw = self.pack_tiled(qw, sc, qz, in_features, group_size)
-        if tw is None:
+        """Fills the tiled fields of descriptor `e`, or clears them where a copy cannot be had; returns what has to stay alive
+        with it."""
+        tw = self._packed_tiled(qw, sc, qz, in_features, group_size)
+        tl = self._packed_tiled_left(L) if tw is not None and L is not None else None
+        if tw is None or (L is not None and tl is None):
+            e.tiled, e.tiled_L, e.tiled_rank = None, None, 0
             return None
-        tl = self.pack_tiled_left(L) if L is not None else None
-        if L is not None and tl is None:
-            return None
-        e.tiled = tw.data_ptr()
-        e.tiled_L = tl.data_ptr() if tl is not None else None
+        e.tiled = tw.out.data_ptr()
+        e.tiled_L = tl.out.data_ptr() if tl is not None else None
         e.tiled_rank = int(L.size(1)) if L is not None else 0
         return (tw, tl)
 
@@ -689,8 +725,17 @@ class PreparedGroup:
             self.Ns.append(N)
             self.keep.append((qw, sc, qz, L, bias, side))
         self.corrected = corrected
-        self._tiled_keep = None  # the tiled copies of the members' weights: built by the first call with five token rows or more
+        # the tiled copies of the members' weights, built by the first call that reads them, and what they were made from: in-place
+        # writes to these tensors (load_state_dict among them) raise their versions, and the next call makes the copies again
+        self._tiled_keep, self._tiled_versions = None, None
+        self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
         self._n_total = sum(self.Ns)
+
+    def _build_tiled(self) -> None:
+        """Brings the tiled copies and the descriptors' pointers to them up to date (pointers are cleared where that cannot be)."""
+        self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
+                            for e, k in zip(self.arr, self.keep)]
+        self._tiled_versions = list(map(_version_of, self._tiled_from))
 
     def run(self, x: torch.Tensor, r: Optional[torch.Tensor] = None, outs: Optional[List[torch.Tensor]] = None,
             project: bool = True, out_dtype: torch.dtype = torch.float16) -> List[torch.Tensor]:
@@ -702,10 +747,9 @@ class PreparedGroup:
             raise RuntimeError("inputs must be contiguous CUDA fp16 [M, IC]")
         M = x.size(0)
         dev = x.device
-        if self._tiled_keep is None and M >= TILED_MIN_ROWS and self.ext.wants_tiled(M, self.K, self._n_total, self.group_size,
-                                                                                    self.arr[0].ldw_i32):
-            self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
-                                for e, k in zip(self.arr, self.keep)]
+        if M >= TILED_MIN_ROWS and (self.ext.wants_tiled(M, self.K, self._n_total, self.group_size, self.arr[0].ldw_i32)
+                                    if self._tiled_keep is None else self._tiled_versions != list(map(_version_of, self._tiled_from))):
+            self._build_tiled()
         Ns = self.Ns
         widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:

@@ -1,0 +1,77 @@
+"""Weights written to in place after their packed copies exist, and the other states that those copies can be met in: every
+forward has to give what a module made with the present weights gives."""
+import pytest
+import torch
+import torch.nn as nn
+
+from glowq_amd import correction as corr
+from glowq_amd import linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True, params=["fp16", "fp32"])
+def outputs(request, monkeypatch):
+    monkeypatch.setenv("W4A16_KERNEL_OUT_DTYPE", request.param)
+    with torch.no_grad():
+        yield request.param
+
+
+def quantised(seed, N=640, K=1024, bias=False):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    lin = nn.Linear(K, N, bias=bias, dtype=torch.float16, device="cuda")
+    for p in lin.parameters():
+        p.normal_(0.0, 0.02, generator=gen)
+    return linear.CudaW4A16Linear.from_float(lin, 128)
+
+
+def corrected(seed, N=640, K=1024, rank=64):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    L = torch.randn(N, rank, device="cuda", generator=gen).mul_(0.1).half()
+    R = torch.randn(rank, K, device="cuda", generator=gen).mul_(K ** -0.5).half()
+    return corr.AddSVDCorrection(quantised(seed, N, K), L, R, "solo", False, None, 1.0)
+
+
+def rows_of(m, K=1024):
+    return torch.randn(m, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).half()
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 64, 65, 300])
+@pytest.mark.parametrize("make", [quantised, corrected])
+def test_weights_written_in_place(make, rows):
+    """load_state_dict, a copy into one buffer, another of the scales and one of the left factor."""
+    mod, other, x = make(1), make(2), rows_of(rows)
+    mod(x)
+    mod.load_state_dict(other.state_dict())
+    if make is corrected:
+        mod.A_q.copy_(other.A_q)
+        mod.B_q.copy_(other.B_q)
+    assert torch.equal(mod(x), other(x))
+    inner, source = (getattr(m, "inner", m) for m in (mod, other))
+    for name in ("scales_f16", "qzeros_i32", "qweight_i32"):
+        getattr(source, name).copy_(getattr(getattr(make(3), "inner", make(3)), name))
+        before = mod(x)
+        getattr(inner, name).copy_(getattr(source, name))
+        after = mod(x)
+        assert not torch.equal(before, after)
+        assert torch.equal(after, other(x))
+    # a module made from the weights as they are now
+    fresh = make(4)
+    fresh.load_state_dict(mod.state_dict())
+    if make is corrected:
+        fresh.A_q.copy_(mod.A_q)
+        fresh.B_q.copy_(mod.B_q)
+    assert torch.equal(mod(x), fresh(x))
+
+
+def test_copies_of_tensors_that_share_weights():
+    """One weight tensor with two sets of scales: writing one set leaves the other module's copy alone."""
+    a, b, x = quantised(1), quantised(2), rows_of(300)
+    b.qweight_i32 = a.qweight_i32
+    want_a = a(x)
+    b(x)
+    b.scales_f16.mul_(2.0)
+    fresh = quantised(5)
+    fresh.load_state_dict(b.state_dict())
+    assert torch.equal(b(x), fresh(x))
+    assert torch.equal(a(x), want_a)
