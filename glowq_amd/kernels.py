@@ -737,6 +737,13 @@ class PreparedGroup:
                             for e, k in zip(self.arr, self.keep)]
         self._tiled_versions = list(map(_version_of, self._tiled_from))
 
+    def _without_tiled(self):
+        """The members' descriptors without the tiled copies."""
+        arr = type(self.arr).from_buffer_copy(self.arr)
+        for e in arr:
+            e.tiled, e.tiled_L, e.tiled_rank = None, None, 0
+        return arr
+
     def run(self, x: torch.Tensor, r: Optional[torch.Tensor] = None, outs: Optional[List[torch.Tensor]] = None,
             project: bool = True, out_dtype: torch.dtype = torch.float16) -> List[torch.Tensor]:
         """x [M, K] contiguous fp16 on the group's device.  With a right factor and `project`, r = x R^T is computed by
@@ -747,19 +754,23 @@ class PreparedGroup:
             raise RuntimeError("inputs must be contiguous CUDA fp16 [M, IC]")
         M = x.size(0)
         dev = x.device
-        if M >= TILED_MIN_ROWS and (self.ext.wants_tiled(M, self.K, self._n_total, self.group_size, self.arr[0].ldw_i32)
-                                    if self._tiled_keep is None else self._tiled_versions != list(map(_version_of, self._tiled_from))):
+        arr = self.arr
+        if M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing():
+            # A recorded GEMM without correction reads the weights themselves: a graph then follows writes to them by itself,
+            # where one that reads the copy needs a call outside the graph to bring it up to date.
+            arr = self._without_tiled()
+        elif M >= TILED_MIN_ROWS and (self.ext.wants_tiled(M, self.K, self._n_total, self.group_size, arr[0].ldw_i32)
+                                      if self._tiled_keep is None else self._tiled_versions != list(map(_version_of, self._tiled_from))):
             self._build_tiled()
         Ns = self.Ns
         widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:
             outs = [torch.empty((M, N), dtype=torch.float32 if widen else torch.float16, device=dev) for N in Ns]
-            for e, y in zip(self.arr, outs):
-                e.y, e.ldy = y.data_ptr(), y.stride(0)
         else:
-            for e, y, N in zip(self.arr, outs, Ns):
+            for y, N in zip(outs, Ns):
                 _check(y.dtype == torch.float16 and tuple(y.shape) == (M, N) and y.stride(1) == 1, "output must be CUDA fp16 [M, OC]")
-                e.y, e.ldy = y.data_ptr(), y.stride(0)
+        for e, y in zip(arr, outs):
+            e.y, e.ldy = y.data_ptr(), y.stride(0)
         if M == 0:
             return outs
         fused = project and self.R is not None
@@ -781,19 +792,19 @@ class PreparedGroup:
             ws, ws_bytes = ext._workspace(dev, M)
             stream = ext._stream(dev)
             if widen:
-                for e in self.arr:
+                for e in arr:
                     e.y_type = Y_FP32
             if fused:
                 rc = self.lib.glowq_w4a16_group_forward_fused_ws(
-                    x.data_ptr(), self.R.data_ptr(), r.data_ptr(), self.arr, len(Ns), M, self.K, self.group_size,
+                    x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
                     self.rank, self.alpha, ws, ws_bytes, stream)
             else:
                 rc = self.lib.glowq_w4a16_group_forward_ws(
-                    x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, self.arr, len(Ns), M,
+                    x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, arr, len(Ns), M,
                     self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
         finally:
             if widen:
-                for e in self.arr:
+                for e in arr:
                     e.y_type = 0
             if ctx is not None:
                 ctx.__exit__(None, None, None)
