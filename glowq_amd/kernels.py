@@ -735,7 +735,9 @@ class PreparedGroup:
         """Brings the tiled copies and the descriptors' pointers to them up to date (pointers are cleared where that cannot be)."""
         self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
                             for e, k in zip(self.arr, self.keep)]
-        self._tiled_versions = list(map(_version_of, self._tiled_from))
+        # copies that cannot be made under a capture are asked for again by the next call
+        made = all(self._tiled_keep) or not torch.cuda.is_current_stream_capturing()
+        self._tiled_versions = list(map(_version_of, self._tiled_from)) if made else None
 
     def _without_tiled(self):
         """The members' descriptors without the tiled copies."""

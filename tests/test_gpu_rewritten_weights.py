@@ -95,3 +95,23 @@ def test_graph_of_a_bare_linear_follows_its_weights(rows):
         want = other(x)
         assert (y.double() - want.double()).norm() <= 1e-3 * want.double().norm()
         assert torch.equal(mod(x), want)
+
+
+@pytest.mark.parametrize("make", [quantised, corrected])
+def test_first_call_under_a_capture(ext, make):
+    """Copies are not made under a capture; the first call outside one makes them."""
+    warm, mod, x = make(1), make(2), rows_of(300)
+    warm(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = mod(x)
+    graph.replay()
+    want = mod(x)
+    assert ext.last_launch()["kernel"].startswith("gemm_tiled_kernel")
+    warm.load_state_dict(mod.state_dict())
+    if make is corrected:
+        warm.A_q.copy_(mod.A_q)
+        warm.B_q.copy_(mod.B_q)
+    assert torch.equal(want, warm(x))
+    assert (y.double() - want.double()).norm() <= 1e-3 * want.double().norm()
