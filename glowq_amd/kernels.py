@@ -125,12 +125,25 @@ _version_of = attrgetter("_version")
 class _Packed:
     """A packed copy `out` of a few tensors, kept on the first of them.  `key` says what it was made from: addresses and
     versions (every in-place write through torch raises a tensor's version), so that a write to a source is seen.  Holding the
-    other sources keeps their addresses from being given to new tensors."""
+    other sources keeps their addresses from being given to new tensors.  The copy is made on `stream`, and other streams
+    wait for `event` before their first read of it."""
 
-    __slots__ = ("key", "others", "out")
+    __slots__ = ("key", "others", "out", "event", "stream", "waited")
 
-    def __init__(self, key, others, out):
-        self.key, self.others, self.out = key, others, out
+    def __init__(self, key, others, out, stream):
+        self.key, self.others, self.out, self.stream, self.waited = key, others, out, stream, set()
+        self.event = torch.cuda.Event()
+        self.event.record(torch.cuda.current_stream(out.device))
+
+    def ready_on(self, stream) -> None:
+        """Orders the current stream of the copy's device (handle `stream`) behind the packing.  Not under a capture, which
+        must not wait for work outside it: a recorded launch runs with a replay, and `torch.cuda.graph` has waited for the
+        whole device before it records."""
+        if stream != self.stream and stream not in self.waited and not torch.cuda.is_current_stream_capturing():
+            current = torch.cuda.current_stream(self.out.device)
+            current.wait_event(self.event)
+            self.out.record_stream(current)
+            self.waited.add(stream)
 
     def __reduce__(self):
         return set, ()  # a deep copy or a saved file of the tensor starts without one
@@ -303,7 +316,9 @@ class W4A16Extension:
         hit = getattr(owner, "_glowq_tiled", None)
         if not isinstance(hit, _Packed):
             hit = None
+        stream = self._stream(owner.device)
         if hit is not None and hit.key == key:
+            hit.ready_on(stream)
             return hit
         if torch.cuda.is_current_stream_capturing():
             return None
@@ -312,10 +327,10 @@ class W4A16Extension:
         else:
             out = torch.empty(nbytes, dtype=torch.uint8, device=owner.device)
         with torch.cuda.device(owner.device):
-            rc = pack(out.data_ptr(), self._stream(owner.device))
-        if rc:
-            self._raise(rc, "pack_tiled")
-        packed = _Packed(key, sources[1:], out)
+            rc = pack(out.data_ptr(), stream)
+            if rc:
+                self._raise(rc, "pack_tiled")
+            packed = _Packed(key, sources[1:], out, stream)
         owner._glowq_tiled = packed
         return packed
 
@@ -728,16 +743,24 @@ class PreparedGroup:
         # the tiled copies of the members' weights, built by the first call that reads them, and what they were made from: in-place
         # writes to these tensors (load_state_dict among them) raise their versions, and the next call makes the copies again
         self._tiled_keep, self._tiled_versions = None, None
+        self._tiled_streams = set()  # streams whose next launch finds the copies complete
         self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
         self._n_total = sum(self.Ns)
 
-    def _build_tiled(self) -> None:
-        """Brings the tiled copies and the descriptors' pointers to them up to date (pointers are cleared where that cannot be)."""
+    def _build_tiled(self, stream) -> None:
+        """Brings the tiled copies and the descriptors' pointers to them up to date for a launch on `stream` (pointers are
+        cleared where that cannot be)."""
+        versions = list(map(_version_of, self._tiled_from))
+        capturing = torch.cuda.is_current_stream_capturing()
         self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
                             for e, k in zip(self.arr, self.keep)]
         # copies that cannot be made under a capture are asked for again by the next call
-        made = all(self._tiled_keep) or not torch.cuda.is_current_stream_capturing()
-        self._tiled_versions = list(map(_version_of, self._tiled_from)) if made else None
+        made = all(self._tiled_keep) or not capturing
+        if versions != self._tiled_versions:
+            self._tiled_streams.clear()
+        self._tiled_versions = versions if made else None
+        if not capturing:
+            self._tiled_streams.add(stream)
 
     def _without_tiled(self):
         """The members' descriptors without the tiled copies."""
@@ -756,14 +779,16 @@ class PreparedGroup:
             raise RuntimeError("inputs must be contiguous CUDA fp16 [M, IC]")
         M = x.size(0)
         dev = x.device
-        arr = self.arr
+        arr, ext = self.arr, self.ext
+        stream = ext._stream(dev)
         if M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing():
             # A recorded GEMM without correction reads the weights themselves: a graph then follows writes to them by itself,
             # where one that reads the copy needs a call outside the graph to bring it up to date.
             arr = self._without_tiled()
-        elif M >= TILED_MIN_ROWS and (self.ext.wants_tiled(M, self.K, self._n_total, self.group_size, arr[0].ldw_i32)
-                                      if self._tiled_keep is None else self._tiled_versions != list(map(_version_of, self._tiled_from))):
-            self._build_tiled()
+        elif M >= TILED_MIN_ROWS and (ext.wants_tiled(M, self.K, self._n_total, self.group_size, arr[0].ldw_i32)
+                                      if self._tiled_keep is None else
+                                      stream not in self._tiled_streams or self._tiled_versions != list(map(_version_of, self._tiled_from))):
+            self._build_tiled(stream)
         Ns = self.Ns
         widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:
@@ -783,7 +808,6 @@ class PreparedGroup:
         elif not (r.dtype is torch.float16 and r.dim() == 2 and r.size(0) == M and r.size(1) == self.rank and r.is_contiguous()):
             raise RuntimeError("r must be fp16 [M, rank]")
         self.last_r = r
-        ext = self.ext
         idx = dev.index
         # the library launches on the current device: switch only when the tensors live on another one
         ctx = None
@@ -792,7 +816,6 @@ class PreparedGroup:
             ctx.__enter__()
         try:
             ws, ws_bytes = ext._workspace(dev, M)
-            stream = ext._stream(dev)
             if widen:
                 for e in arr:
                     e.y_type = Y_FP32

@@ -115,3 +115,31 @@ def test_first_call_under_a_capture(ext, make):
         warm.B_q.copy_(mod.B_q)
     assert torch.equal(want, warm(x))
     assert (y.double() - want.double()).norm() <= 1e-3 * want.double().norm()
+
+
+@pytest.mark.parametrize("rows", [5, 64, 65, 300])
+@pytest.mark.parametrize("make", [quantised, corrected])
+def test_copies_on_another_stream(make, rows):
+    """The stream that makes a copy is behind long work: a call on another stream waits for the copy, after a write as well."""
+    mod, same, x = make(1), make(1), rows_of(rows)
+    want = same(x)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    for stream in (first, second):  # their workspaces
+        with torch.cuda.stream(stream):
+            same(x)
+    for seed in (1, 2):
+        if seed == 2:
+            other = make(2)
+            for m in (mod, same):
+                m.load_state_dict(other.state_dict())
+            want = same(x)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(20_000_000)
+            a = mod(x)
+        with torch.cuda.stream(second):
+            b = mod(x)
+            c = mod(x)
+        torch.cuda.synchronize()
+        for y in (a, b, c):
+            assert torch.equal(y, want)
