@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from operator import attrgetter
 from typing import List, Optional, Sequence
 
@@ -165,6 +166,8 @@ class W4A16Extension:
             fn.argtypes = args
         self.version = lib.glowq_version()
         self._workspaces = {}
+        self._stream_locks = {}
+        self._pack_lock = threading.RLock()
 
     # ------------------------------------------------------------------ helpers
     def _raise(self, rc: int, what: str):
@@ -179,6 +182,13 @@ class W4A16Extension:
     WORKSPACE_BYTES = 64 << 20
 
     HANDOVER_BYTES = 8192
+
+    def _enqueue_lock(self, dev: torch.device, stream: int):
+        """The lock of a stream's workspace, held while a call puts its launches on the stream: the launches of one call hand
+        partial results on through the workspace, and another thread's must not come between them."""
+        key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream)
+        lock = self._stream_locks.get(key)
+        return lock if lock is not None else self._stream_locks.setdefault(key, threading.RLock())
 
     def _workspace(self, dev: torch.device, rows: int):
         """(pointer, bytes) of the workspace of the current stream of `dev`: one per stream, because calls that share
@@ -310,29 +320,30 @@ class W4A16Extension:
         the new one too.  None where it would have to be made under a graph capture (it would come from the graph's own memory
         pool, or be made at every replay)."""
         owner = sources[0]
-        ptrs, versions = [t.data_ptr() for t in sources], [t._version for t in sources]
-        shape_key += (nbytes,)
-        key = (ptrs, versions, shape_key)
-        hit = getattr(owner, "_glowq_tiled", None)
-        if not isinstance(hit, _Packed):
-            hit = None
-        stream = self._stream(owner.device)
-        if hit is not None and hit.key == key:
-            hit.ready_on(stream)
-            return hit
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        if hit is not None and hit.key[0] == ptrs and hit.key[2] == shape_key:
-            out = hit.out
-        else:
-            out = torch.empty(nbytes, dtype=torch.uint8, device=owner.device)
-        with torch.cuda.device(owner.device):
-            rc = pack(out.data_ptr(), stream)
-            if rc:
-                self._raise(rc, "pack_tiled")
-            packed = _Packed(key, sources[1:], out, stream)
-        owner._glowq_tiled = packed
-        return packed
+        with self._pack_lock:
+            ptrs, versions = [t.data_ptr() for t in sources], [t._version for t in sources]
+            shape_key += (nbytes,)
+            key = (ptrs, versions, shape_key)
+            hit = getattr(owner, "_glowq_tiled", None)
+            if not isinstance(hit, _Packed):
+                hit = None
+            stream = self._stream(owner.device)
+            if hit is not None and hit.key == key:
+                hit.ready_on(stream)
+                return hit
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            if hit is not None and hit.key[0] == ptrs and hit.key[2] == shape_key:
+                out = hit.out
+            else:
+                out = torch.empty(nbytes, dtype=torch.uint8, device=owner.device)
+            with torch.cuda.device(owner.device):
+                rc = pack(out.data_ptr(), stream)
+                if rc:
+                    self._raise(rc, "pack_tiled")
+                packed = _Packed(key, sources[1:], out, stream)
+            owner._glowq_tiled = packed
+            return packed
 
     def _packed_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[_Packed]:
         if not tiled_enabled():
@@ -407,9 +418,10 @@ class W4A16Extension:
         if out is None:
             out = torch.empty((M, rank), dtype=torch.float16, device=x.device)
         with torch.cuda.device(x.device):
-            ws, ws_bytes = self._workspace(x.device, M)
-            rc = self.lib.glowq_shared_proj_ws(x.data_ptr(), R.data_ptr(), out.data_ptr(), M, K, rank, ws, ws_bytes,
-                                               self._stream(x.device))
+            stream = self._stream(x.device)
+            with self._enqueue_lock(x.device, stream):
+                ws, ws_bytes = self._workspace(x.device, M)
+                rc = self.lib.glowq_shared_proj_ws(x.data_ptr(), R.data_ptr(), out.data_ptr(), M, K, rank, ws, ws_bytes, stream)
         if rc:
             self._raise(rc, "shared_proj")
         return out
@@ -472,16 +484,17 @@ class W4A16Extension:
         if M == 0:
             return result
         with torch.cuda.device(x.device):
-            if R is not None:
+            stream = self._stream(x.device)
+            with self._enqueue_lock(x.device, stream):
                 ws, ws_bytes = self._workspace(x.device, M)
-                rc = self.lib.glowq_w4a16_group_forward_fused_ws(
-                    x.data_ptr(), R.data_ptr(), r.data_ptr(), arr, len(members), M, K, int(group_size),
-                    int(rank), float(alpha), ws, ws_bytes, self._stream(x.device))
-            else:
-                ws, ws_bytes = self._workspace(x.device, M)
-                rc = self.lib.glowq_w4a16_group_forward_ws(
-                    x.data_ptr(), r.data_ptr() if r is not None else None, arr, len(members), M, K, int(group_size),
-                    int(rank), float(alpha), ws, ws_bytes, self._stream(x.device))
+                if R is not None:
+                    rc = self.lib.glowq_w4a16_group_forward_fused_ws(
+                        x.data_ptr(), R.data_ptr(), r.data_ptr(), arr, len(members), M, K, int(group_size),
+                        int(rank), float(alpha), ws, ws_bytes, stream)
+                else:
+                    rc = self.lib.glowq_w4a16_group_forward_ws(
+                        x.data_ptr(), r.data_ptr() if r is not None else None, arr, len(members), M, K, int(group_size),
+                        int(rank), float(alpha), ws, ws_bytes, stream)
         if rc:
             self._raise(rc, "w4a16_group_forward")
         return result
@@ -740,34 +753,29 @@ class PreparedGroup:
             self.Ns.append(N)
             self.keep.append((qw, sc, qz, L, bias, side))
         self.corrected = corrected
-        # the tiled copies of the members' weights, built by the first call that reads them, and what they were made from: in-place
-        # writes to these tensors (load_state_dict among them) raise their versions, and the next call makes the copies again
-        self._tiled_keep, self._tiled_versions = None, None
-        self._tiled_streams = set()  # streams whose next launch finds the copies complete
+        # The tiled copies of the members' weights, built by the first call that reads them: (descriptors with them, what they keep
+        # alive, the versions of the tensors they were made from, the streams whose next launch finds them complete).
+        # In-place writes (load_state_dict among them) raise the versions, and the next call makes the copies again.  Replaced
+        # as a whole, so that a thread sees one state.
+        self._tiled = None
         self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
         self._n_total = sum(self.Ns)
 
-    def _build_tiled(self, stream) -> None:
+    def _build_tiled(self, stream):
         """Brings the tiled copies and the descriptors' pointers to them up to date for a launch on `stream` (pointers are
-        cleared where that cannot be)."""
+        empty where that cannot be)."""
+        old = self._tiled
         versions = list(map(_version_of, self._tiled_from))
         capturing = torch.cuda.is_current_stream_capturing()
-        self._tiled_keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
-                            for e, k in zip(self.arr, self.keep)]
-        # copies that cannot be made under a capture are asked for again by the next call
-        made = all(self._tiled_keep) or not capturing
-        if versions != self._tiled_versions:
-            self._tiled_streams.clear()
-        self._tiled_versions = versions if made else None
-        if not capturing:
-            self._tiled_streams.add(stream)
-
-    def _without_tiled(self):
-        """The members' descriptors without the tiled copies."""
         arr = type(self.arr).from_buffer_copy(self.arr)
-        for e in arr:
-            e.tiled, e.tiled_L, e.tiled_rank = None, None, 0
-        return arr
+        keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
+                for e, k in zip(arr, self.keep)]
+        streams = set(old[3]) if old is not None and old[2] == versions else set()
+        if not capturing:
+            streams.add(stream)
+        # copies that cannot be made under a capture are asked for again by the next call
+        self._tiled = state = (arr, keep, versions if all(keep) or not capturing else None, streams)
+        return state
 
     def run(self, x: torch.Tensor, r: Optional[torch.Tensor] = None, outs: Optional[List[torch.Tensor]] = None,
             project: bool = True, out_dtype: torch.dtype = torch.float16) -> List[torch.Tensor]:
@@ -779,16 +787,17 @@ class PreparedGroup:
             raise RuntimeError("inputs must be contiguous CUDA fp16 [M, IC]")
         M = x.size(0)
         dev = x.device
-        arr, ext = self.arr, self.ext
+        ext, tiled = self.ext, None
         stream = ext._stream(dev)
-        if M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing():
-            # A recorded GEMM without correction reads the weights themselves: a graph then follows writes to them by itself,
-            # where one that reads the copy needs a call outside the graph to bring it up to date.
-            arr = self._without_tiled()
-        elif M >= TILED_MIN_ROWS and (ext.wants_tiled(M, self.K, self._n_total, self.group_size, arr[0].ldw_i32)
-                                      if self._tiled_keep is None else
-                                      stream not in self._tiled_streams or self._tiled_versions != list(map(_version_of, self._tiled_from))):
-            self._build_tiled(stream)
+        # From 65 rows a recorded launch without correction reads the weights themselves: a graph then follows writes to them by
+        # itself, where one that reads the copies needs a call outside the graph to bring them up to date.
+        if M >= TILED_MIN_ROWS and not (M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing()):
+            tiled = self._tiled
+            if (ext.wants_tiled(M, self.K, self._n_total, self.group_size, self.arr[0].ldw_i32) if tiled is None else
+                    stream not in tiled[3] or tiled[2] != list(map(_version_of, self._tiled_from))):
+                tiled = self._build_tiled(stream)
+        # (a copy of the descriptors: other threads may be in the same group)
+        arr = type(self.arr).from_buffer_copy(tiled[0] if tiled is not None else self.arr)
         Ns = self.Ns
         widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:
@@ -798,6 +807,8 @@ class PreparedGroup:
                 _check(y.dtype == torch.float16 and tuple(y.shape) == (M, N) and y.stride(1) == 1, "output must be CUDA fp16 [M, OC]")
         for e, y in zip(arr, outs):
             e.y, e.ldy = y.data_ptr(), y.stride(0)
+            if widen:
+                e.y_type = Y_FP32
         if M == 0:
             return outs
         fused = project and self.R is not None
@@ -815,22 +826,17 @@ class PreparedGroup:
             ctx = torch.cuda.device(dev)
             ctx.__enter__()
         try:
-            ws, ws_bytes = ext._workspace(dev, M)
-            if widen:
-                for e in arr:
-                    e.y_type = Y_FP32
-            if fused:
-                rc = self.lib.glowq_w4a16_group_forward_fused_ws(
-                    x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
-                    self.rank, self.alpha, ws, ws_bytes, stream)
-            else:
-                rc = self.lib.glowq_w4a16_group_forward_ws(
-                    x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, arr, len(Ns), M,
-                    self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
+            with ext._enqueue_lock(dev, stream):
+                ws, ws_bytes = ext._workspace(dev, M)
+                if fused:
+                    rc = self.lib.glowq_w4a16_group_forward_fused_ws(
+                        x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
+                        self.rank, self.alpha, ws, ws_bytes, stream)
+                else:
+                    rc = self.lib.glowq_w4a16_group_forward_ws(
+                        x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, arr, len(Ns), M,
+                        self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
         finally:
-            if widen:
-                for e in arr:
-                    e.y_type = 0
             if ctx is not None:
                 ctx.__exit__(None, None, None)
         if rc == EUNSUPPORTED and widen:  # not the GEMM's call: nothing has been launched

@@ -221,13 +221,14 @@ class CudaW4A16Linear(nn.Module):
         fold_bias = self.bias is not None and KNOBS.out_dtype == torch.float16
         key = (self.qweight_i32.data_ptr(), self.scales_f16.data_ptr(), self.qzeros_i32.data_ptr(),
                self.bias.data_ptr() if fold_bias else 0)
-        if self._prepared is None or self._prepared[0] != key:
+        prepared = self._prepared
+        if prepared is None or prepared[0] != key:
             from .kernels import PreparedGroup
 
             member = self._member()
             member["bias"] = self.bias.data if fold_bias else None
-            self._prepared = (key, PreparedGroup(self._get_ext(), [member], self.in_features, self.group_size, 0.0))
-        return self._prepared[1]
+            self._prepared = prepared = (key, PreparedGroup(self._get_ext(), [member], self.in_features, self.group_size, 0.0))
+        return prepared[1]
 
     def _prefer_gemv(self, m: int) -> bool:
         KNOBS.sync()

@@ -1,5 +1,7 @@
 """Weights written to in place after their packed copies exist, and the other states that those copies can be met in: every
 forward has to give what a module made with the present weights gives."""
+import threading
+
 import pytest
 import torch
 import torch.nn as nn
@@ -143,3 +145,35 @@ def test_copies_on_another_stream(make, rows):
         torch.cuda.synchronize()
         for y in (a, b, c):
             assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+@pytest.mark.parametrize("rows", [1, 4, 64, 65, 129, 300])
+@pytest.mark.parametrize("make", [quantised, corrected])
+def test_threads_in_one_module(make, rows, own_streams):
+    """Threads with inputs of their own in one module and in another that shares their stream's workspace (K = 4096: cut into
+    slices that are added by a second launch)."""
+    K, threads, calls = 4096, 4, 40
+    mods = [make(seed, N=256, K=K) for seed in (1, 2)]
+    xs = [torch.randn(rows, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(i)).half() for i in range(threads)]
+    wants = [[mod(x) for mod in mods] for x in xs]
+    mods = [make(seed, N=256, K=K) for seed in (1, 2)]
+    torch.cuda.synchronize()
+    got, start = [[] for _ in xs], threading.Barrier(threads)
+
+    def work(i):
+        with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream() if own_streams else torch.cuda.current_stream()):
+            start.wait(timeout=60)
+            for _ in range(calls):
+                got[i].append([mod(xs[i]) for mod in mods])
+
+    pool = [threading.Thread(target=work, args=(i,)) for i in range(threads)]
+    for t in pool:
+        t.start()
+    for t in pool:
+        t.join(timeout=60)
+    torch.cuda.synchronize()
+    for ys, want in zip(got, wants):
+        assert len(ys) == calls
+        for pair in ys:
+            assert all(torch.equal(y, w) for y, w in zip(pair, want))
