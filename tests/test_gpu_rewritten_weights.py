@@ -177,3 +177,19 @@ def test_threads_in_one_module(make, rows, own_streams):
         assert len(ys) == calls
         for pair in ys:
             assert all(torch.equal(y, w) for y, w in zip(pair, want))
+
+
+def test_copies_made_on_a_stream_of_another_library(ext, monkeypatch):
+    """A stream that torch did not make may be gone when a reader on another stream waits: the event is recorded at once."""
+    monkeypatch.setattr(ext, "_homes", {})  # (the handle below is one of torch's own)
+    mod, same, x = quantised(1), quantised(1), rows_of(300)
+    want = same(x)
+    torch.cuda.synchronize()
+    made = torch.cuda.Stream()
+    with torch.cuda.stream(torch.cuda.ExternalStream(made.cuda_stream)):
+        torch.cuda._sleep(20_000_000)
+        a = mod(x)
+    assert mod.qweight_i32._glowq_tiled.event is not None
+    b = mod(x)
+    torch.cuda.synchronize()
+    assert torch.equal(a, want) and torch.equal(b, want)
