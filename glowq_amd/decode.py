@@ -69,6 +69,12 @@ def _row_kernels(*tensors) -> bool:
                 or torch._C._len_torch_dispatch_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling())
 
 
+def _several_rows(x) -> bool:
+    """Whether x is a tensor of several token rows -- asked before anything else of it, because a tracer's stand-in for a tensor
+    has no sizes that a branch could look at."""
+    return type(x) in (torch.Tensor, nn.Parameter) and x.dim() == 2 and x.size(0) > 1
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float):
         super().__init__()
@@ -92,7 +98,7 @@ class RMSNorm(nn.Module):
 
     def _takes_rows(self, *xs) -> bool:
         x = xs[0]
-        return (x.dim() == 2 and x.size(0) > 1 and x.size(1) % 8 == 0 and all(t.shape == x.shape and t.device == x.device for t in xs)
+        return (_several_rows(x) and x.size(1) % 8 == 0 and all(t.shape == x.shape and t.device == x.device for t in xs)
                 and self.weight.device == x.device and self.weight.numel() == x.size(1) and _row_kernels(*xs, self.weight))
 
     def forward_add(self, x, delta):
@@ -131,7 +137,7 @@ class Attention(nn.Module):
                                           cfg.head_dim ** -0.5)
                 return self.o_proj(out)
         q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
-        if (T > 1 and x.dim() == 2 and cfg.head_dim % 16 == 0 and pos_idx.dtype == torch.int64 and pos_idx.device == q.device and tuple(pos_idx.shape) == (T,) and pos_idx.is_contiguous()
+        if (_several_rows(x) and cfg.head_dim % 16 == 0 and pos_idx.dtype == torch.int64 and pos_idx.device == q.device and tuple(pos_idx.shape) == (T,) and pos_idx.is_contiguous()
                 and cos.shape == sin.shape == (T, cfg.head_dim) and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
             # rotary embedding and cache append in one launch; the heads stay side by side in a row
             q_rot, k_rot = torch.empty_like(q), torch.empty_like(k)
@@ -174,7 +180,7 @@ class MLP(nn.Module):
             act = torch.empty_like(gate)
             self.glue.ext.silu_mul(gate, up, act)
             return self.down_proj(act)
-        if x.dim() == 2 and x.size(0) > 1 and gate.shape == up.shape and gate.numel() % 8 == 0 and _row_kernels(gate, up):
+        if _several_rows(x) and gate.shape == up.shape and gate.numel() % 8 == 0 and _row_kernels(gate, up):
             act = torch.empty_like(gate)
             load_w4a16_extension().silu_mul(gate, up, act)
             return self.down_proj(act)
@@ -204,7 +210,7 @@ class DecoderLayer(nn.Module):
             h = self.post_attention_layernorm(x, delta=attn.to(x.dtype))
             return x.add_(self.mlp(h).to(x.dtype))
         attn = self.self_attn(self.input_layernorm(x), cos, sin, cache_k, cache_v, pos_idx, mask)
-        if x.size(0) > 1 and not _hooked(self.post_attention_layernorm):
+        if _several_rows(x) and not _hooked(self.post_attention_layernorm):
             x, h = self.post_attention_layernorm.forward_add(x, attn)  # the residual add rides on the norm's launch
         else:
             x = x + attn
