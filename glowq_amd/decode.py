@@ -59,20 +59,24 @@ class _Glue:
         self.ext, self.cos_t, self.sin_t, self.pos = ext, cos_t, sin_t, pos
 
 
-def _row_kernels(*tensors) -> bool:
-    """Whether several token rows may go through the library's kernels instead of tensor expressions: plain fp16 tensors on the
-    GPU, and nobody who needs to see the expressions -- no gradients in either direction, no tracing, no function transforms."""
-    for t in tensors:
-        if not (t.is_cuda and t.device == tensors[0].device and t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0):
-            return False
-    return not (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
-                or torch._C._len_torch_dispatch_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+def _watched() -> bool:
+    """Whether somebody needs to see tensor expressions: gradients in either direction, tracing, function transforms, modes."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack() > 0)
 
 
 def _several_rows(x) -> bool:
-    """Whether x is a tensor of several token rows -- asked before anything else of it, because a tracer's stand-in for a tensor
-    has no sizes that a branch could look at."""
-    return type(x) in (torch.Tensor, nn.Parameter) and x.dim() == 2 and x.size(0) > 1
+    """Whether x is a tensor of several token rows that nobody watches.  Asked before anything else of it: a tracer's stand-in for a
+    tensor has no sizes that a branch could look at, and a transform's has no address."""
+    return type(x) in (torch.Tensor, nn.Parameter) and not _watched() and x.dim() == 2 and x.size(0) > 1
+
+
+def _row_kernels(*tensors) -> bool:
+    """Whether the library's kernels for several token rows take these tensors: plain fp16 on one GPU."""
+    for t in tensors:
+        if not (t.is_cuda and t.device == tensors[0].device and t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            return False
+    return True
 
 
 class RMSNorm(nn.Module):

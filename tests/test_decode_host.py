@@ -37,3 +37,14 @@ def test_layers_can_be_traced_symbolically(model, part):
         traced = torch.fx.symbolic_trace(mod, {"delta": None} if part == "norm" else None)
         got = traced(*args, None) if part == "norm" else traced(*args)
         assert torch.equal(got, mod(*args))
+
+
+def test_batched_rows_stay_expressions():
+    """A tensor under torch.func.vmap has no address to look at."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode(), torch.no_grad():
+        with torch.device("cuda"):
+            norm = decode.RMSNorm(64, 1e-5)
+        x = torch.empty(3, 5, 64, dtype=torch.float16, device="cuda")
+        assert torch.func.vmap(norm)(x).shape == x.shape

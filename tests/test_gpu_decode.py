@@ -638,3 +638,22 @@ def test_row_norm_rounds_once(fp16_out, M, H, with_delta):
     t = want_x.double()
     want = t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
     assert ((h.double() - want).abs() <= (2.0 ** -11 + 2.0 ** -20) * want.abs() + 2.0 ** -25).all()
+
+
+def test_transforms_of_several_rows(fp16_out):
+    """torch.func.vmap and a whole-graph compile go through the expressions, with the results of a plain call."""
+    cfg = decode.DecoderConfig(hidden=256, layers=1, heads=4, kv_heads=2, head_dim=64, intermediate=512, vocab=64, max_len=32, rank=32)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    norm = decode.RMSNorm(256, 1e-5).cuda()
+    x = torch.randn(3, 5, 256, device="cuda", generator=g).half()
+    got, want = torch.func.vmap(norm)(x), torch.nn.functional.rms_norm(x, (256,), norm.weight, 1e-5)
+    assert (got.double() - want.double()).norm() <= 2e-3 * want.double().norm()  # vmap's own rms_norm rounds between its steps
+    layer = decode.DecoderLayer(cfg).half().cuda()
+    caches = [torch.zeros(2, 32, 64, dtype=torch.float16, device="cuda") for _ in range(2)]
+    ang = torch.rand(5, 64, device="cuda", generator=g)
+    args = (x[0], ang.cos().half(), ang.sin().half(), *caches, torch.arange(5, device="cuda"), None)
+    for mod, inputs in ((norm, args[:1]), (layer.mlp, args[:1]), (layer, args)):
+        got = torch.compile(mod, fullgraph=True, backend="eager")(*inputs)
+        want = mod(*inputs)
+        # the kernels round a few times less than the expressions (2^-11 each)
+        assert (got.double() - want.double()).norm() <= 4e-3 * want.double().norm()
