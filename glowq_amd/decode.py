@@ -27,6 +27,8 @@ from typing import Dict, Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.overrides
+import torch.utils._device
 
 from .correction import AddSVDCorrection, patch_svd_correction_wrappers, patch_svd_correction_wrappers_cumulative
 from .kernels import (CHAIN_ACC_BYTES, CHAIN_EPI_NONE, CHAIN_EPI_RESIDUAL, CHAIN_EPI_SWIGLU, CHAIN_PRO_ACC, CHAIN_PRO_NORM_ACC,
@@ -59,16 +61,26 @@ class _Glue:
         self.ext, self.cos_t, self.sin_t, self.pos = ext, cos_t, sin_t, pos
 
 
-def _watched() -> bool:
-    """Whether somebody needs to see tensor expressions: gradients in either direction, tracing, function transforms, modes."""
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack() > 0)
+# torch has no public way to ask for these; on a torch without one of them everything counts as watched
+_PROBES = (getattr(torch._C, "_are_functorch_transforms_active", None), getattr(torch._C, "_len_torch_dispatch_stack", None),
+           getattr(torch.overrides, "_get_current_function_mode_stack", None))
+_DeviceContext = getattr(torch.utils._device, "DeviceContext", None)
+
+
+def _watched(x) -> bool:
+    """Whether somebody needs to see the tensor expressions on the plain tensor x: gradients in either direction, tracing, function
+    transforms, dispatch or function modes (`torch.set_default_device`, a function mode too, only looks at factories)."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled() or None in _PROBES:
+        return True
+    transforms, dispatch_modes, function_modes = _PROBES
+    return (getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or transforms() or dispatch_modes() > 0
+            or (torch.overrides.has_torch_function_unary(x) and any(type(m) is not _DeviceContext for m in function_modes())))
 
 
 def _several_rows(x) -> bool:
     """Whether x is a tensor of several token rows that nobody watches.  Asked before anything else of it: a tracer's stand-in for a
     tensor has no sizes that a branch could look at, and a transform's has no address."""
-    return type(x) in (torch.Tensor, nn.Parameter) and not _watched() and x.dim() == 2 and x.size(0) > 1
+    return type(x) in (torch.Tensor, nn.Parameter) and not _watched(x) and x.dim() == 2 and x.size(0) > 1
 
 
 def _row_kernels(*tensors) -> bool:
@@ -191,10 +203,15 @@ class MLP(nn.Module):
         return self.down_proj(F.silu(gate) * up)
 
 
+_NORM_CALLS = RMSNorm.forward, RMSNorm.__call__
+
+
 def _hooked(mod: nn.Module) -> bool:
-    """Whether calling `mod` does more than its forward, or it is another module than the decoder's own norm."""
+    """Whether calling `mod` does more than its forward, or that is another one than the decoder's own norm has: hooks, a forward
+    or a call replaced on the module, its class or nn.Module, a compiled call."""
     glob = torch.nn.modules.module
-    return not (type(mod) is RMSNorm and "forward" not in mod.__dict__) or bool(
+    return not (type(mod) is RMSNorm and (RMSNorm.forward, RMSNorm.__call__) == _NORM_CALLS and "forward" not in mod.__dict__
+                and getattr(mod, "_compiled_call_impl", None) is None) or bool(
         mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
         or glob._global_forward_hooks or glob._global_forward_pre_hooks or glob._global_backward_hooks or glob._global_backward_pre_hooks)
 

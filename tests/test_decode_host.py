@@ -2,6 +2,8 @@
 import pytest
 import torch
 import torch.fx
+import torch.nn.functional as F
+from torch.overrides import TorchFunctionMode
 
 from glowq_amd import decode
 
@@ -19,6 +21,52 @@ def model():
 
 def caches(length=CFG.max_len):
     return [tuple(torch.zeros(CFG.kv_heads, length, CFG.head_dim) for _ in range(2))]
+
+
+class Recorder:
+    """Stands in for the library: computes what its row kernels compute and writes down their names."""
+
+    def __init__(self):
+        self.calls = []
+
+    def add_rmsnorm_out(self, x, delta, weight, x_out, h, eps):
+        self.calls.append("norm" if delta is None else "add_norm")
+        if delta is not None:
+            x = x_out.copy_(x + delta)
+        h.copy_(F.rms_norm(x, (x.size(-1),), weight, eps))
+
+    def silu_mul(self, gate, up, out):
+        self.calls.append("gate")
+        out.copy_(F.silu(gate) * up)
+
+    def rope_append(self, q, k, v, cos, sin, pos, q_out, k_out, cache_k, cache_v):
+        self.calls.append("append")
+        T, d = cos.shape
+        for src, dst in ((q, q_out), (k, k_out)):
+            dst.copy_(decode._rope(src.view(T, -1, d).transpose(0, 1), cos, sin).transpose(0, 1).reshape(T, -1))
+        ok = (pos >= 0) & (pos < cache_k.size(1))  # a position outside writes no row
+        cache_k[:, pos[ok]] = k_out.view(T, -1, d)[ok].transpose(0, 1)
+        cache_v[:, pos[ok]] = v.view(T, -1, d)[ok].transpose(0, 1)
+
+
+@pytest.fixture()
+def kernels(monkeypatch):
+    """The row kernels as a recorder, with the CPU's tensors taken for fit."""
+    rec = Recorder()
+    monkeypatch.setattr(decode, "load_w4a16_extension", lambda: rec)
+    monkeypatch.setattr(decode, "_row_kernels", lambda *tensors: True)
+    return rec
+
+
+def forward(model, T=5, length=CFG.max_len, start=0):
+    store = caches(length)
+    cos, sin = model.rope_tables("cpu")
+    with torch.no_grad():
+        logits = model.forward_tokens(torch.arange(T), torch.arange(start, start + T), store, cos, sin, from_empty_cache=True)
+    return [logits, *store[0]]
+
+
+ALL = ["norm", "append", "add_norm", "gate", "norm"]
 
 
 def layer_inputs(model, T=5):
@@ -48,3 +96,58 @@ def test_batched_rows_stay_expressions():
             norm = decode.RMSNorm(64, 1e-5)
         x = torch.empty(3, 5, 64, dtype=torch.float16, device="cuda")
         assert torch.func.vmap(norm)(x).shape == x.shape
+
+
+def test_rows_that_nobody_watches_take_the_kernels(model, kernels, monkeypatch):
+    with_kernels = forward(model)
+    assert kernels.calls == ALL
+    with torch.device("cpu"):  # a function mode that looks at factories only
+        forward(model)
+    assert kernels.calls == 2 * ALL
+    monkeypatch.undo()
+    for a, b in zip(with_kernels, forward(model)):
+        assert torch.allclose(a, b, atol=1e-5)
+    assert kernels.calls == 2 * ALL
+
+
+def test_function_modes_see_the_expressions(model, kernels):
+    seen = []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    with Watch():
+        forward(model)
+    assert kernels.calls == []
+    assert seen.count("rms_norm") == 3 and seen.count("silu") == 1 and seen.count("index_copy_") == 2
+
+
+def test_a_torch_without_the_probes_takes_the_expressions(model, kernels, monkeypatch):
+    monkeypatch.setattr(decode, "_PROBES", (None,) + decode._PROBES[1:])
+    forward(model)
+    assert kernels.calls == []
+
+
+@pytest.mark.parametrize("where", ["class", "instance", "call", "hook", "compiled"])
+def test_a_replaced_norm_is_called(model, kernels, monkeypatch, where):
+    """The residual add rides on the norm's launch only where calling the norm is nothing but its own forward."""
+    norm, own, calls = model.model.layers[0].post_attention_layernorm, decode.RMSNorm.forward, []
+
+    def forward_instead(self, x, delta=None):
+        calls.append(self)
+        return own(self, x, delta)
+    if where == "class":
+        monkeypatch.setattr(decode.RMSNorm, "forward", forward_instead)
+    elif where == "instance":
+        norm.forward = forward_instead.__get__(norm)
+    elif where == "call":
+        call = torch.nn.Module.__call__
+        monkeypatch.setattr(torch.nn.Module, "__call__", lambda self, *a, **kw: (calls.append(self), call(self, *a, **kw))[1])
+    elif where == "hook":
+        norm.register_forward_hook(lambda mod, args, out: calls.append(mod))
+    else:
+        norm._compiled_call_impl = lambda *args: (calls.append(norm), own(norm, *args))[1]
+    forward(model)
+    assert norm in calls and "add_norm" not in kernels.calls
