@@ -91,6 +91,33 @@ def _row_kernels(*tensors) -> bool:
     return True
 
 
+def _positions_end(pos_idx, rows: int, caches) -> int:
+    """A bound that selecting from tables of `rows` rows has checked the positions against.  Where a cache is shorter than the tables
+    that does not keep them inside: positions outside are refused here, on the host, and the bound is theirs."""
+    if all(t.size(1) >= rows for pair in caches for t in pair) or not pos_idx.is_cuda:
+        return rows
+    if torch.cuda.is_current_stream_capturing():
+        return rows  # the host cannot look; the layers append with index_copy_
+    first, last = torch.stack(torch.aminmax(pos_idx)).tolist()
+    shortest = min(t.size(1) for pair in caches for t in pair)
+    if first < 0 or last >= shortest:
+        raise IndexError(f"positions {first}..{last} do not fit a cache of {shortest} rows")
+    return last + 1
+
+
+def _note_positions(cos, pos_idx, end: int) -> None:
+    """Notes on `cos` (the rows of a rotary table at `pos_idx`) that the positions are known to lie in 0..end-1."""
+    cos._glowq_positions = (pos_idx, None if pos_idx.is_inference() else pos_idx._version, end)
+
+
+def _inside_cache(cos, pos_idx, cache_k, cache_v) -> bool:
+    """Whether the positions are known to lie inside the caches.  The append kernel writes no row for a position outside; where
+    one could occur, the append is torch's index_copy_."""
+    noted = getattr(cos, "_glowq_positions", None)
+    return (noted is not None and noted[0] is pos_idx and noted[1] == (None if pos_idx.is_inference() else pos_idx._version)
+            and cache_k.shape == cache_v.shape and cache_k.size(1) >= noted[2])
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float):
         super().__init__()
@@ -154,7 +181,7 @@ class Attention(nn.Module):
                 return self.o_proj(out)
         q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         if (_several_rows(x) and cfg.head_dim % 16 == 0 and pos_idx.dtype == torch.int64 and pos_idx.device == q.device and tuple(pos_idx.shape) == (T,) and pos_idx.is_contiguous()
-                and cos.shape == sin.shape == (T, cfg.head_dim) and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
+                and cos.shape == sin.shape == (T, cfg.head_dim) and _inside_cache(cos, pos_idx, cache_k, cache_v) and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
             # rotary embedding and cache append in one launch; the heads stay side by side in a row
             q_rot, k_rot = torch.empty_like(q), torch.empty_like(k)
             load_w4a16_extension().rope_append(q, k, v, cos, sin, pos_idx, q_rot, k_rot, cache_k, cache_v)
@@ -278,7 +305,11 @@ class Decoder(nn.Module):
         `from_empty_cache`: pos_idx is 0..T-1 and nothing older is cached, so attention needs no mask over the cache."""
         cfg = self.cfg
         x = self.model.embed_tokens(tokens)
+        several = _several_rows(x)
+        end = _positions_end(pos_idx, min(cos_t.size(0), sin_t.size(0)), caches) if several else 0
         cos, sin = cos_t.index_select(0, pos_idx).to(x.dtype), sin_t.index_select(0, pos_idx).to(x.dtype)
+        if several:
+            _note_positions(cos, pos_idx, end)
         mask = None
         if not from_empty_cache:
             col = torch.arange(cfg.max_len, device=tokens.device)

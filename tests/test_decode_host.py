@@ -151,3 +151,33 @@ def test_a_replaced_norm_is_called(model, kernels, monkeypatch, where):
         norm._compiled_call_impl = lambda *args: (calls.append(norm), own(norm, *args))[1]
     forward(model)
     assert norm in calls and "add_norm" not in kernels.calls
+
+
+def test_positions_outside_a_short_cache_are_refused(model, kernels):
+    """A cache shorter than the rotary tables: torch's index_copy_ appends, and refuses a position outside."""
+    expressions = ["norm", "add_norm", "gate", "norm"]
+    short, full = forward(model, length=8), forward(model)
+    assert kernels.calls == expressions + ALL
+    assert torch.allclose(short[0], full[0], atol=1e-5) and torch.allclose(short[1], full[1][:, :8], atol=1e-5)
+    with pytest.raises(IndexError):
+        forward(model, length=8, start=4)
+    with pytest.raises(IndexError):
+        forward(model, length=CFG.max_len, start=CFG.max_len - 2)
+    kernels.calls.clear()
+    forward(model, length=CFG.max_len + 8, start=CFG.max_len - 5)
+    assert kernels.calls == ALL
+
+
+def test_positions_that_nothing_has_checked_are_left_to_index_copy(model, kernels):
+    """A layer called by itself, and rows of the tables that belong to other positions."""
+    x, cos, sin, ck, cv, pos, mask = layer_inputs(model)
+    with torch.no_grad():
+        model.model.layers[0](x, cos, sin, ck, cv, pos, mask)
+        assert "append" not in kernels.calls
+        with pytest.raises(IndexError):
+            model.model.layers[0](x, cos, sin, ck, cv, pos + CFG.max_len - 2, None)
+        decode._note_positions(cos, pos, CFG.max_len)
+        assert decode._inside_cache(cos, pos, ck, cv)
+        assert not decode._inside_cache(cos, pos.clone(), ck, cv) and not decode._inside_cache(cos, pos, ck[:, 1:], cv[:, 1:])
+        pos += CFG.max_len
+        assert not decode._inside_cache(cos, pos, ck, cv)

@@ -657,3 +657,28 @@ def test_transforms_of_several_rows(fp16_out):
         want = mod(*inputs)
         # the kernels round a few times less than the expressions (2^-11 each)
         assert (got.double() - want.double()).norm() <= 4e-3 * want.double().norm()
+
+
+def test_positions_outside_a_short_cache_are_refused(fp16_out):
+    """A cache shorter than the rotary tables: positions inside give what a full cache gives, positions outside raise on the host
+    and touch nothing."""
+    cfg = decode.DecoderConfig(hidden=256, layers=2, heads=4, kv_heads=2, head_dim=64, intermediate=512, vocab=64, max_len=32, rank=32)
+    with torch.device("cuda"):
+        model, _, _ = decode.build_decoder(cfg, seed=6)
+    cos, sin = model.rope_tables("cuda")
+
+    def run(length, first):
+        caches = [tuple(torch.zeros(2, length, 64, dtype=torch.float16, device="cuda") for _ in range(2)) for _ in range(2)]
+        pos = torch.arange(first, first + 5, device="cuda")
+        try:
+            return model.forward_tokens(torch.arange(5, device="cuda"), pos, caches, cos, sin, from_empty_cache=True), caches
+        except IndexError:
+            assert not any(t.any() for pair in caches for t in pair)
+            raise
+
+    (want, full), (got, short) = run(32, 0), run(8, 0)
+    assert torch.equal(got, want)
+    assert all(torch.equal(s, f[:, :8]) for a, b in zip(short, full) for s, f in zip(a, b))
+    for length, first in ((8, 4), (8, 20), (8, -1)):
+        with pytest.raises(IndexError):
+            run(length, first)
