@@ -208,7 +208,7 @@ class W4A16Extension:
         lock = self._stream_locks.get(key)
         return lock if lock is not None else self._stream_locks.setdefault(key, threading.RLock())
 
-    def _workspace(self, dev: torch.device, rows: int):
+    def _workspace(self, dev: torch.device, rows: int, stream: Optional[int] = None):
         """(pointer, bytes) of the workspace of the current stream of `dev`: one per stream, because calls that share
         one must not overlap.  Calls with two and more token rows get the large one (many-row projection, split-K of the
         GEMM and of the skinny kernels, hand-over words of the launches that compute r themselves); single-token calls
@@ -217,7 +217,7 @@ class W4A16Extension:
         its first such call while it is being captured into a graph goes without (the buffer would come from the
         graph's own memory pool)."""
         small = rows <= 1
-        key = (dev.index if dev.index is not None else torch.cuda.current_device(), self._stream(dev), small)
+        key = (dev.index if dev.index is not None else torch.cuda.current_device(), self._stream(dev) if stream is None else stream, small)
         ws = self._workspaces.get(key)
         if ws is None:
             if torch.cuda.is_current_stream_capturing():
@@ -744,7 +744,8 @@ class PreparedGroup:
             _check(R.is_cuda and R.dtype == torch.float16 and R.dim() == 2 and R.is_contiguous()
                    and tuple(R.shape) == (self.rank, self.K), "group: R must be a contiguous CUDA fp16 [rank, K] tensor")
         corrected = self.alpha != 0.0 and any(m.get("L") is not None for m in members)
-        self.arr = (_Member * len(members))()
+        self._array = _Member * len(members)
+        self.arr = self._array()
         self.Ns, self.keep = [], []
         x_probe = torch.empty(0, self.K, dtype=torch.float16, device=dev)
         for e, m in zip(self.arr, members):
@@ -785,7 +786,7 @@ class PreparedGroup:
         old = self._tiled
         versions = list(map(_version_of, self._tiled_from))
         capturing = torch.cuda.is_current_stream_capturing()
-        arr = type(self.arr).from_buffer_copy(self.arr)
+        arr = self._array.from_buffer_copy(self.arr)
         keep = [self.ext._set_tiled(e, k[0], k[1], k[2], k[3] if self.corrected else None, self.K, self.group_size)
                 for e, k in zip(arr, self.keep)]
         streams = set(old[3]) if old is not None and old[2] == versions else set()
@@ -815,7 +816,7 @@ class PreparedGroup:
                     stream not in tiled[3] or tiled[2] != list(map(_version_of, self._tiled_from))):
                 tiled = self._build_tiled(stream)
         # (a copy of the descriptors: other threads may be in the same group)
-        arr = type(self.arr).from_buffer_copy(tiled[0] if tiled is not None else self.arr)
+        arr = self._array.from_buffer_copy(tiled[0] if tiled is not None else self.arr)
         Ns = self.Ns
         widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
         if outs is None:
@@ -845,7 +846,7 @@ class PreparedGroup:
             ctx.__enter__()
         try:
             with ext._enqueue_lock(dev, stream):
-                ws, ws_bytes = ext._workspace(dev, M)
+                ws, ws_bytes = ext._workspace(dev, M, stream)
                 if fused:
                     rc = self.lib.glowq_w4a16_group_forward_fused_ws(
                         x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
