@@ -777,6 +777,7 @@ class PreparedGroup:
         # In-place writes (load_state_dict among them) raise the versions, and the next call makes the copies again.  Replaced
         # as a whole, so that a thread sees one state.
         self._tiled = None
+        self._widens_below = 1 << 31  # token rows from which the library has refused fp32 outputs
         self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
         self._n_total = sum(self.Ns)
 
@@ -818,7 +819,8 @@ class PreparedGroup:
         # (a copy of the descriptors: other threads may be in the same group)
         arr = self._array.from_buffer_copy(tiled[0] if tiled is not None else self.arr)
         Ns = self.Ns
-        widen = out_dtype is torch.float32 and outs is None and M >= GEMM_MIN_ROWS
+        # only the GEMM on the tiled copies widens, and a call of so many rows that it was refused is not asked again
+        widen = out_dtype is torch.float32 and outs is None and GEMM_MIN_ROWS <= M < self._widens_below and tiled is not None and all(tiled[1])
         if outs is None:
             outs = [torch.empty((M, N), dtype=torch.float32 if widen else torch.float16, device=dev) for N in Ns]
         else:
@@ -859,6 +861,7 @@ class PreparedGroup:
             if ctx is not None:
                 ctx.__exit__(None, None, None)
         if rc == EUNSUPPORTED and widen:  # not the GEMM's call: nothing has been launched
+            self._widens_below = M
             return self.run(x, r=r, project=project)
         if rc:
             ext._raise(rc, "w4a16_group_forward")

@@ -8,6 +8,7 @@ import torch.nn as nn
 import glowq_oracle as oracle
 from glowq_amd import correction as corr
 from glowq_amd import linear
+from glowq_amd.kernels import EUNSUPPORTED, Y_FP32
 from helpers import assert_close
 from test_host import Toy, toy_artifacts
 
@@ -238,3 +239,41 @@ def test_fp32_outputs_are_the_fp16_results_widened(monkeypatch, rows, K, Ns, gs)
     for a, b in zip(got["fp16"], got["fp32"]):
         assert a.dtype == torch.float16 and b.dtype == torch.float32
         assert torch.equal(a.float(), b)
+
+
+class Counting:
+    """The library with its group calls counted, and fp32 outputs refused if asked to."""
+
+    def __init__(self, lib, refuse):
+        self.lib, self.refuse, self.calls = lib, refuse, 0
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+        if not name.startswith("glowq_w4a16_group_forward"):
+            return fn
+
+        def call(*args):
+            self.calls += 1
+            if self.refuse and any(getattr(e, "y_type", 0) == Y_FP32 for e in args[2]):
+                return EUNSUPPORTED
+            return fn(*args)
+        return call
+
+
+@pytest.mark.parametrize("K,refuse,first", [(384, False, 1), (512, False, 1), (512, True, 2)])
+def test_fp32_outputs_are_not_asked_for_again_where_they_are_refused(monkeypatch, K, refuse, first):
+    """Without a tiled copy (K % 256) the fp16 call is made at once; a refusal for another reason is remembered."""
+    monkeypatch.setenv("W4A16_KERNEL_OUT_DTYPE", "fp32")
+    torch.manual_seed(K)
+    mod = linear.CudaW4A16Linear.from_float(nn.Linear(K, 96, bias=True).half(), 128).cuda()
+    x = torch.randn(100, K).half()
+    want = _ref(x.numpy(), mod)
+    with torch.no_grad():
+        linear.refresh_env_knobs()
+        group = mod._bare_group()
+        group.lib = Counting(group.lib, refuse)
+        for calls in (first, first + 1, first + 2):
+            y = mod(x.cuda())
+            assert group.lib.calls == calls
+            assert y.dtype == torch.float32
+            assert_close(y.cpu().numpy(), want, f"K={K}")
