@@ -335,9 +335,11 @@ class W4A16Extension:
     def _packed_copy(self, sources, shape_key, nbytes: int, pack) -> Optional[_Packed]:
         """The copy of `sources` kept on the first of them, made by `pack(out, stream)` where there is none or a source has been
         written to since.  After a write the copy is made again in its old place, so that launches recorded into graphs read
-        the new one too.  Where it would have to be made under a graph capture (it would come from the graph's own memory
+        the new one too.  None for inference tensors, whose writes torch does not count.  Where it would have to be made under a graph capture (it would come from the graph's own memory
         pool, or be made at every replay) and where this stream cannot wait for it: False, for now."""
         owner = sources[0]
+        if any(t.is_inference() for t in sources):
+            return None
         with self._pack_lock:
             ptrs, versions = [t.data_ptr() for t in sources], [t._version for t in sources]
             shape_key += (nbytes,)
@@ -779,6 +781,7 @@ class PreparedGroup:
         self._tiled = None
         self._widens_below = 1 << 31  # token rows from which the library has refused fp32 outputs
         self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
+        self._may_tile = not any(t.is_inference() for t in self._tiled_from)  # (an inference tensor has no version)
         self._n_total = sum(self.Ns)
 
     def _build_tiled(self, stream):
@@ -811,7 +814,7 @@ class PreparedGroup:
         stream = ext._stream(dev)
         # From 65 rows a recorded launch without correction reads the weights themselves: a graph then follows writes to them by
         # itself, where one that reads the copies needs a call outside the graph to bring them up to date.
-        if M >= TILED_MIN_ROWS and not (M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing()):
+        if self._may_tile and M >= TILED_MIN_ROWS and not (M >= GEMM_MIN_ROWS and not self.corrected and torch.cuda.is_current_stream_capturing()):
             tiled = self._tiled
             if (ext.wants_tiled(M, self.K, self._n_total, self.group_size, self.arr[0].ldw_i32) if tiled is None else
                     stream not in tiled[3] or tiled[2] != list(map(_version_of, self._tiled_from))):

@@ -277,3 +277,18 @@ def test_fp32_outputs_are_not_asked_for_again_where_they_are_refused(monkeypatch
             assert group.lib.calls == calls
             assert y.dtype == torch.float32
             assert_close(y.cpu().numpy(), want, f"K={K}")
+
+
+@pytest.mark.parametrize("rows", [5, 64, 65, 300])
+def test_linear_made_in_inference_mode(fp16_out, rows):
+    """Inference tensors have no version to tell writes by: such a module stays on its canonical buffers."""
+    torch.manual_seed(0)
+    with torch.inference_mode():
+        mod = linear.CudaW4A16Linear.from_float(nn.Linear(512, 96, bias=True).half(), 128).cuda()
+        assert mod.qweight_i32.is_inference()
+    x = torch.randn(rows, 512).half()
+    for again in range(2):
+        assert_close(mod(x.cuda()).cpu().numpy(), _ref(x.numpy(), mod), f"{rows} rows")
+    with torch.inference_mode():
+        mod.scales_f16.mul_(2.0)
+        assert_close(mod(x.cuda()).cpu().numpy(), _ref(x.numpy(), mod), f"{rows} rows, in inference mode")
