@@ -230,6 +230,11 @@ class CudaW4A16Linear(nn.Module):
             self._prepared = prepared = (key, PreparedGroup(self._get_ext(), [member], self.in_features, self.group_size, 0.0))
         return prepared[1]
 
+    def _plain_buffers(self) -> bool:
+        """Contiguous buffers of at least one output; the GEMM entry point also takes others."""
+        return (self.out_features > 0 and self.qweight_i32.is_contiguous() and self.scales_f16.is_contiguous()
+                and self.qzeros_i32.is_contiguous())
+
     def _prefer_gemv(self, m: int) -> bool:
         KNOBS.sync()
         if KNOBS.force_gemm:
@@ -255,8 +260,8 @@ class CudaW4A16Linear(nn.Module):
         self._require_gpu(x2d)
         KNOBS.sync()
         m = x2d.size(0)
-        if KNOBS.force_gemm or (m <= DEFAULT_GEMV_M_MAX and not self._prefer_gemv(m)):
-            # the GEMM entry point asked for where the row count alone would not take it
+        if KNOBS.force_gemm or (not self._prefer_gemv(m) if m <= DEFAULT_GEMV_M_MAX else not self._plain_buffers()):
+            # the GEMM entry point asked for where the row count alone would not take it, or buffers that descriptors do not take
             out = self._get_ext().w4a16_gemm_forward_cuda(x2d, self.qweight_i32, self.scales_f16, self.qzeros_i32,
                                                           self.group_size, KNOBS.split_k_iters)
             return self._finish(out, lead)

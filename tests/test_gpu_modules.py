@@ -292,3 +292,22 @@ def test_linear_made_in_inference_mode(fp16_out, rows):
     with torch.inference_mode():
         mod.scales_f16.mul_(2.0)
         assert_close(mod(x.cuda()).cpu().numpy(), _ref(x.numpy(), mod), f"{rows} rows, in inference mode")
+
+
+@pytest.mark.parametrize("rows", [65, 300])
+def test_buffers_that_are_not_contiguous(fp16_out, rows):
+    """From 65 rows the GEMM entry point serves them (with copies of its own), as before 65 rows had prepared descriptors."""
+    torch.manual_seed(0)
+    mod = linear.CudaW4A16Linear.from_float(nn.Linear(512, 96, bias=True).half(), 128).cuda()
+    x = torch.randn(rows, 512).half()
+    want = mod(x.cuda())
+    for name in ("qweight_i32", "scales_f16", "qzeros_i32"):
+        buf = getattr(mod, name)
+        wide = torch.empty(buf.size(0), buf.size(1) + 3, dtype=buf.dtype, device="cuda")
+        wide[:, :buf.size(1)] = buf
+        setattr(mod, name, wide[:, :buf.size(1)])
+        assert not getattr(mod, name).is_contiguous()
+        # (another cut of K, hence another rounding of a few outputs)
+        assert_close(mod(x.cuda()).cpu().numpy(), want.cpu().numpy(), name)
+    none = linear.CudaW4A16Linear(512, 0).cuda()
+    assert none(x.cuda()).shape == (rows, 0)
