@@ -27,12 +27,10 @@ from typing import Dict, Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-import torch.overrides
-import torch.utils._device
 
 from .correction import AddSVDCorrection, patch_svd_correction_wrappers, patch_svd_correction_wrappers_cumulative
 from .kernels import (CHAIN_ACC_BYTES, CHAIN_EPI_NONE, CHAIN_EPI_RESIDUAL, CHAIN_EPI_SWIGLU, CHAIN_PRO_ACC, CHAIN_PRO_NORM_ACC,
-                      CHAIN_PRO_PLAIN, PreparedGroup, load_w4a16_extension)
+                      CHAIN_PRO_PLAIN, PreparedGroup, load_w4a16_extension, transformed)
 from .linear import CudaW4A16Linear, convert_to_cuda_w4a16, refresh_env_knobs
 
 
@@ -61,20 +59,9 @@ class _Glue:
         self.ext, self.cos_t, self.sin_t, self.pos = ext, cos_t, sin_t, pos
 
 
-# torch has no public way to ask for these; on a torch without one of them everything counts as watched
-_PROBES = (getattr(torch._C, "_are_functorch_transforms_active", None), getattr(torch._C, "_len_torch_dispatch_stack", None),
-           getattr(torch.overrides, "_get_current_function_mode_stack", None))
-_DeviceContext = getattr(torch.utils._device, "DeviceContext", None)
-
-
 def _watched(x) -> bool:
-    """Whether somebody needs to see the tensor expressions on the plain tensor x: gradients in either direction, tracing, function
-    transforms, dispatch or function modes (`torch.set_default_device`, a function mode too, only looks at factories)."""
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled() or None in _PROBES:
-        return True
-    transforms, dispatch_modes, function_modes = _PROBES
-    return (getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or transforms() or dispatch_modes() > 0
-            or (torch.overrides.has_torch_function_unary(x) and any(type(m) is not _DeviceContext for m in function_modes())))
+    """Whether somebody needs to see the tensor expressions on the plain tensor x: gradients, or what `transformed` names."""
+    return torch.is_grad_enabled() or transformed(x)
 
 
 def _several_rows(x) -> bool:

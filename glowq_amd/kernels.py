@@ -22,6 +22,8 @@ from operator import attrgetter
 from typing import List, Optional, Sequence
 
 import torch
+import torch.overrides
+import torch.utils._device
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libglowq_w4a16.so")
@@ -156,6 +158,22 @@ class _Packed:
 
     def __reduce__(self):
         return set, ()  # a deep copy or a saved file of the tensor starts without one
+
+
+# torch has no public way to ask for these; on a torch without one of them everything counts as watched
+_PROBES = (getattr(torch._C, "_are_functorch_transforms_active", None), getattr(torch._C, "_len_torch_dispatch_stack", None),
+           getattr(torch.overrides, "_get_current_function_mode_stack", None))
+_DeviceContext = getattr(torch.utils._device, "DeviceContext", None)
+
+
+def transformed(x) -> bool:
+    """Whether more than autograd's reverse mode may look at the operations on the plain tensor x: tracing, forward-mode, function
+    transforms, dispatch or function modes (`torch.set_default_device`, a function mode too, only looks at factories)."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or None in _PROBES:
+        return True
+    transforms, dispatch_modes, function_modes = _PROBES
+    return (getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or transforms() or dispatch_modes() > 0
+            or (torch.overrides.has_torch_function_unary(x) and any(type(m) is not _DeviceContext for m in function_modes())))
 
 
 def _check(cond: bool, msg: str) -> None:

@@ -23,7 +23,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from .kernels import load_w4a16_extension
+from .kernels import load_w4a16_extension, transformed
 
 _TRUE = {"1", "true", "yes", "y", "on"}
 
@@ -213,12 +213,21 @@ class CudaW4A16Linear(nn.Module):
         bump_generation()
         return super()._apply(fn, *args, **kwargs)
 
-    def _bare_group(self):
+    def _folds_bias(self, m: int) -> bool:
+        """Whether the bias rides in the kernel's epilogue, y = fp16(acc + bias): where the output stays fp16 -- with fp32 output
+        the reference adds it in fp32 after the cast (linear.py:183-186) and so does `_finish` -- and, from 65 rows,
+        where nobody differentiates or transforms the bias, who needs to see the addition."""
+        bias = self.bias
+        if bias is None or KNOBS.out_dtype != torch.float16:
+            return False
+        return m <= DEFAULT_GEMV_M_MAX or not ((bias.requires_grad and torch.is_grad_enabled())
+                                               or type(bias) not in (torch.Tensor, nn.Parameter) or transformed(bias))
+
+    def _bare_group(self, fold_bias: Optional[bool] = None):
         """The module alone as a prepared group (validated once, side stream packed once); rebuilt when a buffer has
         been replaced since."""
-        # the bias rides in the kernel's epilogue, y = fp16(acc + bias), where the output stays fp16; with fp32 output the
-        # reference adds it in fp32 after the cast (linear.py:183-186) and so does `_finish`
-        fold_bias = self.bias is not None and KNOBS.out_dtype == torch.float16
+        if fold_bias is None:
+            fold_bias = self.bias is not None and KNOBS.out_dtype == torch.float16
         key = (self.qweight_i32.data_ptr(), self.scales_f16.data_ptr(), self.qzeros_i32.data_ptr(),
                self.bias.data_ptr() if fold_bias else 0)
         prepared = self._prepared
@@ -268,7 +277,8 @@ class CudaW4A16Linear(nn.Module):
         # Through descriptors validated once (the bias rides in the kernel's epilogue).  From 65 rows this is the same MFMA
         # GEMM as the entry point above, but on the tiled copy of the weights and with the stream's workspace for its splits
         # of K: two 14B layers with half of their groups bare at 1500 rows 2362 -> 2048 us.
-        return self._finish(self._bare_group().run(x2d, out_dtype=KNOBS.out_dtype)[0], lead, bias_applied=KNOBS.out_dtype == torch.float16)
+        fold_bias = self._folds_bias(m)
+        return self._finish(self._bare_group(fold_bias).run(x2d, out_dtype=KNOBS.out_dtype)[0], lead, bias_applied=fold_bias)
 
     def dequantize(self) -> torch.Tensor:
         """fp16 [out_features, in_features] weight, fp16((code - zero) * scale); the device twin of the

@@ -6,6 +6,7 @@ import torch.nn.functional as F
 from torch.overrides import TorchFunctionMode
 
 from glowq_amd import decode
+from glowq_amd import kernels as kernels_module
 
 CFG = decode.DecoderConfig(hidden=64, layers=1, heads=4, kv_heads=2, head_dim=16, intermediate=128, vocab=32, max_len=24)
 
@@ -125,7 +126,7 @@ def test_function_modes_see_the_expressions(model, kernels):
 
 
 def test_a_torch_without_the_probes_takes_the_expressions(model, kernels, monkeypatch):
-    monkeypatch.setattr(decode, "_PROBES", (None,) + decode._PROBES[1:])
+    monkeypatch.setattr(kernels_module, "_PROBES", (None,) + kernels_module._PROBES[1:])
     forward(model)
     assert kernels.calls == []
 

@@ -311,3 +311,29 @@ def test_buffers_that_are_not_contiguous(fp16_out, rows):
         assert_close(mod(x.cuda()).cpu().numpy(), want.cpu().numpy(), name)
     none = linear.CudaW4A16Linear(512, 0).cuda()
     assert none(x.cuda()).shape == (rows, 0)
+
+
+@pytest.mark.parametrize("rows", [65, 300])
+def test_bias_of_a_bare_linear_is_differentiable(monkeypatch, rows):
+    """From 65 rows the bias of an fp16 output is added where autograd, forward-mode and function transforms see it."""
+    monkeypatch.setenv("W4A16_KERNEL_OUT_DTYPE", "fp16")
+    torch.manual_seed(0)
+    mod = linear.CudaW4A16Linear.from_float(nn.Linear(512, 96, bias=True).half(), 128).cuda()
+    x = torch.randn(rows, 512).half().cuda()
+    y = mod(x)
+    y.sum().backward()
+    assert torch.equal(mod.bias.grad, torch.full_like(mod.bias, rows))
+    with torch.no_grad():
+        folded = mod(x)
+    assert not folded.requires_grad
+    assert_close(y.detach().cpu().numpy(), folded.cpu().numpy(), "added and folded")
+    mod.bias.requires_grad_(False)
+    assert torch.equal(mod(x), folded)  # nobody differentiates it: folded
+    biases = torch.stack((mod.bias, 2 * mod.bias))
+    with torch.no_grad():
+        many = torch.func.vmap(lambda b: torch.func.functional_call(mod, {"bias": b}, (x,)))(biases)
+    assert_close(many[0].cpu().numpy(), folded.cpu().numpy(), "one of several biases")
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(mod.bias.detach(), torch.ones_like(mod.bias))
+        out = torch.func.functional_call(mod, {"bias": dual}, (x,))
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(out).tangent, torch.ones_like(out))
