@@ -1049,6 +1049,7 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   static const int mt_max = getenv("GLOWQ_GEMM_MT") ? atoi(getenv("GLOWQ_GEMM_MT")) : 4;
   int mt_cap = M > 128 ? 8 : (M > 64 ? 4 : (M > 32 ? 2 : 1));
   if (mt_cap > mt_max) mt_cap = mt_max;
+  if (y32 && mt_cap > 4) mt_cap = 4;  // (256-row tiles are there for measurements, without fp32 outputs)
   static const int order[6][2] = {{4, 2}, {2, 2}, {4, 1}, {2, 1}, {1, 2}, {1, 1}};
   int mt = 1, nt = 1;
   long best = -1;
@@ -1184,11 +1185,12 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
 #define GLOWQ_GEMM_TILED_CASE(MT, NT, WK)                                                  \
   if (tiled_ok && mt == MT && nt == NT && wk == WK)                                        \
     return y32 ? launch_gemm_t<MT, NT, true, true, true, WK, float>(gg, stream) : launch_gemm_t<MT, NT, true, true, true, WK>(gg, stream);
-  GLOWQ_GEMM_TILED_CASE(8, 2, 1) GLOWQ_GEMM_TILED_CASE(4, 2, 1) GLOWQ_GEMM_TILED_CASE(2, 2, 1) GLOWQ_GEMM_TILED_CASE(1, 2, 1)
-  GLOWQ_GEMM_TILED_CASE(8, 1, 1) GLOWQ_GEMM_TILED_CASE(4, 1, 1) GLOWQ_GEMM_TILED_CASE(2, 1, 1) GLOWQ_GEMM_TILED_CASE(1, 1, 1)
-  GLOWQ_GEMM_TILED_CASE(4, 2, 2) GLOWQ_GEMM_TILED_CASE(2, 1, 2)
+  GLOWQ_GEMM_TILED_CASE(4, 2, 1) GLOWQ_GEMM_TILED_CASE(2, 2, 1) GLOWQ_GEMM_TILED_CASE(1, 2, 1) GLOWQ_GEMM_TILED_CASE(4, 1, 1)
+  GLOWQ_GEMM_TILED_CASE(2, 1, 1) GLOWQ_GEMM_TILED_CASE(1, 1, 1) GLOWQ_GEMM_TILED_CASE(4, 2, 2) GLOWQ_GEMM_TILED_CASE(2, 1, 2)
 #undef GLOWQ_GEMM_TILED_CASE
   if (y32) return hipErrorInvalidValue;  // (gemm_widens said no)
+  if (tiled_ok && mt == 8 && nt == 2) return launch_gemm_t<8, 2, true, true, true>(gg, stream);
+  if (tiled_ok && mt == 8 && nt == 1) return launch_gemm_t<8, 1, true, true, true>(gg, stream);
 #define GLOWQ_GEMM_CASE(MT, NT)                                                            \
   if (mt == MT && nt == NT) return super ? launch_gemm_t<MT, NT, true, true>(gg, stream) : launch_gemm_t<MT, NT, true>(gg, stream);
   GLOWQ_GEMM_CASE(8, 2) GLOWQ_GEMM_CASE(4, 2) GLOWQ_GEMM_CASE(2, 2) GLOWQ_GEMM_CASE(1, 2)
