@@ -952,7 +952,6 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   if (kWk > 1 && lds < (size_t)BM * BN * sizeof(float)) lds = (size_t)BM * BN * sizeof(float);  // the hand-over of the accumulators
   static LdsLimit lds_limit;
   if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
-  note_launch(0, 0, 256 * kWk, "%s<%d,%d,%d>", kTiled ? "gemm_tiled_kernel" : "gemm_mfma_kernel", kMT, kNT, kWk);
   const int m_blocks = (gg.m[0].M + BM - 1) / BM;
   int total = 0;
   for (int i = 0; i < gg.n; ++i) {
@@ -961,9 +960,12 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   }
   if (!(kQuant && kSuper)) gg.slices = 1;
   if (!(kQuant && kSuper) || gg.slices > 1 || gg.tail_slices < 2 || gg.full < 0 || gg.full >= total) gg.tail_slices = 0;
-  if (gg.tail_slices > 1) {
+  const int tail_wgs = gg.tail_slices > 1 ? gg.full + (total - gg.full) * gg.tail_slices : 0;
+  note_launch(tail_wgs > 0 ? tail_wgs : total, tail_wgs > 0 ? 1 : gg.slices, 256 * kWk, "%s<%d,%d,%d%s>",
+              kTiled ? "gemm_tiled_kernel" : "gemm_mfma_kernel", kMT, kNT, kWk, std::is_same_v<YT, float> ? ",float" : "");
+  if (tail_wgs > 0) {
     const int tail_tiles = total - gg.full;
-    hipLaunchKernelGGL(kern, dim3(gg.full + tail_tiles * gg.tail_slices, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
+    hipLaunchKernelGGL(kern, dim3(tail_wgs, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(tail_tiles, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
     return hipGetLastError();
@@ -1560,8 +1562,9 @@ static hipError_t launch_proj_tile(const half_t* x, const half_t* R, half_t* r, 
   constexpr size_t lds = (size_t)2 * (128 * kA) * kTRow;
   static LdsLimit lds_limit;
   if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((M + 64 * kA - 1) / (64 * kA), (rank + 64 * kA - 1) / (64 * kA), slices), dim3(256), lds, stream, x, R, r, ws, M, K,
-                     rank);
+  const int row_tiles = (M + 64 * kA - 1) / (64 * kA), col_tiles = (rank + 64 * kA - 1) / (64 * kA);
+  note_launch(row_tiles * col_tiles, slices, 256, "proj_tile_kernel<%d>", kA);
+  hipLaunchKernelGGL(kern, dim3(row_tiles, col_tiles, slices), dim3(256), lds, stream, x, R, r, ws, M, K, rank);
   if (hipError_t e = hipGetLastError(); e != hipSuccess || slices == 1) return e;
   const long n4 = (long)M * rank / 4;
   hipLaunchKernelGGL(proj_sum_kernel, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, stream, ws, r, n4, slices);
@@ -1684,6 +1687,7 @@ hipError_t launch_shared_proj_mfma(const half_t* x, const half_t* R, half_t* r, 
     if (t.a == 1) return launch_proj_tile<1>(x, R, r, M, K, rank, t.slices, static_cast<float*>(ws), stream);
     if (t.a == 2) return launch_proj_tile<2>(x, R, r, M, K, rank, t.slices, static_cast<float*>(ws), stream);
   }
+  note_launch((M + 31) / 32 * ((rank + 32 * p.nt - 1) / (32 * p.nt)), p.slices, 256, "proj_mfma_kernel<%d>", p.nt);
   if (p.nt == 2) return launch_proj_t<2>(x, R, r, M, K, rank, p.slices, ws, stream);
   return launch_proj_t<1>(x, R, r, M, K, rank, p.slices, ws, stream);
 }

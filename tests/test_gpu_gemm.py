@@ -359,3 +359,76 @@ def test_shared_proj_tiles(ext, M, K, rank):
     finally:
         ext.WORKSPACE_BYTES = saved
         ext._workspaces.clear()
+
+
+@pytest.mark.parametrize("M,K,Ns,rank,kernel,grid", [
+    (333, 4096, [2900], 32, "gemm_tiled_kernel<1,1,1>", [253, 1]),
+    (700, 2048, [8100], 64, "gemm_tiled_kernel<2,1,1>", [704, 1]),
+    (333, 3584, [3584, 512, 500], 128, "gemm_tiled_kernel<2,1,2>", [216, 1]),
+    (1200, 4096, [6000], 0, "gemm_tiled_kernel<2,2,1>", [456, 1]),
+    (333, 3584, [18900, 18980], 128, "gemm_tiled_kernel<4,2,1>", [447, 1]),
+    (333, 18944, [3500], 128, "gemm_tiled_kernel<4,2,1>", [42, 6]),             # six slices of K and their sum
+    (1500, 5120, [5100, 1000], 0, "gemm_tiled_kernel<4,2,1>", [480, 1]),        # 256 whole tiles, 32 cut into seven
+    (2000, 18944, [3500], 0, "gemm_tiled_kernel<4,2,2>", [224, 1])])
+@pytest.mark.parametrize("bias", [False, True])
+def test_fp32_outputs_of_every_cut(ext, M, K, Ns, rank, kernel, grid, bias):
+    """Tiles inside the output, ragged last rows and columns and sums of slices, stored as fp32: the fp16 results widened, and
+    those as close to 64 bits as the rounding of the output and the fp32 sums leave them."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half() if rank else None
+    members, mods = [], []
+    for N in Ns:
+        lin = torch.nn.Linear(K, N, bias=True, device="cuda", dtype=torch.float16)
+        with torch.no_grad():
+            lin.weight.normal_(0.0, 0.02, generator=g)
+        mod = CudaW4A16Linear.from_float(lin, 128)
+        L = (torch.randn(N, rank, device="cuda", generator=g) * 0.01).half() if rank else None
+        mods.append(mod)
+        members.append({"qweight": mod.qweight_i32, "scales": mod.scales_f16, "qzeros": mod.qzeros_i32, "L": L,
+                        "bias": mod.bias.data if bias else None})
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if rank else 0.0, R=R)
+    y16 = pg.run(x)
+    assert ext.last_launch()["kernel"] == kernel and ext.last_launch()["grid"] == grid
+    y32 = pg.run(x, out_dtype=torch.float32)
+    assert ext.last_launch()["kernel"] == kernel[:-1] + ",float>" and ext.last_launch()["grid"] == grid
+    for a, b, mod, m in zip(y16, y32, mods, members):
+        assert a.dtype == torch.float16 and b.dtype == torch.float32 and torch.equal(a.float(), b)
+        want = x.double() @ mod.dequantize().double().t()
+        if rank:
+            want += (x.double() @ R.double().t()) @ m["L"].double().t()
+        if bias:
+            want += m["bias"].double()
+        assert ((a.double() - want).abs() <= 1e-2 + 1e-3 * want.abs()).all()
+        # |dequantised weight| < 0.1, K terms: fp16 output 2^-11, fp32 sums far below
+        assert (a.double() - want).norm() <= 1e-3 * want.norm()
+
+
+@pytest.mark.parametrize("M,K,rank,kernel,grid", [
+    (1500, 17408, 256, "proj_tile_kernel<2>", [24, 10]), (1500, 17408, 252, "proj_tile_kernel<2>", [24, 10]),
+    (1001, 18944, 260, "proj_tile_kernel<2>", [24, 10]), (1900, 18944, 132, "proj_tile_kernel<2>", [30, 8]),
+    (1000, 18944, 256, "proj_tile_kernel<2>", [16, 15]), (700, 17408, 256, "proj_tile_kernel<1>", [44, 10]),
+    (1300, 12288, 200, "proj_tile_kernel<1>", [84, 6]), (2048, 5120, 256, "proj_mfma_kernel<2>", [256, 1])])
+def test_large_shared_projections(ext, M, K, rank, kernel, grid):
+    """The 128 x 128 tiles of the projection and their neighbours, on rows and ranks that end inside a tile: all of r against
+    64 bits, and every cut that a smaller workspace leaves."""
+    g = torch.Generator(device="cuda").manual_seed(M + rank)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half()
+    want = x.double() @ R.double().t()
+    saved = ext.WORKSPACE_BYTES
+    try:
+        for nbytes in (saved, 6 * M * rank * 4, 3 * M * rank * 4, 16):
+            ext.WORKSPACE_BYTES = nbytes
+            ext._workspaces.clear()
+            # (guard rows behind r: nothing past its end is written)
+            out = torch.full((M + 130, rank), 7.0, dtype=torch.float16, device="cuda")
+            r = ext.shared_proj(x, R, out=out[:M])
+            if nbytes == saved:
+                assert ext.last_launch()["kernel"] == kernel and ext.last_launch()["grid"] == grid
+            # one rounding to fp16 (2^-11), fp32 sums of K terms around K^-1/2: 1e-4 is ten times their error
+            assert ((r.double() - want).abs() <= 2.0 ** -11 * want.abs() + 1e-4).all()
+            assert (out[M:] == 7.0).all()
+    finally:
+        ext.WORKSPACE_BYTES = saved
+        ext._workspaces.clear()
