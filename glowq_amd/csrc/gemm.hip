@@ -863,7 +863,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   }
   if (m0 + BM <= a.M && (bn + 1) * BN <= a.N) {
     // A tile inside the output: no test per element, and a row's address is a scalar base plus one lane offset for all of them.
-    // With a test and a 64-bit address per element the 32 kMT kNT stores of a wave are some twelve instructions each, 3 to 6 us of
+    // With a test and a 64-bit address per element the 16 kMT kNT stores of a wave are some twelve instructions each, 3 to 6 us of
     // a tile that takes 50 (Qwen2.5-7B layer at 2048 rows 965 -> 928 us, 8B o_proj at 2048 rows 74.5 -> 69.5).
     YT* corner = reinterpret_cast<YT*>(a.y) + (size_t)m0 * a.ldy + (bn * BN + wave * (32 * kNT));
     const uint32_t lane_off = (uint32_t)(4 * lh) * (uint32_t)a.ldy + (uint32_t)ln;
@@ -1151,10 +1151,11 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   // From 65 rows on the tiled copy the cut above stands unless another one is predicted 9 % faster: the choice above fills the
   // chip with tiles first and cuts K only where that leaves most of it idle, but up to about a thousand rows one round of
   // workgroups made of smaller tiles and slices of K is often the shorter way (8B o_proj at 100 rows 18.4 -> 15.1 us, down_proj
-  // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  Over the timings behind kGemmCost this takes
-  // 9 % off the mean and costs nowhere more than 1 %; without the margin it costs more than that on 30 pairs of 250.  Cuts that
-  // send more than 32 MB of fp32 tiles through the workspace are not tried: from there the fit scatters by 7 to 11 %
-  // (standard deviation) instead of 3 to 5.
+  // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  With and without this rule, 21 groups of 1.5B
+  // to 14B shapes at 12 row counts: 82 of 189 pairs at 72 to 1024 rows get another cut, 1.25 times as fast in the mean and the
+  // least of them 1.5 % faster; of 63 pairs at 1200 to 2048 rows, past the rows of the fit, 6 do (1.05 to 1.19 times).
+  // Without the margin the rule costs more than 1 % on 30 pairs of the fit.  Cuts that send more than 32 MB of fp32 tiles through
+  // the workspace are not tried: from there the fit scatters by 7 to 11 % (standard deviation) instead of 3 to 5.
   if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
     const int sb_total = gg.m[0].K >> 8;
     float best_us = 0.f;
@@ -1452,7 +1453,7 @@ __global__ __launch_bounds__(256) void proj_reduce_kernel(const float* __restric
   if (m < M && n < rank) r[(size_t)m * rank + n] = (half_t)v;
 }
 
-// ---- shared projection, 65 rows and more: tiles of 64 x 64 or 128 x 128, both operands through LDS --------------------
+// ---- shared projection of many rows: tiles of 64 x 64 or 128 x 128, both operands through LDS --------------------
 // proj_mfma_kernel's 32-row tiles read R once per 32 rows and x once per 32 or 64 columns, 16 or 8 products for every element
 // that a compute unit pulls in, two blocks in flight.  Here a workgroup of four waves (two by two) takes 64 kA rows of x and 64 kB rows
 // of R in stages of 128 columns that go from memory straight into LDS (kSt stages in a ring, swizzled like the activations of
@@ -1534,7 +1535,8 @@ __global__ __launch_bounds__(256) void proj_tile_kernel(const half_t* __restrict
     }
 }
 
-// r = fp16(sum of the slices in slice order); four elements to a thread, one wave to a workgroup (a few hundred waves at most)
+// r = fp16(sum of the slices in slice order); four elements to a thread, one wave to a workgroup (rank 128 at 100 rows: 50
+// of them, rank 256 at 1500 rows: 1500)
 __global__ __launch_bounds__(64) void proj_sum_kernel(const float* __restrict__ partials, half_t* __restrict__ r, long n4, int slices) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n4) return;
@@ -1613,7 +1615,10 @@ static ProjPlan plan_proj(int M, int K, int rank, int num_cus, size_t ws_bytes) 
 // Which of the two kernels, and how the tiles are cut: by what they are predicted to take, in us -- fits over 204 (M, K, rank),
 // 65 to 2048 rows, 7 % rms, of the same form as kGemmCost: a block (256 columns) or stage (128) of K on the first workgroup of
 // a compute unit, on every further one, the second launch, its walk over the slices, the traffic of the fp32 tiles, x.  The
-// tile kernel has to be 7 % ahead; by that rule it takes 18 % off the mean and loses nowhere by more than 1 %.  us, this / 32-row tiles:
+// tile kernel has to be 7 % ahead.  With and without the rule, 12 (K, rank) at 65 to 2048 rows: it takes 87 of 132, 1.32 times as
+// fast in the mean and the least of them 3 % faster.  The plan is also asked at 21 to 64 rows where the small kernel is not used
+// (proj_on_small_kernel), which extrapolates the fit: at 48 rows 1.11 and 1.24 times as fast on the two shapes it gets
+// there (K = 18944 rank 128, K = 17408 rank 256).  us, this / 32-row tiles:
 // K = 18944, rank 128 at 100 / 333 / 2048 rows 11.1 / 14.7, 15.3 / 21.1, 30 / 37; K = 17408, rank 256 at 200 / 1500 rows 14.4 / 26.9,
 // 34 / 78; K = 4096, rank 128 at 100 / 1500 rows 7.3 / 8.6, 12.0 / 17.1; K = 1536, rank 256 at 512 rows 8.9 / 6.9 (not taken).
 struct ProjTilePlan {
