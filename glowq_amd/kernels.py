@@ -15,6 +15,7 @@ library raises, as the reference's loader does (kernels.py:24-32).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -125,16 +126,20 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda id
 _version_of = attrgetter("_version")
 
 
+_SAME_DEVICE = contextlib.nullcontext()  # instead of `torch.cuda.device` where the device is the current one: 3 us less
+
+
 class _Packed:
-    """A packed copy `out` of a few tensors, kept on the first of them.  `key` says what it was made from: addresses and
-    versions (every in-place write through torch raises a tensor's version), so that a write to a source is seen.  Holding the
-    other sources keeps their addresses from being given to new tensors.  The copy is made on the stream `home`; other streams
-    wait for it before their first read (`ready_on`)."""
+    """A packed copy `out` of a tensor and `others`, kept on the tensor.  `key` says where they lie and how they are packed,
+    `versions` what was in them (every in-place write through torch raises a tensor's version), so that a write is seen.
+    Holding the others keeps their addresses from being given to new tensors.  The copy is made on the stream `home`
+    (handle `handle`); other streams wait for it before their first read (`ready_on`)."""
 
-    __slots__ = ("key", "others", "out", "home", "handle", "event", "waited")
+    __slots__ = ("key", "versions", "others", "out", "home", "handle", "event", "waited")
 
-    def __init__(self, key, others, out, home, handle, event):
-        self.key, self.others, self.out, self.home, self.handle, self.event, self.waited = key, others, out, home, handle, event, ()
+    def __init__(self, key, versions, others, out, home, handle, event):
+        self.key, self.versions, self.others, self.out = key, versions, others, out
+        self.home, self.handle, self.event, self.waited = home, handle, event, ()
 
     def ready_on(self, stream) -> bool:
         """Orders the current stream of the copy's device (handle `stream`) behind the packing; False where that cannot be.
@@ -350,37 +355,28 @@ class W4A16Extension:
             self._raise(rc, "pack_side")
         return out
 
-    def _packed_copy(self, sources, shape_key, nbytes: int, pack) -> Optional[_Packed]:
-        """The copy of `sources` kept on the first of them, made by `pack(out, stream)` where there is none or a source has been
-        written to since.  After a write the copy is made again in its old place, so that launches recorded into graphs read
-        the new one too.  None for inference tensors, whose writes torch does not count.  Where it would have to be made under a graph capture (it would come from the graph's own memory
-        pool, or be made at every replay) and where this stream cannot wait for it: False, for now."""
-        owner = sources[0]
-        if any(t.is_inference() for t in sources):
-            return None
+    def _packed_copy(self, owner, others, key, versions, nbytes: int, pack) -> Optional[_Packed]:
+        """The copy kept on `owner` of that tensor and `others`, made by `pack(out, stream)` where there is none or one of them has
+        been written to since.  After a write the copy is made again in its old place, so that launches recorded into graphs read
+        the new one too.  Where it would have to be made under a graph capture (it would come from the graph's own memory pool, or be
+        made at every replay) and where this stream cannot wait for it: False, for now."""
+        dev = owner.device
         with self._pack_lock:
-            ptrs, versions = [t.data_ptr() for t in sources], [t._version for t in sources]
-            shape_key += (nbytes,)
-            key = (ptrs, versions, shape_key)
             hit = getattr(owner, "_glowq_tiled", None)
-            if not isinstance(hit, _Packed):
+            if not isinstance(hit, _Packed) or hit.key != key:
                 hit = None
-            stream = self._stream(owner.device)
-            if hit is not None and hit.key == key:
+            stream = self._stream(dev)
+            if hit is not None and hit.versions == versions:
                 return hit if hit.ready_on(stream) else False
             if torch.cuda.is_current_stream_capturing():
                 return False
-            if hit is not None and hit.key[0] == ptrs and hit.key[2] == shape_key:
-                out = hit.out
-            else:
-                out = torch.empty(nbytes, dtype=torch.uint8, device=owner.device)
-            with torch.cuda.device(owner.device):
+            out = hit.out if hit is not None else torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            with _SAME_DEVICE if dev.index == torch.cuda.current_device() else torch.cuda.device(dev):
                 rc = pack(out.data_ptr(), stream)
                 if rc:
                     self._raise(rc, "pack_tiled")
-                home, event = self._home(owner.device, stream)
-                packed = _Packed(key, sources[1:], out, home, stream, event)
-            owner._glowq_tiled = packed
+                home, event = self._home(dev, stream)
+            packed = owner._glowq_tiled = _Packed(key, versions, others, out, home, stream, event)
             return packed
 
     def _packed_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[_Packed]:
@@ -392,10 +388,15 @@ class W4A16Extension:
             return None
         _check(qweight.dtype == torch.int32 and scales.dtype == torch.float16 and qzeros.dtype == torch.int32 and
                qweight.is_contiguous() and scales.is_contiguous() and qzeros.is_contiguous(), "pack_tiled: contiguous canonical buffers")
+        try:
+            versions = (qweight._version, scales._version, qzeros._version)
+        except RuntimeError:
+            return None  # inference tensors, whose writes torch does not count
+        q, s, z = qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr()
         return self._packed_copy(
-            (qweight, scales, qzeros), (int(in_features), int(group_size)), nbytes,
-            lambda out, stream: self.lib.glowq_pack_tiled(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), out, N, int(in_features),
-                                                          int(group_size), qweight.size(1), scales.size(1), qzeros.size(1), stream))
+            qweight, (scales, qzeros), (q, s, z, int(in_features), int(group_size), nbytes), versions, nbytes,
+            lambda out, stream: self.lib.glowq_pack_tiled(q, s, z, out, N, int(in_features), int(group_size), qweight.size(1),
+                                                          scales.size(1), qzeros.size(1), stream))
 
     def _packed_tiled_left(self, L) -> Optional[_Packed]:
         if not tiled_enabled() or L is None or not L.is_cuda:
@@ -405,8 +406,13 @@ class W4A16Extension:
         if nbytes == 0:
             return None
         _check(L.dtype == torch.float16 and L.is_contiguous(), "pack_tiled_left: contiguous fp16 [OC, rank]")
-        return self._packed_copy((L,), (int(N), int(rank)), nbytes,
-                                 lambda out, stream: self.lib.glowq_pack_tiled_left(L.data_ptr(), out, int(N), int(rank), stream))
+        try:
+            version = L._version
+        except RuntimeError:
+            return None
+        ptr = L.data_ptr()
+        return self._packed_copy(L, (), (ptr, int(N), int(rank)), version, nbytes,
+                                 lambda out, stream: self.lib.glowq_pack_tiled_left(ptr, out, int(N), int(rank), stream))
 
     def pack_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[torch.Tensor]:
         """The tiled copy of a member's weights for the matrix-core routes (a uint8 tensor; layout in csrc/tiled.hpp), or
@@ -799,7 +805,10 @@ class PreparedGroup:
         self._tiled = None
         self._widens_below = 1 << 31  # token rows from which the library has refused fp32 outputs
         self._tiled_from = [t for k in self.keep for t in (k[:4] if corrected else k[:3]) if t is not None]
-        self._may_tile = not any(t.is_inference() for t in self._tiled_from)  # (an inference tensor has no version)
+        try:
+            self._may_tile = bool(list(map(_version_of, self._tiled_from)))
+        except RuntimeError:
+            self._may_tile = False  # an inference tensor has no version
         self._n_total = sum(self.Ns)
 
     def _build_tiled(self, stream):
