@@ -121,6 +121,8 @@ def tiled_enabled() -> bool:
 # The raw handle of torch's current stream of a device: the accessor behind `torch.cuda.current_stream(dev).cuda_stream`,
 # without building the Stream object (a forward makes this call once).
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda idx: torch.cuda.current_stream(idx).cuda_stream)
+# The current device's index, by the accessor behind `torch.cuda.current_device()` (for callers that hold a tensor on the GPU).
+_raw_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 _version_of = attrgetter("_version")
@@ -371,7 +373,7 @@ class W4A16Extension:
             if torch.cuda.is_current_stream_capturing():
                 return False
             out = hit.out if hit is not None else torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            with _SAME_DEVICE if dev.index == torch.cuda.current_device() else torch.cuda.device(dev):
+            with _SAME_DEVICE if dev.index == _raw_device() else torch.cuda.device(dev):
                 rc = pack(out.data_ptr(), stream)
                 if rc:
                     self._raise(rc, "pack_tiled")
@@ -872,22 +874,27 @@ class PreparedGroup:
         self.last_r = r
         idx = dev.index
         # the library launches on the current device: switch only when the tensors live on another one
-        ctx = None
-        if idx is not None and idx != torch.cuda.current_device():
+        ctx = lock = None
+        if idx is not None and idx != _raw_device():
             ctx = torch.cuda.device(dev)
             ctx.__enter__()
         try:
-            with ext._enqueue_lock(dev, stream):
-                ws, ws_bytes = ext._workspace(dev, M, stream)
-                if fused:
-                    rc = self.lib.glowq_w4a16_group_forward_fused_ws(
-                        x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
-                        self.rank, self.alpha, ws, ws_bytes, stream)
-                else:
-                    rc = self.lib.glowq_w4a16_group_forward_ws(
-                        x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, arr, len(Ns), M,
-                        self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
+            if M > 1:  # (a single row's launches hand nothing on through the workspace)
+                held = ext._enqueue_lock(dev, stream)
+                held.acquire()
+                lock = held
+            ws, ws_bytes = ext._workspace(dev, M, stream)
+            if fused:
+                rc = self.lib.glowq_w4a16_group_forward_fused_ws(
+                    x.data_ptr(), self.R.data_ptr(), r.data_ptr(), arr, len(Ns), M, self.K, self.group_size,
+                    self.rank, self.alpha, ws, ws_bytes, stream)
+            else:
+                rc = self.lib.glowq_w4a16_group_forward_ws(
+                    x.data_ptr(), r.data_ptr() if (r is not None and self.corrected) else None, arr, len(Ns), M,
+                    self.K, self.group_size, self.rank if self.corrected else 0, self.alpha, ws, ws_bytes, stream)
         finally:
+            if lock is not None:
+                lock.release()
             if ctx is not None:
                 ctx.__exit__(None, None, None)
         if rc == EUNSUPPORTED and widen:  # not the GEMM's call: nothing has been launched

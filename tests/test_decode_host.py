@@ -111,6 +111,13 @@ def test_rows_that_nobody_watches_take_the_kernels(model, kernels, monkeypatch):
     assert kernels.calls == 2 * ALL
 
 
+def test_rows_in_inference_mode_take_the_kernels(model, kernels):
+    want = forward(model)
+    with torch.inference_mode():
+        got = forward(model)
+    assert kernels.calls == 2 * ALL and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_function_modes_see_the_expressions(model, kernels):
     seen = []
 
