@@ -132,15 +132,15 @@ _SAME_DEVICE = contextlib.nullcontext()  # instead of `torch.cuda.device` where 
 
 
 class _Packed:
-    """A packed copy `out` of a tensor and `others`, kept on the tensor.  `key` says where they lie and how they are packed,
-    `versions` what was in them (every in-place write through torch raises a tensor's version), so that a write is seen.
-    Holding the others keeps their addresses from being given to new tensors.  The copy is made on the stream `home`
-    (handle `handle`); other streams wait for it before their first read (`ready_on`)."""
+    """A packed copy `out` of a tensor and up to two others, kept on the tensor.  `key` says where they lie, how they are packed
+    and what was in them (their versions: every in-place write through torch raises one), so
+    that a write is seen.  Holding the others keeps their addresses from being given to new tensors.  The copy is made on the
+    stream `home` (handle `handle`); other streams wait for it before their first read (`ready_on`)."""
 
-    __slots__ = ("key", "versions", "others", "out", "home", "handle", "event", "waited")
+    __slots__ = ("key", "second", "third", "out", "home", "handle", "event", "waited")
 
-    def __init__(self, key, versions, others, out, home, handle, event):
-        self.key, self.versions, self.others, self.out = key, versions, others, out
+    def __init__(self, key, second, third, out, home, handle, event):
+        self.key, self.second, self.third, self.out = key, second, third, out
         self.home, self.handle, self.event, self.waited = home, handle, event, ()
 
     def ready_on(self, stream) -> bool:
@@ -357,28 +357,28 @@ class W4A16Extension:
             self._raise(rc, "pack_side")
         return out
 
-    def _packed_copy(self, owner, others, key, versions, nbytes: int, pack) -> Optional[_Packed]:
-        """The copy kept on `owner` of that tensor and `others`, made by `pack(out, stream)` where there is none or one of them has
+    def _packed_copy(self, key, fixed: int, nbytes: int, pack, owner, second=None, third=None) -> Optional[_Packed]:
+        """The copy kept on `owner` of that tensor and two others, made by `pack(out, stream)` where there is none or one of them has
         been written to since.  After a write the copy is made again in its old place, so that launches recorded into graphs read
         the new one too.  Where it would have to be made under a graph capture (it would come from the graph's own memory pool, or be
         made at every replay) and where this stream cannot wait for it: False, for now."""
         dev = owner.device
         with self._pack_lock:
             hit = getattr(owner, "_glowq_tiled", None)
-            if not isinstance(hit, _Packed) or hit.key != key:
+            if not isinstance(hit, _Packed):
                 hit = None
             stream = self._stream(dev)
-            if hit is not None and hit.versions == versions:
+            if hit is not None and hit.key == key:
                 return hit if hit.ready_on(stream) else False
             if torch.cuda.is_current_stream_capturing():
                 return False
-            out = hit.out if hit is not None else torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            out = hit.out if hit is not None and hit.key[:fixed] == key[:fixed] else torch.empty(nbytes, dtype=torch.uint8, device=dev)
             with _SAME_DEVICE if dev.index == _raw_device() else torch.cuda.device(dev):
                 rc = pack(out.data_ptr(), stream)
                 if rc:
                     self._raise(rc, "pack_tiled")
                 home, event = self._home(dev, stream)
-            packed = owner._glowq_tiled = _Packed(key, versions, others, out, home, stream, event)
+            packed = owner._glowq_tiled = _Packed(key, second, third, out, home, stream, event)
             return packed
 
     def _packed_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[_Packed]:
@@ -390,15 +390,15 @@ class W4A16Extension:
             return None
         _check(qweight.dtype == torch.int32 and scales.dtype == torch.float16 and qzeros.dtype == torch.int32 and
                qweight.is_contiguous() and scales.is_contiguous() and qzeros.is_contiguous(), "pack_tiled: contiguous canonical buffers")
+        q, s, z = qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr()
         try:
-            versions = (qweight._version, scales._version, qzeros._version)
+            key = (q, s, z, int(in_features), int(group_size), nbytes, qweight._version, scales._version, qzeros._version)
         except RuntimeError:
             return None  # inference tensors, whose writes torch does not count
-        q, s, z = qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr()
         return self._packed_copy(
-            qweight, (scales, qzeros), (q, s, z, int(in_features), int(group_size), nbytes), versions, nbytes,
-            lambda out, stream: self.lib.glowq_pack_tiled(q, s, z, out, N, int(in_features), int(group_size), qweight.size(1),
-                                                          scales.size(1), qzeros.size(1), stream))
+            key, 6, nbytes, lambda out, stream: self.lib.glowq_pack_tiled(q, s, z, out, N, int(in_features), int(group_size), qweight.size(1),
+                                                                          scales.size(1), qzeros.size(1), stream),
+            qweight, scales, qzeros)
 
     def _packed_tiled_left(self, L) -> Optional[_Packed]:
         if not tiled_enabled() or L is None or not L.is_cuda:
@@ -408,13 +408,12 @@ class W4A16Extension:
         if nbytes == 0:
             return None
         _check(L.dtype == torch.float16 and L.is_contiguous(), "pack_tiled_left: contiguous fp16 [OC, rank]")
+        ptr = L.data_ptr()
         try:
-            version = L._version
+            key = (ptr, int(N), int(rank), L._version)
         except RuntimeError:
             return None
-        ptr = L.data_ptr()
-        return self._packed_copy(L, (), (ptr, int(N), int(rank)), version, nbytes,
-                                 lambda out, stream: self.lib.glowq_pack_tiled_left(ptr, out, int(N), int(rank), stream))
+        return self._packed_copy(key, 3, nbytes, lambda out, stream: self.lib.glowq_pack_tiled_left(ptr, out, int(N), int(rank), stream), L)
 
     def pack_tiled(self, qweight, scales, qzeros, in_features: int, group_size: int) -> Optional[torch.Tensor]:
         """The tiled copy of a member's weights for the matrix-core routes (a uint8 tensor; layout in csrc/tiled.hpp), or
