@@ -260,9 +260,9 @@ int glowq_w4a16_route_tiled(int M, int K, int N, int group_size, int ldw_i32);
 
 /*
  * Measurement helpers of bench.py; no counterpart in the reference.
- * glowq_last_launch: what the calling thread's last group launch used -- the kernel with the template arguments of the
- *   instantiation where the launcher records them (the stream GEMV, the tiled-copy kernel), else the route's name --
- *   and its grid and workgroup size (0 where not recorded).
+ * glowq_last_launch: what the calling thread's last group launch, or projection of many rows by itself, used -- the
+ *   kernel with the template arguments of the instantiation where the launcher records them (the stream GEMV, the
+ *   tiled-copy kernel, the GEMM, the projection), else the route's name -- and its grid and workgroup size (0 where not recorded).
  * glowq_probe_stream_read: a kernel that does nothing but read `bytes` (16-byte loads, eight in flight per lane,
  *   workgroup b the b-th contiguous share) with the given grid and workgroup size: the rate a memory-bound kernel of
  *   that launch shape could reach with no arithmetic at all.  `sink` (4 bytes of device memory) is never written.
