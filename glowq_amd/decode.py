@@ -19,6 +19,7 @@ lm_head matmul and the embedding lookup stay torch ops).
 from __future__ import annotations
 
 import argparse
+import itertools
 import json
 import time
 from dataclasses import dataclass
@@ -81,12 +82,12 @@ def _row_kernels(*tensors) -> bool:
 def _positions_end(pos_idx, rows: int, caches) -> int:
     """A bound that selecting from tables of `rows` rows has checked the positions against.  Where a cache is shorter than the tables
     that does not keep them inside: positions outside are refused here, on the host, and the bound is theirs."""
-    if all(t.size(1) >= rows for pair in caches for t in pair) or not pos_idx.is_cuda:
+    shortest = min((t.size(1) for pair in caches for t in pair), default=rows)
+    if shortest >= rows or not pos_idx.is_cuda:
         return rows
     if torch.cuda.is_current_stream_capturing():
         return rows  # the host cannot look; the layers append with index_copy_
     first, last = torch.stack(torch.aminmax(pos_idx)).tolist()
-    shortest = min(t.size(1) for pair in caches for t in pair)
     if first < 0 or last >= shortest:
         raise IndexError(f"positions {first}..{last} do not fit a cache of {shortest} rows")
     return last + 1
@@ -293,7 +294,9 @@ class Decoder(nn.Module):
         cfg = self.cfg
         x = self.model.embed_tokens(tokens)
         several = _several_rows(x)
-        end = _positions_end(pos_idx, min(cos_t.size(0), sin_t.size(0)), caches) if several else 0
+        if several and not isinstance(caches, (list, tuple)):
+            caches = list(itertools.islice(caches, len(self.model.layers)))  # (looked at twice)
+        end = _positions_end(pos_idx, min(cos_t.size(0), sin_t.size(0)), caches[:len(self.model.layers)]) if several else 0
         cos, sin = cos_t.index_select(0, pos_idx).to(x.dtype), sin_t.index_select(0, pos_idx).to(x.dtype)
         if several:
             _note_positions(cos, pos_idx, end)

@@ -1,4 +1,6 @@
 """When the decoder's layers take the library's row kernels and when tensor expressions, on the CPU."""
+import itertools
+
 import pytest
 import torch
 import torch.fx
@@ -189,3 +191,16 @@ def test_positions_that_nothing_has_checked_are_left_to_index_copy(model, kernel
         assert not decode._inside_cache(cos, pos.clone(), ck, cv) and not decode._inside_cache(cos, pos, ck[:, 1:], cv[:, 1:])
         pos += CFG.max_len
         assert not decode._inside_cache(cos, pos, ck, cv)
+
+
+def test_caches_from_an_iterator(model, kernels):
+    """Pairs of caches may come from any iterable, an endless one included; pairs past the layers are not looked at."""
+    want, pair = forward(model), caches()[0]
+    assert decode._positions_end(torch.arange(5), 24, [pair]) == 24
+    cos, sin = model.rope_tables("cpu")
+    with torch.no_grad():
+        logits = model.forward_tokens(torch.arange(5), torch.arange(5), itertools.repeat(pair), cos, sin, from_empty_cache=True)
+    assert all(torch.equal(a, b) for a, b in zip([logits, *pair], want)) and kernels.calls == 2 * ALL
+    with torch.no_grad():
+        again = model.forward_tokens(torch.arange(5), torch.arange(5), [pair, None], cos, sin, from_empty_cache=True)
+    assert torch.equal(again, logits)

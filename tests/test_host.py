@@ -411,3 +411,17 @@ def test_allow_jit_builds_a_missing_library_once(monkeypatch):
     ext = kernels.load_w4a16_extension()
     assert calls == ["build", "build"] and ext.version >= 100
     monkeypatch.setattr(kernels, "_ext", None)
+
+
+def test_a_copied_or_saved_weight_leaves_its_packed_copy_behind(tmp_path):
+    import copy
+    import pickle
+
+    from glowq_amd.kernels import _Packed
+
+    w = torch.arange(6, dtype=torch.int32)
+    w._glowq_tiled = _Packed((w.data_ptr(), w._version), None, None, torch.zeros(3), None, 0, None)
+    for other in (copy.deepcopy(w), pickle.loads(pickle.dumps(w))):
+        assert torch.equal(other, w) and not isinstance(getattr(other, "_glowq_tiled", None), _Packed)
+    torch.save({"w": w}, tmp_path / "w.pt")
+    assert torch.equal(torch.load(tmp_path / "w.pt", weights_only=True)["w"], w)
