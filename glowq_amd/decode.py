@@ -169,7 +169,8 @@ class Attention(nn.Module):
                 return self.o_proj(out)
         q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         if (_several_rows(x) and cfg.head_dim % 16 == 0 and pos_idx.dtype == torch.int64 and pos_idx.device == q.device and tuple(pos_idx.shape) == (T,) and pos_idx.is_contiguous()
-                and cos.shape == sin.shape == (T, cfg.head_dim) and _inside_cache(cos, pos_idx, cache_k, cache_v) and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
+                and cos.shape == sin.shape == (T, cfg.head_dim) and _inside_cache(cos, pos_idx, cache_k, cache_v)
+                and _row_kernels(q, k, v, cos, sin, cache_k, cache_v)):
             # rotary embedding and cache append in one launch; the heads stay side by side in a row
             q_rot, k_rot = torch.empty_like(q), torch.empty_like(k)
             load_w4a16_extension().rope_append(q, k, v, cos, sin, pos_idx, q_rot, k_rot, cache_k, cache_v)
