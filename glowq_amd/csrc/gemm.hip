@@ -546,17 +546,35 @@ void gemm_mfma_kernel(const GemmGroup gg, const int m_blocks) {
 //     LDS -- four rows of 256 bytes, no padding -- so bank conflicts are avoided by the choice of what goes where:
 //     slot c' of row r holds the 16-byte piece c' ^ (r % 16) of that row, and a fragment read of piece c looks in
 //     slot c ^ (r % 16): sixteen consecutive rows land in sixteen different slots.
-//   * The correction runs first as before, with the tiled left factor as B operand (its pairs at positions 2, 3, 6, 7
-//     of every octet are stored times 16, so r is staged through registers with those pairs divided by 16).
+//   * The matrix instructions of a code word and the vector instructions that dequantise the next one are interleaved by hand
+//     (order_word), and the correction runs behind the weights, its sum in registers of its own, r straight into LDS like the
+//     activations: in front, its two round trips came before the first weights, and its staging registers made the 128 x 256
+//     tile spill.  Together 1.04 times as fast in the mean over 15 groups of 1B to 14B shapes at 72 to 2048 rows (8B gate|up at 2048
+//     rows 443 -> 430 us, down_proj at 333 rows 61.7 -> 55.8, 14B o_proj at 100 rows 21.2 -> 18.7, same cuts).
 constexpr int kTRow = 256;  // bytes of a staged row: 128 halves, swizzled instead of padded
-#ifndef GLOWQ_GDBG
-#define GLOWQ_GDBG 0
-#endif
+
+// The order of a word's instructions: behind every matrix instruction its share of the next word's thirteen vector instructions per column
+// tile, the next fragments from LDS in front (few matrix instructions a word) or as soon as a fragment has been used for the last time.
+template <int kMT, int kNT>
+__device__ __forceinline__ void order_word() {
+  constexpr int kShare = (13 * kNT + kMT * kNT - 1) / (kMT * kNT);
+  constexpr bool kReadsFirst = kMT * kNT <= 4;
+  if constexpr (kReadsFirst) __builtin_amdgcn_sched_group_barrier(0x100, kMT, 0);
+#pragma unroll
+  for (int q = 0; q < kMT * kNT; ++q) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, kShare, 0);
+    if (!kReadsFirst && q % kNT == kNT - 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
 
 // kWk = 2: eight waves on the same tile, the second four take the second half of the workgroup's K range with LDS stages
 // of their own, and the two accumulator sets meet in LDS before the epilogue.  For launches with about one tile per
 // compute unit: a SIMD then holds two waves of the one workgroup it has, instead of one wave with nothing to overlap its
 // waits with, and the K loop of a tile takes half as many steps.
+// One super-block of weights and one half-step of activations ahead are enough: four sets of registers and four stages measured the
+// same or slower on every shape at 100 and 333 rows (8B gate|up at 100 rows 41.4 -> 42.2 us, down_proj 28.2 -> 28.9).
 template <int kMT, int kNT, int kWk, typename YT>
 __global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : 2), (kMT * kNT >= 16 ? 1 : 8))))
 void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
@@ -599,14 +617,6 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   const int m0 = bm * BM;
   const int ln = lane & 31, lh = lane >> 5;
 
-  f16v acc[kMT][kNT];
-#pragma unroll
-  for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-    for (int tn = 0; tn < kNT; ++tn)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[tm][tn][i] = 0.f;
-
   const auto rsrc = [](const void* p, size_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(uint32_t)bytes, 0x00020000);
   };
@@ -617,220 +627,237 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
 #pragma unroll
   for (int tn = 0; tn < kNT; ++tn) rb[tn] = min(bn * (BN / 32) + wave * kNT + tn, RB - 1);
 
+  // this workgroup's super-blocks: all of them, or slice `slice` of `nslices`; dealt to the K groups in contiguous halves.
+  // Both groups run the same number of steps (they share the barriers): a step past a group's part reads past the end of
+  // its descriptor -- zero codes at scale zero.
+  const int sb_per = (SB + nslices - 1) / nslices;
+  const int ws0 = min(slice * sb_per, SB), ws1 = min(ws0 + sb_per, SB);
+  const int per_group = (ws1 - ws0 + kWk - 1) / kWk;
+  const int sb0 = min(ws0 + gk * per_group, ws1), sb1 = min(sb0 + per_group, ws1);
+  const int sb_end = sb0 + per_group;  // steps run up to here
+
+  // The correction extends K: behind the last super-block of the last slice the walk goes on over the rank, in steps of 128 columns of
+  // r, dealt to the K groups in turn, with the tiled left factor as B operand.
+  const bool corr = a.r != nullptr && a.lt != nullptr && slice == nslices - 1;
+  const int LB = (a.rank + 63) >> 6;
+  const __amdgpu_buffer_rsrc_t rs_x = rsrc(a.x, (size_t)a.M * a.K * 2);
+  const __amdgpu_buffer_rsrc_t rs_r = rsrc(corr ? a.r : a.x, corr ? (size_t)a.M * a.rank * 2 : 0);
+  const __amdgpu_buffer_rsrc_t rs_w = rsrc(a.wt, (size_t)RB * sb1 * tiled::kChunk);
+  const __amdgpu_buffer_rsrc_t rs_l = rsrc(corr ? a.lt : a.wt, corr ? (size_t)RB * LB * tiled::kLChunk : 0);
+  constexpr uint32_t kPast = 0xFFFF0000u;  // a scalar offset past the end of any descriptor: zeros
+
   // ---- activations: piece q of thread t fills slot (t & 15) of row 16 q + (t >> 4) of the stage, which holds the
-  // 16-byte piece (t & 15) ^ (row % 16) of that row's 256 bytes (row % 16 = (t >> 4) % 16 for every q)
+  // 16-byte piece (t & 15) ^ (row % 16) of that row's 256 bytes (row % 16 = (t >> 4) % 16 for every q); every wave fills the
+  // four rows 16 q + 4 wave + [0, 4) of piece q, one contiguous kilobyte of LDS per load.  Rows past M lie past the end of the descriptor.
   const int srow = tid >> 4;                    // 0..15: the row within a block of sixteen
   const int spiece = (tid & 15) ^ srow;         // the piece of the row this thread moves
-  uint32_t a_row[kAL];
+  const uint32_t x_lane = (uint32_t)srow * (uint32_t)a.K * 2u + (uint32_t)spiece * 16u;
+  const uint32_t r_lane = (uint32_t)srow * (uint32_t)a.rank * 2u + (uint32_t)spiece * 16u;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  // rank columns [128 st, 128 st + 128) of r into stage `stg`; pieces past the rank meet zeros of the left factor and are read as zeros
+  auto load_r = [&](int st, int stg) __attribute__((always_inline)) {
+    const uint32_t off = st * 128 + spiece * 8 < a.rank ? r_lane : kPast;
 #pragma unroll
-  for (int q = 0; q < kAL; ++q) a_row[q] = (uint32_t)min(m0 + srow + 16 * q, a.M - 1);
+    for (int q = 0; q < kAL; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_r, (lds_ptr_t)(smem + (size_t)stg * BM * kTRow + (16 * q + 4 * wave) * kTRow), 16, (int)off,
+                                               (int)((uint32_t)(m0 + 16 * q) * (uint32_t)a.rank * 2u + (uint32_t)st * 256u), 0, 0);
+  };
+  // half-step hs = 2 sb + g of the activations (clamped into the row) into stage `stg`
+  auto load_x = [&](int hs, int stg) __attribute__((always_inline)) {
+    const uint32_t col = (uint32_t)min(hs, 2 * SB - 1) * 256u;
+#pragma unroll
+    for (int q = 0; q < kAL; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr_t)(smem + (size_t)stg * BM * kTRow + (16 * q + 4 * wave) * kTRow), 16, (int)x_lane,
+                                               (int)((uint32_t)(m0 + 16 * q) * (uint32_t)a.K * 2u + col), 0, 0);
+  };
   // A fragment of row tile tm, piece c of the staged row (which 16 columns: see the callers)
   auto read_a = [&](int stage, int tm, int c) __attribute__((always_inline)) {
     return *reinterpret_cast<const h8*>(smem + (size_t)stage * BM * kTRow + (tm * 32 + ln) * kTRow + ((c ^ (ln & 15)) << 4));
   };
+  // The activations of the next stage have landed before the workgroup's barrier: loads return in order, so it is enough
+  // to wait until no more loads are outstanding than were issued behind them.  The scheduling barriers keep the loads where
+  // they are written: left alone, the compiler sinks the refills to the end of the half-step, where nothing hides them.
+  auto wait_loads_but = [&](auto n_const) __attribute__((always_inline)) {
+    constexpr int n = decltype(n_const)::value;
+    __builtin_amdgcn_s_waitcnt((n & 15) | 0x0F70 | ((n >> 4) << 14));  // vmcnt(n), nothing else
+  };
 
+  // ---- weights: two sets of registers take turns; while the pieces of one are dequantised, the same pieces of the other are
+  // refilled with the next super-block (a set refilled in place would have to be copied at the loop's back edge, and a copy waits for
+  // the load)
+  struct BSet {
+    u32x4 w[kNT][4];
+    u32x2 side[kNT];
+  };
+  BSet b[2];
+  const int w_lane = lane * 16;
+  const uint32_t chunk_stride = (uint32_t)RB * (uint32_t)tiled::kChunk;
+  auto load_w = [&](BSet& s, int sb, int piece) __attribute__((always_inline)) {
+#pragma unroll
+    for (int tn = 0; tn < kNT; ++tn)
+      s.w[tn][piece] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, w_lane + piece * 1024, (int)((uint32_t)rb[tn] * (uint32_t)tiled::kChunk + (uint32_t)sb * chunk_stride), 0);
+  };
+  auto load_side = [&](BSet& s, int sb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int tn = 0; tn < kNT; ++tn)
+      s.side[tn] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, tiled::kCodeBytes + ln * 8, (int)((uint32_t)rb[tn] * (uint32_t)tiled::kChunk + (uint32_t)sb * chunk_stride), 0));
+  };
+
+  f16v acc[kMT][kNT];
+#pragma unroll
+  for (int tm = 0; tm < kMT; ++tm)
+#pragma unroll
+    for (int tn = 0; tn < kNT; ++tn)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[tm][tn][i] = 0.f;
+
+  // ---- the quantised K loop, a half of a super-block (128 columns, one quantisation group) per stage --------
+  // Half-step h = 2 sb + g requests the activations of half-step h + 1, then pieces 2 g and 2 g + 1 (and, with g = 0, scale and
+  // zero-point) of super-block sb + 1; its last wait leaves in flight what was requested behind those activations.
+  load_side(b[0], sb0);
+  load_w(b[0], sb0, 0);
+  load_w(b[0], sb0, 1);
+  load_x(2 * sb0, 0);
+  load_w(b[0], sb0, 2);
+  load_w(b[0], sb0, 3);
+  __builtin_amdgcn_sched_barrier(0);
+  wait_loads_but(std::integral_constant<int, 2 * kNT>{});
+  __syncthreads();
+
+  // One code word of every column tile at a time: while the matrix instructions of word t run, the next word is dequantised between
+  // them and its A fragments are on their way from LDS.  Written as word after word the compiler puts a word's thirteen vector
+  // instructions and the wait for its fragments in front of its own matrix instructions, and the two pipes take turns.
+  struct Zero {
+    h2 lo[kNT], hi[kNT], s[kNT];
+  };
+  auto zero_of = [&](const BSet& s, int g) __attribute__((always_inline)) {
+    Zero z;
+#pragma unroll
+    for (int tn = 0; tn < kNT; ++tn) {
+      const uint32_t sw = s.side[tn][g];
+      const float nz = (float)__builtin_bit_cast(half_t, (uint16_t)(sw >> 16)) * 65536.0f;  // -zero
+      const half_t zl = (half_t)(nz - 1024.0f), zh = (half_t)(nz - 64.0f);
+      z.lo[tn] = h2{zl, zl};
+      z.hi[tn] = h2{zh, zh};
+      z.s[tn] = bitcast_u32<h2>(__builtin_amdgcn_perm(sw, sw, 0x01000100u));
+    }
+    return z;
+  };
   int stage = 0;
-  constexpr int kChunk = kMT < 4 ? kMT : 4;  // row tiles whose A fragments are live at once
-
-  // ---- phase 1: the correction, acc = r . L^T, 128 rank columns (two blocks of the tiled left factor) per stage ----------
-  if (a.r != nullptr && a.lt != nullptr && slice == 0) {
-    const int LB = (a.rank + 63) >> 6;
-    const __amdgpu_buffer_rsrc_t rs_r = rsrc(a.r, (size_t)a.M * a.rank * 2);
-    const __amdgpu_buffer_rsrc_t rs_l = rsrc(a.lt, gk == 0 ? (size_t)RB * LB * tiled::kLChunk : 0);  // one K group adds the correction
-    const int steps = (a.rank + 127) >> 7;
-    u32x4 areg[kAL];
-    auto load_r = [&](int st) __attribute__((always_inline)) {
+  Zero zero = zero_of(b[0], 0);  // zero-points and scales of the half the next word lies in
+  h8 bf[kNT];                    // the next word, dequantised
 #pragma unroll
-      for (int q = 0; q < kAL; ++q) {
-        // columns past the rank meet zeros of the left factor
-        const uint32_t col = (uint32_t)st * 128u + (uint32_t)spiece * 8u;
-        areg[q] = __builtin_amdgcn_raw_buffer_load_b128(rs_r, (int)((a_row[q] * (uint32_t)a.rank + min(col, (uint32_t)a.rank - 8u)) * 2u), 0, 0);
-        if (col >= (uint32_t)a.rank) areg[q] = u32x4{0u, 0u, 0u, 0u};
-      }
-    };
-    auto store_r = [&](int stg) __attribute__((always_inline)) {
-      unsigned char* dst = smem + (size_t)stg * BM * kTRow + srow * kTRow + (tid & 15) * 16;
-      const h2 k16 = {(half_t)0.0625f, (half_t)0.0625f};
+  for (int tn = 0; tn < kNT; ++tn) bf[tn] = dequant_word(b[0].w[tn][0][0], zero.lo[tn], zero.hi[tn], zero.s[tn]);
+  // d (the set that holds super-block sb) and g are compile-time constants at every call site
+  auto half_step = [&](int sb, auto d_const, auto g_const) __attribute__((always_inline)) {
+    constexpr int d = decltype(d_const)::value, g = decltype(g_const)::value;
+    const BSet& cur = b[d];
+    BSet& nxt = b[d ^ 1];
+    h8 af[kMT];
 #pragma unroll
-      for (int q = 0; q < kAL; ++q) {
-        u32x4 o = areg[q];
-        o.y = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.y) * k16);
-        o.w = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.w) * k16);
-        *reinterpret_cast<u32x4*>(dst + 16 * q * kTRow) = o;
-      }
-    };
-    load_r(0);
-    store_r(stage);
-    __syncthreads();
-    for (int st = 0; st < steps; ++st) {
-      u32x4 lf[kNT][2][4];
+    for (int u = 0; u < kMT; ++u) af[u] = read_a(stage, u, 8 * lh);
+    load_x(2 * sb + g + 1, stage ^ 1);
+    if (g == 0) load_side(nxt, sb + 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int tn = 0; tn < kNT; ++tn)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int jb = 2 * st + q;
-          // a block past the rank: an offset past the end of the descriptor (zeros)
-          const uint32_t base = jb < LB ? (uint32_t)(rb[tn] * LB + jb) * (uint32_t)tiled::kLChunk : 0xFFFF0000u;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) lf[tn][q][t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, lane * 16 + t * 1024, (int)base, 0);
-        }
-      if (st + 1 < steps) load_r(st + 1);
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int c = 0; c < kMT; c += kChunk) {
-            h8 af[kChunk];
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) af[i] = read_a(stage, c + i, 8 * q + 4 * lh + t);
-#pragma unroll
-            for (int tn = 0; tn < kNT; ++tn)
-#pragma unroll
-              for (int i = 0; i < kChunk; ++i)
-                acc[c + i][tn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], __builtin_bit_cast(h8, lf[tn][q][t]), acc[c + i][tn], 0, 0, 0);
-          }
-      if (st + 1 < steps) store_r(stage ^ 1);
-      __syncthreads();
-      stage ^= 1;
-    }
-    if (a.alpha != 1.0f) {
-#pragma unroll
-      for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < kNT; ++tn)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[tm][tn][i] *= a.alpha;
-    }
-  }
-
-  // ---- phase 2: the quantised K loop, a half of a super-block (128 columns, one quantisation group) per stage --------
-  {
-    const __amdgpu_buffer_rsrc_t rs_x = rsrc(a.x, (size_t)a.M * a.K * 2);
-    // this workgroup's super-blocks: all of them, or slice `slice` of `nslices`; dealt to the K groups in contiguous halves.
-    // Both groups run the same number of steps (they share the barriers): a step past a group's part reads past the end of
-    // its descriptor -- zero codes at scale zero.
-    const int sb_per = (SB + nslices - 1) / nslices;
-    const int ws0 = min(slice * sb_per, SB), ws1 = min(ws0 + sb_per, SB);
-    const int per_group = (ws1 - ws0 + kWk - 1) / kWk;
-    const int sb0 = min(ws0 + gk * per_group, ws1), sb1 = min(sb0 + per_group, ws1);
-    const int sb_end = sb0 + per_group;  // steps run up to here
-    const __amdgpu_buffer_rsrc_t rs_w = rsrc(a.wt, (size_t)RB * sb1 * tiled::kChunk);
-    const uint32_t chunk_stride = (uint32_t)RB * (uint32_t)tiled::kChunk;
-    uint32_t a_off[kAL], w_off[kNT];
-#pragma unroll
-    for (int q = 0; q < kAL; ++q) a_off[q] = (a_row[q] * (uint32_t)a.K + (uint32_t)spiece * 8u) * 2u;
-#pragma unroll
-    for (int tn = 0; tn < kNT; ++tn) w_off[tn] = (uint32_t)rb[tn] * (uint32_t)tiled::kChunk + (uint32_t)lane * 16u;
-    // half-step hs = 2 sb + g (clamped into the slice) of the activations into stage `stg`: every wave fills the four rows
-    // 16 q + 4 wave + [0, 4) of piece q, one contiguous kilobyte of LDS per load
-    auto load_x = [&](int hs, int stg) __attribute__((always_inline)) {
-      const int h = min(hs, 2 * SB - 1);
-      typedef __attribute__((address_space(3))) void* lds_ptr_t;
-#pragma unroll
-      for (int q = 0; q < kAL; ++q)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr_t)(smem + (size_t)stg * BM * kTRow + (16 * q + 4 * wave) * kTRow), 16, (int)a_off[q],
-                                                 h * 256, 0, 0);
-    };
-    // The activations of the next stage have landed before the workgroup's barrier: loads return in order, so it is enough
-    // to wait until no more loads are outstanding than were issued behind them (the refills of this half-step, which
-    // stay in flight).  The scheduling barriers keep the loads where they are written: left alone, the compiler sinks
-    // the refills to the end of the half-step, where nothing hides them.
-    auto wait_loads_but = [&](auto n_const) __attribute__((always_inline)) {
-      constexpr int n = decltype(n_const)::value;
-      __builtin_amdgcn_s_waitcnt((n & 15) | 0x0F70 | ((n >> 4) << 14));  // vmcnt(n), nothing else
-    };
-    // Two sets of weight registers take turns: while the pieces of one are dequantised, the same pieces of the other are
-    // refilled with the next super-block (a set refilled in place would have to be copied at the loop's back edge, and a
-    // copy waits for the load).
-    struct BSet {
-      u32x4 w[kNT][4];
-      u32x2 side[kNT];
-    };
-    BSet b0, b1;
-    const int side_off = tiled::kCodeBytes + ln * 8;
-    if (ws0 < ws1) {
-      load_x(2 * sb0, stage);
-#pragma unroll
-      for (int tn = 0; tn < kNT; ++tn) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b0.w[tn][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, (int)w_off[tn] + j * 1024, sb0 * (int)chunk_stride, 0);
-        b0.side[tn] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, (int)((uint32_t)rb[tn] * (uint32_t)tiled::kChunk) + side_off,
-                                                                                     sb0 * (int)chunk_stride, 0));
-      }
-      wait_loads_but(std::integral_constant<int, 0>{});
-      __syncthreads();
-    }
-    // g is a compile-time constant at every call site; `cur` holds super-block sb, `nxt` receives sb + 1
-    auto half_step = [&](int sb, auto g_const, const BSet& cur, BSet& nxt) __attribute__((always_inline)) {
-      constexpr int g = decltype(g_const)::value;
-      const int sbn = sb + 1;  // (behind the group's last super-block: past the end of the descriptor, zeros nobody uses)
-      if (!(GLOWQ_GDBG & 8)) load_x(2 * sb + g + 1, stage ^ 1);
-      if (g == 1) {
-#pragma unroll
-        for (int tn = 0; tn < kNT; ++tn)
-          nxt.side[tn] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, (int)((uint32_t)rb[tn] * (uint32_t)tiled::kChunk) + side_off,
-                                                                                        sbn * (int)chunk_stride, 0));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      h2 zb_lo[kNT], zb_hi[kNT], s2[kNT];
-#pragma unroll
-      for (int tn = 0; tn < kNT; ++tn) {
-        const uint32_t sw = cur.side[tn][g];
-        const float nz = (float)__builtin_bit_cast(half_t, (uint16_t)(sw >> 16)) * 65536.0f;  // -zero
-        const half_t zl = (half_t)(nz - 1024.0f), zh = (half_t)(nz - 64.0f);
-        zb_lo[tn] = h2{zl, zl};
-        zb_hi[tn] = h2{zh, zh};
-        s2[tn] = bitcast_u32<h2>(__builtin_amdgcn_perm(sw, sw, 0x01000100u));
-      }
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-#pragma unroll
-        for (int tn = 0; tn < kNT; ++tn)
-          nxt.w[tn][2 * g + p] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, (int)w_off[tn] + (2 * g + p) * 1024, sbn * (int)chunk_stride, 0);
+    for (int t = 0; t < 8; ++t) {
+      if ((t & 3) == 0) {
+        load_w(nxt, sb + 1, 2 * g + t / 4);
         __builtin_amdgcn_sched_barrier(0);
+      }
+      h8 an[kMT], bn_[kNT];
+      if (t < 7) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          h8 bf[kNT];
+        for (int u = 0; u < kMT; ++u) an[u] = read_a(stage, u, 8 * lh + t + 1);
+      }
+      if (t == 7) zero = zero_of(g == 0 ? cur : nxt, g ^ 1);
 #pragma unroll
-          for (int tn = 0; tn < kNT; ++tn)
-            bf[tn] = (GLOWQ_GDBG & 1) ? __builtin_bit_cast(h8, u32x4{cur.w[tn][2 * g + p][i], cur.w[tn][2 * g + p][i] ^ cur.side[tn].x, 0u, 0u})
-                                      : dequant_word(cur.w[tn][2 * g + p][i], zb_lo[tn], zb_hi[tn], s2[tn]);
+      for (int tn = 0; tn < kNT; ++tn) {
+        const uint32_t w = t < 7 ? cur.w[tn][2 * g + (t + 1) / 4][(t + 1) & 3] : (g == 0 ? cur.w[tn][2][0] : nxt.w[tn][0][0]);
+        bn_[tn] = dequant_word(w, zero.lo[tn], zero.hi[tn], zero.s[tn]);
+      }
 #pragma unroll
-          for (int c = 0; c < kMT; c += kChunk) {
-            h8 af[kChunk];
+      for (int u = 0; u < kMT; ++u)
 #pragma unroll
-            for (int u = 0; u < kChunk; ++u)
-              af[u] = (GLOWQ_GDBG & 2) ? __builtin_bit_cast(h8, u32x4{(uint32_t)(c + u + i), (uint32_t)p, (uint32_t)lane, 0u})
-                                       : read_a(stage, c + u, 8 * lh + 4 * p + i);
+        for (int tn = 0; tn < kNT; ++tn) acc[u][tn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[u], bf[tn], acc[u][tn], 0, 0, 0);
+      order_word<kMT, kNT>();
 #pragma unroll
-            for (int tn = 0; tn < kNT; ++tn)
+      for (int u = 0; u < kMT; ++u) af[u] = an[u];
 #pragma unroll
-              for (int u = 0; u < kChunk; ++u)
-                acc[c + u][tn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[u], bf[tn], acc[c + u][tn], 0, 0, 0);
-          }
+      for (int tn = 0; tn < kNT; ++tn) bf[tn] = bn_[tn];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wait_loads_but(std::integral_constant<int, 2 * kNT + (g == 0 ? kNT : 0)>{});
+    __syncthreads();
+    stage ^= 1;
+  };
+  auto super_block = [&](int sb, auto d_const) __attribute__((always_inline)) {
+    half_step(sb, d_const, std::integral_constant<int, 0>{});
+    half_step(sb, d_const, std::integral_constant<int, 1>{});
+  };
+
+  int sb = sb0;
+  for (; sb + 1 < sb_end; sb += 2) {
+    super_block(sb, std::integral_constant<int, 0>{});
+    super_block(sb + 1, std::integral_constant<int, 1>{});
+  }
+  if (sb < sb_end) super_block(sb, std::integral_constant<int, 0>{});
+  // requests past the end that are still on their way into the stages have to land before the stages are used for anything else
+  wait_loads_but(std::integral_constant<int, 0>{});
+
+  // ---- the correction, behind the weights: 128 rank columns (two blocks of the tiled left factor) per step, the steps dealt to the K
+  // groups in turn.  Its sum is taken by itself, times alpha.  (The pairs at positions 2, 3, 6, 7 of every octet of the tiled left
+  // factor are stored times 16: the fragments of r are divided by 16 there.)
+  if (corr) {
+    const int mine = (((a.rank + 127) >> 7) + kWk - 1) / kWk;  // (both K groups run the same number: past the rank they add zeros)
+    for (int i = 0; i < mine; ++i) {
+      const int st = gk + kWk * i;
+      __syncthreads();  // the fragment reads of the stage are done
+      load_r(st, 0);
+      u32x4 lf[8];
+#pragma unroll
+      for (int tn = 0; tn < kNT; ++tn) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            lf[4 * q + t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, w_lane + t * 1024, 2 * st + q < LB ? (int)((uint32_t)(rb[tn] * LB + 2 * st + q) * (uint32_t)tiled::kLChunk) : (int)kPast, 0);
+        if (tn == 0) {
+          wait_loads_but(std::integral_constant<int, 8>{});
+          __syncthreads();
+        }
+        constexpr int kPair = kMT > 1 && kMT * kNT < 8 ? 2 : 1;
+        if (kMT * kNT >= 8) __builtin_amdgcn_sched_barrier(0);  // (registers: nothing of the next tile may start early)
+#pragma unroll
+        for (int u = 0; u < kMT; u += kPair) {
+          f16v c[kPair];
+#pragma unroll
+          for (int v = 0; v < kPair; ++v)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) c[v][e] = 0.f;
+#pragma unroll
+          for (int p = 0; p < 8; ++p)
+#pragma unroll
+            for (int v = 0; v < kPair; ++v) {
+              u32x4 f = __builtin_bit_cast(u32x4, read_a(0, u + v, 8 * (p / 4) + 4 * lh + p % 4));
+              const h2 k16 = {(half_t)0.0625f, (half_t)0.0625f};
+              f.y = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(f.y) * k16);
+              f.w = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(f.w) * k16);
+              c[v] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, f), __builtin_bit_cast(h8, lf[p]), c[v], 0, 0, 0);
+            }
+#pragma unroll
+          for (int v = 0; v < kPair; ++v)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[u + v][tn][e] = __builtin_fmaf(a.alpha, c[v][e], acc[u + v][tn][e]);
+          if (kMT * kNT >= 8) __builtin_amdgcn_sched_barrier(0);
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
-      wait_loads_but(std::integral_constant<int, 2 * kNT + (g == 1 ? kNT : 0)>{});
-      if (!(GLOWQ_GDBG & 4)) __syncthreads();
-      stage ^= 1;
-    };
-    int sb = sb0;
-    for (; sb + 1 < sb_end; sb += 2) {
-      half_step(sb, std::integral_constant<int, 0>{}, b0, b1);
-      half_step(sb, std::integral_constant<int, 1>{}, b0, b1);
-      half_step(sb + 1, std::integral_constant<int, 0>{}, b1, b0);
-      half_step(sb + 1, std::integral_constant<int, 1>{}, b1, b0);
-    }
-    if (sb < sb_end) {
-      half_step(sb, std::integral_constant<int, 0>{}, b0, b1);
-      half_step(sb, std::integral_constant<int, 1>{}, b0, b1);
     }
   }
 
-  // ---- the second K group hands its accumulators over through LDS (the stages are free: every wave is past the last barrier)
+  // ---- the second K group hands its accumulators over through LDS, once every wave is done with the stages
   if constexpr (kWk > 1) {
+    __syncthreads();
     float* red = reinterpret_cast<float*>(smem_all);
     if (gk == 1) {
 #pragma unroll
