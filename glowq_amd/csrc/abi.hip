@@ -41,6 +41,7 @@ bool skinny_raw_form(const GroupDev& g);
 hipError_t launch_skinny(GroupDev& g, int num_cus, hipStream_t stream, bool raw);
 bool gemm_supported(const GroupDev& g);
 hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream);
+size_t gemm_handover_bytes();
 bool gemm_widens(const GroupDev& g);
 // misc.hip
 hipError_t launch_probe_read(const void* src, size_t bytes, void* sink, int grid, int block, hipStream_t stream);
@@ -330,6 +331,9 @@ bool tiled_pays(const GroupDev& g) {
 //                   (GLOWQ_PROJ_SPIN_LIMIT; 0: never waits)
 std::atomic<int> g_proj_in_launch{clampi(env_or("GLOWQ_PROJ_IN_LAUNCH", 1), 0, 2)};
 std::atomic<int> g_proj_spin_limit{clampi(env_or("GLOWQ_PROJ_SPIN_LIMIT", 16384), 0, 1 << 24)};
+//   proj_any_cost   1, for tests: launches on the tiled weights compute r themselves wherever they can, not only where that is predicted
+//                   to pay (GLOWQ_PROJ_ANY_COST; 0: where it pays)
+std::atomic<int> g_proj_any_cost{clampi(env_or("GLOWQ_PROJ_ANY_COST", 0), 0, 1)};
 //   small_rows_in_launch  1: a fused call with three or four token rows and a workspace goes to the skinny kernel where its
 //                   launch computes r itself (GLOWQ_SMALL_ROWS_IN_LAUNCH; 0: always the 2..4-row kernels behind a
 //                   projection launch)
@@ -357,6 +361,17 @@ bool skinny_proj_in_launch(const GroupDev& g) {
   bool any_left = false;
   for (int i = 0; i < g.n_members; ++i) any_left = any_left || g.mem[i].L != nullptr;
   return any_left;  // (the launcher still turns down shapes and grids it does not take)
+}
+
+// The same for the GEMM on the tiled weights.
+bool gemm_proj_in_launch(const GroupDev& g) {
+  if (g_proj_in_launch.load(std::memory_order_relaxed) == 0) return false;
+  if (g.ws == nullptr || (reinterpret_cast<uintptr_t>(g.ws) & 15u) != 0 || g.ws_bytes < glowq::gemm_handover_bytes()) return false;
+  if ((g.K & 255) != 0 || (g.rank & 7) != 0 || !aligned16(g.x) || !aligned16(g.R) || !aligned16(g.r_out)) return false;
+  if ((size_t)g.M * g.K * 2 >= (1ull << 32) || (size_t)g.rank * g.K * 2 >= (1ull << 32)) return false;
+  bool any_left = false;
+  for (int i = 0; i < g.n_members; ++i) any_left = any_left || g.mem[i].L != nullptr;
+  return any_left;  // (the launcher still turns down calls without the tiled copy and those it would not pay for)
 }
 
 int pick_route(const GroupDev& g, int force) {
@@ -407,6 +422,12 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
   const int cus = num_cus();
   hipError_t e = hipSuccess;
   g.pub = nullptr;
+  const auto hand_over = [&]() {  // workgroups in front of the launch hand r to the others through the workspace
+    g.pub = static_cast<unsigned long long*>(g.ws);
+    g.pub_spin = (unsigned)g_proj_spin_limit.load(std::memory_order_relaxed);
+    g.pub_mute = g_proj_in_launch.load(std::memory_order_relaxed) == 2;
+    g.pub_any_cost = g_proj_any_cost.load(std::memory_order_relaxed);
+  };
   // r = x R^T ahead of the group as a launch of its own.  (Having every workgroup of the group kernel compute r for
   // itself was measured: the R -> r -> L.r dependency chain then stalls the weight stream for longer than the extra
   // launch costs.)
@@ -430,9 +451,7 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
   if (g.R != nullptr && g.M >= 3 && g.M <= 4 && g_small_rows_in_launch.load(std::memory_order_relaxed) != 0 &&
       (route == kRouteQuad || route == kRouteStream || route == kRouteWaveDot || (route == kRouteQStream && g.K <= 8192)) && skinny_supported(g) &&
       skinny_raw_form(g) && skinny_proj_in_launch(g)) {
-    g.pub = static_cast<unsigned long long*>(g.ws);
-    g.pub_spin = (unsigned)g_proj_spin_limit.load(std::memory_order_relaxed);
-    g.pub_mute = g_proj_in_launch.load(std::memory_order_relaxed) == 2;
+    hand_over();
     note_launch(0, 0, 0, "%s", "skinny_codes_mfma");
     e = launch_skinny(g, cus, stream, true);
     if (e == hipSuccess) return GLOWQ_OK;
@@ -441,12 +460,11 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
     g.pub = nullptr;
   }
   const bool skinny_route = route == kRouteSkinny || route == kRouteSkinnyRaw;
-  if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || route == kRouteSkinnyTiled) && skinny_proj_in_launch(g)))) {
+  if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || route == kRouteSkinnyTiled) && skinny_proj_in_launch(g)) ||
+                         (route == kRouteGemm && gemm_proj_in_launch(g)))) {
     // single token on the stream GEMV, a handful of rows on the skinny kernel: workgroups in front of the group launch
     // produce r and hand it to the others through the workspace (stream_kernel.hpp, skinny.hip), no launch in front
-    g.pub = static_cast<unsigned long long*>(g.ws);
-    g.pub_spin = (unsigned)g_proj_spin_limit.load(std::memory_order_relaxed);
-    g.pub_mute = g_proj_in_launch.load(std::memory_order_relaxed) == 2;
+    hand_over();
   } else if (g.R != nullptr) {
     e = launch_projection();
     if (e != hipSuccess) return fail(GLOWQ_ELAUNCH, "shared_proj launch failed: %s", hipGetErrorString(e));
@@ -471,6 +489,11 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
     e = launch_qstream(g, cus, stream);
   } else if (route == kRouteGemm) {
     e = launch_gemm(g, cus, stream);
+    if (e == hipErrorNotReady && g.pub != nullptr) {
+      e = launch_projection();
+      if (e != hipSuccess) return fail(GLOWQ_ELAUNCH, "shared_proj launch failed: %s", hipGetErrorString(e));
+      e = launch_gemm(g, cus, stream);
+    }
   } else if (route == kRouteSkinnyTiled) {
     e = launch_skinny_tiled(g, cus, stream);
     if (e == hipErrorNotReady && g.pub != nullptr) {
@@ -913,6 +936,7 @@ int glowq_set_tuning(const char* key, int value) {
   else if (strcmp(key, "tiled_max_m") == 0) { slot = &g_tiled_max_m; hi = 64; }
   else if (strcmp(key, "tiled_shape_rule") == 0) { slot = &g_tiled_shape_rule; hi = 1; }
   else if (strcmp(key, "proj_in_launch") == 0) { slot = &g_proj_in_launch; hi = 2; }
+  else if (strcmp(key, "proj_any_cost") == 0) { slot = &g_proj_any_cost; hi = 1; }
   else if (strcmp(key, "proj_spin_limit") == 0) { slot = &g_proj_spin_limit; hi = 1 << 24; }
   else if (strcmp(key, "small_rows_in_launch") == 0) { slot = &g_small_rows_in_launch; hi = 1; }
   if (slot == nullptr) return fail(GLOWQ_EINVAL, "unknown tuning key '%s'", key);

@@ -51,6 +51,7 @@ struct GroupDev {
   unsigned long long* pub;
   unsigned pub_spin;
   int pub_mute;
+  int pub_any_cost;
   MemberDev mem[GLOWQ_MAX_MEMBERS];
   int task_end[GLOWQ_MAX_MEMBERS];  // exclusive prefix of per-member task counts
   int wg_end[GLOWQ_MAX_MEMBERS];    // exclusive prefix of the workgroups assigned to each member

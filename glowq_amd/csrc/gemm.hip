@@ -22,6 +22,8 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "handover.hpp"
+#include "proj_front.hpp"
 #include "tiled.hpp"
 
 namespace glowq {
@@ -66,7 +68,14 @@ struct GemmGroup {
   // leave partials ([slice][tail tile][BM * BN]) for gemm_reduce_kernel.  The last, partly filled round of workgroups
   // of a launch then costs its share of a round instead of a whole one.  tail_slices <= 1: off.
   int full, tail_slices;
+  // the launch computes r itself (kProj of gemm_tiled_kernel, proj_front.hpp): `front.front` workgroups in front of the grid
+  FrontArgs front;
 };
+// A launch that computes r itself keeps at the head of the workspace the words of its workgroups in front and the sums of their slices of
+// r (4 KB each, 32 x 32 tiles); no more workgroups than this do work there.
+constexpr int kMaxFront = 512;
+constexpr size_t kGemmWordBytes = (size_t)kMaxFront * 8;
+constexpr size_t kGemmHandoverBytes = kGemmWordBytes + (size_t)kMaxFront * 4096;
 
 __device__ __forceinline__ h8 permute_for_nibble_order(const h8& v) {
   h8 p;
@@ -575,10 +584,23 @@ __device__ __forceinline__ void order_word() {
 // waits with, and the K loop of a tile takes half as many steps.
 // One super-block of weights and one half-step of activations ahead are enough: four sets of registers and four stages measured the
 // same or slower on every shape at 100 and 333 rows (8B gate|up at 100 rows 41.4 -> 42.2 us, down_proj 28.2 -> 28.9).
-template <int kMT, int kNT, int kWk, typename YT>
-__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : 2), (kMT * kNT >= 16 ? 1 : 8))))
+// kProj: the launch computes r = x R^T itself.  The readers need r behind their K loop, which is when the workgroups in front of the grid are
+// done as a rule; they wait for the words of their rows' tiles (bounded: a reader that gives up computes its r from x and R), and
+// read r past the caches the stores of the workgroups in front have passed.
+template <int kMT, int kNT, int kWk, typename YT, bool kProj>
+__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : (kMT * kNT <= 2 ? 4 : 2)), (kMT * kNT >= 16 ? 1 : 8))))
 void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
-  int wg = (int)blockIdx.x, slice = (int)blockIdx.y, nslices = gg.slices, part_tile = (int)blockIdx.x, part_tiles = (int)gridDim.x;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
+  const int front = kProj ? gg.front.front : 0;
+  unsigned long long tag = 0;
+  if constexpr (kProj) {
+    tag = launch_tag();
+    if ((int)blockIdx.x < front) {
+      if (blockIdx.y == 0) run_front<4 * kWk>(gg.front, (int)blockIdx.x, tag, smem_all);
+      return;
+    }
+  }
+  int wg = (int)blockIdx.x - front, slice = (int)blockIdx.y, nslices = gg.slices, part_tile = wg, part_tiles = (int)gridDim.x - front;
   if (gg.tail_slices > 1) {
     nslices = 1;
     if (wg >= gg.full) {
@@ -587,7 +609,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
       slice = t - part_tile * gg.tail_slices;
       wg = gg.full + part_tile;
       nslices = gg.tail_slices;
-      part_tiles = ((int)gridDim.x - gg.full) / gg.tail_slices;
+      part_tiles = ((int)gridDim.x - front - gg.full) / gg.tail_slices;
     }
   }
   GemmArgs a = gg.m[0];
@@ -601,7 +623,6 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   GLOWQ_PICK(2)
   GLOWQ_PICK(3)
 #undef GLOWQ_PICK
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
   constexpr int BM = 32 * kMT;
   constexpr int BN = 128 * kNT;
   constexpr int kAL = 2 * kMT;  // 16-byte pieces of a stage (BM rows x 256 bytes) per thread
@@ -656,11 +677,33 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // rank columns [128 st, 128 st + 128) of r into stage `stg`; pieces past the rank meet zeros of the left factor and are read as zeros
   auto load_r = [&](int st, int stg) __attribute__((always_inline)) {
+    constexpr int kPastCaches = kProj ? 16 : 0;  // where the workgroups in front left it
     const uint32_t off = st * 128 + spiece * 8 < a.rank ? r_lane : kPast;
 #pragma unroll
     for (int q = 0; q < kAL; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_r, (lds_ptr_t)(smem + (size_t)stg * BM * kTRow + (16 * q + 4 * wave) * kTRow), 16, (int)off,
-                                               (int)((uint32_t)(m0 + 16 * q) * (uint32_t)a.rank * 2u + (uint32_t)st * 256u), 0, 0);
+                                               (int)((uint32_t)(m0 + 16 * q) * (uint32_t)a.rank * 2u + (uint32_t)st * 256u), 0, kPastCaches);
+  };
+  // the same without r: every thread computes the eight entries of its pieces
+  auto compute_r = [&](int st, int stg) {
+#pragma unroll 1
+    for (int q = 0; q < kAL; ++q) {
+      const int row = m0 + srow + 16 * q;
+      h8 own;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int j = st * 128 + spiece * 8 + e;
+        float sum = 0.f;
+        if (row < a.M && j < a.rank) {
+          const h2* xv = reinterpret_cast<const h2*>(a.x + (size_t)row * a.K);
+          const h2* rv = reinterpret_cast<const h2*>(gg.front.R + (size_t)j * a.K);
+#pragma unroll 1
+          for (int k = 0; k < a.K / 2; ++k) sum = __builtin_amdgcn_fdot2(xv[k], rv[k], sum, false);
+        }
+        own[e] = (half_t)sum;
+      }
+      *reinterpret_cast<h8*>(smem + (size_t)stg * BM * kTRow + (16 * q + srow) * kTRow + (tid & 15) * 16) = own;
+    }
   };
   // half-step hs = 2 sb + g of the activations (clamped into the row) into stage `stg`
   auto load_x = [&](int hs, int stg) __attribute__((always_inline)) {
@@ -810,10 +853,17 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   // factor are stored times 16: the fragments of r are divided by 16 there.)
   if (corr) {
     const int mine = (((a.rank + 127) >> 7) + kWk - 1) / kWk;  // (both K groups run the same number: past the rank they add zeros)
+    bool have_r = true;
+    if constexpr (kProj) {
+      // the words of the tiles that cover this workgroup's rows
+      const int side = 32 * gg.front.a, per_row = (a.rank + side - 1) / side * gg.front.slices;
+      have_r = wait_words(gg.front.pub, m0 / side * per_row, (min(m0 + BM, a.M) + side - 1) / side * per_row, gg.front.slices, tag, gg.front.spin);
+    }
     for (int i = 0; i < mine; ++i) {
       const int st = gk + kWk * i;
       __syncthreads();  // the fragment reads of the stage are done
-      load_r(st, 0);
+      if (have_r) load_r(st, 0);  // (each wave's own affair: what it fetches or computes is its rows of the stage)
+      else compute_r(st, 0);
       u32x4 lf[8];
 #pragma unroll
       for (int tn = 0; tn < kNT; ++tn) {
@@ -968,15 +1018,16 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmGroup gg, co
 }
 
 // ---- host side ------------------------------------------------------------------------------------
-template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1, typename YT = half_t>
+template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1, typename YT = half_t, bool kProj = false>
 static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   static_assert(!kTiled || (kQuant && kSuper), "the tiled copy serves the super-block form");
   static_assert(kTiled || (kWk == 1 && std::is_same_v<YT, half_t>), "K groups inside a workgroup and fp32 outputs: the tiled-copy kernel");
   constexpr int BM = 32 * kMT, BN = 128 * kNT;
-  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk, YT> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
+  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk, YT, kProj> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
   size_t lds = kTiled ? (size_t)kWk * 2 * BM * kTRow
                       : (size_t)2 * BM * kARow * sizeof(half_t) + (kSuper ? (size_t)4 * (32 * kNT) * 144 : 0);
   if (kWk > 1 && lds < (size_t)BM * BN * sizeof(float)) lds = (size_t)BM * BN * sizeof(float);  // the hand-over of the accumulators
+  if constexpr (kProj) lds = std::max(lds, front_lds(gg.front));
   static LdsLimit lds_limit;
   if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
   const int m_blocks = (gg.m[0].M + BM - 1) / BM;
@@ -987,17 +1038,18 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   }
   if (!(kQuant && kSuper)) gg.slices = 1;
   if (!(kQuant && kSuper) || gg.slices > 1 || gg.tail_slices < 2 || gg.full < 0 || gg.full >= total) gg.tail_slices = 0;
+  const int front = kProj ? gg.front.front : 0;  // (the launch record names the grid of the tiles)
   const int tail_wgs = gg.tail_slices > 1 ? gg.full + (total - gg.full) * gg.tail_slices : 0;
   note_launch(tail_wgs > 0 ? tail_wgs : total, tail_wgs > 0 ? 1 : gg.slices, 256 * kWk, "%s<%d,%d,%d%s>",
               kTiled ? "gemm_tiled_kernel" : "gemm_mfma_kernel", kMT, kNT, kWk, std::is_same_v<YT, float> ? ",float" : "");
   if (tail_wgs > 0) {
     const int tail_tiles = total - gg.full;
-    hipLaunchKernelGGL(kern, dim3(tail_wgs, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
+    hipLaunchKernelGGL(kern, dim3(front + tail_wgs, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(tail_tiles, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(kern, dim3(total, gg.slices), dim3(256 * kWk), lds, stream, gg, m_blocks);
+  hipLaunchKernelGGL(kern, dim3(front + total, gg.slices), dim3(256 * kWk), lds, stream, gg, m_blocks);
   if (hipError_t e = hipGetLastError(); e != hipSuccess || gg.slices == 1) return e;
   hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(total, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
   return hipGetLastError();
@@ -1065,6 +1117,56 @@ static bool gemm_tiled_form(const GemmGroup& gg) {
   for (int i = 0; i < gg.n; ++i)
     ok = ok && gg.m[i].wt != nullptr && (gg.m[i].r == nullptr || gg.m[i].lt != nullptr) && tiled::weight_bytes(gg.m[i].N, gg.m[i].K) < (1ull << 32);
   return ok;
+}
+
+static float proj_launch_us(int M, int K, int rank, int num_cus, size_t ws_bytes);
+
+// How a launch that computes r itself cuts it, given its own cut; false: r comes from a launch of its own, which is predicted to cost less.
+//  * Tiles of 32 x 32 with K in as many slices as keep six stages each and leave one workgroup a compute unit, or tiles of 64 x 64: 0.45 and
+//    0.65 us a stage of 128 columns, 1.65 times that where every compute unit has work of the launch's own as well, about 2 us at the ends, 2.5
+//    for the sum of slices: measured on launches that waited for r.  What that
+//    costs the launch: what its first readers wait, the places that the workgroups in front keep from others where the launch takes more
+//    than one round, and some of their time where they make it more than one (with fewer slices they may not).  8B q|k|v at 100 rows, us, with one / two / four slices
+//    21.9 / 20.2 / 20.1, projection in front 26.2, r given 19.6; 8B down_proj at 100 rows 64 / 43 / 34, 29.8 with sixteen, 38.1, 27.8.
+//  * Where the launch's own workgroups are no more than one a compute unit and do not all find an empty one beside those in front, the
+//    front is filled up to one a compute unit with workgroups that only hold their places: the others then come out one a compute unit as well.
+//    Otherwise some compute units get two, and the launch takes as long as those: 8B down_proj at 333 rows 72.3 with 220 in front, 57.6
+//    with 264, projection in front 67.6, r given 55.8; 14B down_proj at 512 rows 134 with 128, 106 with 256, 118, 100.
+// 16 groups of 1B to 14B shapes at 65 to 2048 rows: 1.14 times as fast in the mean with the rule as with the projection in front.
+static bool plan_front(GemmGroup& gg, const GemmCost& c, int num_cus, size_t ws_bytes) {
+  FrontArgs& f = gg.front;
+  const int tiles = gemm_tiles(gg, c.mt, c.nt), sb = f.K >> 8, stages = f.K >> 7;
+  const int own = gg.tail_slices > 1 ? gg.full + (tiles - gg.full) * gg.tail_slices : tiles * gg.slices;
+  float best = f.any_cost ? 1e30f : proj_launch_us(f.M, f.K, f.rank, num_cus, ws_bytes);
+  bool found = false;
+  for (int a = 1; a <= 2; ++a) {
+    // workgroups that a compute unit holds: registers, and the LDS that the workgroups in front want (48 or 64 KB of 160)
+    const int per_cu = c.mt == 4 && c.nt == 2 && c.wk == 2 ? 1 : (c.mt * c.nt <= 2 && c.wk == 1 && a == 1 ? 3 : 2);
+    const int slots = num_cus * per_cu, held = std::min((own + num_cus - 1) / num_cus, per_cu);
+    if (a == 2 && per_cu == 2 && c.mt * c.nt <= 2 && own > slots) continue;  // (with 48 KB or less there were three)
+    const float readers = gemm_cost_fixed(gg, c) + (float)(2 * (((sb + gg.slices - 1) / gg.slices + c.wk - 1) / c.wk)) * (c.step + (float)(held - 1) * c.step_more);
+    const long r_tiles = (long)((f.M + 32 * a - 1) / (32 * a)) * ((f.rank + 32 * a - 1) / (32 * a));
+    const long room = per_cu == 1 ? num_cus - own : std::min(num_cus, kMaxFront);
+    if (r_tiles > room) continue;
+    const int most = a == 1 ? std::max(1, std::min({stages / 6, (int)(room / r_tiles), 16})) : 1;
+    const int fitting = std::min(most, (int)((slots - own) / r_tiles));  // slices with which everything is there at once
+    for (const int slices : {most, fitting}) {
+      if (slices < 1) continue;
+      const int count = (int)r_tiles * slices;
+      const float there = 2.f + (a == 1 ? 0.45f : 0.65f) * (own > num_cus ? 1.65f : 1.f) * (float)((stages + slices - 1) / slices) + (slices > 1 ? 2.5f : 0.f);
+      float us = 1.5f + std::max(0.f, 1.25f * there + 1.f - readers);  // (a late r costs far more than the rest)
+      if (own > slots) us += there * (float)count / (float)slots;
+      else if (own + count > slots) us += 0.37f * there;
+      if (us >= best) continue;
+      best = us;
+      found = true;
+      f.a = a;
+      f.slices = slices;
+      f.count = count;
+      f.front = own <= num_cus && count + own > num_cus && per_cu > 1 ? num_cus : count;
+    }
+  }
+  return found;
 }
 
 static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes, bool y32, hipStream_t stream) {
@@ -1212,9 +1314,18 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
       }
     }
   }
+  if (gg.front.pub != nullptr) {
+    bool planned = false;
+    for (const GemmCost& c : kGemmCost)
+      if (tiled_ok && c.mt == mt && c.nt == nt && c.wk == wk) planned = plan_front(gg, c, num_cus, ws_bytes);
+    if (!planned) return hipErrorNotReady;
+  }
 #define GLOWQ_GEMM_TILED_CASE(MT, NT, WK)                                                  \
-  if (tiled_ok && mt == MT && nt == NT && wk == WK)                                        \
-    return y32 ? launch_gemm_t<MT, NT, true, true, true, WK, float>(gg, stream) : launch_gemm_t<MT, NT, true, true, true, WK>(gg, stream);
+  if (tiled_ok && mt == MT && nt == NT && wk == WK) {                                      \
+    if (gg.front.pub != nullptr)                                                           \
+      return y32 ? launch_gemm_t<MT, NT, true, true, true, WK, float, true>(gg, stream) : launch_gemm_t<MT, NT, true, true, true, WK, half_t, true>(gg, stream); \
+    return y32 ? launch_gemm_t<MT, NT, true, true, true, WK, float>(gg, stream) : launch_gemm_t<MT, NT, true, true, true, WK>(gg, stream); \
+  }
   GLOWQ_GEMM_TILED_CASE(4, 2, 1) GLOWQ_GEMM_TILED_CASE(2, 2, 1) GLOWQ_GEMM_TILED_CASE(1, 2, 1) GLOWQ_GEMM_TILED_CASE(4, 1, 1)
   GLOWQ_GEMM_TILED_CASE(2, 1, 1) GLOWQ_GEMM_TILED_CASE(1, 1, 1) GLOWQ_GEMM_TILED_CASE(4, 2, 2) GLOWQ_GEMM_TILED_CASE(2, 1, 2)
 #undef GLOWQ_GEMM_TILED_CASE
@@ -1284,6 +1395,8 @@ bool gemm_widens(const GroupDev& g) {
   return gemm_supported(g) && gemm_tiled_form(gg);
 }
 
+size_t gemm_handover_bytes() { return kGemmHandoverBytes; }
+
 hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
   GemmGroup gg;
   fill_gemm_group(g, gg);
@@ -1291,10 +1404,14 @@ hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
   // workspace; launch_gemm_group turns this into the slice count
   size_t padded = 0;
   for (int i = 0; i < g.n_members; ++i) padded += (size_t)((g.M + 127) / 128 * 128) * ((g.mem[i].N + 255) / 256 * 256);
+  // a launch that computes r itself (run_group set g.pub) keeps its words in front of the partial tiles
   const bool ws_ok = g.ws != nullptr && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0;
-  gg.slices = ws_ok ? (int)std::min<size_t>(g.ws_bytes / (padded * sizeof(float)), 64) : 0;
-  gg.partials = static_cast<float*>(g.ws);
-  return launch_gemm_group(gg, num_cus, ws_ok ? g.ws_bytes : 0, g.mem[0].y32 != 0, stream);
+  const size_t words = g.pub != nullptr ? kGemmHandoverBytes : 0, ws_bytes = ws_ok && g.ws_bytes > words ? g.ws_bytes - words : 0;
+  gg.slices = (int)std::min<size_t>(ws_bytes / (padded * sizeof(float)), 64);
+  gg.partials = reinterpret_cast<float*>(static_cast<unsigned char*>(g.ws) + words);
+  gg.front = FrontArgs{g.x, g.R, g.r_out, g.pub, nullptr, g.M, g.K, g.rank, 0, 0, 1, 1, g.pub_mute ? kNeverRaised : g.pub_spin, g.pub_any_cost};
+  gg.front.partials = gg.partials == nullptr ? nullptr : reinterpret_cast<float*>(static_cast<unsigned char*>(g.ws) + kGemmWordBytes);
+  return launch_gemm_group(gg, num_cus, ws_bytes, g.mem[0].y32 != 0, stream);
 }
 
 // ---- shared projection for many rows: r[M, rank] = fp16(x[M, K] . R[rank, K]^T) ---------------------------
@@ -1650,6 +1767,7 @@ static ProjPlan plan_proj(int M, int K, int rank, int num_cus, size_t ws_bytes) 
 // 34 / 78; K = 4096, rank 128 at 100 / 1500 rows 7.3 / 8.6, 12.0 / 17.1; K = 1536, rank 256 at 512 rows 8.9 / 6.9 (not taken).
 struct ProjTilePlan {
   int a, slices;  // a = 0: the 32-row tiles
+  float us;       // prediction
 };
 static ProjTilePlan plan_proj_tile(const ProjPlan& p, int M, int K, int rank, int num_cus, size_t ws_bytes) {
   const auto rounds_more = [&](long wgs) { return (float)((wgs + num_cus - 1) / num_cus - 1); };
@@ -1660,7 +1778,7 @@ static ProjTilePlan plan_proj_tile(const ProjPlan& p, int M, int K, int rank, in
   float best = 3.9f + per * (p.nt == 1 ? 0.48f : 0.81f) + per * 0.52f * rounds_more(wgs);
   if (p.slices > 1) best += 1.6f + 0.09f * (float)p.slices + 1.5f * slice_mb * (float)p.slices;
   best *= 0.93f;
-  ProjTilePlan plan = {0, 1};
+  ProjTilePlan plan = {0, 1, best};
   for (int a = 1; a <= 2; ++a) {
     const long row_tiles = (M + 64 * a - 1) / (64 * a), col_tiles = (rank + 64 * a - 1) / (64 * a);
     if (row_tiles * col_tiles > 4L * num_cus) continue;
@@ -1674,10 +1792,14 @@ static ProjTilePlan plan_proj_tile(const ProjPlan& p, int M, int K, int rank, in
       if (s > 1 && p.slices == 1) us += 1.5f;  // a second launch where there was none also takes the host's time
       if (us >= best) continue;
       best = us;
-      plan = {a, (stages + depth - 1) / depth};  // no slice without stages
+      plan = {a, (stages + depth - 1) / depth, us};  // no slice without stages
     }
   }
   return plan;
+}
+
+static float proj_launch_us(int M, int K, int rank, int num_cus, size_t ws_bytes) {
+  return plan_proj_tile(plan_proj(M, K, rank, num_cus, ws_bytes), M, K, rank, num_cus, ws_bytes).us;
 }
 
 size_t proj_workspace_bytes(int M, int K, int rank, int num_cus) {

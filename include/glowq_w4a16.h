@@ -182,6 +182,10 @@ int glowq_w4a16_group_forward_fused(const void* x, const void* R, void* r_out, c
  * graph is a launch like any other).  One launch instead of two, the same bits in r_out and in the outputs as the
  * projection launch in front gives; "proj_in_launch" of glowq_set_tuning switches it off.  As everywhere, calls that
  * share a workspace must not overlap.
+ * The GEMM on the tiled weights does the same from 65 token rows on where that is predicted to pay: tiles of r in front of the
+ * grid, a word each; its readers want r behind their weights.  The first 2 101 248 bytes of the workspace hold the words
+ * and fp32 sums of r, the partial tiles of a split of K lie behind them; with less the projection launch stays.  r and outputs agree
+ * with the two-launch form to the rounding of fp32 sums; glowq_last_launch names the grid of the output tiles alone.
  * The skinny MFMA route does the same at 2..32 token rows where its launch leaves enough compute units free for the
  * workgroups that produce r (a workgroup per one or two blocks of four token rows by four rows of R; every group of an 8B
  * layer at 8 and 16 rows): they write r_out with stores that pass the caches private to a part of the chip and raise a
@@ -296,11 +300,12 @@ int glowq_probe_empty_launch(int grid, int block, void* stream);
  * "proj_in_launch" (0 / 1, default 1): a fused single-token call with a workspace computes r inside the group launch
  * where that applies (glowq_w4a16_group_forward_fused_ws); 2, for tests, keeps the producing waves from handing their
  * entries over, so that every reader runs into "proj_spin_limit" (default 16384, 0 = never waits: the number of times
- * a reader looks again for an entry of r that is not there yet before it computes the entry itself).
+ * a reader looks again for an entry of r that is not there yet before it computes the entry itself).  "proj_any_cost" (0 / 1,
+ * default 0), for tests: 1 has launches on the tiled weights compute r wherever they can, not only where that is predicted to pay.
  * Returns the previous value (>= 0) or GLOWQ_EINVAL.  Initial values come from GLOWQ_QUAD_M,
  * GLOWQ_QUAD_MIN_M, GLOWQ_WAVEDOT_M, GLOWQ_SKINNY_M, GLOWQ_SMALL_GROUP_MB, GLOWQ_STREAM_M, GLOWQ_STREAM_SHAPE_RULE,
  * GLOWQ_QSTREAM_M, GLOWQ_QSTREAM_SHAPE_RULE, GLOWQ_SKINNY_CODES_M, GLOWQ_TILED_MIN_M, GLOWQ_TILED_MAX_M,
- * GLOWQ_TILED_SHAPE_RULE, GLOWQ_PROJ_IN_LAUNCH and GLOWQ_PROJ_SPIN_LIMIT.
+ * GLOWQ_TILED_SHAPE_RULE, GLOWQ_PROJ_IN_LAUNCH, GLOWQ_PROJ_ANY_COST and GLOWQ_PROJ_SPIN_LIMIT.
  */
 int glowq_set_tuning(const char* key, int value);
 

@@ -5,6 +5,7 @@ import torch
 
 from glowq_amd.kernels import PreparedGroup
 from glowq_amd.linear import CudaW4A16Linear
+from helpers import tuning
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +60,117 @@ def test_rows_that_are_not_finite_stay_by_themselves(ext, M, K, Ns, rank, bad):
     y = pg.run(x)
     check([v[fine] for v in y], x[fine], pg.last_r[fine], weights, members, 1.0, f"M={M} K={K}")
     assert not any(torch.isfinite(v[rows]).any() for v in y)
+
+
+# ---- launches that compute r = x R^T themselves (workgroups in front of the grid, words in the workspace) ----------------------------
+@pytest.fixture
+def wherever_they_can(ext):
+    with tuning(ext, proj_any_cost=1):
+        yield
+
+
+def computed_r(ext, run):
+    """Whether `run` raised a word of its own at the head of the workspace: a tag of 48 bits, its top bit set (sums left there by other
+    launches have sixteen more bits)."""
+    dev = torch.device("cuda", torch.cuda.current_device())
+    ext._workspace(dev, 65)
+    head = ext._workspaces[(dev.index, ext._stream(dev), False)][:8]
+    head.zero_()
+    run()
+    torch.cuda.synchronize()
+    return int(head.view(torch.int64).item()) >> 47 == 1
+
+
+# 32 x 32 tiles of r with K in one slice and in many, 64 x 64 tiles (more than 256 small ones), both on four and on eight waves, fronts filled
+# up to one workgroup a compute unit, ragged rows and ranks, ranks of several steps, launches of one and of several rounds, tails and slices
+FRONT_CASES = [(65, 256, [130], 8), (65, 768, [200], 40), (100, 3328, [4096, 300], 136), (333, 3584, [3584, 512, 500], 128), (130, 14336, [1000], 64),
+               (333, 14336, [4096], 120), (1500, 2304, [2050], 256), (300, 1024, [20000], 392), (1500, 5120, [5120], 264), (1030, 17408, [5120], 200)]
+
+
+@pytest.mark.parametrize("M,K,Ns,rank", FRONT_CASES)
+def test_launch_computes_r_itself(ext, wherever_they_can, M, K, Ns, rank):
+    print(f"case M={M} K={K} Ns={Ns} rank={rank}", flush=True)
+    x, R, members, weights = make(M + rank, M, K, Ns, rank)
+    if len(Ns) > 1:
+        members[1]["L"] = None if M % 2 else members[1]["L"]  # (a member without correction)
+    pg = PreparedGroup(ext, members, K, 128, 0.75, R=R)
+    pg.run(x)  # (makes the copies)
+    want_r = x.double() @ R.double().t()
+    for _ in range(2):
+        got = []
+        assert computed_r(ext, lambda: got.extend(pg.run(x)))
+        r = pg.last_r
+        # one rounding to fp16 (2^-11), fp32 sums of K terms around K^-1/2
+        assert ((r.double() - want_r).abs() <= 2.0 ** -11 * want_r.abs() + 1e-4).all()
+        for y, w, m in zip(got, weights, members):
+            if m["L"] is None:
+                want = x.double() @ w.double().t()
+                assert ((y.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2e-4).all()
+            else:
+                check([y], x, r, [w], [m], 0.75, f"M={M} K={K} rank={rank}")
+    with tuning(ext, proj_in_launch=0):
+        apart = []
+        assert not computed_r(ext, lambda: apart.extend(pg.run(x)))
+    for a, b in zip(got, apart):
+        assert ((a.double() - b.double()).abs() <= 2.0 ** -10 * b.double().abs() + 4e-4).all()
+
+
+@pytest.mark.parametrize("M,K,Ns,rank", [(65, 768, [200], 40), (333, 3584, [3584, 512, 500], 128), (130, 14336, [1000], 64)])
+def test_readers_that_never_hear_from_the_front(ext, wherever_they_can, M, K, Ns, rank):
+    """Words that never go up: the first slice of a tile walks all of K, and every reader computes its r."""
+    x, R, members, weights = make(M + rank, M, K, Ns, rank)
+    pg = PreparedGroup(ext, members, K, 128, 1.0, R=R)
+    with tuning(ext, proj_in_launch=2, proj_spin_limit=3):
+        y = pg.run(x)
+        torch.cuda.synchronize()
+    want_r = x.double() @ R.double().t()
+    assert ((pg.last_r.double() - want_r).abs() <= 2.0 ** -11 * want_r.abs() + 1e-4).all()
+    for got, w, m in zip(y, weights, members):
+        want = x.double() @ w.double().t() + want_r @ m["L"].double().t()
+        # r of a reader and r_out may round apart: half an ulp of r (2^-11 of a few units) through 8 to 128 entries of L (0.05)
+        assert ((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2e-3).all()
+
+
+def test_replays_and_launches_see_their_own_r(ext, wherever_they_can):
+    """Eager launches and replays in turn through the same words, new activations each time, another group with other tiles between."""
+    M, K, Ns, rank = 100, 3328, [4096, 300], 136
+    x, R, members, weights = make(3, M, K, Ns, rank)
+    x2, R2, members2, weights2 = make(4, 333, 2304, [2050], 64)
+    pg, pg2 = PreparedGroup(ext, members, K, 128, 1.0, R=R), PreparedGroup(ext, members2, 2304, 128, 1.0, R=R2)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        pg.run(x), pg2.run(x2)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            y = pg.run(x)
+            r = pg.last_r
+        g = torch.Generator(device="cuda").manual_seed(9)
+        for it in range(6):
+            x.copy_(torch.randn(M, K, device="cuda", generator=g))
+            graph.replay()
+            side.synchronize()
+            check(y, x, r, weights, members, 1.0, f"replay {it}")
+            want_r = x.double() @ R.double().t()
+            assert ((r.double() - want_r).abs() <= 2.0 ** -11 * want_r.abs() + 1e-4).all(), it
+            x2.copy_(torch.randn(333, 2304, device="cuda", generator=g))
+            y2 = pg2.run(x2)
+            check(y2, x2, pg2.last_r, weights2, members2, 1.0, f"eager {it}")
+    torch.cuda.current_stream().wait_stream(side)
+
+
+def test_calls_without_room_for_the_words_keep_the_projection_launch(ext, wherever_they_can):
+    M, K, Ns, rank = 100, 3328, [4096, 300], 136
+    x, R, members, weights = make(5, M, K, Ns, rank)
+    pg = PreparedGroup(ext, members, K, 128, 1.0, R=R)
+    saved = ext.WORKSPACE_BYTES
+    try:
+        for nbytes in (16, 4096, 1 << 20):
+            ext.WORKSPACE_BYTES = nbytes
+            ext._workspaces.clear()
+            y = pg.run(x)
+            check(y, x, pg.last_r, weights, members, 1.0, f"workspace {nbytes}")
+    finally:
+        ext.WORKSPACE_BYTES = saved
+        ext._workspaces.clear()
