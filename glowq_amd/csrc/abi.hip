@@ -40,7 +40,7 @@ bool skinny_group_form(const GroupDev& g);
 bool skinny_raw_form(const GroupDev& g);
 hipError_t launch_skinny(GroupDev& g, int num_cus, hipStream_t stream, bool raw);
 bool gemm_supported(const GroupDev& g);
-hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream);
+hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream, bool exact = false);
 size_t gemm_handover_bytes();
 bool gemm_widens(const GroupDev& g);
 // misc.hip
@@ -416,10 +416,23 @@ int pick_route_rounded(const GroupDev& g, int force) {
 
 // Runs one group through the chosen route.  Routes with a row capacity smaller than M walk the
 // token rows in chunks (weights are re-read once per chunk).
+// Calls of the route on the tiled copy that run on the GEMM in its unrounded form: all of 33 to 64 rows, and from 17 rows on groups whose
+// 128-column tiles come to between half and all of the compute units (K of 2048 columns and more).  us with the projection, 24 and 32
+// rows, GEMM / the kernel of skinny_tiled.hip: 8B gate|up (224 tiles) 22.6, 22.9 / 26.1, 26.5; 27648 x 5120 (216) 24.4, 23.9 / 30.3, 30.3;
+// 14B gate|up (272: a second round) 40.5, 42.6 / 36.2, 37.4; 14B down_proj (40 tiles in slices of K) 33.0, 34.5 / 31.6, 32.5; 12 and 16 rows 8B gate|up
+// 22.5, 22.8 / 20.5, 20.8.
+bool tiled_route_on_gemm(const GroupDev& g) {
+  if (g.M > 32) return true;
+  long tiles = 0;
+  for (int i = 0; i < g.n_members; ++i) tiles += (g.mem[i].N + 127) / 128;
+  return g.M > 16 && g.K >= 2048 && tiles * 2 > num_cus() && tiles <= num_cus();
+}
+
 int run_group(GroupDev g, int route, hipStream_t stream) {
   for (int i = 0; i < g.n_members; ++i)
     if (g.mem[i].y32 && !(route == kRouteGemm && gemm_widens(g))) return fail(GLOWQ_EUNSUPPORTED, "fp32 outputs: only where the GEMM on the tiled weights takes the call, and for all members alike");
   const int cus = num_cus();
+  const bool on_gemm = route == kRouteSkinnyTiled && tiled_route_on_gemm(g);
   hipError_t e = hipSuccess;
   g.pub = nullptr;
   const auto hand_over = [&]() {  // workgroups in front of the launch hand r to the others through the workspace
@@ -460,8 +473,8 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
     g.pub = nullptr;
   }
   const bool skinny_route = route == kRouteSkinny || route == kRouteSkinnyRaw;
-  if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || route == kRouteSkinnyTiled) && skinny_proj_in_launch(g)) ||
-                         (route == kRouteGemm && gemm_proj_in_launch(g)))) {
+  if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || (route == kRouteSkinnyTiled && !on_gemm)) && skinny_proj_in_launch(g)) ||
+                         ((route == kRouteGemm || on_gemm) && gemm_proj_in_launch(g)))) {
     // single token on the stream GEMV, a handful of rows on the skinny kernel: workgroups in front of the group launch
     // produce r and hand it to the others through the workspace (stream_kernel.hpp, skinny.hip), no launch in front
     hand_over();
@@ -495,11 +508,12 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
       e = launch_gemm(g, cus, stream);
     }
   } else if (route == kRouteSkinnyTiled) {
-    e = launch_skinny_tiled(g, cus, stream);
+    const auto launch = [&]() { return on_gemm ? launch_gemm(g, cus, stream, true) : launch_skinny_tiled(g, cus, stream); };
+    e = launch();
     if (e == hipErrorNotReady && g.pub != nullptr) {
       e = launch_projection();
       if (e != hipSuccess) return fail(GLOWQ_ELAUNCH, "shared_proj launch failed: %s", hipGetErrorString(e));
-      e = launch_skinny_tiled(g, cus, stream);
+      e = launch();
     }
   } else if (skinny_route) {
     e = launch_skinny(g, cus, stream, route == kRouteSkinnyRaw);

@@ -84,8 +84,9 @@ __device__ __forceinline__ h8 permute_for_nibble_order(const h8& v) {
   return p;
 }
 
-// 8 codes of one word -> fp16((code - zero) * scale), in nibble order (0,4,1,5,2,6,3,7).
+// 8 codes of one word -> fp16((code - zero) * scale), in nibble order (0,4,1,5,2,6,3,7); kScaled = false: code - zero, exact.
 // zb_lo = -(1024 + zero), zb_hi = -(64 + zero), both exact in fp16.
+template <bool kScaled = true>
 __device__ __forceinline__ h8 dequant_word(uint32_t w, h2 zb_lo, h2 zb_hi, h2 s2) {
   // the two exponent patterns (1024.0 and 64.0 in both halves) live in vector registers: with the nibble mask as the one
   // scalar operand the mask-and-merge is then a single v_and_or_b32 instead of an AND and an OR
@@ -97,10 +98,13 @@ __device__ __forceinline__ h8 dequant_word(uint32_t w, h2 zb_lo, h2 zb_hi, h2 s2
   const h2 q1 = bitcast_u32<h2>((w & 0x00F000F0u) | e64);
   const h2 q2 = bitcast_u32<h2>((hi & 0x000F000Fu) | e1024);
   const h2 q3 = bitcast_u32<h2>((hi & 0x00F000F0u) | e64);
-  const h2 d0 = (q0 + zb_lo) * s2;
-  const h2 d1 = (q1 + zb_hi) * s2;
-  const h2 d2 = (q2 + zb_lo) * s2;
-  const h2 d3 = (q3 + zb_hi) * s2;
+  h2 d0 = q0 + zb_lo, d1 = q1 + zb_hi, d2 = q2 + zb_lo, d3 = q3 + zb_hi;
+  if constexpr (kScaled) {
+    d0 *= s2;
+    d1 *= s2;
+    d2 *= s2;
+    d3 *= s2;
+  }
   h8 out;
   out[0] = d0[0]; out[1] = d0[1]; out[2] = d1[0]; out[3] = d1[1];
   out[4] = d2[0]; out[5] = d2[1]; out[6] = d3[0]; out[7] = d3[1];
@@ -562,11 +566,11 @@ void gemm_mfma_kernel(const GemmGroup gg, const int m_blocks) {
 //     rows 443 -> 430 us, down_proj at 333 rows 61.7 -> 55.8, 14B o_proj at 100 rows 21.2 -> 18.7, same cuts).
 constexpr int kTRow = 256;  // bytes of a staged row: 128 halves, swizzled instead of padded
 
-// The order of a word's instructions: behind every matrix instruction its share of the next word's thirteen vector instructions per column
-// tile, the next fragments from LDS in front (few matrix instructions a word) or as soon as a fragment has been used for the last time.
-template <int kMT, int kNT>
+// The order of a word's instructions: behind every matrix instruction its share of the next word's kOps vector instructions per column tile,
+// the next fragments from LDS in front (few matrix instructions a word) or as soon as a fragment has been used for the last time.
+template <int kMT, int kNT, int kOps>
 __device__ __forceinline__ void order_word() {
-  constexpr int kShare = (13 * kNT + kMT * kNT - 1) / (kMT * kNT);
+  constexpr int kShare = (kOps * kNT + kMT * kNT - 1) / (kMT * kNT);
   constexpr bool kReadsFirst = kMT * kNT <= 4;
   if constexpr (kReadsFirst) __builtin_amdgcn_sched_group_barrier(0x100, kMT, 0);
 #pragma unroll
@@ -587,8 +591,11 @@ __device__ __forceinline__ void order_word() {
 // kProj: the launch computes r = x R^T itself.  The readers need r behind their K loop, which is when the workgroups in front of the grid are
 // done as a rule; they wait for the words of their rows' tiles (bounded: a reader that gives up computes its r from x and R), and
 // read r past the caches the stores of the workgroups in front have passed.
-template <int kMT, int kNT, int kWk, typename YT, bool kProj>
-__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : (kMT * kNT <= 2 ? 4 : 2)), (kMT * kNT >= 16 ? 1 : 8))))
+// kExact: up to 64 rows, the arithmetic of the kernel of skinny_tiled.hip: the matrix instructions multiply code - zero, and the sum over a
+// half of 128 columns meets its scale in fp32, so the weight is never rounded (nine vector instructions a word and sixteen a
+// half and tile against thirteen a word: as many at two row tiles).
+template <int kMT, int kNT, int kWk, typename YT, bool kProj, bool kExact>
+__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : (kMT * kNT <= 2 && !(kExact && kMT == 2) ? 4 : 2)), (kMT * kNT >= 16 ? 1 : 8))))
 void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
   const int front = kProj ? gg.front.front : 0;
@@ -596,11 +603,18 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   if constexpr (kProj) {
     tag = launch_tag();
     if ((int)blockIdx.x < front) {
-      if (blockIdx.y == 0) run_front<4 * kWk>(gg.front, (int)blockIdx.x, tag, smem_all);
+      run_front<4 * kWk>(gg.front, (int)blockIdx.x, tag, smem_all);
       return;
     }
   }
-  int wg = (int)blockIdx.x - front, slice = (int)blockIdx.y, nslices = gg.slices, part_tile = wg, part_tiles = (int)gridDim.x - front;
+  // (with workgroups in front the slices of K lie behind each other in x: in y every one of them would bring a front that only leaves again)
+  const int across = kProj && gg.slices > 1 ? ((int)gridDim.x - front) / gg.slices : (int)gridDim.x - front;
+  int wg = (int)blockIdx.x - front, slice = (int)blockIdx.y, nslices = gg.slices;
+  if (kProj && gg.slices > 1) {
+    slice = wg / across;
+    wg -= slice * across;
+  }
+  int part_tile = wg, part_tiles = across;
   if (gg.tail_slices > 1) {
     nslices = 1;
     if (wg >= gg.full) {
@@ -772,6 +786,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   // instructions and the wait for its fragments in front of its own matrix instructions, and the two pipes take turns.
   struct Zero {
     h2 lo[kNT], hi[kNT], s[kNT];
+    float scale[kNT];  // kExact
   };
   auto zero_of = [&](const BSet& s, int g) __attribute__((always_inline)) {
     Zero z;
@@ -782,7 +797,8 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
       const half_t zl = (half_t)(nz - 1024.0f), zh = (half_t)(nz - 64.0f);
       z.lo[tn] = h2{zl, zl};
       z.hi[tn] = h2{zh, zh};
-      z.s[tn] = bitcast_u32<h2>(__builtin_amdgcn_perm(sw, sw, 0x01000100u));
+      if constexpr (kExact) z.scale[tn] = (float)__builtin_bit_cast(half_t, (uint16_t)(sw & 0xFFFFu));
+      else z.s[tn] = bitcast_u32<h2>(__builtin_amdgcn_perm(sw, sw, 0x01000100u));
     }
     return z;
   };
@@ -790,12 +806,14 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   Zero zero = zero_of(b[0], 0);  // zero-points and scales of the half the next word lies in
   h8 bf[kNT];                    // the next word, dequantised
 #pragma unroll
-  for (int tn = 0; tn < kNT; ++tn) bf[tn] = dequant_word(b[0].w[tn][0][0], zero.lo[tn], zero.hi[tn], zero.s[tn]);
+  for (int tn = 0; tn < kNT; ++tn) bf[tn] = dequant_word<!kExact>(b[0].w[tn][0][0], zero.lo[tn], zero.hi[tn], zero.s[tn]);
   // d (the set that holds super-block sb) and g are compile-time constants at every call site
   auto half_step = [&](int sb, auto d_const, auto g_const) __attribute__((always_inline)) {
     constexpr int d = decltype(d_const)::value, g = decltype(g_const)::value;
     const BSet& cur = b[d];
     BSet& nxt = b[d ^ 1];
+    f16v half_sum[kExact ? kMT : 1][kExact ? kNT : 1];
+    float scale[kNT];
     h8 af[kMT];
 #pragma unroll
     for (int u = 0; u < kMT; ++u) af[u] = read_a(stage, u, 8 * lh);
@@ -813,21 +831,39 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
 #pragma unroll
         for (int u = 0; u < kMT; ++u) an[u] = read_a(stage, u, 8 * lh + t + 1);
       }
-      if (t == 7) zero = zero_of(g == 0 ? cur : nxt, g ^ 1);
+      if (t == 7) {
+        if constexpr (kExact) {
+#pragma unroll
+          for (int tn = 0; tn < kNT; ++tn) scale[tn] = zero.scale[tn];
+        }
+        zero = zero_of(g == 0 ? cur : nxt, g ^ 1);
+      }
 #pragma unroll
       for (int tn = 0; tn < kNT; ++tn) {
         const uint32_t w = t < 7 ? cur.w[tn][2 * g + (t + 1) / 4][(t + 1) & 3] : (g == 0 ? cur.w[tn][2][0] : nxt.w[tn][0][0]);
-        bn_[tn] = dequant_word(w, zero.lo[tn], zero.hi[tn], zero.s[tn]);
+        bn_[tn] = dequant_word<!kExact>(w, zero.lo[tn], zero.hi[tn], zero.s[tn]);
       }
 #pragma unroll
       for (int u = 0; u < kMT; ++u)
 #pragma unroll
-        for (int tn = 0; tn < kNT; ++tn) acc[u][tn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[u], bf[tn], acc[u][tn], 0, 0, 0);
-      order_word<kMT, kNT>();
+        for (int tn = 0; tn < kNT; ++tn) {
+          f16v& sum = kExact ? half_sum[u][tn] : acc[u][tn];
+          if (kExact && t == 0) sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[u], bf[tn], f16v{}, 0, 0, 0);
+          else sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[u], bf[tn], sum, 0, 0, 0);
+        }
+      order_word<kMT, kNT, kExact ? 9 : 13>();
 #pragma unroll
       for (int u = 0; u < kMT; ++u) af[u] = an[u];
 #pragma unroll
       for (int tn = 0; tn < kNT; ++tn) bf[tn] = bn_[tn];
+    }
+    if constexpr (kExact) {
+#pragma unroll
+      for (int u = 0; u < kMT; ++u)
+#pragma unroll
+        for (int tn = 0; tn < kNT; ++tn)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[u][tn][e] = __builtin_fmaf(scale[tn], half_sum[u][tn][e], acc[u][tn][e]);
     }
     __builtin_amdgcn_sched_barrier(0);
     wait_loads_but(std::integral_constant<int, 2 * kNT + (g == 0 ? kNT : 0)>{});
@@ -1018,12 +1054,12 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmGroup gg, co
 }
 
 // ---- host side ------------------------------------------------------------------------------------
-template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1, typename YT = half_t, bool kProj = false>
+template <int kMT, int kNT, bool kQuant, bool kSuper = false, bool kTiled = false, int kWk = 1, typename YT = half_t, bool kProj = false, bool kExact = false>
 static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   static_assert(!kTiled || (kQuant && kSuper), "the tiled copy serves the super-block form");
   static_assert(kTiled || (kWk == 1 && std::is_same_v<YT, half_t>), "K groups inside a workgroup and fp32 outputs: the tiled-copy kernel");
   constexpr int BM = 32 * kMT, BN = 128 * kNT;
-  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk, YT, kProj> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
+  auto kern = kTiled ? gemm_tiled_kernel<kMT, kNT, kWk, YT, kProj, kExact> : gemm_mfma_kernel<kMT, kNT, kQuant, kSuper>;
   size_t lds = kTiled ? (size_t)kWk * 2 * BM * kTRow
                       : (size_t)2 * BM * kARow * sizeof(half_t) + (kSuper ? (size_t)4 * (32 * kNT) * 144 : 0);
   if (kWk > 1 && lds < (size_t)BM * BN * sizeof(float)) lds = (size_t)BM * BN * sizeof(float);  // the hand-over of the accumulators
@@ -1041,7 +1077,7 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
   const int front = kProj ? gg.front.front : 0;  // (the launch record names the grid of the tiles)
   const int tail_wgs = gg.tail_slices > 1 ? gg.full + (total - gg.full) * gg.tail_slices : 0;
   note_launch(tail_wgs > 0 ? tail_wgs : total, tail_wgs > 0 ? 1 : gg.slices, 256 * kWk, "%s<%d,%d,%d%s>",
-              kTiled ? "gemm_tiled_kernel" : "gemm_mfma_kernel", kMT, kNT, kWk, std::is_same_v<YT, float> ? ",float" : "");
+              kTiled ? "gemm_tiled_kernel" : "gemm_mfma_kernel", kMT, kNT, kWk, kExact ? ",exact" : std::is_same_v<YT, float> ? ",float" : "");
   if (tail_wgs > 0) {
     const int tail_tiles = total - gg.full;
     hipLaunchKernelGGL(kern, dim3(front + tail_wgs, 1), dim3(256 * kWk), lds, stream, gg, m_blocks);
@@ -1049,7 +1085,7 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(tail_tiles, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(kern, dim3(front + total, gg.slices), dim3(256 * kWk), lds, stream, gg, m_blocks);
+  hipLaunchKernelGGL(kern, kProj ? dim3(front + total * gg.slices) : dim3(total, gg.slices), dim3(256 * kWk), lds, stream, gg, m_blocks);
   if (hipError_t e = hipGetLastError(); e != hipSuccess || gg.slices == 1) return e;
   hipLaunchKernelGGL((gemm_reduce_kernel<kMT, kNT, YT>), dim3(total, kMT * kNT), dim3(256), 0, stream, gg, m_blocks);
   return hipGetLastError();
@@ -1069,6 +1105,12 @@ constexpr GemmCost kGemmCost[] = {
     {2, 1, 1, 2.2f, 2.1f, 0.60f, 0.39f, 1.6f, 0.37f, 0.64f}, {2, 1, 2, 2.0f, 3.0f, 0.96f, 0.88f, 2.3f, 0.34f, 0.96f},
     {2, 2, 1, 2.9f, 3.3f, 0.90f, 0.77f, 1.6f, 0.29f, 0.52f}, {4, 1, 1, 3.1f, 2.8f, 1.00f, 0.73f, 1.9f, 0.24f, 0.59f},
     {4, 2, 1, 5.0f, 4.0f, 1.43f, 1.27f, 1.1f, 0.23f, 0.58f}, {4, 2, 2, 6.0f, 5.5f, 2.46f, 3.10f, 1.3f, 0.25f, 0.92f}};
+
+// The same for the unrounded form at 33 to 64 rows: 558 timings of 19 groups of 1B to 14B shapes at 36 and 57 rows, 6 % rms; the cut it picks
+// takes 1.6 % longer than the fastest of them in the mean, 9 % at most.
+constexpr GemmCost kGemmExactCost[] = {{1, 1, 1, 1.9f, 1.0f, 0.43f, 0.21f, 3.1f, 0.47f, 1.63f},
+                                       {2, 1, 1, 1.5f, 1.9f, 0.52f, 0.32f, 3.1f, 0.35f, 1.65f},
+                                       {2, 1, 2, 4.3f, 1.1f, 0.81f, 1.03f, 2.7f, 0.35f, 1.83f}};
 
 static int gemm_tiles(const GemmGroup& gg, int mt, int nt) {
   int cols = 0;
@@ -1120,8 +1162,10 @@ static bool gemm_tiled_form(const GemmGroup& gg) {
 }
 
 static float proj_launch_us(int M, int K, int rank, int num_cus, size_t ws_bytes);
+bool proj_on_small_kernel(int M, int K, int rank);  // abi.hip
 
-// How a launch that computes r itself cuts it, given its own cut; false: r comes from a launch of its own, which is predicted to cost less.
+// How a launch that computes r itself cuts it, given its own cut, and what that is predicted to cost it, in us; `f.count` 0: r comes from a
+// launch of its own, which is predicted to cost less (that cost, then).
 //  * Tiles of 32 x 32 with K in as many slices as keep six stages each and leave one workgroup a compute unit, or tiles of 64 x 64: 0.45 and
 //    0.65 us a stage of 128 columns, 1.65 times that where every compute unit has work of the launch's own as well, about 2 us at the ends, 2.5
 //    for the sum of slices: measured on launches that waited for r.  What that
@@ -1133,15 +1177,15 @@ static float proj_launch_us(int M, int K, int rank, int num_cus, size_t ws_bytes
 //    Otherwise some compute units get two, and the launch takes as long as those: 8B down_proj at 333 rows 72.3 with 220 in front, 57.6
 //    with 264, projection in front 67.6, r given 55.8; 14B down_proj at 512 rows 134 with 128, 106 with 256, 118, 100.
 // 16 groups of 1B to 14B shapes at 65 to 2048 rows: 1.14 times as fast in the mean with the rule as with the projection in front.
-static bool plan_front(GemmGroup& gg, const GemmCost& c, int num_cus, size_t ws_bytes) {
+static float plan_front(GemmGroup& gg, const GemmCost& c, bool exact, int num_cus, float launch_us) {
   FrontArgs& f = gg.front;
   const int tiles = gemm_tiles(gg, c.mt, c.nt), sb = f.K >> 8, stages = f.K >> 7;
   const int own = gg.tail_slices > 1 ? gg.full + (tiles - gg.full) * gg.tail_slices : tiles * gg.slices;
-  float best = f.any_cost ? 1e30f : proj_launch_us(f.M, f.K, f.rank, num_cus, ws_bytes);
-  bool found = false;
+  float best = f.any_cost ? 1e30f : launch_us;
+  f.count = 0;
   for (int a = 1; a <= 2; ++a) {
     // workgroups that a compute unit holds: registers, and the LDS that the workgroups in front want (48 or 64 KB of 160)
-    const int per_cu = c.mt == 4 && c.nt == 2 && c.wk == 2 ? 1 : (c.mt * c.nt <= 2 && c.wk == 1 && a == 1 ? 3 : 2);
+    const int per_cu = (c.mt == 4 && c.nt == 2 && c.wk == 2) || (exact && c.wk == 2) ? 1 : (c.mt * c.nt <= 2 && c.wk == 1 && a == 1 ? 3 : 2);
     const int slots = num_cus * per_cu, held = std::min((own + num_cus - 1) / num_cus, per_cu);
     if (a == 2 && per_cu == 2 && c.mt * c.nt <= 2 && own > slots) continue;  // (with 48 KB or less there were three)
     const float readers = gemm_cost_fixed(gg, c) + (float)(2 * (((sb + gg.slices - 1) / gg.slices + c.wk - 1) / c.wk)) * (c.step + (float)(held - 1) * c.step_more);
@@ -1159,14 +1203,66 @@ static bool plan_front(GemmGroup& gg, const GemmCost& c, int num_cus, size_t ws_
       else if (own + count > slots) us += 0.37f * there;
       if (us >= best) continue;
       best = us;
-      found = true;
       f.a = a;
       f.slices = slices;
       f.count = count;
       f.front = own <= num_cus && count + own > num_cus && per_cu > 1 ? num_cus : count;
     }
   }
-  return found;
+  return best;
+}
+
+// Up to 64 rows in the unrounded form: one row block of 64, or up to two of 32, K cut and dealt as the costs have it.  Group launches, us, this /
+// the kernel of skinny_tiled.hip with 64 rows, which it replaced (consumer and producer waves, five of them on four SIMDs on the wide groups,
+// and every workgroup's x through registers): 57 rows 8B q|k|v 14.5 / 18.3, o_proj 13.0 / 16.1, gate|up 26.2 / 32.4, down_proj 20.9 / 26.5; 14B
+// gate|up 42.8 / 45.4, down_proj 25.2 / 31.5; 15 groups at 33 to 64 rows 1.25 times as fast in the mean.
+static hipError_t launch_gemm_exact(GemmGroup& gg, int num_cus, size_t ws_bytes, hipStream_t stream) {
+  const int sb_total = gg.m[0].K >> 8;
+  const bool fused = gg.front.pub != nullptr;
+  // (the projection launch of these rows: 3.4 us at 32 rows, K = 4096, rank 128, 4.3 at 64 rows, 7.5 at 57 rows, K = 5120, rank 256)
+  const float macs = (float)gg.m[0].M * (float)gg.m[0].K * (float)gg.front.rank;
+  const float launch_us = !fused ? 0.f : proj_on_small_kernel(gg.m[0].M, gg.m[0].K, gg.front.rank) ? 2.3f + 0.065e-6f * macs : proj_launch_us(gg.m[0].M, gg.m[0].K, gg.front.rank, num_cus, ws_bytes);
+  const GemmCost* best = nullptr;
+  float best_us = 0.f;
+  GemmGroup cut = gg;
+  // of each kind of cut (tiles; all of them in slices of K, or those of the last, partly filled round) the cheapest, with what r costs it
+  for (const GemmCost& c : kGemmExactCost)
+    for (const bool tail_only : {false, true}) {
+      const int tiles = gemm_tiles(gg, c.mt, c.nt), tail = tiles % num_cus;
+      if (tail_only && (tiles < num_cus || tail == 0)) continue;
+      const size_t tile_bytes = (size_t)(32 * c.mt) * (128 * c.nt) * sizeof(float);
+      float us = 0.f;
+      int slices = 0;
+      for (int s = tail_only ? 2 : 1; s <= 16 && s * 2 <= std::max(sb_total, 2); ++s) {
+        const int per = (sb_total + s - 1) / s, cut_tiles = tail_only ? tail : tiles;
+        if ((sb_total + per - 1) / per != s) continue;  // a slice without super-blocks
+        if (s > 1 && (cut_tiles * s > (tail_only ? 1 : 3) * num_cus || (size_t)cut_tiles * s * tile_bytes > std::min(ws_bytes, (size_t)32 << 20))) break;
+        const float t = gemm_cost_cut(c, tiles, sb_total, tail_only ? 1 : s, tail_only ? s : 0, num_cus);
+        if (slices != 0 && t >= us) continue;
+        us = t;
+        slices = s;
+      }
+      if (slices == 0) continue;
+      cut.slices = tail_only ? 1 : slices;
+      cut.tail_slices = tail_only ? slices : 0;
+      cut.full = tail_only ? tiles - tail : 0;
+      us += gemm_cost_fixed(gg, c);
+      if (fused) us += plan_front(cut, c, true, num_cus, launch_us);
+      if (best != nullptr && us >= best_us) continue;
+      best = &c;
+      best_us = us;
+      gg.slices = cut.slices;
+      gg.tail_slices = cut.tail_slices;
+      gg.full = cut.full;
+      gg.front = cut.front;
+    }
+  if (fused && gg.front.count == 0) return hipErrorNotReady;
+#define GLOWQ_GEMM_EXACT_CASE(MT, WK)                    \
+  if (best->mt == MT && best->nt == 1 && best->wk == WK) \
+    return fused ? launch_gemm_t<MT, 1, true, true, true, WK, half_t, true, true>(gg, stream) : launch_gemm_t<MT, 1, true, true, true, WK, half_t, false, true>(gg, stream);
+  GLOWQ_GEMM_EXACT_CASE(1, 1) GLOWQ_GEMM_EXACT_CASE(2, 1) GLOWQ_GEMM_EXACT_CASE(2, 2)
+#undef GLOWQ_GEMM_EXACT_CASE
+  return hipErrorInvalidValue;
 }
 
 static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes, bool y32, hipStream_t stream) {
@@ -1317,7 +1413,10 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   if (gg.front.pub != nullptr) {
     bool planned = false;
     for (const GemmCost& c : kGemmCost)
-      if (tiled_ok && c.mt == mt && c.nt == nt && c.wk == wk) planned = plan_front(gg, c, num_cus, ws_bytes);
+      if (tiled_ok && c.mt == mt && c.nt == nt && c.wk == wk) {
+        plan_front(gg, c, false, num_cus, proj_launch_us(M, gg.m[0].K, gg.front.rank, num_cus, ws_bytes));
+        planned = gg.front.count > 0;
+      }
     if (!planned) return hipErrorNotReady;
   }
 #define GLOWQ_GEMM_TILED_CASE(MT, NT, WK)                                                  \
@@ -1397,7 +1496,7 @@ bool gemm_widens(const GroupDev& g) {
 
 size_t gemm_handover_bytes() { return kGemmHandoverBytes; }
 
-hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
+hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream, bool exact) {
   GemmGroup gg;
   fill_gemm_group(g, gg);
   // slices of the padded output (rows to a multiple of 128, columns of every member to a multiple of 256) that fit the
@@ -1411,6 +1510,7 @@ hipError_t launch_gemm(GroupDev& g, int num_cus, hipStream_t stream) {
   gg.partials = reinterpret_cast<float*>(static_cast<unsigned char*>(g.ws) + words);
   gg.front = FrontArgs{g.x, g.R, g.r_out, g.pub, nullptr, g.M, g.K, g.rank, 0, 0, 1, 1, g.pub_mute ? kNeverRaised : g.pub_spin, g.pub_any_cost};
   gg.front.partials = gg.partials == nullptr ? nullptr : reinterpret_cast<float*>(static_cast<unsigned char*>(g.ws) + kGemmWordBytes);
+  if (exact) return launch_gemm_exact(gg, num_cus, ws_bytes, stream);
   return launch_gemm_group(gg, num_cus, ws_bytes, g.mem[0].y32 != 0, stream);
 }
 

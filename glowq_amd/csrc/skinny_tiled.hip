@@ -1,4 +1,4 @@
-// Matrix-core kernel for a handful of token rows (5..64, from 2 on the longest streams) on members that bring the tiled copy of their weights
+// Matrix-core kernel for a handful of token rows (5..32, from 2 on the longest streams) on members that bring the tiled copy of their weights
 // (tiled.hpp): the weights are streamed once, every 16-byte load of a wave is one contiguous kilobyte and lands in
 // the lanes' registers as the B operand of v_mfma_f32_32x32x16_f16 -- no pass through LDS, no per-lane scale and
 // zero-point gather (both ride in the stream).
@@ -38,8 +38,8 @@
 // weight stream to get there -- and read r with loads that pass those caches; one that does not see the word within its
 // bound computes the pieces of r it would have loaded, so every wave ends whatever becomes of the workgroups in front.
 // Few column tiles (o_proj, down_proj): K is also cut into gridDim.y slices, each workgroup leaves its fp32 tile in the
-// caller's workspace and skinny_tiled_reduce_kernel adds the slices in order.  More than 32 token rows: two row tiles
-// per wave, every code word feeds two matrix instructions.
+// caller's workspace and skinny_tiled_reduce_kernel adds the slices in order.  Calls of 33 to 64 rows run in this arithmetic on
+// gemm_tiled_kernel (gemm.hip).
 #include <atomic>
 #include <cstdlib>
 
@@ -133,22 +133,21 @@ __device__ unsigned long long g_tstamps[65536 * 32];
 #define GLOWQ_STAMP(i) do { } while (0)
 #endif
 
-// kRows: token rows a K group stages (8, 16, 32 or 64).  kWk: K groups per workgroup.  kPW: producer waves per K group.
+// kRows: token rows a K group stages (8, 16 or 32).  kWk: K groups per workgroup.  kPW: producer waves per K group.
 // The leading scalar arguments arrive in registers with the wave (kernel-argument preload): what a workgroup of the
 // first member needs to request its first weights and activations, without a round trip to the argument buffer.
-// Consumer waves a K group may have and the workgroup size that goes with it: 768 threads at most, 512 where a wave
-// holds two row tiles (their registers do not fit three waves on a SIMD).
-constexpr int tiled_max_cw(int rows, int wk, int pw) { return wk > 1 ? 4 : (rows > 32 ? 8 - pw : 12 - pw); }
-constexpr int tiled_max_threads(int rows, int wk, int pw) { return (tiled_max_cw(rows, wk, pw) + pw) * 64 * wk; }
+// Consumer waves a K group may have and the workgroup size that goes with it: 768 threads at most.
+constexpr int tiled_max_cw(int wk, int pw) { return wk > 1 ? 4 : 12 - pw; }
+constexpr int tiled_max_threads(int wk, int pw) { return (tiled_max_cw(wk, pw) + pw) * 64 * wk; }
 
 template <int kRows, int kWk, int kPW, bool kProj = false>
-__global__ __launch_bounds__(tiled_max_threads(kRows, kWk, kPW))
+__global__ __launch_bounds__(tiled_max_threads(kWk, kPW))
 void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K, const int slices,
                          const unsigned char* __restrict__ wt0, const int blk_end0, const int N0, const int cw, const TileArgs g) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
-  constexpr int kMT = kRows > 32 ? 2 : 1;        // 32-row tiles per consumer wave
+  static_assert(kRows <= 32, "one 32-row tile per consumer wave");
   constexpr int kPQ = (kRows + 2 * kPW - 1) / (2 * kPW);  // 16-byte pieces of a super-block of x per producer thread
-  constexpr bool kRagged = kPQ * 2 * kPW != kRows;       // three producer waves: the last pass covers part of the rows
+  static_assert(kPQ * 2 * kPW == kRows, "whole passes");
   constexpr int kSigBytes = kRows * 16;          // per 128-column half: a 16-byte fragment of sums per token row
   constexpr int kStage = kRows * kRowBytes + 2 * kSigBytes;
   constexpr int kLiveRegs = kRows >= 32 ? 16 : (kRows >= 16 ? 8 : 4);  // accumulator registers of rows that exist
@@ -266,7 +265,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       const h2 sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
 #pragma unroll
       for (int q = 0; q < kPQ; ++q) {
-        if (kRagged && 2 * kPW * q + prow >= kRows) break;  // (whole groups of sixteen lanes: the row reduction stays among live lanes)
         // the sixteen lanes pcol / 16 hold the 128 columns of one half of the token row: their sum, in fp32
         const h8 v = __builtin_bit_cast(h8, av[q]);
         float sum = __builtin_amdgcn_fdot2(h2{v[0], v[1]}, ones, 0.f, false);
@@ -410,11 +408,9 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   const bool has_l = wg_corr && gk == 0 && mem.lt != nullptr && live;
   const __amdgpu_buffer_rsrc_t rs_l = rsrc(has_l ? mem.lt + (size_t)rb * LBall * tiled::kLChunk : wt, has_l ? (size_t)LBall * tiled::kLChunk : 0);
 
-  f16v acc[kMT];
+  f16v acc;
 #pragma unroll
-  for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[tm][i] = 0.f;
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
   const uint32_t half0 = lh == 0 ? 0xFFFFFFFFu : 0u;  // the zero-point fragment lives in the first lane half
   const int arow = kRows >= 32 ? ln : (ln & (kRows - 1));
   const int arow_off = arow * kRowBytes + 128 * lh;
@@ -443,7 +439,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #endif
 #pragma unroll
     for (int gh = 0; gh < 2; ++gh) {
-      f16v pg[kMT];
+      f16v pg;
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const u32x4 raw = b.w[2 * gh + p];
@@ -452,15 +448,12 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         for (int i = 0; i < 4; ++i) {
           const uint32_t wd = raw[i], hi = wd >> 8;
           const h8 bf = __builtin_bit_cast(h8, u32x4{wd & 0x000F000Fu, wd & 0x00F000F0u, hi & 0x000F000Fu, hi & 0x00F000F0u});
-#pragma unroll
-          for (int tm = 0; tm < kMT; ++tm) {
-            const h8 af = *reinterpret_cast<const h8*>(st + arow_off + tm * 32 * kRowBytes + 256 * gh + 64 * p + 16 * i);
-            if (p == 0 && i == 0) {
-              const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-              pg[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, zero, 0, 0, 0);
-            } else {
-              pg[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, pg[tm], 0, 0, 0);
-            }
+          const h8 af = *reinterpret_cast<const h8*>(st + arow_off + 256 * gh + 64 * p + 16 * i);
+          if (p == 0 && i == 0) {
+            const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            pg = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, zero, 0, 0, 0);
+          } else {
+            pg = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, pg, 0, 0, 0);
           }
         }
       }
@@ -468,13 +461,10 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       const uint32_t sw = side[gh];
       const h8 bz = __builtin_bit_cast(h8, u32x4{__builtin_amdgcn_perm(sw, sw, 0x03020302u) & half0, 0u, 0u, 0u});
       const float sf = (float)__builtin_bit_cast(half_t, (uint16_t)(sw & 0xFFFFu)) * 0x1p24f;
+      const h8 az = *reinterpret_cast<const h8*>(st + sig_off + gh * kSigBytes);
+      pg = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz, pg, 0, 0, 0);
 #pragma unroll
-      for (int tm = 0; tm < kMT; ++tm) {
-        const h8 az = *reinterpret_cast<const h8*>(st + sig_off + tm * 32 * 16 + gh * kSigBytes);
-        pg[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz, pg[tm], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < kLiveRegs; ++i) acc[tm][i] = __builtin_fmaf(sf, pg[tm][i], acc[tm][i]);
-      }
+      for (int i = 0; i < kLiveRegs; ++i) acc[i] = __builtin_fmaf(sf, pg[i], acc[i]);
     }
     if constexpr (kRefill)
       b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sb_next * chunk_stride + tiled::kCodeBytes, kStreamAux));
@@ -521,11 +511,9 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   // stage 0 the first 256 columns of r.  Ranks above 256 take further passes, each with its loads in the open.  K groups
   // other than the first hold zeros in their sets.
   if (wg_corr) {
-    f16v acc2[kMT];
+    f16v acc2;
 #pragma unroll
-    for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc2[tm][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc2[i] = 0.f;
     for (int pass = 0; pass * kD < LBall; ++pass) {
       if (pass > 0) {
         __syncthreads();  // the fragment reads of the pass before are done
@@ -540,17 +528,13 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
       for (int q = 0; q < kD; ++q)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int tm = 0; tm < kMT; ++tm) {
-            const h8 af = *reinterpret_cast<const h8*>(ar + tm * 32 * kRowBytes + 128 * q + 16 * t);
-            acc2[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, __builtin_bit_cast(h8, bs[q].w[t]), acc2[tm], 0, 0, 0);
-          }
+        for (int t = 0; t < 4; ++t) {
+          const h8 af = *reinterpret_cast<const h8*>(ar + 128 * q + 16 * t);
+          acc2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, __builtin_bit_cast(h8, bs[q].w[t]), acc2, 0, 0, 0);
+        }
     }
 #pragma unroll
-    for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[tm][i] = __builtin_fmaf(g.alpha, acc2[tm][i], acc[tm][i]);
+    for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(g.alpha, acc2[i], acc[i]);
   }
 
   GLOWQ_STAMP(5);
@@ -560,21 +544,17 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     float* red = reinterpret_cast<float*>(smem_all);
     if (gk > 0) {
 #pragma unroll
-      for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) red[((((gk - 1) * cw + wave) * kMT + tm) * 16 + i) * 64 + lane] = acc[tm][i];
+      for (int i = 0; i < 16; ++i) red[(((gk - 1) * cw + wave) * 16 + i) * 64 + lane] = acc[i];
     }
     __syncthreads();
     if (gk > 0) return;
 #pragma unroll
     for (int o = 1; o < kWk; ++o)
 #pragma unroll
-      for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[tm][i] += red[((((o - 1) * cw + wave) * kMT + tm) * 16 + i) * 64 + lane];
+      for (int i = 0; i < 16; ++i) acc[i] += red[(((o - 1) * cw + wave) * 16 + i) * 64 + lane];
   }
 
-  // ---- epilogue: accumulator register i of row tile tm is token row 32 tm + 8 (i / 4) + 4 lh + i % 4, column ln of
+  // ---- epilogue: accumulator register i is token row 8 (i / 4) + 4 lh + i % 4, column ln of
   // the wave's row block
   GLOWQ_STAMP(6);
   if (!live) return;
@@ -582,23 +562,19 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   if (slices > 1) {
     float* prow = g.partials + ((size_t)blockIdx.y * M) * g.ldp + mem.col0 + n;
 #pragma unroll
-    for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = 32 * tm + 8 * (i >> 2) + 4 * lh + (i & 3);
-        if (m < M) prow[(size_t)m * g.ldp] = acc[tm][i];
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int m = 8 * (i >> 2) + 4 * lh + (i & 3);
+      if (m < M) prow[(size_t)m * g.ldp] = acc[i];
+    }
     return;
   }
   if (n >= mem.N) return;
   const float bias = mem.bias ? (float)mem.bias[n] : 0.f;
 #pragma unroll
-  for (int tm = 0; tm < kMT; ++tm)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = 32 * tm + 8 * (i >> 2) + 4 * lh + (i & 3);
-      if (m < M) mem.y[(size_t)m * mem.ldy + n] = (half_t)(acc[tm][i] + bias);
-    }
+  for (int i = 0; i < 16; ++i) {
+    const int m = 8 * (i >> 2) + 4 * lh + (i & 3);
+    if (m < M) mem.y[(size_t)m * mem.ldy + n] = (half_t)(acc[i] + bias);
+  }
 }
 
 // y = fp16(sum over the K slices, in slice order, + bias).  One thread per (token row, four columns of the padded row).
@@ -749,25 +725,21 @@ static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes) {
   // a few tiles more than compute units would run as two rounds, the second nearly empty: wider tiles (one K group)
   // where they bring the count down to one round
   if (tiled_tiles(g, 4) > num_cus) {
-    for (int cw = 5; cw <= (g.M <= 32 ? 8 : 6); ++cw)
+    for (int cw = 5; cw <= 8; ++cw)
       if (tiled_tiles(g, cw) <= num_cus) {
         p.cw = cw;
         break;
       }
   }
-  if (env_cw >= 1 && env_cw <= (g.M <= 32 ? 8 : 6)) p.cw = env_cw;
+  if (env_cw >= 1 && env_cw <= 8) p.cw = env_cw;
   // two K groups: up to 16 token rows on tiles that fill the chip by themselves (more rows want four producer waves, and
   // a K range cut into slices is short enough already).  8B shapes, launch with the projection, us, two groups / one:
   // gate|up 8 rows 22.4 / 24.1, 32 rows 26.4 / 26.3; down_proj 32 rows 27.1 / 25.5
   int wk = (SB >= 8 && p.cw <= 4 && g.M <= 16 && tiled_tiles(g, p.cw) * 2 > num_cus) ? 2 : 1;
-  if (env_wk == 1 || (env_wk == 2 && p.cw <= 4 && g.M <= 32)) wk = env_wk;
+  if (env_wk == 1 || (env_wk == 2 && p.cw <= 4)) wk = env_wk;
   p.pw = g.M <= 8 ? 1 : (g.M <= 16 || wk == 2 ? 2 : 4);
-  // two row tiles per wave: 512 threads, their registers allow no more -- four producer waves beside four consumers, three
-  // beside five, two beside six
-  if (g.M > 32) wk = 1, p.pw = p.cw > 5 ? 2 : (p.cw > 4 ? 3 : 4);
   if (env_pw == 2 && g.M > 8) p.pw = 2;
-  if (env_pw == 3 && g.M > 32 && p.cw <= 5) p.pw = 3;
-  if (env_pw == 4 && g.M > 16 && wk == 1 && (g.M <= 32 || p.cw <= 4)) p.pw = 4;
+  if (env_pw == 4 && g.M > 16 && wk == 1) p.pw = 4;
   p.wk = wk;
   const int tiles = tiled_tiles(g, p.cw);
   long ldp = 0;
@@ -789,13 +761,12 @@ size_t tiled_split_workspace_bytes(int M, int num_cus) { return M > 4 ? (size_t)
 template <int kRows, int kWk, int kPW, bool kProj = false>
 static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipStream_t stream) {
   auto kern = skinny_tiled_kernel<kRows, kWk, kPW, kProj>;
-  constexpr int kMT = kRows > 32 ? 2 : 1;
   size_t lds = (size_t)kWk * 2 * (kRows * kRowBytes + 2 * kRows * 16);
-  const size_t red = (size_t)(kWk - 1) * a.cw * kMT * 16 * 64 * sizeof(float);
+  const size_t red = (size_t)(kWk - 1) * a.cw * 16 * 64 * sizeof(float);
   if (lds < red) lds = red;
   static LdsLimit lds_limit;
   if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
-  if (a.cw < 1 || a.cw > tiled_max_cw(kRows, kWk, kPW)) return hipErrorInvalidValue;
+  if (a.cw < 1 || a.cw > tiled_max_cw(kWk, kPW)) return hipErrorInvalidValue;
   const int threads = (a.cw + kPW) * 64 * kWk;
   int grid_x = a.tiles;
   if constexpr (kProj) {
@@ -884,7 +855,7 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   }
   a.tiles = tiles;
   a.ldp = col;
-  const int key = (g.M <= 8 ? 8 : g.M <= 16 ? 16 : g.M <= 32 ? 32 : 64) * 100 + plan.wk * 10 + plan.pw;
+  const int key = (g.M <= 8 ? 8 : g.M <= 16 ? 16 : 32) * 100 + plan.wk * 10 + plan.pw;
   if (proj) {
     if (a.slices != 1) return hipErrorNotReady;
     switch (key) {
@@ -903,9 +874,6 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
     case 3222: return launch_tiled_t<32, 2, 2>(a, g.x, num_cus, stream);
     case 3212: return launch_tiled_t<32, 1, 2>(a, g.x, num_cus, stream);
     case 3214: return launch_tiled_t<32, 1, 4>(a, g.x, num_cus, stream);
-    case 6412: return launch_tiled_t<64, 1, 2>(a, g.x, num_cus, stream);
-    case 6413: return launch_tiled_t<64, 1, 3>(a, g.x, num_cus, stream);
-    case 6414: return launch_tiled_t<64, 1, 4>(a, g.x, num_cus, stream);
   }
   return hipErrorInvalidValue;
 }

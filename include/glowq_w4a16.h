@@ -182,7 +182,7 @@ int glowq_w4a16_group_forward_fused(const void* x, const void* R, void* r_out, c
  * graph is a launch like any other).  One launch instead of two, the same bits in r_out and in the outputs as the
  * projection launch in front gives; "proj_in_launch" of glowq_set_tuning switches it off.  As everywhere, calls that
  * share a workspace must not overlap.
- * The GEMM on the tiled weights does the same from 65 token rows on where that is predicted to pay: tiles of r in front of the
+ * The GEMM on the tiled weights (from 65 token rows, and 33 to 64 in its unrounded form) does the same where that is predicted to pay: tiles of r in front of the
  * grid, a word each; its readers want r behind their weights.  The first 2 101 248 bytes of the workspace hold the words
  * and fp32 sums of r, the partial tiles of a split of K lie behind them; with less the projection launch stays.  r and outputs agree
  * with the two-launch form to the rounding of fp32 sums; glowq_last_launch names the grid of the output tiles alone.

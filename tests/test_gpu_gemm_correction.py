@@ -174,3 +174,40 @@ def test_calls_without_room_for_the_words_keep_the_projection_launch(ext, wherev
     finally:
         ext.WORKSPACE_BYTES = saved
         ext._workspaces.clear()
+
+
+# ---- up to 64 rows: the unrounded form ---------------------------------------------------------------------------------------
+@pytest.mark.parametrize("in_front", [False, True])
+@pytest.mark.parametrize("M,K,Ns,rank,gs", [(33, 256, [32], 8, 128), (64, 512, [130, 40], 40, 256), (57, 5120, [5120, 1024, 1024], 256, 128), (40, 17408, [5120], 264, 128),
+                                            (64, 1280, [34816], 64, 512), (17, 2048, [16600, 9000], 72, 128), (32, 2304, [30000], 128, 128), (49, 3328, [300], 136, 128)])
+def test_unrounded_form(ext, M, K, Ns, rank, gs, in_front):
+    """Weights that are never rounded, to the accuracy of the outputs' rounding: with activations in the hundreds of which rounded weights
+    would be off by more."""
+    print(f"case M={M} K={K} Ns={Ns} rank={rank} gs={gs} {in_front}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = (torch.randn(M, K, device="cuda", generator=g) * 64).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half()
+    members, exact = [], []
+    for N in Ns:
+        codes = torch.randint(0, 16, (N, K), device="cuda", generator=g)
+        zeros = torch.randint(0, 16, (N, (K + gs - 1) // gs), device="cuda", generator=g)
+        scales = (torch.rand(N, zeros.size(1), device="cuda", generator=g) * 0.01 + 0.001).half()
+        qw = sum(codes.view(N, K // 8, 8)[:, :, i] << (4 * i) for i in range(8))
+        zp = torch.nn.functional.pad(zeros, (0, -zeros.size(1) % 8))
+        qz = sum(zp.view(N, -1, 8)[:, :, i] << (4 * i) for i in range(8))
+        members.append({"qweight": qw.to(torch.int32), "qzeros": qz.to(torch.int32), "scales": scales, "bias": None,
+                        "L": (torch.randn(N, rank, device="cuda", generator=g) * 0.05).half()})
+        exact.append((codes - zeros.repeat_interleave(gs, 1)[:, :K]).double() * scales.repeat_interleave(gs, 1)[:, :K].double())
+    pg = PreparedGroup(ext, members, K, gs, 1.0, R=R)
+    with tuning(ext, tiled_shape_rule=0, proj_any_cost=1, proj_in_launch=1 if in_front else 0):
+        for _ in range(2):
+            y = pg.run(x)
+            assert ext.last_launch()["kernel"].startswith("gemm_tiled_kernel") and "exact" in ext.last_launch()["kernel"]
+            r = pg.last_r
+            want_r = x.double() @ R.double().t()
+            assert ((r.double() - want_r).abs() <= 2.0 ** -11 * want_r.abs() + 6e-3).all()
+            for got, w, m in zip(y, exact, members):
+                want = x.double() @ w.t() + r.double() @ m["L"].double().t()
+                # outputs in the hundreds: their own rounding, and fp32 sums of terms up to 64 x 4 x 0.15
+                assert ((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2e-2).all()
+                assert (got.double() - want).norm() <= 3.2e-4 * want.norm()
