@@ -416,16 +416,17 @@ int pick_route_rounded(const GroupDev& g, int force) {
 
 // Runs one group through the chosen route.  Routes with a row capacity smaller than M walk the
 // token rows in chunks (weights are re-read once per chunk).
-// Calls of the route on the tiled copy that run on the GEMM in its unrounded form: all of 33 to 64 rows, and from 17 rows on groups whose
-// 128-column tiles come to between half and all of the compute units (K of 2048 columns and more).  us with the projection, 24 and 32
-// rows, GEMM / the kernel of skinny_tiled.hip: 8B gate|up (224 tiles) 22.6, 22.9 / 26.1, 26.5; 27648 x 5120 (216) 24.4, 23.9 / 30.3, 30.3;
+// Calls of the route on the tiled copy that run on the GEMM in its unrounded form: all of 33 to 64 rows, and from 17 rows on groups with
+// an r to compute whose 128-column tiles come to between half and all of the compute units (K of 2048 columns and more; without r 2 x 14336 x
+// 4096 at 32 rows 21.9 / 18.5).  us with the projection, 24 and 32 rows, GEMM / the kernel of skinny_tiled.hip: 8B gate|up (224 tiles)
+// 22.6, 22.9 / 26.1, 26.5; 27648 x 5120 (216) 24.4, 23.9 / 30.3, 30.3;
 // 14B gate|up (272: a second round) 40.5, 42.6 / 36.2, 37.4; 14B down_proj (40 tiles in slices of K) 33.0, 34.5 / 31.6, 32.5; 12 and 16 rows 8B gate|up
 // 22.5, 22.8 / 20.5, 20.8.
 bool tiled_route_on_gemm(const GroupDev& g) {
   if (g.M > 32) return true;
   long tiles = 0;
   for (int i = 0; i < g.n_members; ++i) tiles += (g.mem[i].N + 127) / 128;
-  return g.M > 16 && g.K >= 2048 && tiles * 2 > num_cus() && tiles <= num_cus();
+  return g.M > 16 && g.R != nullptr && g.K >= 2048 && tiles * 2 > num_cus() && tiles <= num_cus();
 }
 
 int run_group(GroupDev g, int route, hipStream_t stream) {

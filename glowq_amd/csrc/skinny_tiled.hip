@@ -12,6 +12,12 @@
 // thirteen a dequantisation to fp16 takes: the vector ALUs, not memory, bound the dequantising form.
 // (The division by 16 is exact for |x| >= 2^-10; below, x / 16 is a subnormal and x is rounded to a multiple of 2^-20,
 // an absolute error of 2^-21 and less.  The row sums are carried as two halves, good to 2^-22 of their value.)
+// Up to 16 token rows the products are tiles of 16 by 16 (v_mfma_f32_16x16x32_f16: half the matrix time and half the LDS reads of 32 rows
+// that are half empty): v_permlane16_swap trades rows of sixteen lanes between two neighbouring words, after which each holds sixteen
+// columns over the k values of both, and one more product per fragment, against ones, leaves the row sums in fp32 (no sums in the
+// producers, whose vector instructions a step had to wait for).  All eight fragments of a step are asked for at its head.  Launch
+// without a correction, 16 rows, us: 2 x 14336 x 4096 18.4 -> 15.3 (4.0 TB/s), 2 x 17408 x 5120 26.4 -> 23.2, 17408 x 5120 19.7 -> 15.4,
+// 5120 x 17408 20.0 -> 16.3.
 //
 // A workgroup owns 32 cw output columns of one member (a row block of 32 per consumer wave) and all token rows.  Its
 // waves come in K groups that walk contiguous parts of the K range in step and meet in LDS at the end; a K group is
@@ -20,9 +26,10 @@
 //   * Consumers keep kD sets of weight registers in rotation: the set of super-block v is refilled with super-block
 //     v + kD as soon as its words have been masked, so up to kD - 1 super-blocks of a wave are in flight while it
 //     computes.  They wait for nothing but their weights.
-//   * Producers load the activations of the next super-block (token rows x 512 bytes) in memory order (the tiled copy
+//   * Producers load the activations of the super-blocks ahead (token rows x 512 bytes; four sets of registers in rotation -- with one,
+//     every step took an L2 round trip under load: 3 to 17 % of the launches) in memory order (the tiled copy
 //     holds the nibbles of a word in the order the masks deliver them: no permutation), divide the pairs at positions
-//     2, 3 and 6, 7 of every octet by 16, sum every row's two
+//     2, 3 and 6, 7 of every octet by 16, from 17 rows on sum every row's two
 //     128-column halves in fp32, and leave all of it in the LDS stage the consumers do not read (528-byte rows:
 //     conflict-free 16-byte reads).  One barrier per super-block.  A wave's loads return in order: a consumer that
 //     fetched activations as well would have to drain its weight requests with every step.
@@ -40,6 +47,7 @@
 // Few column tiles (o_proj, down_proj): K is also cut into gridDim.y slices, each workgroup leaves its fp32 tile in the
 // caller's workspace and skinny_tiled_reduce_kernel adds the slices in order.  Calls of 33 to 64 rows run in this arithmetic on
 // gemm_tiled_kernel (gemm.hip).
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 
@@ -148,7 +156,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   static_assert(kRows <= 32, "one 32-row tile per consumer wave");
   constexpr int kPQ = (kRows + 2 * kPW - 1) / (2 * kPW);  // 16-byte pieces of a super-block of x per producer thread
   static_assert(kPQ * 2 * kPW == kRows, "whole passes");
-  constexpr int kSigBytes = kRows * 16;          // per 128-column half: a 16-byte fragment of sums per token row
+  constexpr bool kNarrow = kRows <= 16;          // tiles of 16 token rows by 16 columns
+  constexpr int kSigBytes = kNarrow ? 0 : kRows * 16;  // per 128-column half: a 16-byte fragment of sums per token row
   constexpr int kStage = kRows * kRowBytes + 2 * kSigBytes;
   constexpr int kLiveRegs = kRows >= 32 ? 16 : (kRows >= 16 ? 8 : 4);  // accumulator registers of rows that exist
   const int group_threads = (cw + kPW) * 64;  // the consumer waves, then the producer waves
@@ -248,8 +257,11 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     const int prow = pt >> 5, pcol = pt & 31;  // piece q of this thread: token row 2 kPW q + prow, 16-byte piece pcol
     const __amdgpu_buffer_rsrc_t rs_x = rsrc(x, (size_t)M * K * 2);
     const __amdgpu_buffer_rsrc_t rs_r = rsrc(g.r != nullptr ? (const void*)g.r : (const void*)x, g.r != nullptr ? (size_t)M * g.rank * 2 : 0);
-    u32x4 av[kPQ];
-    auto load_a = [&](bool is_r, int idx) __attribute__((always_inline)) {
+    // kXD sets of activation registers in rotation: a piece has kXD - 1 steps to arrive
+    constexpr int kXD = kNarrow || kPQ <= 4 ? 4 : 2;
+    static_assert(kD % kXD == 0, "the sets rotate with the steps of a round");
+    u32x4 avs[kXD][kPQ];
+    auto load_a = [&](u32x4 (&av)[kPQ], bool is_r, int idx) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t rs = is_r ? rs_r : rs_x;
       const uint32_t ld = (uint32_t)(is_r ? g.rank : K);
 #pragma unroll
@@ -258,13 +270,20 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         av[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((row * ld + (uint32_t)pcol * 8u) * 2u), idx * 512, 0);
       }
     };
-    auto store_a = [&](int stage) __attribute__((always_inline)) {
+    auto store_a = [&](const u32x4 (&av)[kPQ], int stage) __attribute__((always_inline)) {
       unsigned char* dst = smem + stage * kStage + prow * kRowBytes + pcol * 16;
       unsigned char* sig = smem + stage * kStage + kRows * kRowBytes + (pcol >> 4) * kSigBytes + prow * 16;
       const h2 ones = {(half_t)1.f, (half_t)1.f};
       const h2 sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
 #pragma unroll
       for (int q = 0; q < kPQ; ++q) {
+        if constexpr (kNarrow) {
+          u32x4 o = av[q];
+          o.y = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.y) * sixteenth);
+          o.w = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.w) * sixteenth);
+          *reinterpret_cast<u32x4*>(dst + 2 * kPW * q * kRowBytes) = o;
+          continue;
+        }
         // the sixteen lanes pcol / 16 hold the 128 columns of one half of the token row: their sum, in fp32
         const h8 v = __builtin_bit_cast(h8, av[q]);
         float sum = __builtin_amdgcn_fdot2(h2{v[0], v[1]}, ones, 0.f, false);
@@ -290,7 +309,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     // stores passed); without the word within the bound, the thread computes the eight entries of each of its pieces
     // `polls`: how often the wave looks before it gives up (one look where it may come back later).  True: the loads
     // are out.
-    auto ask_r_handed = [&](unsigned polls) __attribute__((always_inline)) -> bool {
+    auto ask_r_handed = [&](u32x4 (&av)[kPQ], unsigned polls) __attribute__((always_inline)) -> bool {
       int seen = 0;
       if (lane == 0) {
         for (unsigned spins = 0; !seen && spins < polls && g.spin != 0xFFFFFFFFu; ++spins) {
@@ -308,8 +327,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       }
       return seen != 0;
     };
-    auto load_r_handed = [&]() __attribute__((always_inline)) {
-      if (ask_r_handed(g.spin == 0xFFFFFFFFu ? 0u : g.spin + 1u)) return;
+    auto load_r_handed = [&](u32x4 (&av)[kPQ]) __attribute__((always_inline)) {
+      if (ask_r_handed(av, g.spin == 0xFFFFFFFFu ? 0u : g.spin + 1u)) return;
       for (int q = 0; q < kPQ; ++q) {
         const int row = min(2 * kPW * q + prow, M - 1);
         h8 own;
@@ -326,35 +345,50 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         av[q] = __builtin_bit_cast(u32x4, own);
       }
     };
-    load_a(false, min(sb0, SB - 1));
-    store_a(0);
-    load_a(false, min(sb0 + 1, SB - 1));
+    // what follows the last super-block through the stages (step `steps`) is r
+    const auto fetch = [&](u32x4 (&av)[kPQ], int j) __attribute__((always_inline)) {
+      const bool is_r = j >= steps;
+      if constexpr (kProj) {
+        if (!is_r) load_a(av, false, min(sb0 + j, SB - 1));
+      } else {
+        load_a(av, is_r, is_r ? 0 : min(sb0 + j, SB - 1));  // (past r: once more, never stored)
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < kXD; ++j) fetch(avs[j], j);
+    store_a(avs[0], 0);
+    fetch(avs[0], kXD);
     __syncthreads();
     bool have_r = false;
-    for (int i = 0; i < steps; ++i) {
+    const auto produce = [&](int i, auto set_const) __attribute__((always_inline)) {  // step i: set (i + 1) % kXD
+      constexpr int set = decltype(set_const)::value;
 #if !(GLOWQ_TDBG & 8)
       if constexpr (kProj) {
         // r that was not there a step earlier is waited for during the last super-block, for the stage that super-block
         // does not read
-        if (i + 1 == steps && wg_corr && gk == 0 && !have_r) load_r_handed();
+        if (set == 0 && i + 1 == steps && wg_corr && gk == 0 && !have_r) load_r_handed(avs[0]);
       }
-      store_a((i + 1) & 1);                                   // step i + 1's activations (or r after the last step)
-      const bool next_r = i + 2 >= steps;
+      store_a(avs[set], (i + 1) & 1);  // step i + 1's activations (or r after the last step)
+      fetch(avs[set], i + 1 + kXD);
       if constexpr (kProj) {
-        if (!next_r) load_a(false, min(sb0 + i + 2, SB - 1));
-        // where the other form asks for r, one look: as a rule the workgroups in front are long done
-        else if (i + 2 == steps && wg_corr && gk == 0) have_r = ask_r_handed(1u);
-      } else {
-        load_a(next_r, next_r ? 0 : min(sb0 + i + 2, SB - 1));  // (past the last step: r once more, never stored)
+        // one look a step before: as a rule the workgroups in front are long done
+        if (i + 2 == steps && wg_corr && gk == 0) have_r = ask_r_handed(avs[0], 1u);
       }
 #endif
       __syncthreads();
+    };
+    using std::integral_constant;
+    for (int i = 0; i < steps; i += kD) {
+      produce(i, integral_constant<int, 1 % kXD>{});
+      produce(i + 1, integral_constant<int, 2 % kXD>{});
+      produce(i + 2, integral_constant<int, 3 % kXD>{});
+      produce(i + 3, integral_constant<int, 4 % kXD>{});
     }
     if (wg_corr) {
       for (int pass = 1; pass * kD < LBall; ++pass) {
         __syncthreads();
-        load_a(true, pass);
-        store_a(0);
+        load_a(avs[0], true, pass);
+        store_a(avs[0], 0);
         __syncthreads();
       }
     }
@@ -408,6 +442,17 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   const bool has_l = wg_corr && gk == 0 && mem.lt != nullptr && live;
   const __amdgpu_buffer_rsrc_t rs_l = rsrc(has_l ? mem.lt + (size_t)rb * LBall * tiled::kLChunk : wt, has_l ? (size_t)LBall * tiled::kLChunk : 0);
 
+  // Up to 16 token rows: tiles of 16 rows by 16 columns, two to a row block (acc[c][i]: row 4 (lane / 16) + i, column 16 c + lane % 16).
+  // Rows of sixteen lanes of two neighbouring words change places, and each of the two then holds the codes of sixteen columns over
+  // the 32 k values of both.
+  f4 nacc[2] = {};
+  const auto spread = [](uint32_t a, uint32_t b, uint32_t& lo, uint32_t& hi) __attribute__((always_inline)) {
+    const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    lo = v[0];
+    hi = v[1];
+  };
+  const int nrow_off = (lane & (kRows - 1) & 15) * kRowBytes;
+  const int nq = lane >> 4;  // k octet of the lane: word nq % 2 of a pair, lane half nq / 2
   f16v acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
@@ -437,6 +482,53 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       return;
     }
 #endif
+    if constexpr (kNarrow) {
+      uint32_t sw[2][2];
+      spread(side.x, side.x, sw[0][0], sw[0][1]);
+      spread(side.y, side.y, sw[1][0], sw[1][1]);
+      // the pairs a mask leaves at code * 2^-20 are staged divided by 16
+      const h2 one = {(half_t)1.f, (half_t)1.f}, sixteen = {(half_t)16.f, (half_t)16.f};
+      const uint32_t o1 = __builtin_bit_cast(uint32_t, one), o16 = __builtin_bit_cast(uint32_t, sixteen);
+      const h8 ones = __builtin_bit_cast(h8, u32x4{o1, o16, o1, o16});
+      // all fragments of the step are asked for at once: one LDS round trip for it instead of eight
+      const unsigned char* xs = st + nrow_off + 128 * (nq >> 1) + 16 * (nq & 1);
+      h8 af[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) af[t] = *reinterpret_cast<const h8*>(xs + 256 * (t >> 2) + 32 * (t & 3));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int gh = 0; gh < 2; ++gh) {
+        f4 pg[2] = {}, sx = {};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const u32x4 raw = b.w[2 * gh + p];
+#pragma unroll
+          for (int i = 0; i < 4; i += 2) {
+            const h8 a = af[4 * gh + 2 * p + (i >> 1)];
+            uint32_t w[2];
+            spread(raw[i], raw[i + 1], w[0], w[1]);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const uint32_t hi = w[c] >> 8;
+              const h8 bf = __builtin_bit_cast(h8, u32x4{w[c] & 0x000F000Fu, w[c] & 0x00F000F0u, hi & 0x000F000Fu, hi & 0x00F000F0u});
+              pg[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bf, pg[c], 0, 0, 0);
+            }
+            sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ones, sx, 0, 0, 0);
+          }
+          if constexpr (kRefill) b.w[2 * gh + p] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, b_off + (2 * gh + p) * 1024, sb_next * chunk_stride, kStreamAux);
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float sf = (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] & 0xFFFFu)) * 0x1p24f;
+          const float nz = (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] >> 16)) * 0x1p-8f;  // -zero * 2^-24
+#pragma unroll
+          for (int i = 0; i < 4; ++i) nacc[c][i] = __builtin_fmaf(sf, __builtin_fmaf(nz, sx[i], pg[c][i]), nacc[c][i]);
+        }
+      }
+      if constexpr (kRefill)
+        b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sb_next * chunk_stride + tiled::kCodeBytes, kStreamAux));
+      return;
+    }
 #pragma unroll
     for (int gh = 0; gh < 2; ++gh) {
       f16v pg;
@@ -512,6 +604,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   // other than the first hold zeros in their sets.
   if (wg_corr) {
     f16v acc2;
+    f4 nacc2[2] = {};
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc2[i] = 0.f;
     for (int pass = 0; pass * kD < LBall; ++pass) {
@@ -524,6 +617,26 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
             bs[q].w[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, b_off + t * 1024, (pass * kD + q) * tiled::kLChunk, 0);
         __syncthreads();
       }
+      if constexpr (kNarrow) {
+        const unsigned char* ar = smem + nrow_off + 64 * (nq >> 1) + 16 * (nq & 1);
+#pragma unroll
+        for (int q = 0; q < kD; ++q)
+#pragma unroll
+          for (int t = 0; t < 4; t += 2) {
+            const h8 af = *reinterpret_cast<const h8*>(ar + 128 * q + 16 * t);
+            u32x4 bw[2];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              uint32_t lo, hi;
+              spread(bs[q].w[t][e], bs[q].w[t + 1][e], lo, hi);
+              bw[0][e] = lo;
+              bw[1][e] = hi;
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) nacc2[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, __builtin_bit_cast(h8, bw[c]), nacc2[c], 0, 0, 0);
+          }
+        continue;
+      }
       const unsigned char* ar = smem + arow * kRowBytes + 64 * lh;
 #pragma unroll
       for (int q = 0; q < kD; ++q)
@@ -535,7 +648,13 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(g.alpha, acc2[i], acc[i]);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) nacc[c] += g.alpha * nacc2[c];
   }
+  constexpr int kAccs = kNarrow ? 8 : 16;
+  float out[kAccs];
+#pragma unroll
+  for (int i = 0; i < kAccs; ++i) out[i] = kNarrow ? nacc[(i >> 2) & 1][i & 3] : acc[i];
 
   GLOWQ_STAMP(5);
   // ---- the K groups' accumulators meet in LDS: groups 1.. leave theirs, group 0 adds them in order ---------------
@@ -544,36 +663,38 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     float* red = reinterpret_cast<float*>(smem_all);
     if (gk > 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) red[(((gk - 1) * cw + wave) * 16 + i) * 64 + lane] = acc[i];
+      for (int i = 0; i < kAccs; ++i) red[(((gk - 1) * cw + wave) * kAccs + i) * 64 + lane] = out[i];
     }
     __syncthreads();
     if (gk > 0) return;
 #pragma unroll
     for (int o = 1; o < kWk; ++o)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] += red[(((o - 1) * cw + wave) * 16 + i) * 64 + lane];
+      for (int i = 0; i < kAccs; ++i) out[i] += red[(((o - 1) * cw + wave) * kAccs + i) * 64 + lane];
   }
 
-  // ---- epilogue: accumulator register i is token row 8 (i / 4) + 4 lh + i % 4, column ln of
-  // the wave's row block
+  // ---- epilogue: entry i of a lane is token row 8 (i / 4) + 4 lh + i % 4, column ln of the wave's row block; of the narrow tiles row
+  // 4 nq + i % 4, column 16 (i / 4) + lane % 16
   GLOWQ_STAMP(6);
   if (!live) return;
-  const int n = rb * 32 + ln;
+  const auto row_of = [&](int i) { return kNarrow ? 4 * nq + (i & 3) : 8 * (i >> 2) + 4 * lh + (i & 3); };
+  const auto col_of = [&](int i) { return rb * 32 + (kNarrow ? 16 * (i >> 2) + (lane & 15) : ln); };
   if (slices > 1) {
-    float* prow = g.partials + ((size_t)blockIdx.y * M) * g.ldp + mem.col0 + n;
+    float* prow = g.partials + ((size_t)blockIdx.y * M) * g.ldp + mem.col0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = 8 * (i >> 2) + 4 * lh + (i & 3);
-      if (m < M) prow[(size_t)m * g.ldp] = acc[i];
-    }
+    for (int i = 0; i < kAccs; ++i)
+      if (row_of(i) < M) prow[(size_t)row_of(i) * g.ldp + col_of(i)] = out[i];
     return;
   }
-  if (n >= mem.N) return;
-  const float bias = mem.bias ? (float)mem.bias[n] : 0.f;
+  constexpr int kPer = kNarrow ? 4 : 16;  // entries of a column
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int m = 8 * (i >> 2) + 4 * lh + (i & 3);
-    if (m < M) mem.y[(size_t)m * mem.ldy + n] = (half_t)(acc[i] + bias);
+  for (int i0 = 0; i0 < kAccs; i0 += kPer) {
+    const int n = col_of(i0);
+    if (n >= mem.N) continue;
+    const float bias = mem.bias ? (float)mem.bias[n] : 0.f;
+#pragma unroll
+    for (int i = i0; i < i0 + kPer; ++i)
+      if (row_of(i) < M) mem.y[(size_t)row_of(i) * mem.ldy + n] = (half_t)(out[i] + bias);
   }
 }
 
@@ -703,27 +824,78 @@ bool skinny_tiled_supported(const GroupDev& g) {
 }
 
 // How the launch cuts K and staffs a K group: `wk` K groups inside a workgroup (their sums meet in LDS), `slices`
-// workgroups per tile (their sums meet in the workspace), `pw` producer waves per K group.  A SIMD wants two waves and
-// more (a lone wave issues most vector instructions at half rate), so two K groups wherever K has the depth; slices
-// where the tiles alone leave most of the chip empty.  Workgroups stay at 768 threads and below (a 1024-thread
-// workgroup gets 128 registers per lane and the chip runs such workgroups in two rounds).
+// workgroups per tile (their sums meet in the workspace), `pw` producer waves per K group, `cw` consumer waves (a tile is 32 cw columns).
+// Workgroups stay at 768 threads and below (a 1024-thread workgroup gets 128 registers per lane and the chip runs such workgroups in
+// two rounds).
 struct TiledPlan {
   int wk, slices, pw, cw;
+  bool front;  // the launch computes r itself
 };
 static int tiled_tiles(const GroupDev& g, int cw) {
   int t = 0;
   for (int i = 0; i < g.n_members; ++i) t += ((g.mem[i].N + 31) / 32 + cw - 1) / cw;
   return t;
 }
-static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes) {
-  static const int env_slices = getenv("GLOWQ_TILED_SLICES") ? atoi(getenv("GLOWQ_TILED_SLICES")) : 0;
-  static const int env_wk = getenv("GLOWQ_TILED_WK") ? atoi(getenv("GLOWQ_TILED_WK")) : 0;
-  static const int env_pw = getenv("GLOWQ_TILED_PW") ? atoi(getenv("GLOWQ_TILED_PW")) : 0;
-  static const int env_cw = getenv("GLOWQ_TILED_CW") ? atoi(getenv("GLOWQ_TILED_CW")) : 0;
+static int proj_blocks(int M, int rank) { return ((rank + 3) / 4) * ((M + 3) / 4); }  // of four token rows by four rows of R
+// Up to 16 rows: the cheapest cut by what the launches were seen to take (us): 4.2 and the longer, a fifth of the shorter, of the steps of a
+// K group (whole rotations, 0.34 each and 0.04 per consumer wave; of two K groups 0.49 or 0.72; a compute unit draws a super-block of a row
+// block in 0.11) and the bytes of the group at 4.9 TB/s; 3.3 for slices and the launch that adds them.  r ahead of the launch is 2.3 and its
+// products, inside it 1.0 where the workgroups in front, on the compute units the tiles leave free, are done in time: 4.0 and 0.53 per
+// thousand columns of K for each of the blocks a team of four waves computes (q|k|v of a 14B layer at twelve rows, six blocks each on 32
+// compute units, 22.5 against 14.3 on wider tiles).  Tiles on a quarter of the chip and less are cut in K rather than given a front.
+// Predicted / measured at 16 rows without a correction: 5120 x 5120 10.6 / 9.6, 17408 x 5120 15.5 / 15.4, 2 x 17408 x 5120 24.7 / 23.2,
+// 5120 x 17408 18.2 / 16.7, 4096 x 14336 14.6 / 14.0.
+// (One K group at a wave per SIMD leaves vector and matrix instructions to alternate; two of them pay where the tiles are a row block or
+// two wide: 4096 x 4096 7.9 against 10.2, but 2 x 14336 x 4096 at four 16.9 against 15.5.)
+static TiledPlan narrow_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused) {
   const int SB = g.K >> 8;
-  TiledPlan p{1, 1, 1, 4};
-  // a few tiles more than compute units would run as two rounds, the second nearly empty: wider tiles (one K group)
-  // where they bring the count down to one round
+  const bool corrected = g.r != nullptr || g.R != nullptr;
+  double rows = 0;
+  for (int i = 0; i < g.n_members; ++i) rows += (g.mem[i].N + 31) / 32 * 32;
+  const double stream_us = rows * (g.K * 0.53125 + (corrected ? 2. * g.rank : 0.)) / 4.9e6;
+  TiledPlan best{1, 1, 1, 1, false};
+  double best_us = 1e30;
+  bool one_round = false;
+  for (int cw = 1; cw <= 8; ++cw) {
+    const int tiles = tiled_tiles(g, cw);
+    if (cw < 8 && tiles > num_cus) continue;
+    if (one_round && SB < 8) break;  // (a launch this short: nothing to gain from wider tiles)
+    one_round = true;
+    const double rounds = (double)((tiles + num_cus - 1) / num_cus);
+    const size_t per_slice = (size_t)g.M * tiles * cw * 32 * sizeof(float);
+    for (int wk = 1; wk <= (cw <= 2 && SB >= 4 ? 2 : 1); ++wk) {
+      long top = cw <= 4 ? std::min<long>(num_cus / std::max(tiles, 1), SB / (4 * wk)) : 1;
+      top = std::min<long>(top, (long)(ws_bytes / per_slice));
+      for (int s = 1, last = 0; s == 1 || s <= top; ++s) {
+        const int per = (SB + s - 1) / s, slices = (SB + per - 1) / per;
+        if (slices == last) continue;
+        last = slices;
+        const int steps = ((per + wk - 1) / wk + kD - 1) / kD * kD;
+        const double step_us = rounds * steps * std::max(wk == 1 ? 0.34 + 0.04 * cw : (cw == 1 ? 0.49 : 0.72), cw * wk * 0.11);
+        double us = 4.2 + std::max(step_us, stream_us) + 0.2 * std::min(step_us, stream_us) + (slices > 1 ? 3.3 : 0.);
+        const int pw = fused && g.M > 8 ? 2 : 1;
+        bool front = false;
+        if (g.R != nullptr) {
+          const int threads = (cw + pw) * 64 * wk, free_cus = (num_cus - tiles) & ~3;  // (the front is padded to a multiple of four: handover.hpp)
+          const int blocks = proj_blocks(g.M, g.rank), teams = blocks > free_cus && threads >= 512 ? 2 : 1;
+          front = fused && slices == 1 && threads >= 256 && tiles * 4 > num_cus && free_cus > 0 && (free_cus * kTiledProjBlocks >= blocks || g.pub_mute);
+          if (front) us = 1.0 + std::max(us, 4.0 + 0.53e-3 * g.K * ((blocks + free_cus * teams - 1) / (free_cus * teams)));
+          else us += 2.3 + 0.065e-6 * g.M * (double)g.K * g.rank;
+        }
+        if (us < best_us) best_us = us, best = TiledPlan{wk, slices, pw, cw, front};
+      }
+    }
+  }
+  return best;
+}
+static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused) {
+  if (g.M <= 16) return narrow_plan(g, num_cus, ws_bytes, fused);
+  const int SB = g.K >> 8;
+  // one K group of four consumer and four producer waves (two of two producers, 8B shapes at 32 rows, us: gate|up 26.4 against 26.3,
+  // down_proj 27.1 against 25.5)
+  TiledPlan p{1, 1, 4, 4, false};
+  // a few tiles more than compute units would run as two rounds, the second nearly empty: wider tiles where they bring the count
+  // down to one round
   if (tiled_tiles(g, 4) > num_cus) {
     for (int cw = 5; cw <= 8; ++cw)
       if (tiled_tiles(g, cw) <= num_cus) {
@@ -731,24 +903,11 @@ static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes) {
         break;
       }
   }
-  if (env_cw >= 1 && env_cw <= 8) p.cw = env_cw;
-  // two K groups: up to 16 token rows on tiles that fill the chip by themselves (more rows want four producer waves, and
-  // a K range cut into slices is short enough already).  8B shapes, launch with the projection, us, two groups / one:
-  // gate|up 8 rows 22.4 / 24.1, 32 rows 26.4 / 26.3; down_proj 32 rows 27.1 / 25.5
-  int wk = (SB >= 8 && p.cw <= 4 && g.M <= 16 && tiled_tiles(g, p.cw) * 2 > num_cus) ? 2 : 1;
-  if (env_wk == 1 || (env_wk == 2 && p.cw <= 4)) wk = env_wk;
-  p.pw = g.M <= 8 ? 1 : (g.M <= 16 || wk == 2 ? 2 : 4);
-  if (env_pw == 2 && g.M > 8) p.pw = 2;
-  if (env_pw == 4 && g.M > 16 && wk == 1) p.pw = 4;
-  p.wk = wk;
+  // slices where the tiles alone leave most of the chip empty
   const int tiles = tiled_tiles(g, p.cw);
-  long ldp = 0;
-  for (int i = 0; i < g.n_members; ++i) ldp += ((g.mem[i].N + 31) / 32 + p.cw - 1) / p.cw * p.cw * 32;
-  long s = env_slices > 0 ? env_slices : (tiles * 2 <= num_cus ? num_cus / tiles : 1);
-  if (s > SB / (4 * wk)) s = SB / (4 * wk);
-  const size_t per_slice = (size_t)g.M * ldp * sizeof(float);
-  if (per_slice > 0 && (size_t)s > ws_bytes / per_slice) s = (long)(ws_bytes / per_slice);
-  if (s < 1) s = 1;
+  const size_t per_slice = (size_t)g.M * tiles * p.cw * 32 * sizeof(float);
+  long s = tiles * 2 <= num_cus ? num_cus / std::max(tiles, 1) : 1;
+  s = std::max(1L, std::min(s, std::min((long)SB / 4, per_slice > 0 ? (long)(ws_bytes / per_slice) : 1L)));
   const int per = (SB + (int)s - 1) / (int)s;  // slices of equal depth: no more of them than leave none empty
   p.slices = (SB + per - 1) / per;
   return p;
@@ -761,8 +920,8 @@ size_t tiled_split_workspace_bytes(int M, int num_cus) { return M > 4 ? (size_t)
 template <int kRows, int kWk, int kPW, bool kProj = false>
 static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipStream_t stream) {
   auto kern = skinny_tiled_kernel<kRows, kWk, kPW, kProj>;
-  size_t lds = (size_t)kWk * 2 * (kRows * kRowBytes + 2 * kRows * 16);
-  const size_t red = (size_t)(kWk - 1) * a.cw * 16 * 64 * sizeof(float);
+  size_t lds = (size_t)kWk * 2 * (kRows * kRowBytes + (kRows <= 16 ? 0 : 2 * kRows * 16));
+  const size_t red = (size_t)(kWk - 1) * a.cw * (kRows <= 16 ? 8 : 16) * 64 * sizeof(float);
   if (lds < red) lds = red;
   static LdsLimit lds_limit;
   if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit); e != hipSuccess) return e;
@@ -772,7 +931,7 @@ static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipS
   if constexpr (kProj) {
     // The workgroups in front take places the launch leaves free on the chip, so that every workgroup starts at once and
     // none with a column tile waits behind a producer.  The readers ask for r during their last super-block, so a
-    // producer has most of the launch for its blocks: up to `per_producer` of them (GLOWQ_TILED_PROJ_BLOCKS).
+    // producer has most of the launch for its blocks: up to kTiledProjBlocks of them.
     static std::atomic<long> asked_for{-1};
     static std::atomic<int> resident{0};
     const long shape = (long)lds * 4096 + threads;
@@ -784,19 +943,15 @@ static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipS
       resident.store(per_cu, std::memory_order_relaxed);
       asked_for.store(shape, std::memory_order_release);
     }
-    static const int env_blocks = getenv("GLOWQ_TILED_PROJ_BLOCKS") ? atoi(getenv("GLOWQ_TILED_PROJ_BLOCKS")) : 0;
-    static const int env_producers = getenv("GLOWQ_TILED_PRODUCERS") ? atoi(getenv("GLOWQ_TILED_PRODUCERS")) : 0;
-    const int per_producer = env_blocks > 0 ? env_blocks : kTiledProjBlocks;
     // (one workgroup per compute unit, whatever the occupancy allows: two that share a compute unit share its LDS
     // bandwidth and matrix cores, and the launch gets longer -- gate|up of a 14B layer at eight rows with 131 producers
     // beside 218 tiles 42 us against 30.5)
     const long capacity = per_cu >= 1 ? num_cus : 0;
     long want = (capacity - (long)a.tiles) & ~3L;  // (the front is padded to a multiple of four: handover.hpp)
-    if (env_producers > 0) want = env_producers;
-    const int nblocks = ((a.rank + 3) / 4) * ((a.M + 3) / 4);  // blocks of r: four token rows by four rows of R
+    const int nblocks = proj_blocks(a.M, a.rank);
     if (want > nblocks) want = nblocks;
     if (want > kTiledMaxProducers) want = kTiledMaxProducers;
-    if (threads < 256 || want < 1 || ((long)per_producer * want < nblocks && a.spin != 0xFFFFFFFFu)) return hipErrorNotReady;
+    if (threads < 256 || want < 1 || ((long)kTiledProjBlocks * want < nblocks && a.spin != 0xFFFFFFFFu)) return hipErrorNotReady;
     a.producers = (int)want;
     a.teams = (nblocks > want && threads >= 512) ? 2 : 1;  // two blocks at a time where the workgroup has the waves
     grid_x = front_grid(a.tiles, a.producers);
@@ -834,7 +989,7 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   a.alpha = g.alpha;
   const bool ws_ok = g.ws != nullptr && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0;
   a.partials = ws_ok ? static_cast<float*>(g.ws) : nullptr;
-  const TiledPlan plan = tiled_plan(g, num_cus, ws_ok ? g.ws_bytes : 0);
+  const TiledPlan plan = tiled_plan(g, num_cus, ws_ok ? g.ws_bytes : 0, proj);
   a.slices = plan.slices;
   a.cw = plan.cw;
   int tiles = 0, col = 0;
@@ -857,7 +1012,7 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   a.ldp = col;
   const int key = (g.M <= 8 ? 8 : g.M <= 16 ? 16 : 32) * 100 + plan.wk * 10 + plan.pw;
   if (proj) {
-    if (a.slices != 1) return hipErrorNotReady;
+    if (!plan.front) return hipErrorNotReady;
     switch (key) {
       case 821: return launch_tiled_t<8, 2, 1, true>(a, g.x, num_cus, stream);
       case 811: return launch_tiled_t<8, 1, 1, true>(a, g.x, num_cus, stream);
@@ -869,10 +1024,8 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   switch (key) {
     case 821: return launch_tiled_t<8, 2, 1>(a, g.x, num_cus, stream);
     case 811: return launch_tiled_t<8, 1, 1>(a, g.x, num_cus, stream);
-    case 1622: return launch_tiled_t<16, 2, 2>(a, g.x, num_cus, stream);
-    case 1612: return launch_tiled_t<16, 1, 2>(a, g.x, num_cus, stream);
-    case 3222: return launch_tiled_t<32, 2, 2>(a, g.x, num_cus, stream);
-    case 3212: return launch_tiled_t<32, 1, 2>(a, g.x, num_cus, stream);
+    case 1621: return launch_tiled_t<16, 2, 1>(a, g.x, num_cus, stream);
+    case 1611: return launch_tiled_t<16, 1, 1>(a, g.x, num_cus, stream);
     case 3214: return launch_tiled_t<32, 1, 4>(a, g.x, num_cus, stream);
   }
   return hipErrorInvalidValue;
