@@ -50,7 +50,8 @@ size_t skinny_split_workspace_bytes(int M, int num_cus);  // skinny.hip
 // skinny_tiled.hip
 size_t tiled_split_workspace_bytes(int M, int num_cus);
 bool skinny_tiled_supported(const GroupDev& g);
-hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream);
+bool skinny_words_supported(const GroupDev& g);
+hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream, bool canon);
 hipError_t launch_pack_tiled(const int32_t*, const half_t*, const int32_t*, void*, int, int, int, int, int, int, int, hipStream_t);
 hipError_t launch_pack_tiled_left(const half_t*, void*, int, int, int, hipStream_t);
 hipError_t launch_shared_proj_mfma(const half_t*, const half_t*, half_t*, int, int, int, int, hipStream_t, void* ws,
@@ -429,6 +430,19 @@ bool tiled_route_on_gemm(const GroupDev& g) {
   return g.M > 16 && g.R != nullptr && g.K >= 2048 && tiles * 2 > num_cus() && tiles <= num_cus();
 }
 
+// Groups of the skinny routes whose 5 to 16 token rows run on the narrow tiles over the canonical buffers (skinny_tiled.hip): all without an r to
+// compute, the others where K is short or the stream long enough that r, which the skinny kernels take along for fewer columns, costs them a
+// launch or a part of the chip.  Group call, us at 8 and 16 rows, this / the skinny kernels: without a
+// correction 4096 x 4096 7.2, 8.1 / 7.5, 8.2, 3 x 2048 x 2048 5.6, 6.0 / 6.1, 6.5, 5120 x 5120 9.3, 10.4 / 9.7, 10.8, 18944 x 3584 12.5, 13.4 /
+// 17.9, 20.8; with one 2 x 9472 x 2816 12.8, 13.3 / 17.8, 20.4, 8192 x 2048 7.7, 8.1 / 8.9, 9.4; not q|k|v of an 8B and a 14B layer 9.7, 10.7 /
+// 9.8, 10.2 and 15.7, 17.1 / 14.9, 16.3, nor 4096 x 14336 19.6, 20.9 / 17.7, 19.9.
+bool words_pay(const GroupDev& g) {
+  long rows = 0;
+  for (int i = 0; i < g.n_members; ++i) rows += g.mem[i].N;
+  if (g.R == nullptr) return true;
+  return rows > 2048 && (g.K <= 3072 || (g.K <= 6144 && rows * (long)g.K / 2 >= 25L * 1000 * 1000));
+}
+
 int run_group(GroupDev g, int route, hipStream_t stream) {
   for (int i = 0; i < g.n_members; ++i)
     if (g.mem[i].y32 && !(route == kRouteGemm && gemm_widens(g))) return fail(GLOWQ_EUNSUPPORTED, "fp32 outputs: only where the GEMM on the tiled weights takes the call, and for all members alike");
@@ -474,6 +488,7 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
     g.pub = nullptr;
   }
   const bool skinny_route = route == kRouteSkinny || route == kRouteSkinnyRaw;
+  const bool on_words = skinny_route && skinny_words_supported(g) && words_pay(g);
   if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || (route == kRouteSkinnyTiled && !on_gemm)) && skinny_proj_in_launch(g)) ||
                          ((route == kRouteGemm || on_gemm) && gemm_proj_in_launch(g)))) {
     // single token on the stream GEMV, a handful of rows on the skinny kernel: workgroups in front of the group launch
@@ -509,7 +524,7 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
       e = launch_gemm(g, cus, stream);
     }
   } else if (route == kRouteSkinnyTiled) {
-    const auto launch = [&]() { return on_gemm ? launch_gemm(g, cus, stream, true) : launch_skinny_tiled(g, cus, stream); };
+    const auto launch = [&]() { return on_gemm ? launch_gemm(g, cus, stream, true) : launch_skinny_tiled(g, cus, stream, false); };
     e = launch();
     if (e == hipErrorNotReady && g.pub != nullptr) {
       e = launch_projection();
@@ -517,11 +532,12 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
       e = launch();
     }
   } else if (skinny_route) {
-    e = launch_skinny(g, cus, stream, route == kRouteSkinnyRaw);
+    const auto launch = [&]() { return on_words ? launch_skinny_tiled(g, cus, stream, true) : launch_skinny(g, cus, stream, route == kRouteSkinnyRaw); };
+    e = launch();
     if (e == hipErrorNotReady && g.pub != nullptr) {
       e = launch_projection();
       if (e != hipSuccess) return fail(GLOWQ_ELAUNCH, "shared_proj launch failed: %s", hipGetErrorString(e));
-      e = launch_skinny(g, cus, stream, route == kRouteSkinnyRaw);
+      e = launch();
     }
   } else {
     const int cap = (route == kRouteWaveDot) ? kWaveDotMaxM

@@ -18,6 +18,13 @@
 // producers, whose vector instructions a step had to wait for).  All eight fragments of a step are asked for at its head.  Launch
 // without a correction, 16 rows, us: 2 x 14336 x 4096 18.4 -> 15.3 (4.0 TB/s), 2 x 17408 x 5120 26.4 -> 23.2, 17408 x 5120 19.7 -> 15.4,
 // 5120 x 17408 20.0 -> 16.3.
+// kCanon: the narrow tiles on the canonical buffers, for groups without a tiled copy: a lane takes 16 bytes (four words) of the row that is its
+// column, and word j of all lanes is an operand by itself -- the k values of a product may come in any order that the activations share, which
+// are read from where those words' columns are staged, in the order the masks leave the codes.  A load instruction covers half a cache line of
+// sixteen rows, so the two halves are asked for together and without the non-temporal hint (18944 x 3584, 16 rows: 13.4, with it 14.2; asked
+// for half a step apart 15.9); scales and zero-points come for four super-blocks at a time (with two gathers a super-block 15.2).
+// Launch without a correction, 8 and 16 rows, us, against the kernels of skinny.hip: 14336 x 4096 15.7, 16.9 -> 11.6, 12.5, 18944 x 3584
+// 17.9, 20.8 -> 12.5, 13.4, 1024 x 5120 8.9, 9.8 -> 8.2, 8.4, 4096 x 14336 15.3, 17.5 -> 14.8, 15.3, 8192 x 2048 6.3, 6.9 -> 5.3, 6.3.
 //
 // A workgroup owns 32 cw output columns of one member (a row block of 32 per consumer wave) and all token rows.  Its
 // waves come in K groups that walk contiguous parts of the K range in step and meet in LDS at the end; a K group is
@@ -67,6 +74,10 @@ struct TileMember {
   half_t* y;
   int N, ldy;
   int col0;                 // first column of the member in a row of the partial buffer (members padded to 128)
+  // kCanon: wt is the packed weight itself, lt the left factor [N, rank]
+  const half_t* scales;
+  const int32_t* qzeros;
+  int ldw, lds, ldz;
 };
 
 struct TileArgs {
@@ -148,7 +159,7 @@ __device__ unsigned long long g_tstamps[65536 * 32];
 constexpr int tiled_max_cw(int wk, int pw) { return wk > 1 ? 4 : 12 - pw; }
 constexpr int tiled_max_threads(int wk, int pw) { return (tiled_max_cw(wk, pw) + pw) * 64 * wk; }
 
-template <int kRows, int kWk, int kPW, bool kProj = false>
+template <int kRows, int kWk, int kPW, bool kProj = false, bool kCanon = false>
 __global__ __launch_bounds__(tiled_max_threads(kWk, kPW))
 void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K, const int slices,
                          const unsigned char* __restrict__ wt0, const int blk_end0, const int N0, const int cw, const TileArgs g) {
@@ -157,6 +168,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   constexpr int kPQ = (kRows + 2 * kPW - 1) / (2 * kPW);  // 16-byte pieces of a super-block of x per producer thread
   static_assert(kPQ * 2 * kPW == kRows, "whole passes");
   constexpr bool kNarrow = kRows <= 16;          // tiles of 16 token rows by 16 columns
+  static_assert(kNarrow || !kCanon, "the canonical buffers are read by the narrow tiles");
   constexpr int kSigBytes = kNarrow ? 0 : kRows * 16;  // per 128-column half: a 16-byte fragment of sums per token row
   constexpr int kStage = kRows * kRowBytes + 2 * kSigBytes;
   constexpr int kLiveRegs = kRows >= 32 ? 16 : (kRows >= 16 ? 8 : 4);  // accumulator registers of rows that exist
@@ -267,16 +279,28 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
       for (int q = 0; q < kPQ; ++q) {
         const uint32_t row = (uint32_t)min(2 * kPW * q + prow, M - 1);
-        av[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((row * ld + (uint32_t)pcol * 8u) * 2u), idx * 512, 0);
+        uint32_t off = (row * ld + (uint32_t)pcol * 8u) * 2u;
+        if (is_r && idx * 256 + pcol * 8 >= g.rank) off = 0x80000000u;  // zeros past the rank (not the next row, which may not be finite)
+        av[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, idx * 512, 0);
       }
     };
-    auto store_a = [&](const u32x4 (&av)[kPQ], int stage) __attribute__((always_inline)) {
+    auto store_a = [&](const u32x4 (&av)[kPQ], int stage, bool is_r) __attribute__((always_inline)) {
       unsigned char* dst = smem + stage * kStage + prow * kRowBytes + pcol * 16;
       unsigned char* sig = smem + stage * kStage + kRows * kRowBytes + (pcol >> 4) * kSigBytes + prow * 16;
       const h2 ones = {(half_t)1.f, (half_t)1.f};
       const h2 sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
 #pragma unroll
       for (int q = 0; q < kPQ; ++q) {
+        if constexpr (kCanon) {
+          // columns in the order the masks deliver the codes of a canonical word: (0, 4), (1, 5) / 16, (2, 6), (3, 7) / 16; r as it is
+          const u32x4 v = av[q];
+          u32x4 o = {__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
+                     __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
+          o.y = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.y) * sixteenth);
+          o.w = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.w) * sixteenth);
+          *reinterpret_cast<u32x4*>(dst + 2 * kPW * q * kRowBytes) = is_r ? v : o;
+          continue;
+        }
         if constexpr (kNarrow) {
           u32x4 o = av[q];
           o.y = __builtin_bit_cast(uint32_t, bitcast_u32<h2>(o.y) * sixteenth);
@@ -322,7 +346,9 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
         for (int q = 0; q < kPQ; ++q) {
           const uint32_t row = (uint32_t)min(2 * kPW * q + prow, M - 1);
-          av[q] = __builtin_amdgcn_raw_buffer_load_b128(rs_r, (int)((row * (uint32_t)g.rank + (uint32_t)pcol * 8u) * 2u), 0, 16);
+          uint32_t off = (row * (uint32_t)g.rank + (uint32_t)pcol * 8u) * 2u;
+          if (pcol * 8 >= g.rank) off = 0x80000000u;
+          av[q] = __builtin_amdgcn_raw_buffer_load_b128(rs_r, (int)off, 0, 16);
         }
       }
       return seen != 0;
@@ -356,7 +382,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     };
 #pragma unroll
     for (int j = 0; j < kXD; ++j) fetch(avs[j], j);
-    store_a(avs[0], 0);
+    store_a(avs[0], 0, false);
     fetch(avs[0], kXD);
     __syncthreads();
     bool have_r = false;
@@ -368,7 +394,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         // does not read
         if (set == 0 && i + 1 == steps && wg_corr && gk == 0 && !have_r) load_r_handed(avs[0]);
       }
-      store_a(avs[set], (i + 1) & 1);  // step i + 1's activations (or r after the last step)
+      store_a(avs[set], (i + 1) & 1, i + 1 >= steps);  // step i + 1's activations (or r after the last step)
       fetch(avs[set], i + 1 + kXD);
       if constexpr (kProj) {
         // one look a step before: as a rule the workgroups in front are long done
@@ -388,7 +414,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       for (int pass = 1; pass * kD < LBall; ++pass) {
         __syncthreads();
         load_a(avs[0], true, pass);
-        store_a(avs[0], 0);
+        store_a(avs[0], 0, true);
         __syncthreads();
       }
     }
@@ -418,21 +444,69 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   // chunk (rb, sb) lies at (sb * RB + rb) * kChunk: the descriptor starts at the wave's chunk of super-block 0 and ends
   // behind its chunk of the group's last super-block
   const int chunk_stride = ((mem_N + 31) >> 5) * tiled::kChunk;
-  const __amdgpu_buffer_rsrc_t rs_w = rsrc(wt + (size_t)(live ? rb : 0) * tiled::kChunk, live && sb1 > 0 ? (size_t)(sb1 - 1) * chunk_stride + tiled::kChunk : 0);
+  const int ldw = kCanon ? g.mem[mi].ldw : 0, lds = kCanon ? g.mem[mi].lds : 0, ldz = kCanon ? g.mem[mi].ldz : 0;
+  const int crows = live ? min(32, mem_N - rb * 32) : 0;  // kCanon: rows of the block that exist
+  const size_t crow0 = (size_t)(live ? rb : 0) * 32;
+  const __amdgpu_buffer_rsrc_t rs_w = kCanon ? rsrc(wt + crow0 * ldw * 4, (size_t)crows * ldw * 4)
+                                             : rsrc(wt + (size_t)(live ? rb : 0) * tiled::kChunk, live && sb1 > 0 ? (size_t)(sb1 - 1) * chunk_stride + tiled::kChunk : 0);
   const int b_off = lane * 16;
 
   struct BSet {
-    u32x4 w[4];
-    u32x2 side;  // the lane's column: (scale | -zero * 2^-16) of the two halves
+    u32x4 w[4];  // kCanon: [2 half + c], columns 16 c + lane % 16, k words 4 (lane / 16) .. + 3 of the half
+    u32x2 side;  // the lane's column: (scale | -zero * 2^-16) of the two halves (kCanon: from `turn`)
   };
   BSet bs[kD];
+  const __amdgpu_buffer_rsrc_t rs_s = rsrc(kCanon ? (const void*)(g.mem[mi].scales + crow0 * lds) : (const void*)wt, kCanon ? (size_t)crows * lds * 2 : 0);
+  const __amdgpu_buffer_rsrc_t rs_z = rsrc(kCanon ? (const void*)(g.mem[mi].qzeros + crow0 * ldz) : (const void*)wt, kCanon ? (size_t)crows * ldz * 4 : 0);
+  const int c_row = lane & 15;
+  int w_at[2], s_at[2], z_at[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    w_at[c] = (16 * c + c_row) * ldw * 4 + (lane >> 4) * 16;
+    s_at[c] = (16 * c + c_row) * lds * 2;
+    z_at[c] = (16 * c + c_row) * ldz * 4;
+  }
+  // kCanon: scales and zero-points of the super-blocks of a rotation in columns c = 0, 1 (a gather over sixteen rows, hence four
+  // super-blocks at a time), asked for a rotation ahead.  The four pairs of scales start early enough to lie in the row.
+  struct Side {
+    u32x4 s[2];
+    uint32_t z0[2], z1[2];
+  };
+  Side ahead = {}, now = {};
+  const auto request_side = [&](int sbq) __attribute__((always_inline)) {
+    const int at = min(sbq, SB - kD) * 4, word = min(sbq, SB - 1) >> 2, last = (SB - 1) >> 2;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      ahead.s[c] = __builtin_amdgcn_raw_buffer_load_b128(rs_s, s_at[c], at, 0);
+      ahead.z0[c] = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_at[c], word * 4, 0);
+      ahead.z1[c] = __builtin_amdgcn_raw_buffer_load_b32(rs_z, z_at[c], min(word + 1, last) * 4, 0);
+    }
+  };
+  const auto turn = [&](int sbq, bool more) __attribute__((always_inline)) {
+    const int skip = min(sbq, SB - 1) - min(sbq, SB - kD);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      u32x4 v = ahead.s[c];
+      if (skip & 1) v = u32x4{v.y, v.z, v.w, v.w};
+      if (skip & 2) v = u32x4{v.z, v.w, v.w, v.w};
+      now.s[c] = v;
+      now.z0[c] = __builtin_amdgcn_alignbit(ahead.z1[c], ahead.z0[c], 8 * (sbq & 3));
+    }
+    if (more) request_side(sbq + kD);
+  };
   auto request = [&](BSet& b, int sbq) __attribute__((always_inline)) {
+    if constexpr (kCanon) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b.w[2 * (j & 1) + (j >> 1)] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, w_at[j >> 1], sbq * 128 + (j & 1) * 64, 0);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) b.w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, b_off + j * 1024, sbq * chunk_stride, kStreamAux);
     b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sbq * chunk_stride + tiled::kCodeBytes, kStreamAux));
   };
   // two super-blocks up front, the other two once the first activations are staged: with all four at once the whole
   // chip asks for half a long matrix before any wave can begin
+  if constexpr (kCanon) request_side(sb0);
   request(bs[0], sb0);
   request(bs[1], sb0 + 1);
   GLOWQ_STAMP(1);
@@ -440,8 +514,21 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   // a member without a left factor (GlowQ-S) reads zeros for its correction blocks
   const TileMember mem = g.mem[mi];
   const bool has_l = wg_corr && gk == 0 && mem.lt != nullptr && live;
-  const __amdgpu_buffer_rsrc_t rs_l = rsrc(has_l ? mem.lt + (size_t)rb * LBall * tiled::kLChunk : wt, has_l ? (size_t)LBall * tiled::kLChunk : 0);
+  const __amdgpu_buffer_rsrc_t rs_l = kCanon ? rsrc(has_l ? mem.lt + crow0 * g.rank * 2 : wt, has_l ? (size_t)crows * g.rank * 2 : 0) : rsrc(has_l ? mem.lt + (size_t)rb * LBall * tiled::kLChunk : wt, has_l ? (size_t)LBall * tiled::kLChunk : 0);
 
+  // block q (64 columns of the rank) of the left factor into a set
+  const auto request_left = [&](BSet& b, int q) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if constexpr (kCanon) {  // w[2 t + c]: columns 32 t + 8 (lane / 16) .. + 7 of the block
+        const int col = q * 64 + (t >> 1) * 32 + (lane >> 4) * 8;
+        const int at = ((16 * (t & 1) + c_row) * g.rank + col) * 2;
+        b.w[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, col < g.rank ? at : (int)0x80000000u, 0, 0);
+      } else {
+        b.w[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, b_off + t * 1024, q * tiled::kLChunk, 0);
+      }
+    }
+  };
   // Up to 16 token rows: tiles of 16 rows by 16 columns, two to a row block (acc[c][i]: row 4 (lane / 16) + i, column 16 c + lane % 16).
   // Rows of sixteen lanes of two neighbouring words change places, and each of the two then holds the codes of sixteen columns over
   // the 32 k values of both.
@@ -463,7 +550,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 
   // One super-block: the codes of the register set `b` against the staged rows, half by half.
   // kRefill: each register of the set is refilled with super-block sb_next as soon as its words have been masked.
-  auto compute = [&](int sb_next, int stage, BSet& b, auto refill_const) __attribute__((always_inline)) {
+  auto compute = [&](auto d_const, int sb_next, BSet& b, auto refill_const) __attribute__((always_inline)) {
+    constexpr int d = decltype(d_const)::value, stage = d & 1;
     constexpr bool kRefill = decltype(refill_const)::value;
     const unsigned char* st = smem + stage * kStage;
     const u32x2 side = b.side;
@@ -483,24 +571,42 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     }
 #endif
     if constexpr (kNarrow) {
-      uint32_t sw[2][2];
-      spread(side.x, side.x, sw[0][0], sw[0][1]);
-      spread(side.y, side.y, sw[1][0], sw[1][1]);
+      uint32_t sw[2][2];  // [half][c]
+      if constexpr (kCanon) {
+        sw[0][0] = now.s[0][d], sw[0][1] = now.s[1][d], sw[1][0] = sw[0][0] >> 16, sw[1][1] = sw[0][1] >> 16;
+      } else {
+        spread(side.x, side.x, sw[0][0], sw[0][1]);
+        spread(side.y, side.y, sw[1][0], sw[1][1]);
+      }
       // the pairs a mask leaves at code * 2^-20 are staged divided by 16
       const h2 one = {(half_t)1.f, (half_t)1.f}, sixteen = {(half_t)16.f, (half_t)16.f};
       const uint32_t o1 = __builtin_bit_cast(uint32_t, one), o16 = __builtin_bit_cast(uint32_t, sixteen);
       const h8 ones = __builtin_bit_cast(h8, u32x4{o1, o16, o1, o16});
       // all fragments of the step are asked for at once: one LDS round trip for it instead of eight
-      const unsigned char* xs = st + nrow_off + 128 * (nq >> 1) + 16 * (nq & 1);
+      const unsigned char* xs = st + nrow_off + (kCanon ? 64 * nq : 128 * (nq >> 1) + 16 * (nq & 1));
       h8 af[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) af[t] = *reinterpret_cast<const h8*>(xs + 256 * (t >> 2) + 32 * (t & 3));
+      for (int t = 0; t < 8; ++t) af[t] = *reinterpret_cast<const h8*>(xs + 256 * (t >> 2) + (kCanon ? 16 : 32) * (t & 3));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int gh = 0; gh < 2; ++gh) {
         f4 pg[2] = {}, sx = {};
+        if constexpr (kCanon) {
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
+          for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const uint32_t wd = b.w[2 * gh + c][j], hi = wd >> 8;
+              const h8 bf = __builtin_bit_cast(h8, u32x4{wd & 0x000F000Fu, wd & 0x00F000F0u, hi & 0x000F000Fu, hi & 0x00F000F0u});
+              pg[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j], bf, pg[c], 0, 0, 0);
+            }
+            sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j], ones, sx, 0, 0, 0);
+          }
+          if constexpr (kRefill)
+            if (gh == 1) request(b, sb_next);  // (both halves of a cache line together)
+        }
+#pragma unroll
+        for (int p = 0; p < (kCanon ? 0 : 2); ++p) {
           const u32x4 raw = b.w[2 * gh + p];
 #pragma unroll
           for (int i = 0; i < 4; i += 2) {
@@ -520,12 +626,13 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const float sf = (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] & 0xFFFFu)) * 0x1p24f;
-          const float nz = (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] >> 16)) * 0x1p-8f;  // -zero * 2^-24
+          const float nz = kCanon ? (float)((now.z0[c] >> (8 * d + 4 * gh)) & 15u) * -0x1p-24f
+                                  : (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] >> 16)) * 0x1p-8f;  // -zero * 2^-24
 #pragma unroll
           for (int i = 0; i < 4; ++i) nacc[c][i] = __builtin_fmaf(sf, __builtin_fmaf(nz, sx[i], pg[c][i]), nacc[c][i]);
         }
       }
-      if constexpr (kRefill)
+      if constexpr (kRefill && !kCanon)
         b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sb_next * chunk_stride + tiled::kCodeBytes, kStreamAux));
       return;
     }
@@ -574,11 +681,10 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     constexpr int d = decltype(d_const)::value;
     constexpr bool kLast = decltype(last_const)::value;
     if constexpr (kLast) {
-      if (sb < sb1) compute(0, d & 1, bs[d], std::false_type{});
-#pragma unroll
-      for (int t = 0; t < 4; ++t) bs[d].w[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, b_off + t * 1024, d * tiled::kLChunk, 0);
+      if (sb < sb1) compute(d_const, 0, bs[d], std::false_type{});
+      request_left(bs[d], d);
     } else {
-      compute(sb + kD, d & 1, bs[d], std::true_type{});
+      compute(d_const, sb + kD, bs[d], std::true_type{});
     }
     GLOWQ_STAMP(8 + min(sb - sb0, 11) * 2);
     __syncthreads();
@@ -587,12 +693,14 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   using std::integral_constant;
   int sb = sb0;
   for (int rd = 0; rd < rounds - 1; ++rd, sb += kD) {
+    if constexpr (kCanon) turn(sb, true);
     step(sb, integral_constant<int, 0>{}, std::false_type{});
     step(sb + 1, integral_constant<int, 1>{}, std::false_type{});
     step(sb + 2, integral_constant<int, 2>{}, std::false_type{});
     step(sb + 3, integral_constant<int, 3>{}, std::false_type{});
   }
   GLOWQ_STAMP(3);
+  if constexpr (kCanon) turn(sb, false);
   step(sb, integral_constant<int, 0>{}, std::true_type{});
   GLOWQ_STAMP(4);
   step(sb + 1, integral_constant<int, 1>{}, std::true_type{});
@@ -611,22 +719,19 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       if (pass > 0) {
         __syncthreads();  // the fragment reads of the pass before are done
 #pragma unroll
-        for (int q = 0; q < kD; ++q)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            bs[q].w[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, b_off + t * 1024, (pass * kD + q) * tiled::kLChunk, 0);
+        for (int q = 0; q < kD; ++q) request_left(bs[q], pass * kD + q);
         __syncthreads();
       }
       if constexpr (kNarrow) {
-        const unsigned char* ar = smem + nrow_off + 64 * (nq >> 1) + 16 * (nq & 1);
+        const unsigned char* ar = smem + nrow_off + (kCanon ? 16 * nq : 64 * (nq >> 1) + 16 * (nq & 1));
 #pragma unroll
         for (int q = 0; q < kD; ++q)
 #pragma unroll
           for (int t = 0; t < 4; t += 2) {
-            const h8 af = *reinterpret_cast<const h8*>(ar + 128 * q + 16 * t);
-            u32x4 bw[2];
+            const h8 af = *reinterpret_cast<const h8*>(ar + 128 * q + (kCanon ? 32 : 16) * t);
+            u32x4 bw[2] = {bs[q].w[t], bs[q].w[t + 1]};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < (kCanon ? 0 : 4); ++e) {
               uint32_t lo, hi;
               spread(bs[q].w[t][e], bs[q].w[t + 1][e], lo, hi);
               bw[0][e] = lo;
@@ -823,6 +928,22 @@ bool skinny_tiled_supported(const GroupDev& g) {
   return true;
 }
 
+// The narrow tiles on the canonical buffers: 5 to 16 token rows, K in four and more whole super-blocks, groups of 128 columns, and what the loads need of
+// pointers and strides (codes and left factor 16 bytes, scales and zero-points four).
+bool skinny_words_supported(const GroupDev& g) {
+  if (g.M < 5 || g.M > 16 || (g.K & 255) != 0 || g.K < 1024 || g.group_size != 128) return false;
+  const half_t* r = g.r != nullptr ? g.r : (g.R != nullptr ? g.r_out : nullptr);
+  if (r != nullptr && ((g.rank & 7) != 0 || g.rank < 8 || (reinterpret_cast<uintptr_t>(r) & 15u) != 0)) return false;
+  if ((reinterpret_cast<uintptr_t>(g.x) & 15u) != 0 || (size_t)g.M * g.K * 2 >= (1ull << 31)) return false;
+  for (int i = 0; i < g.n_members; ++i) {
+    const MemberDev& m = g.mem[i];
+    if ((reinterpret_cast<uintptr_t>(m.qweight) & 15u) != 0 || (m.ldw & 3) != 0 || m.ldw < g.K / 8 || (size_t)m.ldw * 128 >= (1ull << 31)) return false;
+    if ((reinterpret_cast<uintptr_t>(m.scales) & 3u) != 0 || (m.lds & 1) != 0 || (reinterpret_cast<uintptr_t>(m.qzeros) & 3u) != 0) return false;
+    if (m.L != nullptr && r != nullptr && (reinterpret_cast<uintptr_t>(m.L) & 15u) != 0) return false;
+  }
+  return true;
+}
+
 // How the launch cuts K and staffs a K group: `wk` K groups inside a workgroup (their sums meet in LDS), `slices`
 // workgroups per tile (their sums meet in the workspace), `pw` producer waves per K group, `cw` consumer waves (a tile is 32 cw columns).
 // Workgroups stay at 768 threads and below (a 1024-thread workgroup gets 128 registers per lane and the chip runs such workgroups in
@@ -847,7 +968,7 @@ static int proj_blocks(int M, int rank) { return ((rank + 3) / 4) * ((M + 3) / 4
 // 5120 x 17408 18.2 / 16.7, 4096 x 14336 14.6 / 14.0.
 // (One K group at a wave per SIMD leaves vector and matrix instructions to alternate; two of them pay where the tiles are a row block or
 // two wide: 4096 x 4096 7.9 against 10.2, but 2 x 14336 x 4096 at four 16.9 against 15.5.)
-static TiledPlan narrow_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused) {
+static TiledPlan narrow_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused, bool canon) {
   const int SB = g.K >> 8;
   const bool corrected = g.r != nullptr || g.R != nullptr;
   double rows = 0;
@@ -873,7 +994,7 @@ static TiledPlan narrow_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bo
         const int steps = ((per + wk - 1) / wk + kD - 1) / kD * kD;
         const double step_us = rounds * steps * std::max(wk == 1 ? 0.34 + 0.04 * cw : (cw == 1 ? 0.49 : 0.72), cw * wk * 0.11);
         double us = 4.2 + std::max(step_us, stream_us) + 0.2 * std::min(step_us, stream_us) + (slices > 1 ? 3.3 : 0.);
-        const int pw = fused && g.M > 8 ? 2 : 1;
+        const int pw = (fused || canon) && g.M > 8 ? 2 : 1;  // (one wave with all pieces of 16 rows and more to do runs out of registers)
         bool front = false;
         if (g.R != nullptr) {
           const int threads = (cw + pw) * 64 * wk, free_cus = (num_cus - tiles) & ~3;  // (the front is padded to a multiple of four: handover.hpp)
@@ -888,8 +1009,8 @@ static TiledPlan narrow_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bo
   }
   return best;
 }
-static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused) {
-  if (g.M <= 16) return narrow_plan(g, num_cus, ws_bytes, fused);
+static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes, bool fused, bool canon) {
+  if (g.M <= 16) return narrow_plan(g, num_cus, ws_bytes, fused, canon);
   const int SB = g.K >> 8;
   // one K group of four consumer and four producer waves (two of two producers, 8B shapes at 32 rows, us: gate|up 26.4 against 26.3,
   // down_proj 27.1 against 25.5)
@@ -917,9 +1038,9 @@ static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes, boo
 // groups have tiles of four consumer waves (128 columns): one 128-column fp32 tile per token row for each of them.
 size_t tiled_split_workspace_bytes(int M, int num_cus) { return M > 4 ? (size_t)num_cus * (size_t)M * 128 * sizeof(float) : 0; }
 
-template <int kRows, int kWk, int kPW, bool kProj = false>
+template <int kRows, int kWk, int kPW, bool kProj = false, bool kCanon = false>
 static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipStream_t stream) {
-  auto kern = skinny_tiled_kernel<kRows, kWk, kPW, kProj>;
+  auto kern = skinny_tiled_kernel<kRows, kWk, kPW, kProj, kCanon>;
   size_t lds = (size_t)kWk * 2 * (kRows * kRowBytes + (kRows <= 16 ? 0 : 2 * kRows * 16));
   const size_t red = (size_t)(kWk - 1) * a.cw * (kRows <= 16 ? 8 : 16) * 64 * sizeof(float);
   if (lds < red) lds = red;
@@ -958,14 +1079,37 @@ static hipError_t launch_tiled_t(TileArgs& a, const half_t* x, int num_cus, hipS
   }
   hipLaunchKernelGGL(kern, dim3(grid_x, a.slices), dim3(threads), lds, stream, x, a.M, a.K, a.slices, a.mem[0].wt,
                      a.blk_end[0], a.mem[0].N, a.cw, a);
-  note_launch(grid_x, a.slices, threads, kProj ? "skinny_tiled_kernel<%d,%d,%d,1> with %d consumer waves" : "skinny_tiled_kernel<%d,%d,%d> with %d consumer waves",
-              kRows, kWk, kPW, a.cw);
+  note_launch(grid_x, a.slices, threads, kProj ? "%s<%d,%d,%d,1> with %d consumer waves" : "%s<%d,%d,%d> with %d consumer waves",
+              kCanon ? "skinny_words_kernel" : "skinny_tiled_kernel", kRows, kWk, kPW, a.cw);
   if (hipError_t e = hipGetLastError(); e != hipSuccess || a.slices == 1) return e;
   hipLaunchKernelGGL(skinny_tiled_reduce_kernel, dim3((a.ldp / 4 + 255) / 256, a.M), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
-hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
+template <bool kCanon>
+static hipError_t launch_narrow(TileArgs& a, const half_t* x, const TiledPlan& plan, bool proj, int num_cus, hipStream_t stream) {
+  const int key = (a.M <= 8 ? 8 : 16) * 100 + plan.wk * 10 + plan.pw;
+  if (proj) {
+    if (!plan.front) return hipErrorNotReady;
+    switch (key) {
+      case 821: return launch_tiled_t<8, 2, 1, true, kCanon>(a, x, num_cus, stream);
+      case 811: return launch_tiled_t<8, 1, 1, true, kCanon>(a, x, num_cus, stream);
+      case 1622: return launch_tiled_t<16, 2, 2, true, kCanon>(a, x, num_cus, stream);
+      case 1612: return launch_tiled_t<16, 1, 2, true, kCanon>(a, x, num_cus, stream);
+    }
+    return hipErrorInvalidValue;
+  }
+  switch (key) {
+    case 821: return launch_tiled_t<8, 2, 1, false, kCanon>(a, x, num_cus, stream);
+    case 811: return launch_tiled_t<8, 1, 1, false, kCanon>(a, x, num_cus, stream);
+    case 1620 + (kCanon ? 2 : 1): return launch_tiled_t<16, 2, kCanon ? 2 : 1, false, kCanon>(a, x, num_cus, stream);
+    case 1610 + (kCanon ? 2 : 1): return launch_tiled_t<16, 1, kCanon ? 2 : 1, false, kCanon>(a, x, num_cus, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+// `canon`: the narrow tiles on the canonical buffers (skinny_words_supported)
+hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream, bool canon) {
   TileArgs a;
   a.r = g.r;
   // the launch computes r itself (run_group set g.pub to the head of the workspace): up to 16 token rows and rank 256 (r
@@ -989,15 +1133,20 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   a.alpha = g.alpha;
   const bool ws_ok = g.ws != nullptr && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0;
   a.partials = ws_ok ? static_cast<float*>(g.ws) : nullptr;
-  const TiledPlan plan = tiled_plan(g, num_cus, ws_ok ? g.ws_bytes : 0, proj);
+  const TiledPlan plan = tiled_plan(g, num_cus, ws_ok ? g.ws_bytes : 0, proj, canon);
   a.slices = plan.slices;
   a.cw = plan.cw;
   int tiles = 0, col = 0;
   for (int i = 0; i < g.n_members; ++i) {
     const MemberDev& m = g.mem[i];
     TileMember& t = a.mem[i];
-    t.wt = static_cast<const unsigned char*>(m.tiled);
-    t.lt = (m.L != nullptr && (g.r != nullptr || proj)) ? static_cast<const unsigned char*>(m.tiled_L) : nullptr;
+    t.wt = canon ? reinterpret_cast<const unsigned char*>(m.qweight) : static_cast<const unsigned char*>(m.tiled);
+    t.lt = (m.L != nullptr && (g.r != nullptr || proj)) ? (canon ? reinterpret_cast<const unsigned char*>(m.L) : static_cast<const unsigned char*>(m.tiled_L)) : nullptr;
+    t.scales = m.scales;
+    t.qzeros = m.qzeros;
+    t.ldw = m.ldw;
+    t.lds = m.lds;
+    t.ldz = m.ldz;
     t.bias = m.bias;
     t.y = m.y;
     t.N = m.N;
@@ -1010,25 +1159,8 @@ hipError_t launch_skinny_tiled(GroupDev& g, int num_cus, hipStream_t stream) {
   }
   a.tiles = tiles;
   a.ldp = col;
-  const int key = (g.M <= 8 ? 8 : g.M <= 16 ? 16 : 32) * 100 + plan.wk * 10 + plan.pw;
-  if (proj) {
-    if (!plan.front) return hipErrorNotReady;
-    switch (key) {
-      case 821: return launch_tiled_t<8, 2, 1, true>(a, g.x, num_cus, stream);
-      case 811: return launch_tiled_t<8, 1, 1, true>(a, g.x, num_cus, stream);
-      case 1622: return launch_tiled_t<16, 2, 2, true>(a, g.x, num_cus, stream);
-      case 1612: return launch_tiled_t<16, 1, 2, true>(a, g.x, num_cus, stream);
-    }
-    return hipErrorNotReady;
-  }
-  switch (key) {
-    case 821: return launch_tiled_t<8, 2, 1>(a, g.x, num_cus, stream);
-    case 811: return launch_tiled_t<8, 1, 1>(a, g.x, num_cus, stream);
-    case 1621: return launch_tiled_t<16, 2, 1>(a, g.x, num_cus, stream);
-    case 1611: return launch_tiled_t<16, 1, 1>(a, g.x, num_cus, stream);
-    case 3214: return launch_tiled_t<32, 1, 4>(a, g.x, num_cus, stream);
-  }
-  return hipErrorInvalidValue;
+  if (g.M <= 16) return canon ? launch_narrow<true>(a, g.x, plan, proj, num_cus, stream) : launch_narrow<false>(a, g.x, plan, proj, num_cus, stream);
+  return launch_tiled_t<32, 1, 4>(a, g.x, num_cus, stream);
 }
 
 }  // namespace glowq

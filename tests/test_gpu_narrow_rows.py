@@ -1,0 +1,134 @@
+"""GPU parity of the 16 x 16 tiles for up to sixteen token rows, on the tiled copy of the weights and on the canonical buffers: both staged row
+counts, ragged row blocks and members, K groups and slices of unequal depth, ranks around the blocks and past a pass, r inside the launch
+and ahead of it, strided buffers, rows that are not finite, and replays of a graph."""
+import pytest
+import torch
+
+from glowq_amd.kernels import PreparedGroup
+from helpers import tuning
+
+pytestmark = pytest.mark.gpu
+
+
+def make(seed, M, K, Ns, rank, gs=128):
+    """Activations in the hundreds (rounded weights would be off by more than the outputs are), weights as stored and in fp64."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = (torch.randn(M, K, device="cuda", generator=g) * 64).half()
+    R = (torch.randn(rank, K, device="cuda", generator=g) * K ** -0.5).half() if rank else None
+    members, exact = [], []
+    for N in Ns:
+        codes = torch.randint(0, 16, (N, K), device="cuda", generator=g)
+        zeros = torch.randint(0, 16, (N, K // gs), device="cuda", generator=g)
+        scales = (torch.rand(N, K // gs, device="cuda", generator=g) * 0.01 + 0.001).half()
+        qw = sum(codes.view(N, K // 8, 8)[:, :, i] << (4 * i) for i in range(8))
+        zp = torch.nn.functional.pad(zeros, (0, -zeros.size(1) % 8))
+        qz = sum(zp.view(N, -1, 8)[:, :, i] << (4 * i) for i in range(8))
+        members.append({"qweight": qw.to(torch.int32), "qzeros": qz.to(torch.int32), "scales": scales, "bias": None,
+                        "L": (torch.randn(N, rank, device="cuda", generator=g) * 0.05).half() if rank else None})
+        exact.append((codes - zeros.repeat_interleave(gs, 1)).double() * scales.repeat_interleave(gs, 1).double())
+    return x, R, members, exact
+
+
+def check(y, x, r, exact, members, rows=slice(None)):
+    for got, w, m in zip(y, exact, members):
+        want = x.double() @ w.t()
+        if m["L"] is not None:
+            want = want + r.double() @ m["L"].double().t()
+        got, want = got.double()[rows], want[rows]
+        # outputs in the hundreds: their own rounding, and fp32 sums of terms up to 64 x 4 x 0.15
+        assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 2e-2).all()
+        assert (got - want).norm() <= 3.2e-4 * want.norm()
+
+
+@pytest.fixture(params=["tiled", "words"])
+def form(request, ext):
+    limits = {"tiled_shape_rule": 0} if request.param == "tiled" else {"tiled_max_m": 0}
+    with tuning(ext, **limits):
+        yield request.param
+
+
+def launched(ext, form):
+    return ext.last_launch()["kernel"].startswith(f"skinny_{form}_kernel")
+
+
+SHAPES = [(256, [4000], 8), (512, [130, 2040], 40), (1024, [4100, 3000], 40), (1280, [2600, 33], 72), (2304, [2336], 256), (5120, [5120, 1024, 1024], 256),
+          (17408, [5120], 264), (768, [34000], 136), (4096, [28672], 64), (1024, [1], 0), (3328, [40, 7], 0), (14336, [4096], 0), (2816, [9472, 9472], 0)]
+
+
+@pytest.mark.parametrize("K,Ns,rank", SHAPES)
+@pytest.mark.parametrize("M", [5, 8, 9, 16])
+def test_against_fp64(ext, form, M, K, Ns, rank):
+    print(f"case M={M} K={K} Ns={Ns} rank={rank} {form}", flush=True)
+    x, R, members, exact = make(M + K, M, K, Ns, rank)
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if rank else 0.0, R=R)
+    for in_front in (0, 1):
+        with tuning(ext, proj_in_launch=in_front):
+            y = pg.run(x)
+        if form == "words" and (rank or K < 1024) and ext.last_launch()["kernel"].startswith("skinny_") and not launched(ext, form):
+            continue  # a group that the skinny kernel keeps
+        assert launched(ext, form), ext.last_launch()
+        r = pg.last_r
+        if rank:
+            want_r = x.double() @ R.double().t()
+            assert ((r.double() - want_r).abs() <= 2.0 ** -11 * want_r.abs() + 6e-3).all()
+        check(y, x, r, exact, members)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("K,Ns,rank", [(2304, [2336], 40), (14336, [4096], 0), (2816, [9472, 9472], 256)])
+def test_rows_that_are_not_finite_stay_by_themselves(ext, form, K, Ns, rank, bad):
+    M = 13
+    x, R, members, exact = make(K, M, K, Ns, rank)
+    x[[1, 11]] = bad
+    fine = [m for m in range(M) if m not in (1, 11)]
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if rank else 0.0, R=R)
+    y = pg.run(x)
+    assert launched(ext, form)
+    for out in y:
+        assert not torch.isfinite(out[[1, 11]]).any()
+        assert torch.isfinite(out[fine]).all()
+    xs, r = x[fine], pg.last_r[fine] if rank else None
+    check([o[fine] for o in y], xs, r, exact, members)
+
+
+def test_strided_buffers_and_bias(ext):
+    """Members inside wider buffers (row strides above the shape's) on the canonical form, with a bias."""
+    M, K, N = 11, 1280, 2600
+    x, _, (m,), exact = make(3, M, K, [N], 0)
+    wide = {k: torch.full((N, m[k].size(1) + pad), 7, dtype=m[k].dtype, device="cuda") for k, pad in (("qweight", 4), ("scales", 2), ("qzeros", 1))}
+    for k, w in wide.items():
+        w[:, :m[k].size(1)] = m[k]
+    bias = (torch.randn(N, device="cuda") * 100).half()
+    with tuning(ext, tiled_max_m=0):
+        pg = PreparedGroup(ext, [{**m, "bias": bias}], K, 128, 0.0)
+        e = pg.arr[0]
+        for k, (ptr, ld) in {"qweight": ("qweight", "ldw_i32"), "scales": ("scales", "lds"), "qzeros": ("qzeros", "ldz_i32")}.items():
+            setattr(e, ptr, wide[k].data_ptr())
+            setattr(e, ld, wide[k].size(1))
+        (y,) = pg.run(x)
+        assert launched(ext, "words")
+    want = x.double() @ exact[0].t() + bias.double()
+    assert ((y.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2e-2).all()
+
+
+def test_replays_follow_rows_and_weights(ext):
+    """A recorded call on the canonical buffers: replays with new activations and after writes to the weights."""
+    M, K, Ns, rank = 12, 2048, [2048, 2048, 2048], 64
+    x, R, members, exact = make(5, M, K, Ns, rank)
+    pg = PreparedGroup(ext, members, K, 128, 1.0, R=R)
+    pg.run(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = pg.run(x)
+        r = pg.last_r
+    assert launched(ext, "words")
+    for seed in (6, 7, 8):
+        x2, R2, members2, exact2 = make(seed, M, K, Ns, rank)
+        x.copy_(x2), R.copy_(R2)
+        for a, b in zip(members, members2):
+            for k in ("qweight", "qzeros", "scales", "L"):
+                a[k].copy_(b[k])
+        graph.replay()
+        torch.cuda.synchronize()
+        check(y, x, r, exact2, members)
