@@ -257,8 +257,8 @@ int glowq_static_scratch_prepare(void);
  * eight token rows).
  */
 int glowq_w4a16_route(int M, int K, int N, int group_size, int ldw_i32);
-/* The same for a member that brings the tiled copy of its weights (glowq_pack_tiled): 8 = the matrix-core kernel that
- * streams the tiled copy: 33..64 token rows, and 5..32 where the group's codes are 40 MB and more (24 MB from 17 rows);
+/* The same for a member that brings the tiled copy of its weights (glowq_pack_tiled): 8 = the matrix-core kernels that
+ * read the tiled copy in unrounded arithmetic: 33..64 token rows, and 5..32 where the group's codes are 40 MB and more (24 MB from 17 rows);
  * "tiled_min_m" / "tiled_max_m" / "tiled_shape_rule" of glowq_set_tuning. */
 int glowq_w4a16_route_tiled(int M, int K, int N, int group_size, int ldw_i32);
 
