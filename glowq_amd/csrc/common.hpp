@@ -50,8 +50,7 @@ struct GroupDev {
   // 64-bit word per entry, and the number of polls a reader spends on one before it computes the entry itself
   unsigned long long* pub;
   unsigned pub_spin;
-  int pub_mute;
-  int pub_any_cost;
+  short pub_mute, pub_any_cost;  // (one word between them: `mem` stays where the kernels that take this struct read it fastest)
   MemberDev mem[GLOWQ_MAX_MEMBERS];
   int task_end[GLOWQ_MAX_MEMBERS];  // exclusive prefix of per-member task counts
   int wg_end[GLOWQ_MAX_MEMBERS];    // exclusive prefix of the workgroups assigned to each member
