@@ -23,6 +23,11 @@
 // are read from where those words' columns are staged, in the order the masks leave the codes.  A load instruction covers half a cache line of
 // sixteen rows, so the two halves are asked for together and without the non-temporal hint (18944 x 3584, 16 rows: 13.4, with it 14.2; asked
 // for half a step apart 15.9); scales and zero-points come for four super-blocks at a time (with two gathers a super-block 15.2).
+// From 9 rows on (kWhole) the activations stay whole, as in the rounding kernel of skinny.hip that has these rows otherwise: the masks of two neighbouring
+// words make one operand of the low nibbles and one of the high ones, with sums of their own (error of the output at |x| around 1e-4, against
+// x / 16 in fp16: 2.1e-4 / 2.0e-3; same matrix and vector instructions: 14336 x 4096 at 16 rows 12.8 us / 12.6, 1024 x 5120 9.2 / 9.5, 4096 x 14336
+// 19.5 / 19.7.  As code - zero, nine vector instructions a word instead of five: 13.4, 9.6, 20.2).  At 8 rows two sums cost 2 to 5 % more, and
+// the raw-code form of skinny.hip divides by 16 as well.
 // Launch without a correction, 8 and 16 rows, us, against the kernels of skinny.hip: 14336 x 4096 15.7, 16.9 -> 11.6, 12.5, 18944 x 3584
 // 17.9, 20.8 -> 12.5, 13.4, 1024 x 5120 8.9, 9.8 -> 8.2, 8.4, 4096 x 14336 15.3, 17.5 -> 14.8, 15.3, 8192 x 2048 6.3, 6.9 -> 5.3, 6.3.
 //
@@ -169,6 +174,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   static_assert(kPQ * 2 * kPW == kRows, "whole passes");
   constexpr bool kNarrow = kRows <= 16;          // tiles of 16 token rows by 16 columns
   static_assert(kNarrow || !kCanon, "the canonical buffers are read by the narrow tiles");
+  constexpr bool kWhole = kCanon && kRows > 8;   // activations are not divided by 16
   constexpr int kSigBytes = kNarrow ? 0 : kRows * 16;  // per 128-column half: a 16-byte fragment of sums per token row
   constexpr int kStage = kRows * kRowBytes + 2 * kSigBytes;
   constexpr int kLiveRegs = kRows >= 32 ? 16 : (kRows >= 16 ? 8 : 4);  // accumulator registers of rows that exist
@@ -291,6 +297,20 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       const h2 sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
 #pragma unroll
       for (int q = 0; q < kPQ; ++q) {
+        if constexpr (kWhole) {
+          // the pairs of columns that a mask leaves in the low bits of a byte, (0, 4) and (2, 6), of two neighbouring words, then those it leaves
+          // in the high bits, (1, 5) and (3, 7): a piece of the stage holds one kind; r as it is
+          const u32x4 v = av[q];
+          unsigned char* piece = dst + 2 * kPW * q * kRowBytes;
+          if (is_r) {
+            *reinterpret_cast<u32x4*>(piece) = v;
+          } else {
+            piece -= 8 * (pcol & 1);
+            *reinterpret_cast<u32x2*>(piece) = u32x2{__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x05040100u)};
+            *reinterpret_cast<u32x2*>(piece + 16) = u32x2{__builtin_amdgcn_perm(v.z, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
+          }
+          continue;
+        }
         if constexpr (kCanon) {
           // columns in the order the masks deliver the codes of a canonical word: (0, 4), (1, 5) / 16, (2, 6), (3, 7) / 16; r as it is
           const u32x4 v = av[q];
@@ -578,10 +598,10 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         spread(side.x, side.x, sw[0][0], sw[0][1]);
         spread(side.y, side.y, sw[1][0], sw[1][1]);
       }
-      // the pairs a mask leaves at code * 2^-20 are staged divided by 16
+      // the pairs a mask leaves at code * 2^-20 are staged divided by 16 (but kWhole)
       const h2 one = {(half_t)1.f, (half_t)1.f}, sixteen = {(half_t)16.f, (half_t)16.f};
       const uint32_t o1 = __builtin_bit_cast(uint32_t, one), o16 = __builtin_bit_cast(uint32_t, sixteen);
-      const h8 ones = __builtin_bit_cast(h8, u32x4{o1, o16, o1, o16});
+      const h8 ones = __builtin_bit_cast(h8, u32x4{o1, kWhole ? o1 : o16, o1, kWhole ? o1 : o16});
       // all fragments of the step are asked for at once: one LDS round trip for it instead of eight
       const unsigned char* xs = st + nrow_off + (kCanon ? 64 * nq : 128 * (nq >> 1) + 16 * (nq & 1));
       h8 af[8];
@@ -591,6 +611,33 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
       for (int gh = 0; gh < 2; ++gh) {
         f4 pg[2] = {}, sx = {};
+        if constexpr (kWhole) {
+          // codes * 2^-24 and codes * 2^-20 into sums of their own, so that the activations stay whole
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            f4 pl = {}, ph = {};
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+              const uint32_t wa = b.w[2 * gh + c][j], wb = b.w[2 * gh + c][j + 1], ha = wa >> 8, hb = wb >> 8;
+              const h8 lo = __builtin_bit_cast(h8, u32x4{wa & 0x000F000Fu, ha & 0x000F000Fu, wb & 0x000F000Fu, hb & 0x000F000Fu});
+              const h8 hi = __builtin_bit_cast(h8, u32x4{wa & 0x00F000F0u, ha & 0x00F000F0u, wb & 0x00F000F0u, hb & 0x00F000F0u});
+              pl = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j], lo, pl, 0, 0, 0);
+              ph = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j + 1], hi, ph, 0, 0, 0);
+              if (c == 0) {
+                sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j], ones, sx, 0, 0, 0);
+                sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * gh + j + 1], ones, sx, 0, 0, 0);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const float sf = (float)__builtin_bit_cast(half_t, (uint16_t)(sw[gh][c] & 0xFFFFu)) * 0x1p24f;
+            const float nz = (float)((now.z0[c] >> (8 * d + 4 * gh)) & 15u) * -0x1p-24f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) nacc[c][i] = __builtin_fmaf(sf, __builtin_fmaf(nz, sx[i], __builtin_fmaf(0.0625f, ph[i], pl[i])), nacc[c][i]);
+          }
+          if constexpr (kRefill)
+            if (gh == 1) request(b, sb_next);  // (both halves of a cache line together)
+          continue;
+        }
         if constexpr (kCanon) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {

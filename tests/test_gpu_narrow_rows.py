@@ -132,3 +132,30 @@ def test_replays_follow_rows_and_weights(ext):
         graph.replay()
         torch.cuda.synchronize()
         check(y, x, r, exact2, members)
+
+
+@pytest.mark.parametrize("std", [1e-4, 3e-5])
+@pytest.mark.parametrize("K,Ns,rank", [(4096, [300], 0), (2816, [3000, 40], 40)])
+@pytest.mark.parametrize("M", [5, 8, 9, 16])
+def test_small_activations(ext, form, M, K, Ns, rank, std):
+    """Activations far below 2^-10 keep their bits on the canonical buffers from 9 rows on, where the rounding kernel has the other groups.  The tiled
+    copy and fewer rows take half of the columns as x / 16, in fp16 multiples of 2^-24: an error of at most 2^-21 in x, evenly spread."""
+    x, R, members, exact = make(M + K, M, K, Ns, rank)
+    x = (x.float() * (std / 64)).half()
+    for m in members:  # outputs of order one
+        m["scales"] *= 2048
+    exact = [2048 * w for w in exact]
+    if rank:
+        R *= 2048
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if rank else 0.0, R=R)
+    y = pg.run(x)
+    assert launched(ext, form), ext.last_launch()
+    of_x = 2.0 ** -20 / 24 ** 0.5 / std if form == "tiled" or M <= 8 else 0.0
+    for got, w, m in zip(y, exact, members):
+        want = x.double() @ w.t()
+        if m["L"] is not None:
+            want = want + pg.last_r.double() @ m["L"].double().t()
+        # the output's own rounding: at most 2^-11 of a value and 0.29 / 0.5 of that in the mean.  Both norms of the rest hang on the sums of the
+        # K / 128 groups of a row (a weight's mean over its group is as large as its spread): 110 of them in the smallest case, 7 % of
+        # deviation each, 10 % of the ratio; four deviations
+        assert (got.double() - want).norm() <= (3.2e-4 ** 2 + (1.4 * of_x) ** 2) ** 0.5 * want.norm()
