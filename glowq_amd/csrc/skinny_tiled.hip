@@ -26,8 +26,9 @@
 // From 9 rows on (kWhole) the activations stay whole, as in the rounding kernel of skinny.hip that has these rows otherwise: the masks of two neighbouring
 // words make one operand of the low nibbles and one of the high ones, with sums of their own (error of the output at |x| around 1e-4, against
 // x / 16 in fp16: 2.1e-4 / 2.0e-3; same matrix and vector instructions: 14336 x 4096 at 16 rows 12.8 us / 12.6, 1024 x 5120 9.2 / 9.5, 4096 x 14336
-// 19.5 / 19.7.  As code - zero, nine vector instructions a word instead of five: 13.4, 9.6, 20.2).  At 8 rows two sums cost 2 to 5 % more, and
-// the raw-code form of skinny.hip divides by 16 as well.
+// 19.5 / 19.7.  As code - zero, nine vector instructions a word instead of five: 13.4, 9.6, 20.2), and sums that are not finite are taken again
+// with code - zero, which gives an infinite activation's products their signs.  At 8 rows two sums cost 2 to 5 % more, and the
+// raw-code form of skinny.hip divides by 16 as well.
 // Launch without a correction, 8 and 16 rows, us, against the kernels of skinny.hip: 14336 x 4096 15.7, 16.9 -> 11.6, 12.5, 18944 x 3584
 // 17.9, 20.8 -> 12.5, 13.4, 1024 x 5120 8.9, 9.8 -> 8.2, 8.4, 4096 x 14336 15.3, 17.5 -> 14.8, 15.3, 8192 x 2048 6.3, 6.9 -> 5.3, 6.3.
 //
@@ -66,6 +67,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "dequant.hpp"
 #include "handover.hpp"
 #include "proj_block.hpp"
 #include "tiled.hpp"
@@ -753,6 +755,46 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   step(sb + 1, integral_constant<int, 1>{}, std::true_type{});
   step(sb + 2, integral_constant<int, 2>{}, std::true_type{});
   step(sb + 3, integral_constant<int, 3>{}, std::true_type{});
+
+  // kWhole, a sum that is not finite: an infinite activation makes infinities of both signs of sum code * x and -zero * sum x, and no number of
+  // their sum.  The wave walks its part of K again with code - zero as the operand, whose products have the signs they should have
+  // (words and activations straight from memory: such a call has worse things than this walk to wait for).
+  if constexpr (kWhole) {
+    float size = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) size += __builtin_fabsf(nacc[i >> 2][i & 3]);
+    if (live && __builtin_amdgcn_ballot_w64(!(size < __builtin_inff())) != 0) {
+      const half_t* xr = x + (size_t)min(lane & 15, M - 1) * K + 32 * nq;
+      nacc[0] = nacc[1] = f4{};
+#pragma unroll 1
+      for (int again = sb0; again < sb1; ++again) {
+        BSet b;
+        request(b, again);
+#pragma unroll 1
+        for (int gh = 0; gh < 2; ++gh) {
+          const int grp = 2 * again + gh;
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const size_t row = crow0 + min(16 * c + c_row, crows - 1);
+            const uint32_t z = nibble((uint32_t)g.mem[mi].qzeros[row * ldz + (grp >> 3)], grp & 7);
+            const h2 zb_lo = bitcast_u32<h2>(z * 0x00010001u + 0xE400E400u), zb_hi = bitcast_u32<h2>(z * 0x00100010u + 0xD400D400u);
+            f4 sum = {};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const u32x4 v = *reinterpret_cast<const u32x4*>(xr + again * 256 + gh * 128 + 8 * j);
+              const u32x4 o = {__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
+                               __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
+              const uint32_t wd = gh == 0 ? b.w[c][j] : b.w[2 + c][j];
+              sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, o), dequant_word<false>(wd, zb_lo, zb_hi, h2{}), sum, 0, 0, 0);
+            }
+            const float sc = (float)g.mem[mi].scales[row * lds + grp];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) nacc[c][i] = __builtin_fmaf(sc, sum[i], nacc[c][i]);
+          }
+        }
+      }
+    }
+  }
 
   // ---- the correction: set q holds block q of the tiled left factor (B fragments of its four k-steps as they are),
   // stage 0 the first 256 columns of r.  Ranks above 256 take further passes, each with its loads in the open.  K groups

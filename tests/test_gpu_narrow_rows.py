@@ -159,3 +159,24 @@ def test_small_activations(ext, form, M, K, Ns, rank, std):
         # K / 128 groups of a row (a weight's mean over its group is as large as its spread): 110 of them in the smallest case, 7 % of
         # deviation each, 10 % of the ratio; four deviations
         assert (got.double() - want).norm() <= (3.2e-4 ** 2 + (1.4 * of_x) ** 2) ** 0.5 * want.norm()
+
+
+@pytest.mark.parametrize("K,Ns,rank", [(4096, [300], 0), (2816, [3000, 40], 40)])
+@pytest.mark.parametrize("M", [9, 16])
+def test_an_infinite_activation_keeps_its_sign(ext, M, K, Ns, rank):
+    """On the canonical buffers from 9 rows on an infinite activation makes outputs of the sign of its weight, and no number where that is zero."""
+    x, R, members, exact = make(M + K, M, K, Ns, rank)
+    x[1, 5], x[M - 1, K - 3] = float("inf"), float("-inf")
+    with tuning(ext, tiled_max_m=0):
+        for m in members:
+            m["L"] = None  # (r of these rows is infinite or no number, whatever the weights are)
+        pg = PreparedGroup(ext, members, K, 128, 0.0)
+        y = pg.run(x)
+        assert launched(ext, "words"), ext.last_launch()
+    for got, w in zip(y, exact):
+        want = torch.where(torch.isfinite(x), x, 0).double() @ w.t()
+        for row, col in ((1, 5), (M - 1, K - 3)):
+            want[row] = x[row, col].double() * w[:, col]
+        finite = torch.isfinite(want)
+        assert torch.equal(got.double()[~finite].nan_to_num(nan=1.0), want[~finite].nan_to_num(nan=1.0))
+        assert ((got.double() - want)[finite].abs() <= 2.0 ** -11 * want[finite].abs() + 2e-2).all()
