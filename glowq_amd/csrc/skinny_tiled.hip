@@ -469,7 +469,9 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   const int ldw = kCanon ? g.mem[mi].ldw : 0, lds = kCanon ? g.mem[mi].lds : 0, ldz = kCanon ? g.mem[mi].ldz : 0;
   const int crows = live ? min(32, mem_N - rb * 32) : 0;  // kCanon: rows of the block that exist
   const size_t crow0 = (size_t)(live ? rb : 0) * 32;
-  const __amdgpu_buffer_rsrc_t rs_w = kCanon ? rsrc(wt + crow0 * ldw * 4, (size_t)crows * ldw * 4)
+  // kCanon: the last row may be the end of its buffer whatever the stride (a member cut from a wider one), and requests run past K
+  const auto span = [&](size_t ld, int used) { return crows > 0 ? (size_t)(crows - 1) * ld + used : 0; };
+  const __amdgpu_buffer_rsrc_t rs_w = kCanon ? rsrc(wt + crow0 * ldw * 4, span(ldw, K / 8) * 4)
                                              : rsrc(wt + (size_t)(live ? rb : 0) * tiled::kChunk, live && sb1 > 0 ? (size_t)(sb1 - 1) * chunk_stride + tiled::kChunk : 0);
   const int b_off = lane * 16;
 
@@ -478,8 +480,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     u32x2 side;  // the lane's column: (scale | -zero * 2^-16) of the two halves (kCanon: from `turn`)
   };
   BSet bs[kD];
-  const __amdgpu_buffer_rsrc_t rs_s = rsrc(kCanon ? (const void*)(g.mem[mi].scales + crow0 * lds) : (const void*)wt, kCanon ? (size_t)crows * lds * 2 : 0);
-  const __amdgpu_buffer_rsrc_t rs_z = rsrc(kCanon ? (const void*)(g.mem[mi].qzeros + crow0 * ldz) : (const void*)wt, kCanon ? (size_t)crows * ldz * 4 : 0);
+  const __amdgpu_buffer_rsrc_t rs_s = rsrc(kCanon ? (const void*)(g.mem[mi].scales + crow0 * lds) : (const void*)wt, kCanon ? span(lds, 2 * SB) * 2 : 0);
+  const __amdgpu_buffer_rsrc_t rs_z = rsrc(kCanon ? (const void*)(g.mem[mi].qzeros + crow0 * ldz) : (const void*)wt, kCanon ? span(ldz, (2 * SB + 7) / 8) * 4 : 0);
   const int c_row = lane & 15;
   int w_at[2], s_at[2], z_at[2];
 #pragma unroll
@@ -1028,6 +1030,7 @@ bool skinny_words_supported(const GroupDev& g) {
     const MemberDev& m = g.mem[i];
     if ((reinterpret_cast<uintptr_t>(m.qweight) & 15u) != 0 || (m.ldw & 3) != 0 || m.ldw < g.K / 8 || (size_t)m.ldw * 128 >= (1ull << 31)) return false;
     if ((reinterpret_cast<uintptr_t>(m.scales) & 3u) != 0 || (m.lds & 1) != 0 || (reinterpret_cast<uintptr_t>(m.qzeros) & 3u) != 0) return false;
+    if ((size_t)m.lds * 64 >= (1ull << 31) || (size_t)m.ldz * 128 >= (1ull << 31)) return false;
     if (m.L != nullptr && r != nullptr && (reinterpret_cast<uintptr_t>(m.L) & 15u) != 0) return false;
   }
   return true;

@@ -91,20 +91,25 @@ def test_rows_that_are_not_finite_stay_by_themselves(ext, form, K, Ns, rank, bad
     check([o[fine] for o in y], xs, r, exact, members)
 
 
-def test_strided_buffers_and_bias(ext):
-    """Members inside wider buffers (row strides above the shape's) on the canonical form, with a bias."""
-    M, K, N = 11, 1280, 2600
+@pytest.mark.parametrize("at_end", [False, True])
+@pytest.mark.parametrize("M", [5, 11])
+def test_strided_buffers_and_bias(ext, M, at_end):
+    """Members inside wider buffers (row strides above the shape's) on the canonical form, with a bias: the first columns of a buffer, and the
+    last ones, so that nothing lies behind the last row."""
+    K, N = 1280, 2600
     x, _, (m,), exact = make(3, M, K, [N], 0)
-    wide = {k: torch.full((N, m[k].size(1) + pad), 7, dtype=m[k].dtype, device="cuda") for k, pad in (("qweight", 4), ("scales", 2), ("qzeros", 1))}
-    for k, w in wide.items():
-        w[:, :m[k].size(1)] = m[k]
+    wide = {}
+    for k, pad in (("qweight", 4), ("scales", 2), ("qzeros", 1)):
+        whole = torch.full((N, m[k].size(1) + pad), 7, dtype=m[k].dtype, device="cuda")
+        wide[k] = whole[:, pad:] if at_end else whole[:, :m[k].size(1)]
+        wide[k].copy_(m[k])
     bias = (torch.randn(N, device="cuda") * 100).half()
     with tuning(ext, tiled_max_m=0):
         pg = PreparedGroup(ext, [{**m, "bias": bias}], K, 128, 0.0)
         e = pg.arr[0]
         for k, (ptr, ld) in {"qweight": ("qweight", "ldw_i32"), "scales": ("scales", "lds"), "qzeros": ("qzeros", "ldz_i32")}.items():
             setattr(e, ptr, wide[k].data_ptr())
-            setattr(e, ld, wide[k].size(1))
+            setattr(e, ld, wide[k].stride(0))
         (y,) = pg.run(x)
         assert launched(ext, "words")
     want = x.double() @ exact[0].t() + bias.double()
