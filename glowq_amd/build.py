@@ -12,6 +12,8 @@ import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
 
+from . import isa_lint
+
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libglowq_w4a16.so")
@@ -47,6 +49,10 @@ def _hipcc() -> str:
 NO_SCRATCH = {"gemv_stream.hip": "gemv_stream_kernel", "gemv_chain.hip": "gemv_stream_kernel",
               "gemv_qstream.hip": "gemv_qstream_kernel"}
 
+# Sources whose kernels wait for their direct-to-LDS loads by the number of loads requested behind them: in the assembly that
+# order has to be the source's (isa_lint.py).
+COUNTED_WAITS = {"gemm.hip": "gemm_tiled_kernel"}
+
 
 def _check_no_scratch(src: str, kernel: str, remarks: str) -> None:
     name = None
@@ -60,10 +66,8 @@ def _check_no_scratch(src: str, kernel: str, remarks: str) -> None:
                                    "must stay in registers")
 
 
-def _check_in_flight_registers(src: str, kernel: str, asm_dir: str) -> None:
-    """The device assembly the compile left in `asm_dir` through the lint of isa_lint.py."""
-    from .isa_lint import lint
-
+def _check_assembly(src: str, kernel: str, asm_dir: str, lint, claim: str) -> None:
+    """The device assembly the compile left in `asm_dir` through a check of isa_lint.py."""
     stem = os.path.splitext(src)[0]
     listings = [f for f in os.listdir(asm_dir) if f.startswith(stem + "-hip-amdgcn") and f.endswith(".s")]
     if not listings:
@@ -72,8 +76,7 @@ def _check_in_flight_registers(src: str, kernel: str, asm_dir: str) -> None:
         with open(os.path.join(asm_dir, f)) as fh:
             found = lint(fh.read(), kernel)
         if found:
-            raise RuntimeError(f"{src}: registers of loads in flight are touched before their wait "
-                               f"({len(found)} places), first:\n  " + "\n  ".join(found[:3]))
+            raise RuntimeError(f"{src}: {claim} ({len(found)} places), first:\n  " + "\n  ".join(found[:3]))
 
 
 def _compile(src: str, obj_dir: str, extra) -> str:
@@ -81,12 +84,13 @@ def _compile(src: str, obj_dir: str, extra) -> str:
     cmd = [_hipcc(), *HIPCC_FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     if src in NO_SCRATCH:
         cmd.insert(1, "-Rpass-analysis=kernel-resource-usage")
+    if src in NO_SCRATCH or src in COUNTED_WAITS:
         cmd.insert(1, "-save-temps=obj")  # keeps the device assembly beside the object
     res = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     if src in NO_SCRATCH and res.returncode == 0:
         _check_no_scratch(src, NO_SCRATCH[src], res.stderr)
-        _check_in_flight_registers(src, NO_SCRATCH[src], obj_dir)
+        _check_assembly(src, NO_SCRATCH[src], obj_dir, isa_lint.lint, "registers of loads in flight are touched before their wait")
         kept, skip = [], 0
         for l in res.stderr.splitlines():  # a remark is its own line plus the source line and the caret under it
             if "-Rpass-analysis=kernel-resource-usage" in l:
@@ -96,6 +100,8 @@ def _compile(src: str, obj_dir: str, extra) -> str:
             elif "remarks generated" not in l and not l.startswith("In file included from"):
                 kept.append(l)
         res.stderr = "\n".join(kept)
+    if src in COUNTED_WAITS and res.returncode == 0:
+        _check_assembly(src, COUNTED_WAITS[src], obj_dir, isa_lint.counted_waits, "waits leave loads to LDS in flight")
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src}:\n{err}")

@@ -710,6 +710,8 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   // they are written: left alone, the compiler sinks the refills to the end of the half-step, where nothing hides them.
   auto wait_loads_but = [&](auto n_const) __attribute__((always_inline)) {
     constexpr int n = decltype(n_const)::value;
+    // (a comment in the assembly: the build checks that the n loads in front of it are none of those that go to LDS, isa_lint.py)
+    asm volatile("; loads to LDS are followed by %0 others" ::"n"(n));
     __builtin_amdgcn_s_waitcnt((n & 15) | 0x0F70 | ((n >> 4) << 14));  // vmcnt(n), nothing else
   };
 
@@ -749,6 +751,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   load_w(b[0], sb0, 0);
   load_w(b[0], sb0, 1);
   load_x(2 * sb0, 0);
+  __builtin_amdgcn_sched_barrier(0);
   load_w(b[0], sb0, 2);
   load_w(b[0], sb0, 3);
   __builtin_amdgcn_sched_barrier(0);
@@ -781,9 +784,10 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   h8 bf[kNT];                    // the next word, dequantised
 #pragma unroll
   for (int tn = 0; tn < kNT; ++tn) bf[tn] = dequant_word<!kExact>(b[0].w[tn][0][0], zero.lo[tn], zero.hi[tn], zero.s[tn]);
-  // d (the set that holds super-block sb) and g are compile-time constants at every call site
-  auto half_step = [&](int sb, auto d_const, auto g_const) __attribute__((always_inline)) {
+  // d (the set that holds super-block sb), g and whether another super-block follows are compile-time constants at every call site
+  auto half_step = [&](int sb, auto d_const, auto g_const, auto more_const) __attribute__((always_inline)) {
     constexpr int d = decltype(d_const)::value, g = decltype(g_const)::value;
+    constexpr bool kMore = decltype(more_const)::value;
     const BSet& cur = b[d];
     BSet& nxt = b[d ^ 1];
     f16v half_sum[kExact ? kMT : 1][kExact ? kNT : 1];
@@ -791,12 +795,13 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
     h8 af[kMT];
 #pragma unroll
     for (int u = 0; u < kMT; ++u) af[u] = read_a(stage, u, 8 * lh);
-    load_x(2 * sb + g + 1, stage ^ 1);
-    if (g == 0) load_side(nxt, sb + 1);
+    if (g == 0 || kMore) load_x(2 * sb + g + 1, stage ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (g == 0 && kMore) load_side(nxt, sb + 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      if ((t & 3) == 0) {
+      if ((t & 3) == 0 && kMore) {
         load_w(nxt, sb + 1, 2 * g + t / 4);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -810,10 +815,10 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
 #pragma unroll
           for (int tn = 0; tn < kNT; ++tn) scale[tn] = zero.scale[tn];
         }
-        zero = zero_of(g == 0 ? cur : nxt, g ^ 1);
+        if (g == 0 || kMore) zero = zero_of(g == 0 ? cur : nxt, g ^ 1);
       }
 #pragma unroll
-      for (int tn = 0; tn < kNT; ++tn) {
+      for (int tn = 0; tn < (t < 7 || g == 0 || kMore ? kNT : 0); ++tn) {
         const uint32_t w = t < 7 ? cur.w[tn][2 * g + (t + 1) / 4][(t + 1) & 3] : (g == 0 ? cur.w[tn][2][0] : nxt.w[tn][0][0]);
         bn_[tn] = dequant_word<!kExact>(w, zero.lo[tn], zero.hi[tn], zero.s[tn]);
       }
@@ -840,21 +845,22 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
           for (int e = 0; e < 16; ++e) acc[u][tn][e] = __builtin_fmaf(scale[tn], half_sum[u][tn][e], acc[u][tn][e]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    wait_loads_but(std::integral_constant<int, 2 * kNT + (g == 0 ? kNT : 0)>{});
+    wait_loads_but(std::integral_constant<int, kMore ? 2 * kNT + (g == 0 ? kNT : 0) : 0>{});
     __syncthreads();
     stage ^= 1;
   };
-  auto super_block = [&](int sb, auto d_const) __attribute__((always_inline)) {
-    half_step(sb, d_const, std::integral_constant<int, 0>{});
-    half_step(sb, d_const, std::integral_constant<int, 1>{});
+  auto super_block = [&](int sb, auto d_const, auto more_const) __attribute__((always_inline)) {
+    half_step(sb, d_const, std::integral_constant<int, 0>{}, more_const);
+    half_step(sb, d_const, std::integral_constant<int, 1>{}, more_const);
   };
 
   int sb = sb0;
   for (; sb + 1 < sb_end; sb += 2) {
-    super_block(sb, std::integral_constant<int, 0>{});
-    super_block(sb + 1, std::integral_constant<int, 1>{});
+    super_block(sb, std::integral_constant<int, 0>{}, std::true_type{});
+    super_block(sb + 1, std::integral_constant<int, 1>{}, std::true_type{});
   }
-  if (sb < sb_end) super_block(sb, std::integral_constant<int, 0>{});
+  // (nothing uses what an odd last one would request: the compiler drops those loads, and a count of them would leave the activations in flight)
+  if (sb < sb_end) super_block(sb, std::integral_constant<int, 0>{}, std::false_type{});
   // requests past the end that are still on their way into the stages have to land before the stages are used for anything else
   wait_loads_but(std::integral_constant<int, 0>{});
 
@@ -874,6 +880,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
       __syncthreads();  // the fragment reads of the stage are done
       if (have_r) load_r(st, 0);  // (each wave's own affair: what it fetches or computes is its rows of the stage)
       else compute_r(st, 0);
+      __builtin_amdgcn_sched_barrier(0);  // (the wait below counts the loads of the left factor behind those of r)
       u32x4 lf[8];
 #pragma unroll
       for (int tn = 0; tn < kNT; ++tn) {
@@ -883,6 +890,7 @@ void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
           for (int t = 0; t < 4; ++t)
             lf[4 * q + t] = __builtin_amdgcn_raw_buffer_load_b128(rs_l, w_lane + t * 1024, 2 * st + q < LB ? (int)((uint32_t)(rb[tn] * LB + 2 * st + q) * (uint32_t)tiled::kLChunk) : (int)kPast, 0);
         if (tn == 0) {
+          __builtin_amdgcn_sched_barrier(0);
           wait_loads_but(std::integral_constant<int, 8>{});
           __syncthreads();
         }

@@ -79,6 +79,34 @@ def lint(asm: str, kernel_substring: str) -> List[str]:
     return problems
 
 
+_COUNTED = re.compile(r"^\s*; loads to LDS are followed by (\d+) others")
+_VMEM = re.compile(r"^\s*(?:global|buffer|flat)_(?:load|store|atomic)_\w+")
+
+
+def counted_waits(asm: str, kernel_substring: str) -> List[str]:
+    """Waits that leave a load to LDS in flight, in the kernels of `asm` whose symbol contains `kernel_substring`.
+
+    In front of a hand-counted wait the source leaves the comment "loads to LDS are followed by n others" (gemm.hip): the last n
+    vector-memory instructions before it, in its own straight line, have to be loads to registers, whatever order the compiler gave them."""
+    problems: List[str] = []
+    name, recent = None, []
+    for i, raw in enumerate(asm.splitlines()):
+        label = _LABEL.match(raw)
+        if label:
+            if not raw.startswith("."):
+                name = label.group(1)
+            recent = []
+        elif (m := _COUNTED.match(raw)) and name and kernel_substring in name:
+            n = int(m.group(1))
+            behind = recent[len(recent) - n:] if n else []
+            if len(behind) < n or any(behind):
+                problems.append(f"{name}: line {i + 1}: {n} loads are counted behind the ones to LDS, but the last ones are "
+                                + "".join("L" if to_lds else "r" for to_lds in recent[-16:]) + " (L: to LDS, r: to registers)")
+        elif _VMEM.match(raw):
+            recent.append(raw.split(";")[0].rstrip().endswith(" lds"))
+    return problems
+
+
 if __name__ == "__main__":
     import sys
 
