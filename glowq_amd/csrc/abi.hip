@@ -300,6 +300,23 @@ std::atomic<int> g_skinny_codes_max_m{clampi(env_or("GLOWQ_SKINNY_CODES_M", 8), 
 
 int pick_route_rounded(const GroupDev& g, int force);
 
+//   words_max_m     token rows (5..16) up to which groups of the skinny routes run on the narrow tiles over the canonical buffers
+//                   (skinny_tiled.hip), in unrounded arithmetic, where that pays (GLOWQ_WORDS_M); 0, or 0 for skinny_codes_max_m: the kernels
+//                   of skinny.hip.  Reported as the raw-code route, whose arithmetic it is.
+// It pays for all groups without an r to compute, and for the others where K is short or the stream long enough that r, which the skinny
+// kernels take along for fewer columns, costs them a launch or a part of the chip.  Group call, us at 8 and 16 rows, this / the skinny kernels: without a
+// correction 4096 x 4096 7.2, 8.1 / 7.5, 8.2, 3 x 2048 x 2048 5.6, 6.0 / 6.1, 6.5, 5120 x 5120 9.3, 10.4 / 9.7, 10.8, 18944 x 3584 12.5, 13.4 /
+// 17.9, 20.8; with one 2 x 9472 x 2816 12.8, 13.3 / 17.8, 20.4, 8192 x 2048 7.7, 8.1 / 8.9, 9.4; not q|k|v of an 8B and a 14B layer 9.7, 10.7 /
+// 9.8, 10.2 and 15.7, 17.1 / 14.9, 16.3, nor 4096 x 14336 19.6, 20.9 / 17.7, 19.9.
+std::atomic<int> g_words_max_m{clampi(env_or("GLOWQ_WORDS_M", 16), 0, 16)};
+bool words_pay(const GroupDev& g, bool computes_r) {
+  if (g.M > g_words_max_m.load(std::memory_order_relaxed) || g_skinny_codes_max_m.load(std::memory_order_relaxed) == 0 || !skinny_words_supported(g)) return false;
+  if (!computes_r) return true;
+  long rows = 0;
+  for (int i = 0; i < g.n_members; ++i) rows += g.mem[i].N;
+  return rows > 2048 && (g.K <= 3072 || (g.K <= 6144 && rows * (long)g.K / 2 >= 25L * 1000 * 1000));
+}
+
 //   tiled_min_m / tiled_max_m  token rows served by the matrix-core kernel that reads the tiled copy of the weights, where
 //                   every member of the group brings one (GLOWQ_TILED_MIN_M, GLOWQ_TILED_MAX_M; max 0 switches it off)
 std::atomic<int> g_tiled_min_m{clampi(env_or("GLOWQ_TILED_MIN_M", 2), 1, 64)};
@@ -375,14 +392,16 @@ bool gemm_proj_in_launch(const GroupDev& g) {
   return any_left;  // (the launcher still turns down calls without the tiled copy and those it would not pay for)
 }
 
-int pick_route(const GroupDev& g, int force) {
+int pick_route(const GroupDev& g, int force, bool computes_r) {
   if (force < 0 && g.M >= g_tiled_min_m.load(std::memory_order_relaxed) && g.M <= g_tiled_max_m.load(std::memory_order_relaxed) &&
       skinny_tiled_supported(g) && tiled_pays(g))
     return kRouteSkinnyTiled;
   const int route = pick_route_rounded(g, force);
-  if (route == kRouteSkinny && force < 0 && g.M <= g_skinny_codes_max_m.load(std::memory_order_relaxed) && skinny_raw_form(g)) return kRouteSkinnyRaw;
+  if (route == kRouteSkinny && force < 0 && ((g.M <= g_skinny_codes_max_m.load(std::memory_order_relaxed) && skinny_raw_form(g)) || words_pay(g, computes_r)))
+    return kRouteSkinnyRaw;
   return route;
 }
+int pick_route(const GroupDev& g, int force) { return pick_route(g, force, g.R != nullptr); }
 
 int pick_route_rounded(const GroupDev& g, int force) {
   if (!fast_layout(g)) return kRouteGeneric;
@@ -415,8 +434,6 @@ int pick_route_rounded(const GroupDev& g, int force) {
   return kRouteGeneric;
 }
 
-// Runs one group through the chosen route.  Routes with a row capacity smaller than M walk the
-// token rows in chunks (weights are re-read once per chunk).
 // Calls of the route on the tiled copy that run on the GEMM in its unrounded form: all of 33 to 64 rows, and from 17 rows on groups with
 // an r to compute whose 128-column tiles come to between half and all of the compute units (K of 2048 columns and more; without r 2 x 14336 x
 // 4096 at 32 rows 21.9 / 18.5).  us with the projection, 24 and 32 rows, GEMM / the kernel of skinny_tiled.hip: 8B gate|up (224 tiles)
@@ -430,19 +447,8 @@ bool tiled_route_on_gemm(const GroupDev& g) {
   return g.M > 16 && g.R != nullptr && g.K >= 2048 && tiles * 2 > num_cus() && tiles <= num_cus();
 }
 
-// Groups of the skinny routes whose 5 to 16 token rows run on the narrow tiles over the canonical buffers (skinny_tiled.hip): all without an r to
-// compute, the others where K is short or the stream long enough that r, which the skinny kernels take along for fewer columns, costs them a
-// launch or a part of the chip.  Group call, us at 8 and 16 rows, this / the skinny kernels: without a
-// correction 4096 x 4096 7.2, 8.1 / 7.5, 8.2, 3 x 2048 x 2048 5.6, 6.0 / 6.1, 6.5, 5120 x 5120 9.3, 10.4 / 9.7, 10.8, 18944 x 3584 12.5, 13.4 /
-// 17.9, 20.8; with one 2 x 9472 x 2816 12.8, 13.3 / 17.8, 20.4, 8192 x 2048 7.7, 8.1 / 8.9, 9.4; not q|k|v of an 8B and a 14B layer 9.7, 10.7 /
-// 9.8, 10.2 and 15.7, 17.1 / 14.9, 16.3, nor 4096 x 14336 19.6, 20.9 / 17.7, 19.9.
-bool words_pay(const GroupDev& g) {
-  long rows = 0;
-  for (int i = 0; i < g.n_members; ++i) rows += g.mem[i].N;
-  if (g.R == nullptr) return true;
-  return rows > 2048 && (g.K <= 3072 || (g.K <= 6144 && rows * (long)g.K / 2 >= 25L * 1000 * 1000));
-}
-
+// Runs one group through the chosen route.  Routes with a row capacity smaller than M walk the
+// token rows in chunks (weights are re-read once per chunk).
 int run_group(GroupDev g, int route, hipStream_t stream) {
   for (int i = 0; i < g.n_members; ++i)
     if (g.mem[i].y32 && !(route == kRouteGemm && gemm_widens(g))) return fail(GLOWQ_EUNSUPPORTED, "fp32 outputs: only where the GEMM on the tiled weights takes the call, and for all members alike");
@@ -488,7 +494,7 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
     g.pub = nullptr;
   }
   const bool skinny_route = route == kRouteSkinny || route == kRouteSkinnyRaw;
-  const bool on_words = skinny_route && skinny_words_supported(g) && words_pay(g);
+  const bool on_words = route == kRouteSkinnyRaw && words_pay(g, g.R != nullptr);
   if (g.R != nullptr && ((route == kRouteStream && proj_in_launch(g)) || ((skinny_route || (route == kRouteSkinnyTiled && !on_gemm)) && skinny_proj_in_launch(g)) ||
                          ((route == kRouteGemm || on_gemm) && gemm_proj_in_launch(g)))) {
     // single token on the stream GEMV, a handful of rows on the skinny kernel: workgroups in front of the group launch
@@ -532,7 +538,7 @@ int run_group(GroupDev g, int route, hipStream_t stream) {
       e = launch();
     }
   } else if (skinny_route) {
-    const auto launch = [&]() { return on_words ? launch_skinny_tiled(g, cus, stream, true) : launch_skinny(g, cus, stream, route == kRouteSkinnyRaw); };
+    const auto launch = [&]() { return on_words ? launch_skinny_tiled(g, cus, stream, true) : launch_skinny(g, cus, stream, route == kRouteSkinnyRaw && skinny_raw_form(g)); };
     e = launch();
     if (e == hipErrorNotReady && g.pub != nullptr) {
       e = launch_projection();
@@ -918,7 +924,7 @@ static int route_query(int M, int K, int N, int group_size, int ldw_i32, bool wi
   g.mem[0].N = N;
   g.mem[0].ldw = ldw_i32;
   if (with_tiled && tiled::applies(K, group_size)) g.mem[0].tiled = reinterpret_cast<const void*>(uintptr_t{16});  // never read
-  return pick_route(g, -1);
+  return pick_route(g, -1, true);
 }
 
 int glowq_w4a16_route(int M, int K, int N, int group_size, int ldw_i32) { return route_query(M, K, N, group_size, ldw_i32, false); }
@@ -962,6 +968,7 @@ int glowq_set_tuning(const char* key, int value) {
   else if (strcmp(key, "qstream_max_m") == 0) { slot = &g_qstream_max_m; hi = 4; }
   else if (strcmp(key, "qstream_shape_rule") == 0) { slot = &g_qstream_shape_rule; hi = 1; }
   else if (strcmp(key, "skinny_codes_max_m") == 0) { slot = &g_skinny_codes_max_m; hi = 64; }
+  else if (strcmp(key, "words_max_m") == 0) { slot = &g_words_max_m; }
   else if (strcmp(key, "stream_shape_rule") == 0) { slot = &g_stream_shape_rule; hi = 1; }
   else if (strcmp(key, "tiled_min_m") == 0) { slot = &g_tiled_min_m; lo = 1; hi = 64; }
   else if (strcmp(key, "tiled_max_m") == 0) { slot = &g_tiled_max_m; hi = 64; }

@@ -723,7 +723,7 @@ class W4A16Extension:
     def set_tuning(self, key: str, value: int) -> int:
         """Sets a route limit of the process ("quad_max_m", "quad_min_m", "wave_dot_max_m", "skinny_max_m",
         "small_group_mb", "stream_max_m", "stream_shape_rule", "qstream_max_m", "qstream_shape_rule",
-        "skinny_codes_max_m"); returns the old value."""
+        "skinny_codes_max_m", "words_max_m"); returns the old value."""
         old = self.lib.glowq_set_tuning(key.encode(), int(value))
         if old < 0:
             raise ValueError(self.lib.glowq_last_error().decode())

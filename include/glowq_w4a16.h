@@ -70,9 +70,10 @@ const char* glowq_last_error(void);
  * Replaces `w4a16_gemv_forward_cuda` (src/cuda_w4a16/csrc/gemv_w4a16.cu:146-214; pybind
  * src/cuda_w4a16/csrc/pybind.cpp:19-23).  Any M is accepted; all M rows share one pass over the weights.
  * Weight rounding by row count: the GEMV kernels (1 token row; 2..4 rows by group size, see glowq_set_tuning) keep
- * (code - zero) * scale unrounded, as the reference's GEMV does (gemv_w4a16.cu:96-112), and so does the raw-code
- * form of the skinny MFMA kernel (route 7: 5..8 rows by default, where K is a multiple of 256 and the groups have 128
- * columns).  On the other MFMA routes (1 and 2, glowq_w4a16_route tells) the dequantised weight is rounded once to fp16
+ * (code - zero) * scale unrounded, as the reference's GEMV does (gemv_w4a16.cu:96-112), and so do the raw-code
+ * forms of the skinny MFMA route (route 7, where K is a multiple of 256 and the groups have 128 columns: 5..8 rows by default, and
+ * up to 16 rows from K = 1024 on on the narrow tiles over the canonical buffers, "words_max_m" of glowq_set_tuning) and the kernels on the
+ * tiled copy up to 64 rows (route 8).  On the other MFMA routes (1 and 2, glowq_w4a16_route tells) the dequantised weight is rounded once to fp16
  * before the multiply, which is the arithmetic of the reference's dequantise-then-matmul route (gemm_w4a16.cu:46-49,132)
  * -- the reference itself switches to that arithmetic only above 128 rows.  On activations of order one the two differ
  * by far less than 1e-2 + 1e-3 |y|; with outlier channels in the thousands they differ by more than that, in the
@@ -254,7 +255,10 @@ int glowq_static_scratch_prepare(void);
  * wave in flight up front; the default at one token row), 6 = the 4x4x4 matrix-core GEMV under the stream GEMV's
  * memory schedule (the default at two to four token rows), 7 = skinny MFMA with the int4 codes fed to the matrix
  * cores as they are and scale and zero-point applied to each group's sum (unrounded arithmetic; the default at five to
- * eight token rows).
+ * eight token rows, and at nine to sixteen where the narrow tiles over the canonical buffers pay).
+ * The answer is that for a call that computes a correction (glowq_w4a16_group_forward_fused).  At nine to sixteen rows it takes the narrow
+ * tiles where K is at most 3072, or at most 6144 and the codes 25 MB and more, with more than 2048 rows out; a call
+ * without a correction, or with r given, takes them wherever they apply.  What a call ran on, glowq_last_launch names ("skinny_words_kernel").
  */
 int glowq_w4a16_route(int M, int K, int N, int group_size, int ldw_i32);
 /* The same for a member that brings the tiled copy of its weights (glowq_pack_tiled): 8 = the matrix-core kernels that
@@ -266,7 +270,7 @@ int glowq_w4a16_route_tiled(int M, int K, int N, int group_size, int ldw_i32);
  * Measurement helpers of bench.py; no counterpart in the reference.
  * glowq_last_launch: what the calling thread's last group launch, or projection of many rows by itself, used -- the
  *   kernel with the template arguments of the instantiation where the launcher records them (the stream GEMV, the
- *   tiled-copy kernel, the GEMM, the projection), else the route's name -- and its grid and workgroup size (0 where not recorded).
+ *   tiled-copy kernel, the narrow tiles over the canonical buffers, the GEMM, the projection), else the route's name -- and its grid and workgroup size (0 where not recorded).
  * glowq_probe_stream_read: a kernel that does nothing but read `bytes` (16-byte loads, eight in flight per lane,
  *   workgroup b the b-th contiguous share) with the given grid and workgroup size: the rate a memory-bound kernel of
  *   that launch shape could reach with no arithmetic at all.  `sink` (4 bytes of device memory) is never written.
@@ -293,6 +297,9 @@ int glowq_probe_empty_launch(int grid, int block, void* stream);
  * was measured faster on (1, the default) or for every shape it can take (0).
  * "skinny_codes_max_m" (0..64, default 8): token rows up to which the skinny MFMA kernel runs in its raw-code form
  * (route 7) where that applies; above it is slower than dequantising first (the work on the sums grows with the rows).
+ * "words_max_m" (0..16, default 16): token rows, from five, up to which groups of the skinny MFMA route run on narrow tiles (16 x 16) over
+ * the canonical buffers instead, in the same arithmetic, where that applies and pays (route 7 as well; K a multiple of 256 from 1024 on, groups of 128
+ * columns); 0 for either of the two limits switches that off.
  * "tiled_min_m" / "tiled_max_m" (default 2 / 64; max 0 switches the route off): token rows served by the kernel that
  * streams the tiled copy of the weights where every member brings one; "tiled_shape_rule" (0 / 1): up to 32 rows only
  * for groups whose stream is long enough to pay for its start-up (1, the default: 80 MB of codes up to 4 rows, 40 MB up to
@@ -304,7 +311,7 @@ int glowq_probe_empty_launch(int grid, int block, void* stream);
  * default 0), for tests: 1 has launches on the tiled weights compute r wherever they can, not only where that is predicted to pay.
  * Returns the previous value (>= 0) or GLOWQ_EINVAL.  Initial values come from GLOWQ_QUAD_M,
  * GLOWQ_QUAD_MIN_M, GLOWQ_WAVEDOT_M, GLOWQ_SKINNY_M, GLOWQ_SMALL_GROUP_MB, GLOWQ_STREAM_M, GLOWQ_STREAM_SHAPE_RULE,
- * GLOWQ_QSTREAM_M, GLOWQ_QSTREAM_SHAPE_RULE, GLOWQ_SKINNY_CODES_M, GLOWQ_TILED_MIN_M, GLOWQ_TILED_MAX_M,
+ * GLOWQ_QSTREAM_M, GLOWQ_QSTREAM_SHAPE_RULE, GLOWQ_SKINNY_CODES_M, GLOWQ_WORDS_M, GLOWQ_TILED_MIN_M, GLOWQ_TILED_MAX_M,
  * GLOWQ_TILED_SHAPE_RULE, GLOWQ_PROJ_IN_LAUNCH, GLOWQ_PROJ_ANY_COST and GLOWQ_PROJ_SPIN_LIMIT.
  */
 int glowq_set_tuning(const char* key, int value);

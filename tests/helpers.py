@@ -58,6 +58,14 @@ def assert_close(got, want64, what=""):
     return float(err.max())
 
 
+def rounds_weights(ext):
+    """Whether the kernel of the last call rounds (code - zero) * scale to fp16 (the others keep it as it is)."""
+    name = ext.last_launch()["kernel"]
+    if name.startswith("skinny_group_kernel<"):  # r inside the launch; the fourth argument: raw codes
+        return name.split(",")[3] == "0"
+    return name.startswith(("skinny_mfma", "gemm_mfma_kernel", "gemm_tiled_kernel")) and ",exact" not in name
+
+
 @contextlib.contextmanager
 def tuning(ext, **limits):
     """Route limits of the library set for the body of a `with` and put back afterwards."""

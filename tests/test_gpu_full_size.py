@@ -6,7 +6,7 @@ the full-size launch on the same buffers, and size-independent properties cover 
 dequantised columns exactly, a group launch equals its members launched alone bit for bit, token rows of a batched
 launch equal single-row launches within tolerance, and the result is additive in x within tolerance.
 
-Yardstick by kernel route: the GEMV routes and the kernels that feed the codes to the matrix cores as they are keep the
+Yardstick by the kernel that ran: the GEMV routes and the kernels that feed the codes to the matrix cores as they are keep the
 dequantised weight unrounded (`corrected_linear_exact`), the dequantising MFMA routes round it to fp16 once like the
 reference's dequantise-then-matmul (`corrected_linear_rounded_exact`); tolerance
 |a - b| <= 1e-2 + 1e-3 |b| in both cases."""
@@ -15,7 +15,7 @@ import pytest
 import torch
 
 import glowq_oracle as oracle
-from helpers import assert_close
+from helpers import assert_close, rounds_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -30,7 +30,6 @@ MODELS = {
                       "down": (17408, [5120])}),
 }
 GROUPS = ["qkv", "o", "gate_up", "down"]
-UNROUNDED = {"wave_dot_gemv", "quad_mfma_gemv", "generic", "stream_gemv", "quad_stream_gemv", "skinny_codes_mfma", "skinny_tiled_mfma"}
 
 
 def _layer(model, name, M, seed, bias=False):
@@ -55,15 +54,15 @@ def _sample_rows(N, seed):
     return np.unique(np.concatenate(([0, 1, 2, 3, N - 4, N - 3, N - 2, N - 1], rng.integers(0, N, 24))))
 
 
-def _oracle_rows(x, R, mem, rows, route, alpha=1.0):
+def _oracle_rows(x, R, mem, rows, rounded, alpha=1.0):
     """float64 yardstick of the sampled output rows of one member for the token rows in `x`."""
     idx = torch.from_numpy(rows).cuda()
     qw, qz, sc = (mem[k][idx].cpu().numpy() for k in ("qweight", "qzeros", "scales"))
     xh = x.cpu().numpy()
     if mem["L"] is None:
-        want = (oracle.linear_exact if route in UNROUNDED else oracle.linear_rounded_exact)(xh, qw, qz, sc, GS)
+        want = (oracle.linear_rounded_exact if rounded else oracle.linear_exact)(xh, qw, qz, sc, GS)
     else:
-        fn = oracle.corrected_linear_exact if route in UNROUNDED else oracle.corrected_linear_rounded_exact
+        fn = oracle.corrected_linear_rounded_exact if rounded else oracle.corrected_linear_exact
         want = fn(xh, qw, qz, sc, GS, R.cpu().numpy(), mem["L"][idx].cpu().numpy(), alpha)
     if mem.get("bias") is not None:
         want = want + mem["bias"][idx].cpu().numpy().astype(np.float64)[None, :]
@@ -72,14 +71,14 @@ def _oracle_rows(x, R, mem, rows, route, alpha=1.0):
 
 def _check_sampled(ext, model, name, M, x, R, members, outs, tokens=None):
     K, Ns = MODELS[model][1][name]
-    route = ext.route(M, K, sum(Ns))
+    route, rounded = ext.route(M, K, sum(Ns)), rounds_weights(ext)
     tok = np.arange(M) if tokens is None else np.asarray(tokens)
     tix = torch.from_numpy(tok).cuda()
     for i, (mem, y) in enumerate(zip(members, outs)):
         rows = _sample_rows(mem["qweight"].size(0), 10 * M + i)
-        want = _oracle_rows(x[tix], R, mem, rows, route)
+        want = _oracle_rows(x[tix], R, mem, rows, rounded)
         got = y[tix][:, torch.from_numpy(rows).cuda()].cpu().numpy()
-        assert_close(got, want, f"{model} {name} member {i} M={M} route {route}")
+        assert_close(got, want, f"{model} {name} member {i} M={M} route {route} rounded {rounded}")
     return route
 
 
@@ -259,7 +258,7 @@ def test_chained_layer_at_full_size(ext, model):
         """Sampled rows of a launch's own outputs (where it wrote them) against the oracle."""
         for mem, y in zip(layers[name][2], outs_or_none):
             rows = _sample_rows(mem["qweight"].size(0), 5)
-            want = _oracle_rows(x[None, :], R[name], mem, rows, "stream_gemv")[0]
+            want = _oracle_rows(x[None, :], R[name], mem, rows, False)[0]
             assert_close(y.cpu().numpy()[rows], want, f"{model} {name}")
 
     for mode in ("full", "mlp"):

@@ -139,6 +139,22 @@ def test_replays_follow_rows_and_weights(ext):
         check(y, x, r, exact2, members)
 
 
+@pytest.mark.parametrize("limit", ["words_max_m", "skinny_codes_max_m"])
+def test_switched_off_the_weights_are_rounded(ext, limit):
+    """Without the narrow tiles, or without raw codes at all, sixteen rows take the kernel that rounds the weights: further from fp64 than they are
+    with unrounded ones (here 2e-4), as near as half an ulp of a weight allows."""
+    M, K, N = 16, 2048, 3000
+    x, _, members, (w,) = make(9, M, K, [N], 0)
+    pg = PreparedGroup(ext, members, K, 128, 0.0)
+    want = x.double() @ w.t()
+    with tuning(ext, tiled_max_m=0, **{limit: 0}):
+        (y,) = pg.run(x)
+        assert ext.last_launch()["kernel"] == "skinny_mfma"
+    rounded = x.double() @ w.half().double().t()
+    near = (y.double() - rounded).norm() / want.norm()
+    assert near <= 3.2e-4 and (y.double() - want).norm() / want.norm() > near
+
+
 @pytest.mark.parametrize("std", [1e-4, 3e-5])
 @pytest.mark.parametrize("K,Ns,rank", [(4096, [300], 0), (2816, [3000, 40], 40)])
 @pytest.mark.parametrize("M", [5, 8, 9, 16])

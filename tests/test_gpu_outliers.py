@@ -4,7 +4,7 @@
 On such inputs the reference's two routes differ from each other by more than the tolerance (shown on the CPU in
 tests/test_oracle.py::test_two_reference_semantics_part_on_outlier_activations), so each kernel is judged against the
 semantics it implements:
-  * the stream, wave-dot and 4x4x4 GEMV, the skinny kernel's raw-code form and the kernel that streams the tiled copy of
+  * the stream, wave-dot and 4x4x4 GEMV, the skinny kernel's raw-code form, the narrow tiles and the kernel that streams the tiled copy of
     the weights keep the dequantised weight unrounded, like the reference's GEMV kernel
     (src/cuda_w4a16/csrc/gemv_w4a16.cu:96-112): yardstick `corrected_linear_exact`;
   * the skinny MFMA kernel and the tiled MFMA GEMM round the dequantised weight to fp16 once, like the reference's
@@ -17,7 +17,7 @@ import pytest
 import torch
 
 import glowq_oracle as oracle
-from helpers import ABS_TOL, REL_TOL, dev, make_group, outlier_activations
+from helpers import ABS_TOL, REL_TOL, dev, make_group, outlier_activations, rounds_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +35,7 @@ CASES = [
     (8, 4096, [512], 128, "default"), (8, 4096, [512], 128, "quad"), (4, 4096, [512], 128, "qstream"),
     (4, 14336, [8192], 128, "qstream"), (3, 4096, [2048, 2048], 256, "qstream"),
     (16, 14336, [256], 128, "default"), (16, 4096, [1024, 256], 128, "quad"),
+    (9, 2048, [2048, 512], 64, "default"), (16, 2048, [2048, 512], 64, "default"), (16, 2048, [512], 64, "default"),
     (64, 4096, [512, 96], 256, "default"), (130, 2048, [512], 128, "default"), (300, 4096, [256, 128], 128, "default"),
 ]
 
@@ -75,10 +76,11 @@ def test_outlier_channels_against_the_semantics_of_the_route(ext, tuned, case):
     r = torch.empty(M, rank, dtype=torch.float16, device="cuda")
     outs = ext.group_forward(dev(x), r, mem, 128, 1.0, R=dev(R))
     torch.cuda.synchronize()
-    route = ext.route(M, K, sum(Ns))
+    route, rounded = ext.route(M, K, sum(Ns)), rounds_weights(ext)
+    assert rounded == (route not in UNROUNDED), ext.last_launch()
     r64 = x.astype(np.float64) @ R.astype(np.float64).T
     assert np.all(np.abs(r.cpu().numpy().astype(np.float64) - r64) <= ABS_TOL + REL_TOL * np.abs(r64))
-    yardstick = oracle.corrected_linear_exact if route in UNROUNDED else oracle.corrected_linear_rounded_exact
+    yardstick = oracle.corrected_linear_rounded_exact if rounded else oracle.corrected_linear_exact
     for j, (m, y) in enumerate(zip(members, outs)):
         got = y.cpu().numpy()
         assert np.isfinite(got).all()
@@ -90,6 +92,6 @@ def test_outlier_channels_against_the_semantics_of_the_route(ext, tuned, case):
         assert np.all(err <= bound), (f"member {j} on {route}: err {err[worst]:.4f} > bound {bound[worst]:.4f} at {worst} "
                                       f"(max |y| {np.abs(want).max():.1f})")
         # and the check tells the two semantics apart where it matters: the other yardstick is further away
-        other = (oracle.corrected_linear_rounded_exact if route in UNROUNDED else oracle.corrected_linear_exact)(
+        other = (oracle.corrected_linear_exact if rounded else oracle.corrected_linear_rounded_exact)(
             x, m["qweight"], m["qzeros"], m["scales"], 128, R, m["L"], 1.0)
         assert np.abs(got.astype(np.float64) - want).mean() <= np.abs(got.astype(np.float64) - other).mean() + 1e-3

@@ -14,6 +14,7 @@ import torch.nn as nn
 import glowq_oracle as oracle
 from glowq_amd import correction as corr
 from glowq_amd import kernels, linear
+from helpers import tuning
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -284,6 +285,23 @@ def test_library_exports_every_declared_symbol():
     assert set(kernels._SIGNATURES) == declared
     assert ctypes.sizeof(kernels._Member) == 6 * 8 + 6 * 4 + 8 + 2 * 8 + 2 * 4  # matches glowq_member_t
     assert kernels._Member.side.offset == 72 and kernels._Member.side_rank.offset == 68
+
+
+def test_the_route_names_the_arithmetic_of_the_narrow_tiles():
+    """Five to sixteen rows of a corrected group on the narrow tiles over the canonical buffers: reported as unrounded, with a limit of their own,
+    and none of them where raw codes are switched off."""
+    ext = kernels.load_w4a16_extension()
+    with tuning(ext, quad_max_m=0):
+        for M in (9, 16):
+            assert ext.route(M, 2048, 2560, tiled=False) == "skinny_codes_mfma" and ext.route(M, 4096, 28672, tiled=False) == "skinny_codes_mfma"
+            # as for groups that compute a correction: short streams and long K stay on the rounding kernel
+            assert ext.route(M, 4096, 4096, tiled=False) == "skinny_mfma" and ext.route(M, 2048, 2048, tiled=False) == "skinny_mfma"
+            assert ext.route(M, 14336, 4096, tiled=False) == "skinny_mfma" and ext.route(M, 2048, 2560, group_size=64, tiled=False) == "skinny_mfma"
+        assert ext.route(17, 2048, 2560, tiled=False) == "skinny_mfma"
+        with tuning(ext, words_max_m=12):
+            assert ext.route(12, 2048, 2560, tiled=False) == "skinny_codes_mfma" and ext.route(13, 2048, 2560, tiled=False) == "skinny_mfma"
+        with tuning(ext, skinny_codes_max_m=0):
+            assert ext.route(8, 2048, 2560, tiled=False) == "skinny_mfma" and ext.route(16, 2048, 2560, tiled=False) == "skinny_mfma"
 
 
 def test_abi_rejects_bad_arguments_without_a_gpu():
