@@ -53,6 +53,9 @@ def launched(ext, form):
 
 SHAPES = [(256, [4000], 8), (512, [130, 2040], 40), (1024, [4100, 3000], 40), (1280, [2600, 33], 72), (2304, [2336], 256), (5120, [5120, 1024, 1024], 256),
           (17408, [5120], 264), (768, [34000], 136), (4096, [28672], 64), (1024, [1], 0), (3328, [40, 7], 0), (14336, [4096], 0), (2816, [9472, 9472], 0)]
+# K of those with a correction that have r inside their launch, where the call allows it, on the tiled copy and on the canonical buffers (the canonical
+# form leaves all other corrected ones, and those with K below 1024, to the skinny kernel)
+INSIDE = {"tiled": {768, 1024, 1280, 2304, 4096, 5120}, "words": {1024, 1280, 2304, 4096}}
 
 
 @pytest.mark.parametrize("K,Ns,rank", SHAPES)
@@ -64,9 +67,12 @@ def test_against_fp64(ext, form, M, K, Ns, rank):
     for in_front in (0, 1):
         with tuning(ext, proj_in_launch=in_front):
             y = pg.run(x)
-        if form == "words" and (rank or K < 1024) and ext.last_launch()["kernel"].startswith("skinny_") and not launched(ext, form):
+        if form == "words" and rank and K not in INSIDE[form]:
+            assert ext.last_launch()["kernel"].startswith(("skinny_codes_mfma", "skinny_mfma", "skinny_group_kernel<"))
             continue  # a group that the skinny kernel keeps
         assert launched(ext, form), ext.last_launch()
+        inside = ext.last_launch()["kernel"].split(">")[0].count(",") == 3  # rows, K groups, producer waves and, with r inside, a 1
+        assert inside == bool(in_front and rank and K in INSIDE[form]), ext.last_launch()
         r = pg.last_r
         if rank:
             want_r = x.double() @ R.double().t()

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import glowq_oracle as oracle
-from helpers import assert_close, dev, make_group
+from helpers import assert_close, dev, make_group, tuning
 
 pytestmark = pytest.mark.gpu
 
@@ -16,9 +16,15 @@ ROUTE = 7  # skinny_codes_mfma
 
 @pytest.fixture()
 def codes(ext):
-    old = ext.set_tuning("skinny_codes_max_m", 64)
-    yield ext
-    ext.set_tuning("skinny_codes_max_m", old)
+    # (the narrow tiles would take some of the groups of 5 to 16 rows, the tiled copy those above 32)
+    with tuning(ext, skinny_codes_max_m=64, words_max_m=0, tiled_max_m=0):
+        yield ext
+
+
+def launched(ext):
+    """Whether the last call ran on the skinny kernel in its raw-code form (with r inside the launch it names its arguments)."""
+    name = ext.last_launch()["kernel"]
+    return name == "skinny_codes_mfma" or (name.startswith("skinny_group_kernel<") and name.endswith(",1,1>"))
 
 
 CASES = [
@@ -67,6 +73,7 @@ def test_skinny_codes_group_matches_oracle(codes, case):
         bufs = [wide[:, int(a):int(a) + n] for a, n in zip(starts, Ns)]
         r = torch.empty(M, rank, dtype=torch.float16, device="cuda") if rank else None
         outs = ext.group_forward(dev(x), r, mem, gs, 0.5, outs=bufs, R=dev(R) if rank else None)
+        assert launched(ext), ext.last_launch()
         torch.cuda.synchronize()
     finally:
         if saved is not None:
@@ -91,6 +98,7 @@ def test_skinny_codes_is_exact_on_integer_inputs(codes):
     sc = np.full((N, K // gs), 1.0 / 64, dtype=np.float16)
     assert ext.lib.glowq_w4a16_route(M, K, N, gs, K // 8) == ROUTE
     y = ext.w4a16_gemv_forward_cuda(dev(x), dev(qw), dev(sc), dev(qz), gs)
+    assert launched(ext), ext.last_launch()
     torch.cuda.synchronize()
     want = oracle.linear_exact(x, qw, qz, sc, gs)
     assert np.array_equal(y.cpu().numpy(), want.astype(np.float16))
