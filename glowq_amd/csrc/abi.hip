@@ -303,18 +303,26 @@ int pick_route_rounded(const GroupDev& g, int force);
 //   words_max_m     token rows (5..16) up to which groups of the skinny routes run on the narrow tiles over the canonical buffers
 //                   (skinny_tiled.hip), in unrounded arithmetic, where that pays (GLOWQ_WORDS_M); 0, or 0 for skinny_codes_max_m: the kernels
 //                   of skinny.hip.  Reported as the raw-code route, whose arithmetic it is.
-// It pays for all groups without an r to compute, and for the others where K is short or the stream long enough that r, which the skinny
-// kernels take along for fewer columns, costs them a launch or a part of the chip.  Group call, us at 8 and 16 rows, this / the skinny kernels: without a
-// correction 4096 x 4096 7.2, 8.1 / 7.5, 8.2, 3 x 2048 x 2048 5.6, 6.0 / 6.1, 6.5, 5120 x 5120 9.3, 10.4 / 9.7, 10.8, 18944 x 3584 12.5, 13.4 /
-// 17.9, 20.8; with one 2 x 9472 x 2816 12.8, 13.3 / 17.8, 20.4, 8192 x 2048 7.7, 8.1 / 8.9, 9.4; not q|k|v of an 8B and a 14B layer 9.7, 10.7 /
-// 9.8, 10.2 and 15.7, 17.1 / 14.9, 16.3, nor 4096 x 14336 19.6, 20.9 / 17.7, 19.9.
+// It pays for all groups of more than 8192 rows.  Group call, us at 8 and 16 rows, this / the skinny kernels: without a correction 14336 x 4096 11.3,
+// 12.2 / 13.8, 15.6, 2 x 18944 x 3584 18.4, 19.3 / 26.3, 29.4; with r given 11.7, 12.6 / 13.7, 15.3, 19.4, 20.7 / 28.1, 31.3.
+// Up to 8192 rows a workgroup has one row block, and K of more than 6144 columns has to be cut into slices: 4096 x 14336 with the workspace 14.3,
+// 14.9 / 14.3, 16.5, without it 17.4, 18.8 / 15.9, 18.3, 2048 x 8192 10.2, 10.5 / 11.5, 12.9, without 11.7, 12.5 / 11.5, 13.0.  With r given these launches
+// wait for r and L at their end: q|k|v of an 8B layer 8.6, 9.2 / 8.2, 8.9, 4096 x 4096 7.9, 8.6 / 7.7, 8.4 (without a correction 8.3, 8.8 / 8.1, 8.9,
+// 7.6, 8.2 / 7.7, 8.6), and up to 8 rows K from 12288 columns on where the skinny kernel cuts it as well, 4096 x 14336 14.6 / 14.0.
+// r to compute: where K is short or the stream long enough that r, which the skinny kernels take along for fewer columns, costs them a
+// launch or a part of the chip: 2 x 9472 x 2816 11.8, 13.0 / 16.2, 18.8, 8192 x 2048 7.7, 8.6 / 9.0, 9.5; not q|k|v of an 8B and a 14B layer 9.7,
+// 10.7 / 9.8, 10.2 and 15.7, 17.1 / 14.9, 16.3, nor 4096 x 14336 19.6, 20.9 / 17.7, 19.9.
 std::atomic<int> g_words_max_m{clampi(env_or("GLOWQ_WORDS_M", 16), 0, 16)};
 bool words_pay(const GroupDev& g, bool computes_r) {
   if (g.M > g_words_max_m.load(std::memory_order_relaxed) || g_skinny_codes_max_m.load(std::memory_order_relaxed) == 0 || !skinny_words_supported(g)) return false;
-  if (!computes_r) return true;
   long rows = 0;
   for (int i = 0; i < g.n_members; ++i) rows += g.mem[i].N;
-  return rows > 2048 && (g.K <= 3072 || (g.K <= 6144 && rows * (long)g.K / 2 >= 25L * 1000 * 1000));
+  if (computes_r) return rows > 2048 && (g.K <= 3072 || (g.K <= 6144 && rows * (long)g.K / 2 >= 25L * 1000 * 1000));
+  if (rows > 8192) return true;
+  const bool slices = g.ws != nullptr && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0 && g.ws_bytes >= glowq::tiled_split_workspace_bytes(g.M, num_cus());
+  if (g.K > 6144 && !slices) return false;
+  if (g.r == nullptr || g.K < 2048) return true;
+  return g.K > 6144 && (g.M > 8 || g.K < 12288 || rows > 16L * num_cus());
 }
 
 //   tiled_min_m / tiled_max_m  token rows served by the matrix-core kernel that reads the tiled copy of the weights, where

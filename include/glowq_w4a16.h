@@ -258,7 +258,8 @@ int glowq_static_scratch_prepare(void);
  * eight token rows, and at nine to sixteen where the narrow tiles over the canonical buffers pay).
  * The answer is that for a call that computes a correction (glowq_w4a16_group_forward_fused).  At nine to sixteen rows it takes the narrow
  * tiles where K is at most 3072, or at most 6144 and the codes 25 MB and more, with more than 2048 rows out; a call
- * without a correction, or with r given, takes them wherever they apply.  What a call ran on, glowq_last_launch names ("skinny_words_kernel").
+ * without a correction, or with r given, takes them from 8192 rows out on, and below that where K is at most 6144 (with r given: below
+ * 2048) or the workspace holds its slices.  What a call ran on, glowq_last_launch names ("skinny_words_kernel").
  */
 int glowq_w4a16_route(int M, int K, int N, int group_size, int ldw_i32);
 /* The same for a member that brings the tiled copy of its weights (glowq_pack_tiled): 8 = the matrix-core kernels that

@@ -145,6 +145,32 @@ def test_replays_follow_rows_and_weights(ext):
         check(y, x, r, exact2, members)
 
 
+@pytest.mark.parametrize("K,Ns,given,workspace,words", [
+    (4096, [2048, 512], False, False, True), (4096, [2048, 512], True, True, False), (1024, [2048, 512], True, False, True),
+    (4096, [8000, 400], True, False, True), (14336, [4096], False, False, False), (14336, [4096], False, True, True), (14336, [4096], True, True, True),
+    (8192, [2048], True, False, False), (8192, [2048], True, True, True)])
+@pytest.mark.parametrize("M", [5, 16])
+def test_short_groups_with_r_given_and_long_k_without_slices(ext, M, K, Ns, given, workspace, words):
+    """Which calls without an r to compute take the canonical form; the others stay on the skinny kernel, and both are right."""
+    rank = 40 if given else 0
+    words = words and not (given and M <= 8 and K >= 12288)  # (the skinny kernel cuts that K itself)
+    x, R, members, exact = make(M + K, M, K, Ns, rank)
+    r = (torch.randn(M, rank, device="cuda") * 64).half() if given else None
+    pg = PreparedGroup(ext, members, K, 128, 1.0 if given else 0.0)
+    outs = [torch.empty(M, N, dtype=torch.float16, device="cuda") for N in Ns]
+    for e, y in zip(pg.arr, outs):
+        e.y, e.ldy = y.data_ptr(), y.stride(0)
+    ws = torch.empty((8 << 20) if workspace else 16, dtype=torch.uint8, device="cuda")
+    with tuning(ext, tiled_max_m=0):
+        assert ext.lib.glowq_w4a16_group_forward_ws(x.data_ptr(), r.data_ptr() if given else None, pg.arr, len(Ns), M, K, 128, rank, 1.0,
+                                                    ws.data_ptr(), ws.numel() if workspace else 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert launched(ext, "words") == words, ext.last_launch()
+    if words or M <= 8:
+        check(outs, x, r, exact, members)
+    else:  # rounded weights
+        check(outs, x, r, [w.half().double() for w in exact], members)
+
+
 @pytest.mark.parametrize("limit", ["words_max_m", "skinny_codes_max_m"])
 def test_switched_off_the_weights_are_rounded(ext, limit):
     """Without the narrow tiles, or without raw codes at all, sixteen rows take the kernel that rounds the weights: further from fp64 than they are
