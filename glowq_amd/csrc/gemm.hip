@@ -569,7 +569,7 @@ __device__ __forceinline__ void order_word() {
 // half of 128 columns meets its scale in fp32, so the weight is never rounded (nine vector instructions a word and sixteen a
 // half and tile against thirteen a word: as many at two row tiles).
 template <int kMT, int kNT, int kWk, typename YT, bool kProj, bool kExact>
-__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT >= 16 ? 1 : (kMT * kNT <= 2 && !(kExact && kMT == 2) ? 4 : 2)), (kMT * kNT >= 16 ? 1 : 8))))
+__global__ __launch_bounds__(256 * kWk) __attribute__((amdgpu_waves_per_eu((kMT * kNT <= 2 && !(kExact && kMT == 2) ? 4 : 2), 8)))
 void gemm_tiled_kernel(const GemmGroup gg, const int m_blocks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
   const int front = kProj ? gg.front.front : 0;
@@ -1258,7 +1258,7 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   static const int mt_max = getenv("GLOWQ_GEMM_MT") ? atoi(getenv("GLOWQ_GEMM_MT")) : 4;
   int mt_cap = M > 128 ? 8 : (M > 64 ? 4 : (M > 32 ? 2 : 1));
   if (mt_cap > mt_max) mt_cap = mt_max;
-  if (y32 && mt_cap > 4) mt_cap = 4;  // (256-row tiles are there for measurements, without fp32 outputs)
+  if (y32 && mt_cap > 4) mt_cap = 4;  // (256-row tiles are there for measurements, on the canonical buffers, which have no fp32 outputs)
   static const int order[6][2] = {{4, 2}, {2, 2}, {4, 1}, {2, 1}, {1, 2}, {1, 1}};
   int mt = 1, nt = 1;
   long best = -1;
@@ -1411,8 +1411,6 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   GLOWQ_GEMM_TILED_CASE(2, 1, 1) GLOWQ_GEMM_TILED_CASE(1, 1, 1) GLOWQ_GEMM_TILED_CASE(4, 2, 2) GLOWQ_GEMM_TILED_CASE(2, 1, 2)
 #undef GLOWQ_GEMM_TILED_CASE
   if (y32) return hipErrorInvalidValue;  // (gemm_widens said no)
-  if (tiled_ok && mt == 8 && nt == 2) return launch_gemm_t<8, 2, true, true, true>(gg, stream);
-  if (tiled_ok && mt == 8 && nt == 1) return launch_gemm_t<8, 1, true, true, true>(gg, stream);
 #define GLOWQ_GEMM_CASE(MT, NT)                                                            \
   if (mt == MT && nt == NT) return super ? launch_gemm_t<MT, NT, true, true>(gg, stream) : launch_gemm_t<MT, NT, true>(gg, stream);
   GLOWQ_GEMM_CASE(8, 2) GLOWQ_GEMM_CASE(4, 2) GLOWQ_GEMM_CASE(2, 2) GLOWQ_GEMM_CASE(1, 2)

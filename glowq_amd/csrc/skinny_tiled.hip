@@ -26,7 +26,7 @@
 // From 9 rows on (kWhole) the activations stay whole, as in the rounding kernel of skinny.hip that has these rows otherwise: the masks of two neighbouring
 // words make one operand of the low nibbles and one of the high ones, with sums of their own (error of the output at |x| around 1e-4, against
 // x / 16 in fp16: 2.1e-4 / 2.0e-3; same matrix and vector instructions: 14336 x 4096 at 16 rows 12.8 us / 12.6, 1024 x 5120 9.2 / 9.5, 4096 x 14336
-// 19.5 / 19.7.  As code - zero, nine vector instructions a word instead of five: 13.4, 9.6, 20.2), and sums that are not finite are taken again
+// 19.5 / 19.7, 2 x 14336 x 4096 15.9 / 15.2, with r inside 19.9 / 18.2.  As code - zero, nine vector instructions a word instead of five: 13.4, 9.6, 20.2), and sums that are not finite are taken again
 // with code - zero, which gives an infinite activation's products their signs.  At 8 rows two sums cost 2 to 5 % more, and the
 // raw-code form of skinny.hip divides by 16 as well.
 // Launch without a correction, 8 and 16 rows, us, against the kernels of skinny.hip: 14336 x 4096 15.7, 16.9 -> 11.6, 12.5, 18944 x 3584
@@ -149,16 +149,6 @@ constexpr int kStreamAux = GLOWQ_TILED_AUX;  // cache policy of the weight loads
 
 }  // namespace
 
-#ifndef GLOWQ_TDBG
-#define GLOWQ_TDBG 0
-#endif
-#if GLOWQ_TDBG & 32
-__device__ unsigned long long g_tstamps[65536 * 32];
-#define GLOWQ_STAMP(i) do { if (lane == 0 && !producer) g_tstamps[(((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 16 + (threadIdx.x >> 6)) * 32 + (i)] = wall_clock64(); } while (0)
-#else
-#define GLOWQ_STAMP(i) do { } while (0)
-#endif
-
 // kRows: token rows a K group stages (8, 16 or 32).  kWk: K groups per workgroup.  kPW: producer waves per K group.
 // The leading scalar arguments arrive in registers with the wave (kernel-argument preload): what a workgroup of the
 // first member needs to request its first weights and activations, without a round trip to the argument buffer.
@@ -179,7 +169,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   constexpr bool kWhole = kCanon && kRows > 8;   // activations are not divided by 16
   constexpr int kSigBytes = kNarrow ? 0 : kRows * 16;  // per 128-column half: a 16-byte fragment of sums per token row
   constexpr int kStage = kRows * kRowBytes + 2 * kSigBytes;
-  constexpr int kLiveRegs = kRows >= 32 ? 16 : (kRows >= 16 ? 8 : 4);  // accumulator registers of rows that exist
   const int group_threads = (cw + kPW) * 64;  // the consumer waves, then the producer waves
   const int gk = kWk > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >= group_threads ? 1 : 0) : 0;
   static_assert(kWk <= 2, "gk is a comparison");
@@ -189,7 +178,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   const bool producer = wave >= cw;
   const int ln = lane & 31, lh = lane >> 5;
   unsigned char* smem = smem_all + gk * 2 * kStage;
-  GLOWQ_STAMP(0);
 
   int tile = (int)blockIdx.x;
   unsigned long long tag = 0;
@@ -410,7 +398,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     bool have_r = false;
     const auto produce = [&](int i, auto set_const) __attribute__((always_inline)) {  // step i: set (i + 1) % kXD
       constexpr int set = decltype(set_const)::value;
-#if !(GLOWQ_TDBG & 8)
       if constexpr (kProj) {
         // r that was not there a step earlier is waited for during the last super-block, for the stage that super-block
         // does not read
@@ -422,7 +409,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
         // one look a step before: as a rule the workgroups in front are long done
         if (i + 2 == steps && wg_corr && gk == 0) have_r = ask_r_handed(avs[0], 1u);
       }
-#endif
       __syncthreads();
     };
     using std::integral_constant;
@@ -533,7 +519,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   if constexpr (kCanon) request_side(sb0);
   request(bs[0], sb0);
   request(bs[1], sb0 + 1);
-  GLOWQ_STAMP(1);
 
   // a member without a left factor (GlowQ-S) reads zeros for its correction blocks
   const TileMember mem = g.mem[mi];
@@ -568,9 +553,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
   const uint32_t half0 = lh == 0 ? 0xFFFFFFFFu : 0u;  // the zero-point fragment lives in the first lane half
-  const int arow = kRows >= 32 ? ln : (ln & (kRows - 1));
-  const int arow_off = arow * kRowBytes + 128 * lh;
-  const int sig_off = kRows * kRowBytes + arow * 16;
+  const int arow_off = ln * kRowBytes + 128 * lh;  // 32-row tiles
+  const int sig_off = kRows * kRowBytes + ln * 16;
 
   // One super-block: the codes of the register set `b` against the staged rows, half by half.
   // kRefill: each register of the set is refilled with super-block sb_next as soon as its words have been masked.
@@ -579,21 +563,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     constexpr bool kRefill = decltype(refill_const)::value;
     const unsigned char* st = smem + stage * kStage;
     const u32x2 side = b.side;
-#if GLOWQ_TDBG & 1
-    {
-      uint32_t f = side.x ^ side.y;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const u32x4 raw = b.w[j];
-        if constexpr (kRefill) b.w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, b_off + j * 1024, sb_next * chunk_stride, kStreamAux);
-        f ^= raw.x ^ raw.y ^ raw.z ^ raw.w;
-      }
-      acc[0][0] += __builtin_bit_cast(float, f & 0x3FFFFFFFu) + *reinterpret_cast<const float*>(st + arow_off);
-      if constexpr (kRefill)
-        b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sb_next * chunk_stride + tiled::kCodeBytes, kStreamAux));
-      return;
-    }
-#endif
     if constexpr (kNarrow) {
       uint32_t sw[2][2];  // [half][c]
       if constexpr (kCanon) {
@@ -714,7 +683,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
       const h8 az = *reinterpret_cast<const h8*>(st + sig_off + gh * kSigBytes);
       pg = __builtin_amdgcn_mfma_f32_32x32x16_f16(az, bz, pg, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < kLiveRegs; ++i) acc[i] = __builtin_fmaf(sf, pg[i], acc[i]);
+      for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(sf, pg[i], acc[i]);
     }
     if constexpr (kRefill)
       b.side = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, ln * 8, sb_next * chunk_stride + tiled::kCodeBytes, kStreamAux));
@@ -723,7 +692,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
   __syncthreads();
   request(bs[2], sb0 + 2);
   request(bs[3], sb0 + 3);
-  GLOWQ_STAMP(2);
 
   // step d of a rotation at super-block sb: compute on stage d % 2; barrier.  Last rotation: a step past the group's
   // part is skipped, and the sets are refilled with the blocks of the tiled left factor (set q: block q; past the rank
@@ -737,9 +705,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     } else {
       compute(d_const, sb + kD, bs[d], std::true_type{});
     }
-    GLOWQ_STAMP(8 + min(sb - sb0, 11) * 2);
     __syncthreads();
-    GLOWQ_STAMP(9 + min(sb - sb0, 11) * 2);
   };
   using std::integral_constant;
   int sb = sb0;
@@ -750,10 +716,8 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
     step(sb + 2, integral_constant<int, 2>{}, std::false_type{});
     step(sb + 3, integral_constant<int, 3>{}, std::false_type{});
   }
-  GLOWQ_STAMP(3);
   if constexpr (kCanon) turn(sb, false);
   step(sb, integral_constant<int, 0>{}, std::true_type{});
-  GLOWQ_STAMP(4);
   step(sb + 1, integral_constant<int, 1>{}, std::true_type{});
   step(sb + 2, integral_constant<int, 2>{}, std::true_type{});
   step(sb + 3, integral_constant<int, 3>{}, std::true_type{});
@@ -833,7 +797,7 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
           }
         continue;
       }
-      const unsigned char* ar = smem + arow * kRowBytes + 64 * lh;
+      const unsigned char* ar = smem + ln * kRowBytes + 64 * lh;
 #pragma unroll
       for (int q = 0; q < kD; ++q)
 #pragma unroll
@@ -852,7 +816,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 #pragma unroll
   for (int i = 0; i < kAccs; ++i) out[i] = kNarrow ? nacc[(i >> 2) & 1][i & 3] : acc[i];
 
-  GLOWQ_STAMP(5);
   // ---- the K groups' accumulators meet in LDS: groups 1.. leave theirs, group 0 adds them in order ---------------
   if constexpr (kWk > 1) {
     __syncthreads();  // every group is done with its stages
@@ -871,7 +834,6 @@ void skinny_tiled_kernel(const half_t* __restrict__ x, const int M, const int K,
 
   // ---- epilogue: entry i of a lane is token row 8 (i / 4) + 4 lh + i % 4, column ln of the wave's row block; of the narrow tiles row
   // 4 nq + i % 4, column 16 (i / 4) + lane % 16
-  GLOWQ_STAMP(6);
   if (!live) return;
   const auto row_of = [&](int i) { return kNarrow ? 4 * nq + (i & 3) : 8 * (i >> 2) + 4 * lh + (i & 3); };
   const auto col_of = [&](int i) { return rb * 32 + (kNarrow ? 16 * (i >> 2) + (lane & 15) : ln); };
@@ -975,12 +937,6 @@ __global__ __launch_bounds__(256) void pack_tiled_left_kernel(const half_t* __re
 }
 
 // ---- host side ----------------------------------------------------------------------------------------------
-#if GLOWQ_TDBG & 32
-extern "C" int glowq_debug_stamps(void* host, size_t bytes, int clear) {
-  if (clear) { void* p; hipGetSymbolAddress(&p, HIP_SYMBOL(g_tstamps)); return (int)hipMemset(p, 0, sizeof(g_tstamps)); }
-  return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(g_tstamps), bytes < sizeof(g_tstamps) ? bytes : sizeof(g_tstamps));
-}
-#endif
 hipError_t launch_pack_tiled(const int32_t* qweight, const half_t* scales, const int32_t* qzeros, void* out, int N, int K,
                              int group_size, int ldw, int lds, int ldz, int num_cus, hipStream_t stream) {
   const long total = (long)((N + 31) >> 5) * (K >> 8) * 64;
@@ -1126,8 +1082,8 @@ static TiledPlan tiled_plan(const GroupDev& g, int num_cus, size_t ws_bytes, boo
   return p;
 }
 
-// The most workspace tiled_plan asks for: it cuts K only where tiles x slices stay within num_cus workgroups, and such
-// groups have tiles of four consumer waves (128 columns): one 128-column fp32 tile per token row for each of them.
+// The most workspace tiled_plan and narrow_plan ask for: they cut K only where tiles x slices stay within num_cus workgroups, and into slices only
+// tiles of up to four consumer waves (128 columns): one 128-column fp32 tile per token row for each of them.
 size_t tiled_split_workspace_bytes(int M, int num_cus) { return M > 4 ? (size_t)num_cus * (size_t)M * 128 * sizeof(float) : 0; }
 
 template <int kRows, int kWk, int kPW, bool kProj = false, bool kCanon = false>
