@@ -560,8 +560,9 @@ __device__ __forceinline__ void order_word() {
 // of their own, and the two accumulator sets meet in LDS before the epilogue.  For launches with about one tile per
 // compute unit: a SIMD then holds two waves of the one workgroup it has, instead of one wave with nothing to overlap its
 // waits with, and the K loop of a tile takes half as many steps.
-// One super-block of weights and one half-step of activations ahead are enough: four sets of registers and four stages measured the
-// same or slower on every shape at 100 and 333 rows (8B gate|up at 100 rows 41.4 -> 42.2 us, down_proj 28.2 -> 28.9).
+// One super-block of weights and one half-step of activations are ahead.  Four sets of registers and four stages measured the same or slower
+// on every shape at 100 and 333 rows (8B gate|up at 100 rows 41.4 -> 42.2 us, down_proj 28.2 -> 28.9), but that says nothing of more activations in
+// flight: in front of a barrier the compiler waits for every load to LDS (see proj_front.hpp), whatever the wait above it leaves.
 // kProj: the launch computes r = x R^T itself.  The readers need r behind their K loop, which is when the workgroups in front of the grid are
 // done as a rule; they wait for the words of their rows' tiles (bounded: a reader that gives up computes its r from x and R), and
 // read r past the caches the stores of the workgroups in front have passed.
@@ -1074,7 +1075,9 @@ static hipError_t launch_gemm_t(GemmGroup& gg, hipStream_t stream) {
 }
 
 // What a launch of gemm_tiled_kernel takes, in us: a fit over 250 (group, rows) pairs -- 21 groups of 1.5B to 14B shapes,
-// 65 to 1024 rows, with and without slices of K, 8400 timings, 7 % rms -- used to compare ways to cut one product.  A half-step
+// 65 to 1024 rows, with and without slices of K, 8400 timings, 7 % rms -- used to compare ways to cut one product.  The timings are those of the
+// loop before its instructions were interleaved, with the correction in front; of the present one, on the cuts it picks for 24 groups at 72 to 2048
+// rows with r given and without, the sums are 9 % off (rms), 4 % too short in the mean (10 % of 32-row tiles and of K groups, 2 % of the others).  A half-step
 // (128 columns of K) of a tile costs `step` on the first workgroup of a compute unit and `step_more` on every further one
 // (they share its matrix cores, but fill each other's waits); a split of K pays the launch that adds the slices and the
 // traffic of their fp32 tiles.
@@ -1088,8 +1091,9 @@ constexpr GemmCost kGemmCost[] = {
     {2, 2, 1, 2.9f, 3.3f, 0.90f, 0.77f, 1.6f, 0.29f, 0.52f}, {4, 1, 1, 3.1f, 2.8f, 1.00f, 0.73f, 1.9f, 0.24f, 0.59f},
     {4, 2, 1, 5.0f, 4.0f, 1.43f, 1.27f, 1.1f, 0.23f, 0.58f}, {4, 2, 2, 6.0f, 5.5f, 2.46f, 3.10f, 1.3f, 0.25f, 0.92f}};
 
-// The same for the unrounded form at 33 to 64 rows: 558 timings of 19 groups of 1B to 14B shapes at 36 and 57 rows, 6 % rms; the cut it picks
-// takes 1.6 % longer than the fastest of them in the mean, 9 % at most.
+// The same for the unrounded form at 33 to 64 rows: 558 timings of 19 groups of 1B to 14B shapes at 36 and 57 rows, 6 % rms.  Of 24 groups at 33, 48
+// and 64 rows, with r given and without, with a workspace and without, the cut it picks takes 1.6 % longer than the fastest of twelve in the mean,
+// 19 % at most (3584 x 3584 with r given).
 constexpr GemmCost kGemmExactCost[] = {{1, 1, 1, 1.9f, 1.0f, 0.43f, 0.21f, 3.1f, 0.47f, 1.63f},
                                        {2, 1, 1, 1.5f, 1.9f, 0.52f, 0.32f, 3.1f, 0.35f, 1.65f},
                                        {2, 1, 2, 4.3f, 1.1f, 0.81f, 1.03f, 2.7f, 0.35f, 1.83f}};
@@ -1158,7 +1162,7 @@ bool proj_on_small_kernel(int M, int K, int rank);  // abi.hip
 //    front is filled up to one a compute unit with workgroups that only hold their places: the others then come out one a compute unit as well.
 //    Otherwise some compute units get two, and the launch takes as long as those: 8B down_proj at 333 rows 72.3 with 220 in front, 57.6
 //    with 264, projection in front 67.6, r given 55.8; 14B down_proj at 512 rows 134 with 128, 106 with 256, 118, 100.
-// 16 groups of 1B to 14B shapes at 65 to 2048 rows: 1.14 times as fast in the mean with the rule as with the projection in front.
+// 24 groups of 1B to 14B shapes at 72 to 2048 rows: 1.14 times as fast in the mean with the rule as with the projection in front, 1.5 % slower at most.
 static float plan_front(GemmGroup& gg, const GemmCost& c, bool exact, int num_cus, float launch_us) {
   FrontArgs& f = gg.front;
   const int tiles = gemm_tiles(gg, c.mt, c.nt), sb = f.K >> 8, stages = f.K >> 7;
@@ -1361,7 +1365,7 @@ static hipError_t launch_gemm_group(GemmGroup& gg, int num_cus, size_t ws_bytes,
   // 35.7 -> 30.5, 14B q|k|v 31.6 -> 25.3, 14B down_proj at 512 rows 123 -> 108).  With and without this rule, 21 groups of 1.5B
   // to 14B shapes at 12 row counts: 82 of 189 pairs at 72 to 1024 rows get another cut, 1.25 times as fast in the mean and the
   // least of them 1.5 % faster; of 63 pairs at 1200 to 2048 rows, past the rows of the fit, 6 do (1.05 to 1.19 times).
-  // Without the margin the rule costs more than 1 % on 30 pairs of the fit.  Cuts that send more than 32 MB of fp32 tiles through
+  // Without the margin the rule costs more than 1 % on 30 pairs of the fit (all of these timed with the loop that the costs were fitted to).  Cuts that send more than 32 MB of fp32 tiles through
   // the workspace are not tried: from there the fit scatters by 7 to 11 % (standard deviation) instead of 3 to 5.
   if (tiled_ok && mt_cap >= 4 && nt_cap == 2 && force_mt == 0 && force_nt == 0 && env_wk == 0) {
     const int sb_total = gg.m[0].K >> 8;
@@ -1687,7 +1691,7 @@ template <int kA>
 __global__ __launch_bounds__(256) void proj_tile_kernel(const half_t* __restrict__ x, const half_t* __restrict__ R, half_t* __restrict__ r,
                                                         float* __restrict__ partials, int M, int K, int rank) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int kB = kA, kSt = 2;  // (three and four stages measured the same or slower; the second workgroup of a compute unit fills the waits)
+  constexpr int kB = kA, kSt = 2;  // (three and four stages: never in flight, the barrier's wait is for all loads to LDS; a second workgroup of a compute unit fills the waits)
   constexpr int BM = 64 * kA, BN = 64 * kB;
   constexpr int kStage = (BM + BN) * kTRow;
   constexpr int kLoads = (BM + BN) / 16;  // 16-byte loads of a thread per stage

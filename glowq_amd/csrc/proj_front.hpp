@@ -6,8 +6,9 @@
 // of this part of the chip, acknowledged before the tile's word goes up.
 // Long K is cut over `slices` workgroups of a tile: all but the first leave their fp32 sums in the workspace and raise words of their own,
 // and the first adds them in slice order (bounded: without them it walks all of K by itself).
-// What bounds such a workgroup is what one compute unit pulls, 128 kA K bytes with kStages - 1 stages in flight: it has most of the group
-// launch's time for it.  A launch of its own for r takes two dependent launches from some twenty rows on (tiles with K cut over
+// What bounds such a workgroup is a memory round trip a stage: the compiler waits for all loads to LDS in front of a barrier (the release of
+// __syncthreads covers LDS writes, which it takes them for), so a stage is in flight only while the one before it is multiplied,
+// however many the ring holds.  It has most of the group launch's time for it.  A launch of its own for r takes two dependent launches from some twenty rows on (tiles with K cut over
 // workgroups, their sum).
 // K % 128 == 0, rank % 8 == 0, 16-byte aligned x, R and r, x and R below 4 GiB.
 #pragma once
@@ -51,7 +52,8 @@ template <int kWaves, int kA>
 struct ProjFront {
   static_assert((kWaves == 4 || kWaves == 8) && (kA == 1 || kA == 2), "four or eight waves, tiles of 32 or 64");
   static constexpr int kRow = 256;  // bytes of a staged row
-  // (five stages of the small tiles: no faster, and 80 KB of LDS leave two workgroups on a compute unit where there were three)
+  // (five stages of the small tiles: 80 KB of LDS leave two workgroups on a compute unit where there were three, and with the wait above the further
+  // ones were never in flight: no faster)
   static constexpr int kStages = kA == 1 ? 3 : 2;
   static constexpr int kStageBytes = 64 * kA * kRow;
   static constexpr int kLds = kStages * kStageBytes;

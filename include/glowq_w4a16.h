@@ -123,7 +123,8 @@ int glowq_shared_proj(const void* x, const void* R, void* r, int M, int K, int r
  * small launch adds them in slice order (results do not depend on scheduling) and writes r.
  * `workspace`: 16-byte aligned device memory, contents irrelevant; glowq_proj_workspace_bytes gives the size that the
  * 32-row tiles split through -- a smaller one splits less, NULL or 0 bytes is glowq_shared_proj.  The tile kernel for many rows
- * takes up to 32 slices of 4 M rank bytes where a larger one holds them.
+ * takes up to 32 slices of 4 M rank bytes where a larger one holds them.  The size is the projection's alone: what the group calls below do with
+ * a workspace, and how much of it they want, stands with them.
  * Calls that share a workspace must not overlap (one workspace per stream).
  */
 int glowq_shared_proj_ws(const void* x, const void* R, void* r, int M, int K, int rank, void* workspace,
@@ -183,7 +184,7 @@ int glowq_w4a16_group_forward_fused(const void* x, const void* R, void* r_out, c
  * graph is a launch like any other).  One launch instead of two, the same bits in r_out and in the outputs as the
  * projection launch in front gives; "proj_in_launch" of glowq_set_tuning switches it off.  As everywhere, calls that
  * share a workspace must not overlap.
- * The GEMM on the tiled weights (from 65 token rows, and 33 to 64 in its unrounded form) does the same where that is predicted to pay: tiles of r in front of the
+ * The GEMM on the tiled weights (from 65 token rows, and 17 to 64 in its unrounded form) does the same where that is predicted to pay: tiles of r in front of the
  * grid, a word each; its readers want r behind their weights.  The first 2 101 248 bytes of the workspace hold the words
  * and fp32 sums of r, the partial tiles of a split of K lie behind them; with less the projection launch stays.  r and outputs agree
  * with the two-launch form to the rounding of fp32 sums; glowq_last_launch names the grid of the output tiles alone.
@@ -201,7 +202,8 @@ int glowq_w4a16_group_forward_fused(const void* x, const void* R, void* r_out, c
  * The kernel that streams the tiled copy does it at 5..16 token rows and ranks up to 256 where its grid is not cut into
  * slices of K and leaves compute units free (gate|up): producers in front as above, and the waves that stage the
  * activations of each workgroup look for the ready word when r is due in the stages, behind the last columns of K.  Same
- * 8192 bytes at the head of the workspace; the same bits in r_out and in the outputs as the two-launch form.
+ * 8192 bytes at the head of the workspace; the same bits in r_out as the two-launch form, outputs to the rounding of fp32 sums (the two may cut
+ * K differently).  The narrow tiles over the canonical buffers do it in the same way.
  */
 int glowq_w4a16_group_forward_ws(const void* x, const void* r, const glowq_member_t* members, int n_members, int M,
                                  int K, int group_size, int rank, float alpha, void* workspace, size_t workspace_bytes,
@@ -213,7 +215,7 @@ int glowq_w4a16_group_forward_fused_ws(const void* x, const void* R, void* r_out
 /*
  * Tiled copy of a member's weights for the matrix-core routes (5..64 token rows, from 2 on groups of 80 MB of codes and more): the codes of 32 output rows and 256
  * input columns at a time in the order in which one coalesced 16-byte-per-lane load hands every lane the B operand of
- * the 32x32x16 matrix instruction, with each lane's scale and -(1024 + zero-point) behind them (4352 bytes per
+ * the 32x32x16 matrix instruction, with each column's scale and -zero-point * 2^-16 behind them (4352 bytes per
  * (row block, super-block); layout in glowq_amd/csrc/tiled.hpp).  A deterministic function of the canonical buffers,
  * which stay the state-dict form and what every other route reads; the reference has no counterpart (its large-M
  * route writes a dequantised fp16 copy of the whole weight on every call, src/cuda_w4a16/csrc/gemm_w4a16.cu:106-129).
